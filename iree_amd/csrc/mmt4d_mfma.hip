@@ -17,9 +17,53 @@ struct Plan {
   int kind;
   bool rhs_i4;
   bool narrow;  // 16-bit output, rounded once at the end
-  int gather;   // 16 or 4
+  int gather;   // bytes of a row piece, 16 for 16 and more
+  int wave_shape;  // tile of the kernel that splits K over wavefronts, or -1: a block kernel
   MfmaArgs args;
 };
+
+// Estimates in microseconds, fitted to a sweep of M 16..1024 x N 256..16384 x K 256..8192 for every type and row piece
+// (weights that the last-level cache holds, one launch after another): the kernel that they pick is within 2 % of the
+// faster one in the mean, and 14 % at worst.
+//
+// A block kernel takes a fixed time per 64-byte chunk of K, whatever the number of tiles up to one per compute unit.
+double block_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
+  const bool direct = mfma_direct_covers(m, gather, rhs_i4);
+  if (gather == 16 && (kind == kF16 || kind == kBF16) && direct && split_k_covers(m)) return 4.5 + 0.235 * m.chunks;
+  const TileChoice* t;
+  choose_tile(m, rhs_i4, direct, &t);
+  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
+  const int64_t tiles = ((rows + 64 * t->am - 1) / (64 * t->am)) * ((cols + 64 * t->bn - 1) / (64 * t->bn));
+  double per_chunk = t->us_per_chunk;
+  if (kind == kF32) per_chunk *= 2.3;                                   // bound by the matrix pipe
+  if (gather == 2) per_chunk *= t->am * t->bn == 1 ? 2.0 : 1.45;        // 2-byte pieces: more LDS reads per step
+  if (!direct) per_chunk *= 2.2;                                        // staged through registers
+  return 3.3 + (double)((tiles + 255) / 256) * m.chunks * per_chunk;
+}
+
+// The kernel that splits K over wavefronts is bound by the bytes a workgroup loads; workgroups beyond one per compute
+// unit run beside each other where their registers and LDS allow it (not those of the 64x64 tile).
+double wave_k_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather, const WaveKShape& s) {
+  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
+  const int64_t tiles = ((rows + 16 * s.fa - 1) / (16 * s.fa)) * ((cols + 16 * s.fb - 1) / (16 * s.fb));
+  const double row_kb = 1e-3 * m.K * m.lhs_rb, rhs_share = rhs_i4 ? 0.5 : 1.0;
+  double tile_us = 16 * (s.fa + s.fb * rhs_share) * row_kb / (gather < 16 ? 75 : 110);
+  if (kind == kF32) tile_us = tile_us > 0.0234 * s.fa * s.fb * m.chunks ? tile_us : 0.0234 * s.fa * s.fb * m.chunks;
+  double us = 2.9 + 0.07 * s.fa * s.fb + 5e-5 * (rows + cols * rhs_share) * row_kb;
+  if (tiles <= 256) return us + tile_us;
+  const double rounds = tiles / 256.0;
+  if (tiles > (s.fa * s.fb >= 16 ? 256 : 1024)) us += 1e3 * rounds;
+  return us + (rounds + 0.8) * tile_us + 0.8 * rounds;
+}
+
+// Whether the kernel that splits K over wavefronts covers the problem: 16-byte aligned operands whose 16 contiguous
+// bytes belong to one k step.
+bool wave_k_covers(const MfmaArgs& m, int gather, bool rhs_i4) {
+  if (gather == 1 || (rhs_i4 && m.rhs_rb < 16)) return false;
+  if (gather < 16 && ((gather << m.log2_M0) < 16 || (gather << m.log2_N0) < 16)) return false;
+  return (uintptr_t)m.lhs % 16 == 0 && (uintptr_t)m.rhs % 16 == 0 && (m.M == 1 || m.lhs_stride_bytes % 16 == 0) &&
+         (m.N == 1 || m.rhs_stride_bytes % 16 == 0);
+}
 
 // Fills `plan` if the problem is covered. With `probe_only` only type and tile
 // shape are looked at.
@@ -77,13 +121,8 @@ bool make_plan(const Mmt4dArgs& a, bool probe_only, Plan* plan) {
   plan->gather = gather;
   if (probe_only) return true;
 
-  // Alignment of every vector access the kernel makes.
-  const int lhs_align = gather == 4 ? 4 : 16;  // (also for 1-, 2- and 8-byte pieces: 16 bytes per lane)
-  const int rhs_align = i4 ? 8 : lhs_align;
   const int64_t lhs_stride_bytes = a.lhs_stride0 * elem_bytes;
   const int64_t rhs_stride_bytes = i4 ? a.rhs_stride0 / 2 : a.rhs_stride0 * elem_bytes;
-  if (((uintptr_t)a.lhs % lhs_align) || (a.M > 1 && lhs_stride_bytes % lhs_align)) return false;
-  if (((uintptr_t)a.rhs % rhs_align) || (a.N > 1 && rhs_stride_bytes % rhs_align)) return false;
   // (four consecutive outputs per store: 16 bytes, 8 with a 16-bit output)
   if (((uintptr_t)a.out % (narrow ? 8 : 16)) || (a.M > 1 && a.out_stride0 % 4)) return false;
   // Per-piece offsets from a workgroup's first tile are kept in 32 bits.
@@ -106,13 +145,69 @@ bool make_plan(const Mmt4dArgs& a, bool probe_only, Plan* plan) {
   m.log2_lhs_rb = llrb; m.log2_rhs_rb = lrrb;
   m.chunks = (int32_t)(((int64_t)a.K * lhs_rb + 63) / 64);
   m.accumulate = (a.flags & IREE_UK_FLAG_MMT4D_ACCUMULATE) ? 1 : 0;
+
+  // Alignment of every vector access the block kernels make.
+  const int lhs_align = gather == 4 ? 4 : 16;  // (also for 1-, 2- and 8-byte pieces: 16 bytes per lane)
+  const int rhs_align = i4 ? 8 : lhs_align;
+  if (((uintptr_t)a.lhs % lhs_align) || (a.M > 1 && lhs_stride_bytes % lhs_align)) return false;
+  if (((uintptr_t)a.rhs % rhs_align) || (a.N > 1 && rhs_stride_bytes % rhs_align)) return false;
   if ((gather == 1 || gather == 2 || gather == 8) && !mfma_direct_covers(m, gather, i4)) return false;
+  plan->wave_shape = -1;
+  if (!wave_k_covers(m, gather, i4)) return true;
+  double best = block_cost(m, kind, i4, gather);
+  for (int s = 0; s < (int)(sizeof kWaveKShapes / sizeof kWaveKShapes[0]); ++s) {
+    const double cost = wave_k_cost(m, kind, i4, gather, kWaveKShapes[s]);
+    if (cost < best) {
+      best = cost;
+      plan->wave_shape = s;
+    }
+  }
   return true;
+}
+
+// What iree_uk_mi355x_last_kernel reports for a problem that is worked off by the kernel that splits K over wavefronts:
+// names go by the problem's class (the block tile that its size calls for, or few of them against a long K), not by the
+// tile of that kernel, so that a caller that watches the names is not told of a different class after every retuning.
+const char* class_name(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
+  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
+  const int64_t row_bytes = (int64_t)m.K * m.lhs_rb;
+  const bool direct = mfma_direct_covers(m, gather, rhs_i4);
+  if (direct && gather == 16 && !rhs_i4 && kind != kF32) {
+    if (((rows + 63) / 64) * ((cols + 63) / 64) <= 128 && row_bytes % 256 == 0 && row_bytes >= 4096)
+      return "mmt4d_mfma_64x64_split_k";
+    if (kind != kI8 && split_k_covers(m)) return "mmt4d_mfma_128x64_split_k";
+  }
+  static const char* const kNames[] = {"mmt4d_mfma_256x256", "mmt4d_mfma_256x128", "mmt4d_mfma_128x128",
+                                       "mmt4d_mfma_128x64",  "mmt4d_mfma_64x64",   "mmt4d_mfma_64x128"};
+  const TileChoice* tile;
+  return kNames[choose_tile(m, rhs_i4, direct, &tile)];
+}
+
+hipError_t launch_wave_k(const Plan& plan, hipStream_t stream, const char** name) {
+  const MfmaArgs& m = plan.args;
+  const WaveKShape& shape = kWaveKShapes[plan.wave_shape];
+  *name = class_name(m, plan.kind, plan.rhs_i4, plan.gather);
+  // Weights that one row of tiles reads once and the last-level cache (256 MiB, shared with whatever else the program
+  // keeps) is not likely to hold from one call to the next are streamed past the caches: bf16 64 x 14336 x 4096 (117
+  // MB) 27.9 -> 24.8 us. Smaller ones must not be: 64 x 4096 x 4096 (34 MB) 9.0 -> 12.1 us.
+  const bool streamed = ((int64_t)m.M << m.log2_M0) <= 16 * shape.fa &&
+                        (((int64_t)m.N * m.K * m.rhs_rb) << m.log2_N0) > (64ll << 20);
+  switch (plan.kind) {
+    case kI8: return launch_wave_k_i8(m, plan.gather, plan.rhs_i4, plan.wave_shape, streamed, stream);
+    case kF16:
+      return plan.narrow ? launch_wave_k_f16_narrow(m, plan.gather, plan.wave_shape, streamed, stream)
+                         : launch_wave_k_f16(m, plan.gather, plan.wave_shape, streamed, stream);
+    case kBF16:
+      return plan.narrow ? launch_wave_k_bf16_narrow(m, plan.gather, plan.wave_shape, streamed, stream)
+                         : launch_wave_k_bf16(m, plan.gather, plan.wave_shape, streamed, stream);
+    default: return launch_wave_k_f32(m, plan.gather, plan.wave_shape, streamed, stream);
+  }
 }
 
 hipError_t launch_mfma(const Mmt4dArgs& a, hipStream_t stream, const char** name) {
   Plan plan;
   if (!make_plan(a, false, &plan)) return hipErrorInvalidValue;
+  if (plan.wave_shape >= 0) return launch_wave_k(plan, stream, name);
   const MfmaArgs& m = plan.args;
   switch (plan.kind) {
     case kI8: return launch_mfma_i8(m, plan.gather, plan.rhs_i4, stream, name);

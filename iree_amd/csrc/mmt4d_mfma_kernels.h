@@ -81,6 +81,72 @@ hipError_t launch_mfma_bf16_narrow(const MfmaArgs& m, int gather, hipStream_t st
 // `gather` bytes (2 and 8 have no other MFMA kernel).
 bool mfma_direct_covers(const MfmaArgs& m, int gather, bool rhs_i4);
 
+// The kernel that splits K over a workgroup's wavefronts (mmt4d_wave_k_kernels.h): its tiles, smallest first, and its
+// entry per translation unit. `shape` numbers the tiles; `streamed`: read the rhs with non-temporal loads.
+struct WaveKShape {
+  int fa, fb;  // 16-row fragments of the lhs and of the rhs
+};
+constexpr WaveKShape kWaveKShapes[] = {{1, 1}, {1, 2}, {2, 2}, {2, 4}, {4, 2}, {4, 4}};
+hipError_t launch_wave_k_i8(const MfmaArgs& m, int gather, bool rhs_i4, int shape, bool streamed, hipStream_t stream);
+hipError_t launch_wave_k_f16(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);
+hipError_t launch_wave_k_bf16(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);
+hipError_t launch_wave_k_f32(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);
+hipError_t launch_wave_k_f16_narrow(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);
+hipError_t launch_wave_k_bf16_narrow(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);
+
+// The block tiles of the block kernels, and which of them a problem takes. The estimate is
+//   (workgroups per compute unit, rounded up) x (tile area) / (tile efficiency),
+// with the efficiencies measured at saturation on bf16 16x16x8 operands
+// (TFLOP/s at 2048 x 14336 x 4096: 256x256 1003, 256x128 905, 128x128 851,
+// 128x64 607, 64x64 529). It reproduces the measured best tile on every shape
+// tried (128 .. 4096 rows against 14336 columns, 1024^2 .. 4096^2 squares).
+// Larger tiles move fewer operand bytes per multiply through L2 -> LDS and run
+// the matrix pipe longer between barriers, smaller ones spread a problem over
+// more compute units.
+struct TileChoice {
+  int am, bn;
+  float efficiency;
+  bool direct_only;   // no register-staged instantiation of this shape
+  float us_per_chunk; // one workgroup per compute unit, 64 bytes of K per row (bf16 and int8, direct-to-LDS kernel)
+};
+
+// The 128x64 tile with K split over its wavefronts (mmt4d_mfma_split_k_kernel): 65 to 128 lhs rows, one row of tiles.
+// (bf16 128 x 14336 x 4096 27 -> 25 us, 96 rows 27 -> 23 us, 128 x 8192 x 8192 40 -> 36 us. Not with less K per
+// row, where the prologue and the summing of the partial tiles cost what the steps gain; not with more tiles than
+// compute units, where 128x128 tiles win: bf16 128 x 28672 x 4096 41 -> 49 us.)
+inline bool split_k_covers(const MfmaArgs& m) {
+  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
+  const int64_t row_bytes = (int64_t)m.K * m.lhs_rb;
+  return rows > 64 && rows <= 128 && cols <= 256 * 64 && row_bytes % 128 == 0 && row_bytes >= 8192;
+}
+
+inline int choose_tile(const MfmaArgs& m, bool rhs_i4, bool direct, const TileChoice** chosen) {
+  static const TileChoice kTiles[] = {
+      {4, 4, 1003.f, false, 0.52f}, {4, 2, 905.f, true, 0.34f}, {2, 2, 851.f, false, 0.40f},
+      {2, 1, 607.f, true, 0.23f}, {1, 1, 529.f, false, 0.135f}, {1, 2, 600.f, true, 0.22f}};
+  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
+  int best = -1;
+  double best_cost = 0;
+  for (int i = 0; i < (int)(sizeof kTiles / sizeof kTiles[0]); ++i) {
+    const TileChoice& t = kTiles[i];
+    if (t.direct_only && !direct) continue;
+    if (rhs_i4 && t.bn < 2 && t.direct_only) continue;  // the int4 direct path needs a rhs fragment per wavefront
+    if (!rhs_i4 && t.am == 1 && t.bn == 2) continue;    // 64x128 exists for the int4 rhs only (in place of 128x64)
+    // The int4 64x64 tile exists only register-staged, at less than half the
+    // rate of the direct 64x128 one on the same problem.
+    if (rhs_i4 && direct && t.am == 1 && t.bn == 1) continue;
+    const int64_t br = 64 * t.am, bc = 64 * t.bn;
+    const int64_t workgroups = ((rows + br - 1) / br) * ((cols + bc - 1) / bc);
+    const double cost = (double)((workgroups + 255) / 256) * (double)(br * bc) / t.efficiency;
+    if (best < 0 || cost < best_cost) {
+      best = i;
+      best_cost = cost;
+    }
+  }
+  *chosen = &kTiles[best];
+  return best;
+}
+
 #ifdef UK_MFMA_KERNEL_BODIES
 namespace {
 
@@ -1504,38 +1570,32 @@ __device__ __forceinline__ void set_from_bits(int32_t& v, uint32_t bits) { v = (
 __device__ __forceinline__ void set_from_bits(float& v, uint32_t bits) { v = __uint_as_float(bits); }
 
 // ---------------------------------------------------------------------------
-// Block tiles whose four wavefronts split K instead of the tile, for problems
-// with few block tiles: few rhs rows against a long K (say 128 x 4096 x 14336,
-// 128 tiles of 64x64), or at most 128 lhs rows (one tile row of 128x64). There
-// the kernel above is bound by the latency of one pipeline step (counter wait,
-// barrier, LDS reads; about 140 ns) per 64 bytes of K per workgroup, and with
-// few tiles half the compute units have no workgroup at all. Here every
-// wavefront multiplies the whole tile ((32*AMF) x 64, AMF x 2 fragments) over
-// its quarter of the step's K bytes, so a workgroup streams more per step, and
-// the four partial tiles are summed through LDS at the end, in wavefront order
-// (deterministic). Row pieces of 16 bytes or more, int8 / f16 / bf16.
-//   AMF == 2: 64x64 tile, 256 bytes of K per row and step (two MFMA K-steps per
-//     wavefront), ring of 4 stages of 32 KiB. 128 x 4096 x 14336 bf16 62 -> 41 us.
-//   AMF == 4: 128x64 tile, 128 bytes of K per row and step (one K-step per
-//     wavefront), ring of 6 stages of 24 KiB.
-// What bounds them is what a compute unit's load path moves (64 bytes per
-// cycle at best; a stage takes about 500 resp. 400 cycles).
+// A 128x64 block tile whose four wavefronts split K instead of the tile, for 65 to
+// 128 lhs rows against a long K (one tile row). The kernel above is then bound by
+// the latency of one pipeline step (counter wait, barrier, LDS reads; about 140
+// ns) per 64 bytes of K per workgroup. Here every wavefront multiplies the whole
+// tile (4 x 2 fragments) over its quarter of the step's K bytes (one MFMA K-step
+// of the 128 bytes per row and step; ring of 6 stages of 24 KiB), so a workgroup
+// streams more per step, and the four partial tiles are summed through LDS at the
+// end, in wavefront order (deterministic). Row pieces of 16 bytes or more, f16 /
+// bf16. What bounds it is what a compute unit's load path moves (a stage takes
+// about 400 cycles). Problems with fewer tiles go to mmt4d_wave_k_kernels.h.
 //
 // LDS stage: per operand four slices (one per wavefront's share of K, 16*COLS
 // bytes per row, COLS = 2 * K-steps per wavefront) of fragments in the layout
 // of the kernel above (G == 16) with COLS 16-byte columns: slot p of a
 // fragment holds rows 16*(p / (16*COLS)) + (p & 15), column (p >> 4) & (COLS-1).
 // A load fills 64 consecutive slots of one slice.
-template <int KIND, bool NARROW, int AMF>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, AMF == 2 ? 2 : 1)))
+template <int KIND, bool NARROW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void mmt4d_mfma_split_k_kernel(const MfmaArgs a) {
   typedef typename AccType<KIND>::type acc_t;
-  static_assert(KIND != kF32, "one MFMA per fragment pair");
-  static_assert(AMF == 2 || AMF == 4, "64 or 128 lhs rows");
-  constexpr int KKW = AMF == 2 ? 2 : 1;       // MFMA K-steps per wavefront and step
+  static_assert(KIND == kF16 || KIND == kBF16, "16-bit floats");
+  constexpr int AMF = 4;                      // 32-row lhs fragments
+  constexpr int KKW = 1;                      // MFMA K-steps per wavefront and step
   constexpr int COLS = 2 * KKW;               // 16-byte columns of a slice
   constexpr int CHUNK_BYTES = 4 * 16 * COLS;  // of K per row and step
-  constexpr int STAGES = AMF == 2 ? 4 : 6, AHEAD = STAGES - 1;  // (a fifth stage of the 64x64 tile changed nothing)
+  constexpr int STAGES = 6, AHEAD = STAGES - 1;
   constexpr int FRAG_SLOTS = 32 * COLS;
   constexpr int A_SLICE = AMF * FRAG_SLOTS, B_SLICE = 2 * FRAG_SLOTS;  // slots per slice
   constexpr int A_PIECES = 4 * A_SLICE, B_PIECES = 4 * B_SLICE;
@@ -1786,26 +1846,12 @@ hipError_t launch_direct(MfmaArgs m, hipStream_t stream, bool staggered_tail = t
   return hipGetLastError();
 }
 
-// The tiles with K split over the wavefronts. Returns the number of 32-row lhs fragments of the tile to use (2:
-// few 64x64 tiles and a long K; 4: at most 128 lhs rows, one row of 128x64 tiles), or 0 for the ordinary kernels.
-inline int split_k_tile(const MfmaArgs& m, bool int8) {
-  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
-  const int64_t row_bytes = (int64_t)m.K * m.lhs_rb;
-  if (((rows + 63) / 64) * ((cols + 63) / 64) <= 128 && row_bytes % 256 == 0 && row_bytes >= 4096) return 2;
-  // (bf16 128 x 14336 x 4096 27 -> 25 us, 96 rows 27 -> 23 us, 128 x 8192 x 8192 40 -> 36 us. Not with less K per
-  // row, where the prologue and the summing of the partial tiles cost what the steps gain; not for int8, which does
-  // twice the MFMA work per byte: 128 x 14336 x 8192 29 -> 31 us; not with more tiles than compute units, where
-  // 128x128 tiles win: bf16 128 x 28672 x 4096 41 -> 49 us.)
-  if (!int8 && rows > 64 && rows <= 128 && cols <= 256 * 64 && row_bytes % 128 == 0 && row_bytes >= 8192) return 4;
-  return 0;
-}
-
-template <int KIND, bool NARROW, int AMF>
+template <int KIND, bool NARROW>
 hipError_t launch_split_k(MfmaArgs m, hipStream_t stream) {
   unsigned grid;
-  set_tile_grid(&m, 32 * AMF, 64, &grid);
-  constexpr int lds_bytes = AMF == 2 ? 4 * 32768 : 6 * 24576;
-  auto kernel = mmt4d_mfma_split_k_kernel<KIND, NARROW, AMF>;
+  set_tile_grid(&m, 128, 64, &grid);
+  constexpr int lds_bytes = 6 * 24576;
+  auto kernel = mmt4d_mfma_split_k_kernel<KIND, NARROW>;
   const hipError_t attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
   if (attr != hipSuccess) return attr;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds_bytes, stream, m);
@@ -1834,64 +1880,17 @@ hipError_t launch_staged(MfmaArgs m, hipStream_t stream) {
   }
 }
 
-// Picks the block tile. Larger tiles move fewer operand bytes per multiply
-// through L2 -> LDS and run the matrix pipe longer between barriers, smaller
-// ones spread a problem over more compute units. The estimate is
-//   (workgroups per compute unit, rounded up) x (tile area) / (tile efficiency),
-// with the efficiencies measured at saturation on bf16 16x16x8 operands
-// (TFLOP/s at 2048 x 14336 x 4096: 256x256 1003, 256x128 905, 128x128 851,
-// 128x64 607, 64x64 529). It reproduces the measured best tile on every shape
-// tried (128 .. 4096 rows against 14336 columns, 1024^2 .. 4096^2 squares).
-struct TileChoice {
-  int am, bn;
-  float efficiency;
-  bool direct_only;  // no register-staged instantiation of this shape
-};
-
-template <bool RHS_I4>
-int choose_tile(const MfmaArgs& m, bool direct, const TileChoice** chosen) {
-  static const TileChoice kTiles[] = {
-      {4, 4, 1003.f, false}, {4, 2, 905.f, true}, {2, 2, 851.f, false}, {2, 1, 607.f, true}, {1, 1, 529.f, false},
-      {1, 2, 600.f, true}};
-  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
-  int best = -1;
-  double best_cost = 0;
-  for (int i = 0; i < (int)(sizeof kTiles / sizeof kTiles[0]); ++i) {
-    const TileChoice& t = kTiles[i];
-    if (t.direct_only && !direct) continue;
-    if (RHS_I4 && t.bn < 2 && t.direct_only) continue;  // the int4 direct path needs a rhs fragment per wavefront
-    if (!RHS_I4 && t.am == 1 && t.bn == 2) continue;    // 64x128 exists for the int4 rhs only (in place of 128x64)
-    // The int4 64x64 tile exists only register-staged, at less than half the
-    // rate of the direct 64x128 one on the same problem.
-    if (RHS_I4 && direct && t.am == 1 && t.bn == 1) continue;
-    const int64_t br = 64 * t.am, bc = 64 * t.bn;
-    const int64_t workgroups = ((rows + br - 1) / br) * ((cols + bc - 1) / bc);
-    const double cost = (double)((workgroups + 255) / 256) * (double)(br * bc) / t.efficiency;
-    if (best < 0 || cost < best_cost) {
-      best = i;
-      best_cost = cost;
-    }
-  }
-  *chosen = &kTiles[best];
-  return best;
-}
-
 template <int KIND, bool RHS_I4, int G, bool NARROW>
 hipError_t launch_variant(const MfmaArgs& m, hipStream_t stream, const char** name) {
   const bool direct = direct_covers<RHS_I4, G>(m);
-  if constexpr (G == 16 && !RHS_I4 && KIND != kF32) {
-    const int split = direct ? split_k_tile(m, KIND == kI8) : 0;
-    if (split == 2) {
-      *name = "mmt4d_mfma_64x64_split_k";
-      return launch_split_k<KIND, NARROW, 2>(m, stream);
-    }
-    if (split == 4) {
+  if constexpr (G == 16 && (KIND == kF16 || KIND == kBF16)) {
+    if (direct && split_k_covers(m)) {
       *name = "mmt4d_mfma_128x64_split_k";
-      return launch_split_k<KIND, NARROW, 4>(m, stream);
+      return launch_split_k<KIND, NARROW>(m, stream);
     }
   }
   const TileChoice* tile;
-  switch (choose_tile<RHS_I4>(m, direct, &tile)) {
+  switch (choose_tile(m, RHS_I4, direct, &tile)) {
     case 0:
       *name = "mmt4d_mfma_256x256";
 #ifndef UK_STAGES_256

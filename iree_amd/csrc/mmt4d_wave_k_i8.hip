@@ -1,0 +1,17 @@
+// Kernel instantiations of the wave-split mmt4d for one operand type (see
+// mmt4d_wave_k_kernels.h).
+#include "mmt4d_wave_k_kernels.h"
+
+namespace uk {
+
+hipError_t launch_wave_k_i8(const MfmaArgs& m, int gather, bool rhs_i4, int shape, bool streamed, hipStream_t stream) {
+  if (rhs_i4) return launch_wave_k_piece<kI8, true, false, 16>(m, shape, streamed, stream);
+  switch (gather) {
+    case 16: return launch_wave_k_piece<kI8, false, false, 16>(m, shape, streamed, stream);
+    case 8: return launch_wave_k_piece<kI8, false, false, 8>(m, shape, streamed, stream);
+    case 4: return launch_wave_k_piece<kI8, false, false, 4>(m, shape, streamed, stream);
+    default: return launch_wave_k_piece<kI8, false, false, 2>(m, shape, streamed, stream);
+  }
+}
+
+}  // namespace uk

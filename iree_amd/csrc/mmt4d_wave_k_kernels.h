@@ -1,0 +1,372 @@
+// MFMA mmt4d for problems with few output tiles (batched decode, small layers,
+// few rows against a long K): K is split over the wavefronts of a workgroup.
+//
+// The block kernels (mmt4d_mfma_kernels.h) walk K one 64-byte chunk per
+// workgroup barrier, about 150 ns a chunk whatever the tile, and a problem with
+// fewer tiles than compute units has nothing to hide that behind. Here a
+// workgroup of 8 wavefronts owns a (16*FA) x (16*FB) tile and every wavefront
+// multiplies the WHOLE tile over its own contiguous share of K: operands go from
+// global memory straight to the MFMA's registers, a batch of UNROLL 64-byte
+// steps in flight while the previous batch is multiplied, with no LDS and no
+// barrier until the partial tiles are summed through LDS at the end, in
+// wavefront order (results do not depend on scheduling). A workgroup thus has
+// 128 to 256 KiB of loads in flight and is bound by what a compute unit's load
+// path moves, 64 bytes per cycle, i.e. by (16*FA + 16*FB) * 64 bytes per step.
+//
+// Operand registers. Fragments are 16 rows x 64 bytes of K
+// (v_mfma_i32_16x16x64_i8, v_mfma_f32_16x16x32_{f16,bf16}, four
+// v_mfma_f32_16x16x4_f32): lane 16*q + r holds 16 bytes of row r. Which k those
+// are is free as long as lhs and rhs agree. A load is 16 contiguous bytes per
+// lane and covers one fragment's step, 1 KiB. G = bytes of a row piece:
+//   16 (or more): lane 16*q + r loads 16-byte column q of row r: the operand.
+//   8, 4, 2: 16 contiguous bytes are 16 / G rows of one k step. They pass through
+//     1 KiB of LDS that only this wavefront uses (no barrier), as [k][16 rows][G
+//     bytes], and come back as the pieces of k steps 4*d + q of row r (8, 4: reads
+//     linear in the lane number) resp. 16*d + 4*q + {0..3} (2: the transposing
+//     read ds_read_b64_tr_b16). Loaded piece by piece instead, without LDS, an
+//     instruction covers short stretches of several tiles, and where these lie a
+//     multiple of 64 KiB apart (int8 8x8x4 at K = 8192) everything took 5 times as long.
+//   int4 rhs (K0 = 32 or 64): a step is 128 values of K; a lane's 16 bytes are 32
+//     nibbles, widened to two int8 operands of 16x the values, against two
+//     16-byte pieces of the lhs; the sums are shifted right by 4 at the end.
+// K may end inside a step: the last steps are loaded with a check per piece, and
+// what lies beyond K is zero in both operands.
+#ifndef IREE_AMD_CSRC_MMT4D_WAVE_K_KERNELS_H_
+#define IREE_AMD_CSRC_MMT4D_WAVE_K_KERNELS_H_
+
+#include <type_traits>
+
+#define UK_MFMA_KERNEL_BODIES
+#include "mmt4d_mfma_kernels.h"
+
+namespace uk {
+namespace {
+
+typedef float v4f32 __attribute__((ext_vector_type(4)));
+
+template <int KIND> struct Acc16 { typedef v4f32 type; };
+template <> struct Acc16<kI8> { typedef v4i32 type; };
+
+// Product of two 16-row x 64-byte fragments.
+template <int KIND>
+__device__ __forceinline__ typename Acc16<KIND>::type mfma16(uint4 row_operand, uint4 col_operand,
+                                                             typename Acc16<KIND>::type acc) {
+  if constexpr (KIND == kI8) {
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i32, row_operand),
+                                                 __builtin_bit_cast(v4i32, col_operand), acc, 0, 0, 0);
+  } else if constexpr (KIND == kF16) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8f16, row_operand),
+                                                  __builtin_bit_cast(v8f16, col_operand), acc, 0, 0, 0);
+  } else if constexpr (KIND == kBF16) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf16, row_operand),
+                                                   __builtin_bit_cast(v8bf16, col_operand), acc, 0, 0, 0);
+  } else {
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(row_operand.x), __uint_as_float(col_operand.x), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(row_operand.y), __uint_as_float(col_operand.y), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(row_operand.z), __uint_as_float(col_operand.z), acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(row_operand.w), __uint_as_float(col_operand.w), acc, 0, 0, 0);
+  }
+}
+
+// 8 bytes per lane from LDS, transposed within each group of 16 lanes (ds_read_b64_tr_b16): the lanes' 8-byte chunks
+// are taken as 4 rows of 32 bytes (chunks 4j .. 4j + 3 make row j), and lane i of the group receives the i-th 16-bit
+// element of every row.
+__device__ __forceinline__ uint2 lds_read_transposed_b16(const uint8_t* p) {
+  typedef short v4i16 __attribute__((ext_vector_type(4)));
+  const v4i16 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)(p));
+  return __builtin_bit_cast(uint2, v);
+}
+
+// One operand of a workgroup's tile: F fragments, pieces of G bytes. WIDE: the int8 operand that meets an int4 one,
+// two 16-byte pieces per fragment and step.
+template <int G, int F, bool WIDE>
+struct Operand {
+  static constexpr int RAW = WIDE ? 2 * F : F;  // 16-byte registers that hold what one step loads
+  const uint8_t* base;   // uniform: the tile's first row of tiles, k = 0
+  uint32_t off[F];       // per lane, from base, at step 0
+  uint32_t step_bytes;   // from one step to the next
+  int32_t k_lane;        // k step (within a step) of what this lane loads
+  uint32_t lds_slot;     // G < 16: where in a fragment's 1 KiB the lane's 16 bytes go
+
+  // What step `s` holds. CHECKED: pieces from k step `K` on read as zero (`k0` = the step's first k step).
+  // STREAMED: the caller reads every byte once (non-temporal loads).
+  template <bool CHECKED, bool STREAMED>
+  __device__ __forceinline__ void load(int32_t s, int32_t k0, int32_t K, uint4 (&raw)[RAW]) const {
+    const uint8_t* p = base + (uint64_t)(uint32_t)s * step_bytes;
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+#pragma unroll
+      for (int w = 0; w < RAW / F; ++w) {
+        uint4& to = raw[(RAW / F) * f + w];
+        if (CHECKED) to = make_uint4(0, 0, 0, 0);
+        if (!CHECKED || k0 + k_lane < K) {
+          const v4i32* from = (const v4i32*)(p + off[f] + 16 * w);
+          if constexpr (STREAMED) to = __builtin_bit_cast(uint4, __builtin_nontemporal_load(from));
+          else to = __builtin_bit_cast(uint4, *from);
+        }
+      }
+    }
+  }
+
+  // G < 16: the loaded 16 bytes of every fragment into the wavefront's LDS, and fragment f back out of it.
+  __device__ __forceinline__ void to_lds(const uint4 (&raw)[RAW], uint8_t* lds) const {
+#pragma unroll
+    for (int f = 0; f < F; ++f) *(uint4*)(lds + 1024 * f + lds_slot) = raw[f];
+  }
+  __device__ __forceinline__ uint4 from_lds(const uint8_t* lds, int f, int lane) const {
+    const uint8_t* p = lds + 1024 * f;
+    if constexpr (G == 8) {
+      const uint2 lo = *(const uint2*)(p + 8 * lane), hi = *(const uint2*)(p + 512 + 8 * lane);
+      return make_uint4(lo.x, lo.y, hi.x, hi.y);
+    } else if constexpr (G == 4) {
+      return make_uint4(*(const uint32_t*)(p + 4 * lane), *(const uint32_t*)(p + 256 + 4 * lane),
+                        *(const uint32_t*)(p + 512 + 4 * lane), *(const uint32_t*)(p + 768 + 4 * lane));
+    } else {
+      const uint2 lo = lds_read_transposed_b16(p + 8 * lane), hi = lds_read_transposed_b16(p + 512 + 8 * lane);
+      return make_uint4(lo.x, lo.y, hi.x, hi.y);
+    }
+  }
+};
+
+template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int UNROLL, bool STREAMED>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, FA * FB >= 16 ? 2 : 4)))
+void mmt4d_wave_k_kernel(const MfmaArgs a) {
+  typedef typename Acc16<KIND>::type acc_t;
+  typedef Operand<G, FA, RHS_I4> lhs_t;
+  typedef Operand<G, FB, false> rhs_t;
+  constexpr bool STAGED = G < 16;  // operands pass through LDS
+  static_assert(!RHS_I4 || (KIND == kI8 && G == 16), "int4 rhs");
+  // The wavefronts' staging of narrow row pieces, [WAVES][UNROLL][FA + FB][1 KiB]; then [WAVES][FA * FB][64] partial sums.
+  extern __shared__ uint4 ring[];
+
+  int tile_row, tile_col;
+  if (!locate_block(a, &tile_row, &tile_col)) return;
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t total_rows = (int64_t)a.M << a.log2_M0, total_cols = (int64_t)a.N << a.log2_N0;
+  const int64_t first_row = (int64_t)tile_row * (16 * FA), first_col = (int64_t)tile_col * (16 * FB);
+
+  // Tiles past the end of the matrix are redirected to its last one: computed, never stored.
+  auto set_up = [&](auto& op, const uint8_t* base, int64_t first, int32_t tiles, int log2_t0, int64_t stride, int32_t rb,
+                    int log2_rb, int32_t lane_bytes) {
+    const int64_t kstep = (int64_t)rb << log2_t0;
+    const int32_t first_tile = (int32_t)(first >> log2_t0);
+    op.base = uniform_pointer(base + first_tile * stride);
+    op.step_bytes = (uint32_t)(4 * lane_bytes) << log2_t0;
+    int32_t row;  // of the fragment
+    int64_t lane_off;
+    if constexpr (G == 16) {
+      row = r;
+      op.k_lane = (lane_bytes * q) >> log2_rb;
+      lane_off = op.k_lane * kstep + ((lane_bytes * q) & (rb - 1));
+      op.lds_slot = 0;
+    } else {
+      // Lanes go along a tile's step (64 bytes per row, contiguous), then to the fragment's next tile.
+      const int32_t in_tile = lane & ((4 << log2_t0) - 1);
+      const int32_t log2_lanes_per_kstep = log2_t0 + log2_rb - 4;  // (16 bytes of one k step at least: the host's check)
+      const int32_t group = in_tile & ((1 << log2_lanes_per_kstep) - 1);
+      op.k_lane = in_tile >> log2_lanes_per_kstep;
+      row = ((lane >> (2 + log2_t0)) << log2_t0) + group * (16 / G);
+      lane_off = op.k_lane * kstep;
+      op.lds_slot = (uint32_t)(op.k_lane * 16 + row) * G;
+    }
+#pragma unroll
+    for (int f = 0; f < (int)(sizeof op.off / sizeof op.off[0]); ++f) {
+      const int32_t tile = min(first_tile + ((16 * f + row) >> log2_t0), tiles - 1) - first_tile;
+      op.off[f] = (uint32_t)(tile * stride + (row & ((1 << log2_t0) - 1)) * rb + lane_off);
+    }
+  };
+  lhs_t lhs;
+  rhs_t rhs;
+  set_up(lhs, a.lhs, first_row, a.M, a.log2_M0, a.lhs_stride_bytes, a.lhs_rb, a.log2_lhs_rb, RHS_I4 ? 32 : 16);
+  set_up(rhs, a.rhs, first_col, a.N, a.log2_N0, a.rhs_stride_bytes, a.rhs_rb, a.log2_rhs_rb, 16);
+  uint8_t* const staging = (uint8_t*)ring + wave * (UNROLL * (FA + FB) * 1024);  // (narrow pieces only)
+
+  acc_t acc[FA][FB];
+#pragma unroll
+  for (int i = 0; i < FA; ++i)
+#pragma unroll
+    for (int j = 0; j < FB; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+
+  // Batches of UNROLL steps, whose loads are in flight together, are dealt out to the wavefronts in turn: at any time
+  // the workgroup reads one contiguous stretch of every row panel. (A contiguous share of K per wavefront puts all
+  // loads of a launch at the same few offsets modulo the share: 5 to 10 % slower.)
+  const int32_t ksteps_per_step = (RHS_I4 ? 128 : 64) >> a.log2_lhs_rb;
+  const int32_t steps = (a.K + ksteps_per_step - 1) / ksteps_per_step;
+  const int32_t all_batches = a.K / ksteps_per_step / UNROLL;
+  const int32_t batches = (all_batches - wave + WAVES - 1) / WAVES;
+
+  struct Batch {
+    uint4 l[UNROLL][lhs_t::RAW], r[UNROLL][rhs_t::RAW];
+  };
+  auto fetch = [&](int32_t b, Batch& to) {
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const int32_t s = (b * WAVES + wave) * UNROLL + u;
+      rhs.template load<false, STREAMED>(s, 0, 0, to.r[u]);
+      lhs.template load<false, false>(s, 0, 0, to.l[u]);
+    }
+  };
+  // What is left after the full batches (at most UNROLL steps, K's end among them) goes to the last wavefront.
+  const bool has_rest = wave == WAVES - 1 && all_batches * UNROLL < steps;
+  auto fetch_rest = [&](Batch& to) {
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const int32_t s = all_batches * UNROLL + u;
+      const int32_t K = s < steps ? a.K : 0;
+      rhs.template load<true, false>(s, s * ksteps_per_step, K, to.r[u]);
+      lhs.template load<true, false>(s, s * ksteps_per_step, K, to.l[u]);
+    }
+  };
+  auto multiply = [&](const Batch& from) {
+    if constexpr (STAGED) {
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        lhs.to_lds(from.l[u], staging + u * (FA + FB) * 1024);
+        rhs.to_lds(from.r[u], staging + u * (FA + FB) * 1024 + FA * 1024);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      if constexpr (RHS_I4) {
+#pragma unroll
+        for (int j = 0; j < FB; ++j) {
+          const uint4 w = from.r[u][j];
+          const uint4 lo = widen_i4_times16(make_uint2(w.x, w.y)), hi = widen_i4_times16(make_uint2(w.z, w.w));
+#pragma unroll
+          for (int i = 0; i < FA; ++i) {
+            acc[i][j] = mfma16<KIND>(lo, from.l[u][2 * i], acc[i][j]);
+            acc[i][j] = mfma16<KIND>(hi, from.l[u][2 * i + 1], acc[i][j]);
+          }
+        }
+      } else {
+        uint8_t* const lds = staging + u * (FA + FB) * 1024;
+        uint4 fa[FA];
+#pragma unroll
+        for (int i = 0; i < FA; ++i) {
+          if constexpr (STAGED) fa[i] = lhs.from_lds(lds, i, lane); else fa[i] = from.l[u][i];
+        }
+#pragma unroll
+        for (int j = 0; j < FB; ++j) {
+          uint4 fb;
+          if constexpr (STAGED) fb = rhs.from_lds(lds + FA * 1024, j, lane); else fb = from.r[u][j];
+#pragma unroll
+          for (int i = 0; i < FA; ++i) acc[i][j] = mfma16<KIND>(fb, fa[i], acc[i][j]);
+        }
+      }
+    }
+  };
+  {
+    Batch p, n;
+    int32_t b = 0;
+    if (batches > 0) {
+      fetch(0, p);
+      for (; b + 2 < batches; b += 2) {
+        fetch(b + 1, n);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(p);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(b + 2, p);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(n);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (b + 1 < batches) {
+        fetch(b + 1, n);
+        multiply(p);
+        if (has_rest) fetch_rest(p);
+        multiply(n);
+        if (has_rest) multiply(p);
+      } else {
+        if (has_rest) fetch_rest(n);
+        multiply(p);
+        if (has_rest) multiply(n);
+      }
+    } else if (has_rest) {
+      fetch_rest(p);
+      multiply(p);
+    }
+  }
+
+  if constexpr (STAGED) __syncthreads();  // the staging memory takes the partial sums
+  acc_t* partial = (acc_t*)ring;
+#pragma unroll
+  for (int i = 0; i < FA; ++i)
+#pragma unroll
+    for (int j = 0; j < FB; ++j) partial[(wave * (FA * FB) + i * FB + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+
+  // The sums, and the output: lane 16*q + r of fragment (i, j) holds lhs row r and rhs rows 4*q .. 4*q + 3 of the
+  // fragments, four consecutive j0 of one output row.
+  const int32_t M0 = 1 << a.log2_M0, N0 = 1 << a.log2_N0;
+  auto total_of = [&](int f) -> acc_t {
+    acc_t v = partial[f * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) v += partial[(w * (FA * FB) + f) * 64 + lane];
+    if constexpr (RHS_I4) v = acc_t{v.x >> 4, v.y >> 4, v.z >> 4, v.w >> 4};
+    return v;
+  };
+  auto store_quad = [&](int64_t row, int64_t col, acc_t v) {
+    if (row >= total_rows || col >= total_cols) return;
+    const int64_t index = (row >> a.log2_M0) * a.out_stride0 + ((col >> a.log2_N0) << (a.log2_M0 + a.log2_N0)) +
+                          ((row & (M0 - 1)) << a.log2_N0) + (col & (N0 - 1));
+    if constexpr (NARROW) {
+      constexpr int EBITS = KIND == kF16 ? 5 : 8;
+      uint2* dst = (uint2*)(a.out + 2 * index);
+      if (a.accumulate) {
+        const uint2 old = *dst;
+        v += acc_t{widen16<EBITS>((uint16_t)old.x), widen16<EBITS>((uint16_t)(old.x >> 16)),
+                   widen16<EBITS>((uint16_t)old.y), widen16<EBITS>((uint16_t)(old.y >> 16))};
+      }
+      *dst = make_uint2((uint32_t)narrow16<EBITS>(v.x) | ((uint32_t)narrow16<EBITS>(v.y) << 16),
+                        (uint32_t)narrow16<EBITS>(v.z) | ((uint32_t)narrow16<EBITS>(v.w) << 16));
+    } else {
+      acc_t* dst = (acc_t*)(a.out + 4 * index);
+      if (a.accumulate) v += *dst;
+      *dst = v;
+    }
+  };
+  for (int f = wave; f < FA * FB; f += WAVES) {
+    const int i = f / FB, j = f % FB;
+    store_quad(first_row + 16 * i + r, first_col + 16 * j + 4 * q, total_of(f));
+  }
+}
+
+template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int UNROLL>
+hipError_t launch_wave_k_tile(MfmaArgs m, bool streamed, hipStream_t stream) {
+  unsigned grid;
+  set_tile_grid(&m, 16 * FA, 16 * FB, &grid);
+  constexpr int staging_kib = G < 16 ? WAVES * UNROLL * (FA + FB) : 0, partial_kib = WAVES * FA * FB;
+  constexpr int lds_bytes = 1024 * (staging_kib > partial_kib ? staging_kib : partial_kib);
+  auto kernel = mmt4d_wave_k_kernel<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, false>;
+  if constexpr (G == 16) {
+    if (streamed) kernel = mmt4d_wave_k_kernel<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, true>;
+  }
+  if (lds_bytes > 65536) {
+    const hipError_t attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    if (attr != hipSuccess) return attr;
+  }
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * WAVES), lds_bytes, stream, m);
+  return hipGetLastError();
+}
+
+template <int KIND, bool RHS_I4, bool NARROW, int G>
+hipError_t launch_wave_k_piece(const MfmaArgs& m, int shape, bool streamed, hipStream_t stream) {
+  // (8 wavefronts; steps in flight per wavefront such that two batches of the small tiles fit 128 registers, which
+  // leaves room for a second workgroup on the compute unit: 128 x 4096 x 4096 bf16 in 32x32 tiles 15.6 -> 13.7 us.)
+  switch (shape) {
+    case 0: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 1, 8, 4>(m, streamed, stream);
+    case 1: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 2, 8, 2>(m, streamed, stream);
+    case 2: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 2, 2, 8, 2>(m, streamed, stream);
+    case 3: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 2, 4, 8, 1>(m, streamed, stream);
+    case 4: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 4, 2, 8, 1>(m, streamed, stream);
+    case 5: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 4, 4, 8, 1>(m, streamed, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace
+}  // namespace uk
+
+#endif  // IREE_AMD_CSRC_MMT4D_WAVE_K_KERNELS_H_

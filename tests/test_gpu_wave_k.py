@@ -1,0 +1,42 @@
+"""The mmt4d kernel that splits K over the wavefronts of a workgroup (mmt4d_wave_k_kernels.h): every type, row piece size
+and output type it is instantiated for, at sizes that its tiles (16 to 64 rows and columns) do not divide, with K from
+less than a batch of steps per wavefront to many, ending on a step and inside one, strided and accumulating.
+
+Integers are compared bit for bit with a float64 product, floats within 1e-3 of max(|ref|, rms(ref)): sums of at most
+5000 products of unit-scale values in 32 bits differ by about 1e-6 of that in any order, 16-bit results by one unit in
+their last place besides.
+"""
+import pytest
+
+from iree_amd import abi
+from test_gpu_big_tiles import gpu_lib, run_case  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+LAYOUTS = [
+    (abi.MMT4D_TYPE_S8S8S32, 16, 16, 64), (abi.MMT4D_TYPE_S8S8S32, 8, 8, 4), (abi.MMT4D_TYPE_S8S8S32, 16, 16, 2),
+    (abi.MMT4D_TYPE_S8S8S32, 8, 16, 2), (abi.MMT4D_TYPE_S8S8S32, 2, 16, 8), (abi.MMT4D_TYPE_S8S8S32, 1, 16, 32),
+    (abi.MMT4D_TYPE_F16F16F32, 16, 16, 16), (abi.MMT4D_TYPE_F16F16F32, 16, 16, 1), (abi.MMT4D_TYPE_F16F16F32, 8, 8, 1),
+    (abi.MMT4D_TYPE_BF16BF16F32, 8, 8, 4), (abi.MMT4D_TYPE_BF16BF16F32, 4, 16, 2), (abi.MMT4D_TYPE_BF16BF16F32, 1, 4, 16),
+    (abi.MMT4D_TYPE_F32F32F32, 16, 16, 4), (abi.MMT4D_TYPE_F32F32F32, 16, 16, 1), (abi.MMT4D_TYPE_F32F32F32, 4, 8, 2),
+    (abi.MMT4D_TYPE_F16F16F16, 16, 16, 16), (abi.MMT4D_TYPE_F16F16F16, 16, 16, 1), (abi.MMT4D_TYPE_BF16BF16BF16, 16, 16, 2),
+    (abi.MMT4D_TYPE_BF16BF16BF16, 8, 8, 4), (abi.MMT4D_TYPE_S8S4S32, 16, 16, 32), (abi.MMT4D_TYPE_S8S4S32, 4, 16, 64),
+]
+
+
+@pytest.mark.parametrize("flags,M0,N0,K0", LAYOUTS)
+def test_edges_of_tiles_and_of_K(gpu_lib, flags, M0, N0, K0):  # noqa: F811
+    e = {abi.MMT4D_TYPE_S8S8S32: 1, abi.MMT4D_TYPE_S8S4S32: 1, abi.MMT4D_TYPE_F32F32F32: 4}.get(flags, 2)
+    row_piece = K0 * e
+    i4 = flags == abi.MMT4D_TYPE_S8S4S32
+    for n, (rows, cols, row_bytes) in enumerate([(16, 16, 64), (20, 4000, 1100), (17, 40, 5000), (48, 1000, 2000),
+                                                 (70, 264, 4500), (200, 520, 800), (1000, 1000, 1400)]):
+        K = -(-row_bytes // row_piece)
+        if i4 and K0 == 32:
+            K |= 1
+        elif not i4 and K * row_piece % 256 == 0:
+            K += 1  # (whole 256-byte stretches of a long K are another class to the names)
+        pad = 32 // e if n % 2 else 0
+        run_case(gpu_lib, flags, -(-rows // M0), -(-cols // N0), K, M0, N0, K0,
+                 "mmt4d_mfma_64x128" if i4 and K0 == 64 else "mmt4d_mfma_64x64", lhs_pad=pad, rhs_pad=pad,
+                 out_pad=4 if n % 2 else 0, offsets=(pad, pad, 4 if n % 2 else 0), accumulate=n % 3 == 1, seed=n)

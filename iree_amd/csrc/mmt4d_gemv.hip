@@ -583,8 +583,7 @@ bool launch_resident_lhs(const GemvArgs& g, hipStream_t stream, hipError_t* stat
     int used = units;
     for (int u = units; u >= units - units / 16; --u)
       if (g.N % u == 0) { used = u; break; }
-    hipLaunchKernelGGL(kernel, dim3(used), dim3(64 * waves), lds_bytes, stream, g);
-    *status = hipGetLastError();
+    *status = launch_kernel<GemvArgs>(kernel, used, 64 * waves, lds_bytes, stream, g);
   };
   // (8 wavefronts with 16 loads each in flight twice over; 16 wavefronts x 8 measured no better than the kernel above.)
   switch (g.steps) {
@@ -604,9 +603,7 @@ hipError_t launch_kind(const GemvArgs& g, hipStream_t stream, const char** name)
   // One rhs tile per workgroup (most workgroups, best balance over the CUs),
   // 4 wavefronts splitting K, 16 KiB of rhs in flight per wavefront.
   constexpr int TN = 1, UNROLL = 16, WAVES = 4;
-  hipLaunchKernelGGL((mmt4d_gemv_kernel<KIND, TN, UNROLL, WAVES>), dim3((g.N + TN - 1) / TN),
-                     dim3(64 * WAVES), 0, stream, g);
-  return hipGetLastError();
+  return launch_kernel<GemvArgs>(mmt4d_gemv_kernel<KIND, TN, UNROLL, WAVES>, (g.N + TN - 1) / TN, 64 * WAVES, 0, stream, g);
 }
 
 hipError_t launch_gemv(const Mmt4dArgs& a, hipStream_t stream, const char** name) {
@@ -631,17 +628,12 @@ hipError_t launch_gemv(const Mmt4dArgs& a, hipStream_t stream, const char** name
       const hipError_t attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
       if (attr != hipSuccess) return attr;
       *name = "mmt4d_gemv_resident_lhs";
-      hipLaunchKernelGGL(kernel, dim3(units), dim3(g.steps == 64 ? 1024 : 512), lds_bytes, stream, g);
-      return hipGetLastError();
+      return launch_kernel(kernel, units, g.steps == 64 ? 1024 : 512, lds_bytes, stream, g);
     }
     // More than 4 lhs rows: two rhs tiles per workgroup (measured on 16 rows x
     // 65536 x 8192: 4.5 TB/s with one, 5.9 with two, 4.9 with four).
-    if ((g.M << g.log2_M0) > 4) {
-      hipLaunchKernelGGL((mmt4d_gemv_i4_kernel<2, 8, 4>), dim3((g.N + 1) / 2), dim3(256), 0, stream, g);
-    } else {
-      hipLaunchKernelGGL((mmt4d_gemv_i4_kernel<1, 8, 4>), dim3(g.N), dim3(256), 0, stream, g);
-    }
-    return hipGetLastError();
+    if ((g.M << g.log2_M0) > 4) return launch_kernel<GemvArgs>(mmt4d_gemv_i4_kernel<2, 8, 4>, (g.N + 1) / 2, 256, 0, stream, g);
+    return launch_kernel<GemvArgs>(mmt4d_gemv_i4_kernel<1, 8, 4>, g.N, 256, 0, stream, g);
   }
   if (kind == kI8) return launch_kind<kI8>(g, stream, name);
   if (kind == kF16) return launch_kind<kF16>(g, stream, name);

@@ -1842,8 +1842,7 @@ hipError_t launch_direct(MfmaArgs m, hipStream_t stream, bool staggered_tail = t
         hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
     if (attr != hipSuccess) return attr;
   }
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds_bytes, stream, m);
-  return hipGetLastError();
+  return launch_kernel<MfmaArgs>(kernel, grid, 256, lds_bytes, stream, m);
 }
 
 template <int KIND, bool NARROW>
@@ -1854,8 +1853,7 @@ hipError_t launch_split_k(MfmaArgs m, hipStream_t stream) {
   auto kernel = mmt4d_mfma_split_k_kernel<KIND, NARROW>;
   const hipError_t attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds_bytes, stream, m);
-  return hipGetLastError();
+  return launch_kernel<MfmaArgs>(kernel, grid, 256, lds_bytes, stream, m);
 }
 
 // Register-staged kernel (any K, any alignment the plan admits).
@@ -1869,14 +1867,9 @@ hipError_t launch_staged(MfmaArgs m, hipStream_t stream) {
   set_tile_grid(&m, 64 * AM, 64 * BN, &grid);
   // K ending inside a chunk needs the kernel variant with the zero-filling tail step.
   const bool tail = ((int64_t)m.K * m.lhs_rb) % 64 != 0;
-  if (tail) {
-    hipLaunchKernelGGL((mmt4d_mfma_kernel<KIND, RHS_I4, NARROW, G, AM, BN, MIN_BLOCKS, true>), dim3(grid),
-                       dim3(256), 0, stream, m);
-  } else {
-    hipLaunchKernelGGL((mmt4d_mfma_kernel<KIND, RHS_I4, NARROW, G, AM, BN, MIN_BLOCKS, false>), dim3(grid),
-                       dim3(256), 0, stream, m);
-  }
-  return hipGetLastError();
+  return launch_kernel<MfmaArgs>(tail ? mmt4d_mfma_kernel<KIND, RHS_I4, NARROW, G, AM, BN, MIN_BLOCKS, true>
+                                      : mmt4d_mfma_kernel<KIND, RHS_I4, NARROW, G, AM, BN, MIN_BLOCKS, false>,
+                                 grid, 256, 0, stream, m);
   }
 }
 

@@ -449,15 +449,15 @@ template <int KIND, int G, bool NARROW>
 hipError_t launch_piece(const SkinnyArgs& all_rows, hipStream_t stream) {
   // Fewer lhs rows leave registers for more of the rhs stream in flight. More
   // than 8 rows: one launch per slab of 8.
-  const dim3 grid((unsigned)all_rows.N), block(256);
+  void (*kernel)(const SkinnyArgs);
   SkinnyArgs s = all_rows;
   for (s.row0 = 0; s.row0 < s.rows; s.row0 += 8) {
     const int left = s.rows - s.row0;
-    if (left <= 1) hipLaunchKernelGGL((mmt4d_skinny_kernel<KIND, G, 1, 16, NARROW>), grid, block, 0, stream, s);
-    else if (left <= 2) hipLaunchKernelGGL((mmt4d_skinny_kernel<KIND, G, 2, 16, NARROW>), grid, block, 0, stream, s);
-    else if (left <= 4) hipLaunchKernelGGL((mmt4d_skinny_kernel<KIND, G, 4, 8, NARROW>), grid, block, 0, stream, s);
-    else hipLaunchKernelGGL((mmt4d_skinny_kernel<KIND, G, 8, 4, NARROW>), grid, block, 0, stream, s);
-    const hipError_t e = hipGetLastError();
+    if (left <= 1) kernel = mmt4d_skinny_kernel<KIND, G, 1, 16, NARROW>;
+    else if (left <= 2) kernel = mmt4d_skinny_kernel<KIND, G, 2, 16, NARROW>;
+    else if (left <= 4) kernel = mmt4d_skinny_kernel<KIND, G, 4, 8, NARROW>;
+    else kernel = mmt4d_skinny_kernel<KIND, G, 8, 4, NARROW>;
+    const hipError_t e = launch_kernel(kernel, (unsigned)all_rows.N, 256, 0, stream, s);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

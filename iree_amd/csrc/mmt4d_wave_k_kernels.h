@@ -347,8 +347,7 @@ hipError_t launch_wave_k_tile(MfmaArgs m, bool streamed, hipStream_t stream) {
     const hipError_t attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     if (attr != hipSuccess) return attr;
   }
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * WAVES), lds_bytes, stream, m);
-  return hipGetLastError();
+  return launch_kernel<MfmaArgs>(kernel, grid, 64 * WAVES, lds_bytes, stream, m);
 }
 
 template <int KIND, bool RHS_I4, bool NARROW, int G>

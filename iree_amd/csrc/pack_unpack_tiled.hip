@@ -32,9 +32,7 @@
 // Anything this file does not cover (non power-of-two tiles, unaligned tiled
 // buffers) goes to the generic kernels.
 #include <cstdlib>
-#include <mutex>
 #include <type_traits>
-#include <vector>
 
 #include "uk_internal.h"
 
@@ -749,6 +747,33 @@ void host_row_col(const TiledArgs& a, int32_t e, int32_t* row, int32_t* col) {
   *col = (o1l << a.log2_t1) + t1;
 }
 
+// What the host searches below find for a block geometry, kept from one call to the next: the searches take
+// microseconds (choose_pitch) to a millisecond, more than the launch. A few entries per thread, the newest one in
+// the place of whichever shared its slot.
+struct LdsLayout {
+  uint64_t key = 0;
+  int32_t pitch_bytes, log2_lpr, log2_period, pad_bytes;
+};
+
+template <typename Search>
+const LdsLayout& lds_layout(uint64_t key, Search search) {
+  constexpr int kSlots = 64;
+  thread_local LdsLayout known[kSlots];
+  LdsLayout& l = known[(key * 0x9E3779B97F4A7C15ull) >> 58];
+  if (l.key != key) {
+    search(&l);
+    l.key = key;
+  }
+  return l;
+}
+
+// Everything that the searches look at; never 0.
+uint64_t geometry_key(const TiledArgs& a, int elem_bytes, int kind, int piece_bytes, int extra_cols) {
+  return 1ull | (uint64_t)elem_bytes << 1 | (uint64_t)a.log2_t0 << 4 | (uint64_t)a.log2_t1 << 8 | (uint64_t)a.log2_s3 << 12 |
+         (uint64_t)a.log2_br << 16 | (uint64_t)a.log2_bc << 21 | (uint64_t)a.tr_inner << 26 | (uint64_t)a.tr_outer << 27 |
+         (uint64_t)kind << 28 | (uint64_t)piece_bytes << 32 | (uint64_t)extra_cols << 40;
+}
+
 // LDS row pitch: the block width plus the padding (in 16-byte steps) that
 // spreads one wavefront's tiled-side accesses over the most of the 64 banks.
 // (extra_cols: columns of the following tiles that the image holds as well.)
@@ -870,7 +895,9 @@ bool make_plan(const uint8_t* flat, const uint8_t* tiled, int64_t flat_stride0, 
   a.ext_cols = 0;
   if (plan->line_aligned) a.ext_cols = (int32_t)(T1 > 128 / E ? T1 : 128 / E);
   if (plan->line_aligned && tr_outer && a.ext_cols * br * E / 16 > 512) plan->line_aligned = false, a.ext_cols = 0;
-  a.pitch_bytes = choose_pitch(a, E, piece, a.ext_cols);
+  a.pitch_bytes = lds_layout(geometry_key(a, E, 0, piece, a.ext_cols), [&](LdsLayout* found) {
+    found->pitch_bytes = choose_pitch(a, E, piece, a.ext_cols);
+  }).pitch_bytes;
   a.blocks1 = (int32_t)((size1 + bc - 1) / bc);
   // Blocks must cover every tile of the tiled side, not only the 2-D extent
   // (pack writes whole tiles of padding beyond it).
@@ -912,30 +939,13 @@ bool make_plan(const uint8_t* flat, const uint8_t* tiled, int64_t flat_stride0, 
 
 // Lane arrangement and LDS skew for pack_transposing_kernel: the combination
 // with the fewest bank conflicts among the dword writes of one wavefront
-// (32 lanes per pass over 32 banks), found by trying them on the host. The
-// search takes about a millisecond, so results are kept per block geometry.
-struct TransposingChoice {
-  uint32_t key;
-  int32_t log2_lpr, log2_period, pad_bytes;
-};
-
-void choose_transposing(TiledArgs* a, int elem_bytes, int rq) {
-  static std::mutex mutex;
-  static std::vector<TransposingChoice> known;
-  const uint32_t key = (uint32_t)elem_bytes | (uint32_t)a->log2_t0 << 4 | (uint32_t)a->log2_t1 << 8 |
-                       (uint32_t)a->log2_br << 12 | (uint32_t)a->log2_bc << 17 | (uint32_t)a->tr_outer << 22 |
-                       (uint32_t)rq << 23;
-  std::lock_guard<std::mutex> lock(mutex);
-  for (const TransposingChoice& c : known) {
-    if (c.key == key) {
-      a->log2_lpr = c.log2_lpr; a->log2_period = c.log2_period; a->pad_bytes = c.pad_bytes;
-      return;
-    }
-  }
+// (32 lanes per pass over 32 banks), found by trying them on the host.
+void search_transposing(const TiledArgs* a, int elem_bytes, int rq, LdsLayout* found) {
   const int ve = 16 / elem_bytes;
   const int cq = 4 / (elem_bytes * rq);
   const int log2_cg = a->log2_bc + (elem_bytes == 2 ? 1 : 0) - 4;
-  TransposingChoice best{key, 0, 14, 0};
+  LdsLayout& best = *found;
+  best.log2_lpr = 0; best.log2_period = 14; best.pad_bytes = 0;
   long best_cost = -1;
   TiledArgs t = *a;
   for (t.log2_lpr = log2_cg < 2 ? log2_cg : 2; t.log2_lpr <= log2_cg; ++t.log2_lpr) {
@@ -967,26 +977,14 @@ void choose_transposing(TiledArgs* a, int elem_bytes, int rq) {
       }
     }
   }
-  known.push_back(best);
-  a->log2_lpr = best.log2_lpr; a->log2_period = best.log2_period; a->pad_bytes = best.pad_bytes;
 }
 
 // The LDS skew for pack_transposing_wide_kernel: fewest bank conflicts among a
 // wavefront's 128-bit writes (8 lanes per pass, 4 of the 32 banks each).
-void choose_transposing_wide(TiledArgs* a, int elem_bytes) {
-  static std::mutex mutex;
-  static std::vector<TransposingChoice> known;
-  const uint32_t key = (uint32_t)elem_bytes | (uint32_t)a->log2_t0 << 4 | (uint32_t)a->log2_t1 << 8 |
-                       (uint32_t)a->log2_br << 12 | (uint32_t)a->log2_bc << 17 | (uint32_t)a->tr_outer << 22;
-  std::lock_guard<std::mutex> lock(mutex);
-  for (const TransposingChoice& c : known) {
-    if (c.key == key) {
-      a->log2_lpr = 0; a->log2_period = c.log2_period; a->pad_bytes = c.pad_bytes;
-      return;
-    }
-  }
+void search_transposing_wide(const TiledArgs* a, int elem_bytes, LdsLayout* found) {
   const int rq = 4 / elem_bytes, ve = 16 / elem_bytes;
-  TransposingChoice best{key, 0, 14, 0};
+  LdsLayout& best = *found;
+  best.log2_lpr = 0; best.log2_period = 14; best.pad_bytes = 0;
   long best_cost = -1;
   TiledArgs t = *a;
   for (t.log2_period = 6; t.log2_period <= 14; ++t.log2_period) {
@@ -1013,8 +1011,14 @@ void choose_transposing_wide(TiledArgs* a, int elem_bytes) {
       }
     }
   }
-  known.push_back(best);
-  a->log2_lpr = 0; a->log2_period = best.log2_period; a->pad_bytes = best.pad_bytes;
+}
+
+// `rq`: rows per dword of pack_transposing_kernel; 0: pack_transposing_wide_kernel.
+void choose_transposing(TiledArgs* a, int elem_bytes, int rq) {
+  const LdsLayout& l = lds_layout(geometry_key(*a, elem_bytes, 1 + rq, 0, 0), [&](LdsLayout* found) {
+    if (rq) search_transposing(a, elem_bytes, rq, found); else search_transposing_wide(a, elem_bytes, found);
+  });
+  a->log2_lpr = l.log2_lpr; a->log2_period = l.log2_period; a->pad_bytes = l.pad_bytes;
 }
 
 // Whether one of the transposing kernels takes the planned call (0: no,
@@ -1036,7 +1040,7 @@ int plan_transposing(Plan* p) {
   int which = 1;
   if (a.log2_t0 >= log2_ve && a.log2_bc + log2_e >= 8 && a.log2_br >= log2_ve) {
     which = 2;
-    choose_transposing_wide(&a, E);
+    choose_transposing(&a, E, 0);
   } else {
     choose_transposing(&a, E, 4 / E);
   }
@@ -1059,14 +1063,11 @@ void limit_resident_blocks(Plan* p) {
 
 template <int E, int W, bool UNPACK>
 hipError_t launch_pw(const Plan& p, hipStream_t stream) {
-  const dim3 grid(p.grid), block(256);
   switch (p.piece_bytes) {
 #define UK_PIECE(PB)                                                                         \
   case PB:                                                                                   \
     if constexpr (PB >= E) {                                                                 \
-      hipLaunchKernelGGL((tiled_kernel<E, W, PB, UNPACK>), grid, block, p.lds_bytes, stream, \
-                         p.args);                                                            \
-      return hipGetLastError();                                                              \
+      return launch_kernel<TiledArgs>(tiled_kernel<E, W, PB, UNPACK>, p.grid, 256, p.lds_bytes, stream, p.args); \
     }                                                                                        \
     return hipErrorInvalidValue
     UK_PIECE(16);
@@ -1183,19 +1184,10 @@ hipError_t launch_pack(const PackArgs& original, hipStream_t stream, const char*
   limit_resident_blocks(&plan);
   if (which) {
     *name = "pack_transposing";
-    const dim3 grid(plan.grid), block(256);
-    if (which == 2 && plan.elem_bytes == 1) {
-      hipLaunchKernelGGL(pack_transposing_wide_kernel<1>, grid, block, plan.lds_bytes, stream, plan.args);
-    } else if (which == 2) {
-      hipLaunchKernelGGL(pack_transposing_wide_kernel<2>, grid, block, plan.lds_bytes, stream, plan.args);
-    } else if (which == 3) {
-      hipLaunchKernelGGL((pack_transposing_kernel<1, 2>), grid, block, plan.lds_bytes, stream, plan.args);
-    } else if (plan.elem_bytes == 1) {
-      hipLaunchKernelGGL((pack_transposing_kernel<1, 4>), grid, block, plan.lds_bytes, stream, plan.args);
-    } else {
-      hipLaunchKernelGGL((pack_transposing_kernel<2, 2>), grid, block, plan.lds_bytes, stream, plan.args);
-    }
-    return hipGetLastError();
+    void (*kernel)(const TiledArgs) = which == 2 ? (plan.elem_bytes == 1 ? pack_transposing_wide_kernel<1> : pack_transposing_wide_kernel<2>)
+                                      : which == 3 ? pack_transposing_kernel<1, 2>
+                                      : plan.elem_bytes == 1 ? pack_transposing_kernel<1, 4> : pack_transposing_kernel<2, 2>;
+    return launch_kernel(kernel, plan.grid, 256, plan.lds_bytes, stream, plan.args);
   }
   *name = "pack_tiled";
   return launch_plan<false>(plan, stream);
@@ -1223,7 +1215,6 @@ hipError_t launch_unpack(const UnpackArgs& original, hipStream_t stream, const c
   limit_resident_blocks(&plan);
   *name = "unpack_tiled";
   if (plan.line_aligned) {
-    const dim3 grid(plan.grid), block(256);
     void (*kernel)(const TiledArgs) = nullptr;
 #define UK_LINE_ALIGNED_KERNEL(E, MODE)                                                                        \
   (plan.piece_bytes == 16 ? tiled_kernel<E, 16, 16, true, MODE>                                                 \
@@ -1232,8 +1223,7 @@ hipError_t launch_unpack(const UnpackArgs& original, hipStream_t stream, const c
     if (plan.elem_bytes == 4) kernel = tr_outer ? UK_LINE_ALIGNED_KERNEL(4, 2) : UK_LINE_ALIGNED_KERNEL(4, 1);
     else kernel = tr_outer ? UK_LINE_ALIGNED_KERNEL(2, 2) : UK_LINE_ALIGNED_KERNEL(2, 1);
 #undef UK_LINE_ALIGNED_KERNEL
-    hipLaunchKernelGGL(kernel, grid, block, plan.lds_bytes, stream, plan.args);
-    return hipGetLastError();
+    return launch_kernel(kernel, plan.grid, 256, plan.lds_bytes, stream, plan.args);
   }
   return launch_plan<true>(plan, stream);
 }

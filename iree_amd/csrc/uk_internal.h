@@ -48,6 +48,15 @@ struct UnpackArgs {
   int elem_bytes;
 };
 
+// Enqueues a kernel that takes one argument struct. (Half a hundred nanoseconds each of the triple-bracket form's
+// configuration stack and of hipGetLastError are left out: the call itself returns the launch's status.)
+template <typename Args>
+hipError_t launch_kernel(void (*kernel)(const Args), unsigned grid, unsigned block, size_t lds_bytes, hipStream_t stream,
+                         const Args& a) {
+  void* args[] = {const_cast<Args*>(&a)};
+  return hipLaunchKernel((const void*)kernel, dim3(grid), dim3(block), args, lds_bytes, stream);
+}
+
 // A launcher enqueues one operation on `stream` and returns the HIP status of
 // the launch. `name` receives a static string naming the kernel variant.
 typedef hipError_t (*Mmt4dLauncher)(const Mmt4dArgs& a, hipStream_t stream, const char** name);

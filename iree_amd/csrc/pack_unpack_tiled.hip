@@ -162,6 +162,43 @@ struct __attribute__((packed, aligned(1))) Dwords4 {
   uint32_t x, y, z, w;
 };
 
+// How the kernels use the caches. All of them read and write every byte once, but the last-level cache (256 MiB, on the
+// memory's side of the L2s) may hold what an earlier kernel left there and what a later one wants:
+//   kKeep: plain loads; stores written through to memory as they are issued (sc1), which leaves the lines in the
+//     last-level cache without leaving them dirty in an L2, to be written back when the kernel ends. What a pack
+//     writes the product reads next: bf16 pack -> mmt4d -> unpack of 777 x 4095 x 4100 58.4 -> 46.6 us, f32 [2048, 2049]
+//     packed and unpacked 17.7 -> 13.6 (with plain stores 15.2, with non-temporal ones 15.6).
+//   kKeepLoads: plain loads, non-temporal stores. f32 [4096, 4097] packed 24.8 -> 21.0 us, bf16 6000^2 transposed 28.5 -> 22.6.
+//   kStream: both non-temporal, for matrices that the cache cannot hold anyway (f32 8192^2 86 against 90 and 95 us).
+// Pack: kKeep up to 40 MiB of output (beyond that a pack by itself loses what the product after it gains), then
+// kKeepLoads up to 96 MiB of input. Unpack: kKeepLoads up to 96 MiB; its stores stay non-temporal (written through:
+// +10 to 25 % from 64 MB on, nothing below).
+enum CachePolicy { kKeep = 0, kKeepLoads = 1, kStream = 2 };
+constexpr int64_t kKeepOutputBytes = 40ll << 20, kKeepInputBytes = 96ll << 20;
+
+typedef int v4i32 __attribute__((ext_vector_type(4)));
+
+// 16 bytes that this call reads once: of the 2-D side at any alignment, of the tiled side at 16.
+template <int POLICY>
+__device__ __forceinline__ v4i32 load_flat(const uint8_t* p) {
+  typedef int v4a1 __attribute__((ext_vector_type(4), aligned(1)));
+  if constexpr (POLICY == kStream) return __builtin_nontemporal_load((const v4a1*)p);
+  else return *(const v4a1*)p;
+}
+template <int POLICY>
+__device__ __forceinline__ uint4 load_tiled(const uint8_t* p) {
+  if constexpr (POLICY == kStream) return __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4i32*)p));
+  else return *(const uint4*)p;
+}
+
+// A whole vector of the tiled side (pack).
+template <int POLICY>
+__device__ __forceinline__ void store_tiled(uint4 vec, uint8_t* p) {
+  const v4i32 v = __builtin_bit_cast(v4i32, vec);
+  if constexpr (POLICY == kKeep) asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
+  else __builtin_nontemporal_store(v, (v4i32*)p);
+}
+
 constexpr int kBlockBytes = 16384;  // bytes of the 2-D matrix per workgroup
 
 // E: element bytes. W: vector bytes on the 2-D side (16 needs 4-byte aligned
@@ -184,7 +221,7 @@ constexpr int kBlockBytes = 16384;  // bytes of the 2-D matrix per workgroup
 // requested on the tiled side cost what is left, whether or not the loads are
 // masked down to the rows that are used, and although the lines shared by two
 // blocks come from HBM only once.
-template <int E, int W, int PL_BYTES, bool UNPACK, int LINE_ALIGNED = 0>  // (1: line-aligned unpack, 2: the same with an outer transpose)
+template <int E, int W, int PL_BYTES, bool UNPACK, int POLICY, int LINE_ALIGNED = 0>  // (1: line-aligned unpack, 2: the same with an outer transpose)
 __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
   static_assert(!LINE_ALIGNED || (UNPACK && W == 16), "line-aligned windows are for unpack");
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -237,11 +274,8 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
         const int64_t row = row_base + r, col = col_base + (int64_t)cv * EPV;
         const uint8_t* g = a.src + (row * a.flat_stride0 + (STRIDED ? col * a.flat_stride1 : col)) * E;
         if (!STRIDED && row < a.size0 && col + EPV <= a.size1) {
-          // Every byte is read once: streaming (non-temporal) accesses on both
-          // sides leave the caches to the other side's partial lines.
           if constexpr (W == 16) {
-            typedef int v4a4 __attribute__((ext_vector_type(4), aligned(1)));
-            const v4a4 t = __builtin_nontemporal_load((const v4a4*)g);
+            const v4i32 t = load_flat<POLICY>(g);
             regs[u].vec = Dwords4{(uint32_t)t.x, (uint32_t)t.y, (uint32_t)t.z, (uint32_t)t.w};
           } else {
             regs[u].vec = *(const flat_vec_t*)g;
@@ -318,8 +352,7 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
       first[u] = tiled_coord(a, e, tile0_base, tile1_base);
       if constexpr (UNPACK) {
         if (first[u].in_range) {
-          typedef int v4 __attribute__((ext_vector_type(4)));
-          regs[u].vec = __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4*)(a.src + first[u].global_elem * E)));
+          regs[u].vec = load_tiled<POLICY>(a.src + first[u].global_elem * E);
         }
       }
     }
@@ -339,9 +372,7 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
         if constexpr (UNPACK) *l = regs[u].piece[q]; else regs[u].piece[q] = *l;
       }
       if constexpr (!UNPACK) {
-        // Whole tiles, written once, never read back here: streaming store.
-        typedef int v4 __attribute__((ext_vector_type(4)));
-        __builtin_nontemporal_store(__builtin_bit_cast(v4, regs[u].vec), (v4*)(a.dst + first[u].global_elem * E));
+        store_tiled<POLICY>(regs[u].vec, a.dst + first[u].global_elem * E);
       }
     }
   };
@@ -365,7 +396,6 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
     // loads leave their lines in the cache for the other one, the rest stream.
     // A thread's vectors are 256 vectors apart, a whole number of tiles (the
     // host sees to that): all of them are the same pieces of their tiles.
-    typedef int v4 __attribute__((ext_vector_type(4)));
     const int32_t e0 = tid * VE, w0 = e0 & ((1 << log2_tile) - 1);
     const uint8_t* const tile_row = a.src + (tile0_base * a.tiled_stride0 + w0) * E;
     const int32_t total_vecs = ((bc + a.ext_cols) << a.log2_br) / VE;
@@ -385,7 +415,7 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
           if (first[u].col < 128 / E || first[u].col >= bc)
             regs[u].vec = *(const uint4*)g;
           else
-            regs[u].vec = __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4*)g));
+            regs[u].vec = load_tiled<POLICY>(g);
         }
       }
 #pragma unroll
@@ -412,7 +442,7 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
         if (col0 < 128 / E || col0 >= bc)
           regs[u].vec = *(const uint4*)g;
         else
-          regs[u].vec = __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4*)g));
+          regs[u].vec = load_tiled<POLICY>(g);
       }
     }
     int32_t lds_base[PIECES];
@@ -514,7 +544,7 @@ __host__ __device__ __forceinline__ void transposing_unit(const TiledArgs& a, in
 // columns. After the byte transposes that is one whole 16-byte vector of the
 // tiled side per column: 4 / E 128-bit LDS writes per lane instead of 16 / E
 // dword writes, and a quarter of the address arithmetic.
-template <int E>
+template <int E, int POLICY>
 __global__ __launch_bounds__(256) void pack_transposing_wide_kernel(const TiledArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   typedef typename std::conditional<E == 1, uint8_t, uint16_t>::type elem_t;
@@ -552,8 +582,7 @@ __global__ __launch_bounds__(256) void pack_transposing_wide_kernel(const TiledA
       const int64_t row = row_base + patch_row[u] + lane_row * RQ + j, col = col_base + patch_col[u] + cg * VE;
       const uint8_t* g = a.src + (row * a.flat_stride0 + col) * E;
       if (row < a.size0 && col + VE <= a.size1) {
-        typedef int v4a4 __attribute__((ext_vector_type(4), aligned(1)));
-        const v4a4 t = __builtin_nontemporal_load((const v4a4*)g);
+        const v4i32 t = load_flat<POLICY>(g);
         regs[u][j].dword[0] = t.x; regs[u][j].dword[1] = t.y; regs[u][j].dword[2] = t.z; regs[u][j].dword[3] = t.w;
       } else {
 #pragma unroll
@@ -612,9 +641,7 @@ __global__ __launch_bounds__(256) void pack_transposing_wide_kernel(const TiledA
     const int32_t q = tid + 256 * u;
     const TiledCoord c = tiled_coord(a, q * VE, tile0_base, tile1_base);
     if (!c.in_range) continue;
-    typedef int v4 __attribute__((ext_vector_type(4)));
-    const v4 vec = *(const v4*)(lds + skewed(a, (uint32_t)q * 16));
-    __builtin_nontemporal_store(vec, (v4*)(a.dst + c.global_elem * E));
+    store_tiled<POLICY>(*(const uint4*)(lds + skewed(a, (uint32_t)q * 16)), a.dst + c.global_elem * E);
   }
 }
 
@@ -623,7 +650,7 @@ __global__ __launch_bounds__(256) void pack_transposing_wide_kernel(const TiledA
 // adjacent columns: RQ = 4 / E rows of one column for tiles at least that
 // tall, or, for int8 tiles two rows tall (the [N0][2] layouts of the x86
 // dot-product tiles), 2 rows of 2 columns.
-template <int E, int RQ>
+template <int E, int RQ, int POLICY>
 __global__ __launch_bounds__(256) void pack_transposing_kernel(const TiledArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   typedef typename std::conditional<E == 1, uint8_t, uint16_t>::type elem_t;
@@ -656,8 +683,7 @@ __global__ __launch_bounds__(256) void pack_transposing_kernel(const TiledArgs a
       const int64_t row = row_base + row0[u] + j, col = col_base + col0[u];
       const uint8_t* g = a.src + (row * a.flat_stride0 + col) * E;
       if (row < a.size0 && col + VE <= a.size1) {
-        typedef int v4a4 __attribute__((ext_vector_type(4), aligned(1)));
-        const v4a4 t = __builtin_nontemporal_load((const v4a4*)g);
+        const v4i32 t = load_flat<POLICY>(g);
         regs[u][j].dword[0] = t.x; regs[u][j].dword[1] = t.y; regs[u][j].dword[2] = t.z; regs[u][j].dword[3] = t.w;
       } else {
 #pragma unroll
@@ -705,9 +731,7 @@ __global__ __launch_bounds__(256) void pack_transposing_kernel(const TiledArgs a
     const int32_t q = tid + 256 * u;
     const TiledCoord c = tiled_coord(a, q * VE, tile0_base, tile1_base);
     if (!c.in_range) continue;
-    typedef int v4 __attribute__((ext_vector_type(4)));
-    const v4 vec = *(const v4*)(lds + skewed(a, (uint32_t)q * 16));
-    __builtin_nontemporal_store(vec, (v4*)(a.dst + c.global_elem * E));
+    store_tiled<POLICY>(*(const uint4*)(lds + skewed(a, (uint32_t)q * 16)), a.dst + c.global_elem * E);
   }
 }
 
@@ -1061,40 +1085,59 @@ void limit_resident_blocks(Plan* p) {
   if (p->elem_bytes == 4 && p->args.total_blocks >= 8192 && p->lds_bytes < kLdsAskedFor) p->lds_bytes = kLdsAskedFor;
 }
 
-template <int E, int W, bool UNPACK>
-hipError_t launch_pw(const Plan& p, hipStream_t stream) {
+template <int E, bool UNPACK, int POLICY>
+hipError_t launch_e(const Plan& p, hipStream_t stream) {
+  void (*kernel)(const TiledArgs) = nullptr;
   switch (p.piece_bytes) {
-#define UK_PIECE(PB)                                                                         \
-  case PB:                                                                                   \
-    if constexpr (PB >= E) {                                                                 \
-      return launch_kernel<TiledArgs>(tiled_kernel<E, W, PB, UNPACK>, p.grid, 256, p.lds_bytes, stream, p.args); \
-    }                                                                                        \
-    return hipErrorInvalidValue
+#define UK_PIECE(PB) \
+  case PB:           \
+    if constexpr (PB >= E) kernel = tiled_kernel<E, 16, PB, UNPACK, POLICY>; \
+    break
     UK_PIECE(16);
     UK_PIECE(8);
     UK_PIECE(4);
     UK_PIECE(2);
     UK_PIECE(1);
 #undef UK_PIECE
-    default:
-      return hipErrorInvalidValue;
   }
+  if (!kernel) return hipErrorInvalidValue;
+  return launch_kernel(kernel, p.grid, 256, p.lds_bytes, stream, p.args);
 }
 
-template <int E, bool UNPACK>
-hipError_t launch_e(const Plan& p, hipStream_t stream) {
-  if (p.flat_vec_bytes != 16) return hipErrorInvalidValue;
-  return launch_pw<E, 16, UNPACK>(p, stream);
-}
-
-template <bool UNPACK>
+template <bool UNPACK, int POLICY>
 hipError_t launch_plan(const Plan& p, hipStream_t stream) {
+  if (p.flat_vec_bytes != 16) return hipErrorInvalidValue;
   switch (p.elem_bytes) {
-    case 1: return launch_e<1, UNPACK>(p, stream);
-    case 2: return launch_e<2, UNPACK>(p, stream);
-    case 4: return launch_e<4, UNPACK>(p, stream);
+    case 1: return launch_e<1, UNPACK, POLICY>(p, stream);
+    case 2: return launch_e<2, UNPACK, POLICY>(p, stream);
+    case 4: return launch_e<4, UNPACK, POLICY>(p, stream);
     default: return hipErrorInvalidValue;
   }
+}
+
+// (`which` as plan_transposing says, 0: the plain kernel.)
+template <int POLICY>
+hipError_t launch_pack_plan(const Plan& p, int which, hipStream_t stream) {
+  if (!which) return launch_plan<false, POLICY>(p, stream);
+  void (*kernel)(const TiledArgs) =
+      which == 2 ? (p.elem_bytes == 1 ? pack_transposing_wide_kernel<1, POLICY> : pack_transposing_wide_kernel<2, POLICY>)
+      : which == 3 ? pack_transposing_kernel<1, 2, POLICY>
+      : p.elem_bytes == 1 ? pack_transposing_kernel<1, 4, POLICY> : pack_transposing_kernel<2, 2, POLICY>;
+  return launch_kernel(kernel, p.grid, 256, p.lds_bytes, stream, p.args);
+}
+
+template <int POLICY>
+hipError_t launch_unpack_plan(const Plan& p, hipStream_t stream) {
+  if (!p.line_aligned) return launch_plan<true, POLICY>(p, stream);
+  void (*kernel)(const TiledArgs) = nullptr;
+#define UK_LINE_ALIGNED_KERNEL(E, MODE)                                                                \
+  (p.piece_bytes == 16 ? tiled_kernel<E, 16, 16, true, POLICY, MODE>                                    \
+   : p.piece_bytes == 8 ? tiled_kernel<E, 16, 8, true, POLICY, MODE>                                    \
+   : (p.piece_bytes == 4 || E == 4) ? tiled_kernel<E, 16, 4, true, POLICY, MODE> : tiled_kernel<E, 16, E, true, POLICY, MODE>)
+  if (p.elem_bytes == 4) kernel = p.args.tr_outer ? UK_LINE_ALIGNED_KERNEL(4, 2) : UK_LINE_ALIGNED_KERNEL(4, 1);
+  else kernel = p.args.tr_outer ? UK_LINE_ALIGNED_KERNEL(2, 2) : UK_LINE_ALIGNED_KERNEL(2, 1);
+#undef UK_LINE_ALIGNED_KERNEL
+  return launch_kernel(kernel, p.grid, 256, p.lds_bytes, stream, p.args);
 }
 
 }  // namespace
@@ -1182,15 +1225,12 @@ hipError_t launch_pack(const PackArgs& original, hipStream_t stream, const char*
   plan.args.padding_value = a.padding_value;
   const int which = plan_transposing(&plan);
   limit_resident_blocks(&plan);
-  if (which) {
-    *name = "pack_transposing";
-    void (*kernel)(const TiledArgs) = which == 2 ? (plan.elem_bytes == 1 ? pack_transposing_wide_kernel<1> : pack_transposing_wide_kernel<2>)
-                                      : which == 3 ? pack_transposing_kernel<1, 2>
-                                      : plan.elem_bytes == 1 ? pack_transposing_kernel<1, 4> : pack_transposing_kernel<2, 2>;
-    return launch_kernel(kernel, plan.grid, 256, plan.lds_bytes, stream, plan.args);
-  }
-  *name = "pack_tiled";
-  return launch_plan<false>(plan, stream);
+  *name = which ? "pack_transposing" : "pack_tiled";
+  const int64_t in_bytes = a.in_size0 * a.in_size1 * a.elem_bytes;
+  const int64_t out_bytes = a.out_size0 * a.out_size1 * a.out_size2 * a.out_size3 * a.elem_bytes;
+  if (out_bytes <= kKeepOutputBytes) return launch_pack_plan<kKeep>(plan, which, stream);
+  return in_bytes <= kKeepInputBytes ? launch_pack_plan<kKeepLoads>(plan, which, stream)
+                                     : launch_pack_plan<kStream>(plan, which, stream);
 }
 
 hipError_t launch_unpack(const UnpackArgs& original, hipStream_t stream, const char** name) {
@@ -1214,18 +1254,8 @@ hipError_t launch_unpack(const UnpackArgs& original, hipStream_t stream, const c
   plan.args.padding_value = 0;
   limit_resident_blocks(&plan);
   *name = "unpack_tiled";
-  if (plan.line_aligned) {
-    void (*kernel)(const TiledArgs) = nullptr;
-#define UK_LINE_ALIGNED_KERNEL(E, MODE)                                                                        \
-  (plan.piece_bytes == 16 ? tiled_kernel<E, 16, 16, true, MODE>                                                 \
-   : plan.piece_bytes == 8 ? tiled_kernel<E, 16, 8, true, MODE>                                                 \
-   : (plan.piece_bytes == 4 || E == 4) ? tiled_kernel<E, 16, 4, true, MODE> : tiled_kernel<E, 16, E, true, MODE>)
-    if (plan.elem_bytes == 4) kernel = tr_outer ? UK_LINE_ALIGNED_KERNEL(4, 2) : UK_LINE_ALIGNED_KERNEL(4, 1);
-    else kernel = tr_outer ? UK_LINE_ALIGNED_KERNEL(2, 2) : UK_LINE_ALIGNED_KERNEL(2, 1);
-#undef UK_LINE_ALIGNED_KERNEL
-    return launch_kernel(kernel, plan.grid, 256, plan.lds_bytes, stream, plan.args);
-  }
-  return launch_plan<true>(plan, stream);
+  return a.out_size0 * a.out_size1 * a.elem_bytes <= kKeepInputBytes ? launch_unpack_plan<kKeepLoads>(plan, stream)
+                                                                      : launch_unpack_plan<kStream>(plan, stream);
 }
 
 }  // namespace uk

@@ -122,8 +122,8 @@ inline bool split_k_covers(const MfmaArgs& m) {
 
 inline int choose_tile(const MfmaArgs& m, bool rhs_i4, bool direct, const TileChoice** chosen) {
   static const TileChoice kTiles[] = {
-      {4, 4, 1003.f, false, 0.52f}, {4, 2, 905.f, true, 0.34f}, {2, 2, 851.f, false, 0.40f},
-      {2, 1, 607.f, true, 0.23f}, {1, 1, 529.f, false, 0.135f}, {1, 2, 600.f, true, 0.22f}};
+      {4, 4, 1003.f, false, 0.50f}, {4, 2, 905.f, true, 0.31f}, {2, 2, 851.f, false, 0.25f},
+      {2, 1, 607.f, true, 0.168f}, {1, 1, 529.f, false, 0.122f}, {1, 2, 600.f, true, 0.19f}};
   const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
   int best = -1;
   double best_cost = 0;

@@ -59,8 +59,15 @@ __device__ __forceinline__ typename Acc<KIND>::type mfma16(uint4 row_operand, ui
   }
 }
 
+// 16 bytes of the rhs, which a call reads once. STREAMED: past the caches (see streamed_rhs).
+template <bool STREAMED>
+__device__ __forceinline__ uint4 load_rhs(const uint8_t* p) {
+  if constexpr (STREAMED) return __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4i32*)p));
+  else return *(const uint4*)p;
+}
+
 // TN: rhs tiles per workgroup. UNROLL: K-steps whose loads are in flight together.
-template <int KIND, int TN, int UNROLL, int kWaves>
+template <int KIND, int TN, int UNROLL, int kWaves, bool STREAMED>
 __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_kernel(const GemvArgs a) {
   typedef typename Acc<KIND>::type acc_t;
   __shared__ acc_t partial[kWaves][TN][64];
@@ -108,7 +115,7 @@ __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_kernel(const GemvArgs 
       l[u] = make_uint4(0, 0, 0, 0);
       if (lhs_valid) l[u] = *(const uint4*)(lhs_lane + k1 * lhs_kstep);
 #pragma unroll
-      for (int t = 0; t < TN; ++t) r[u][t] = __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4i32*)(rhs_lane[t] + k1 * rhs_kstep)));
+      for (int t = 0; t < TN; ++t) r[u][t] = load_rhs<STREAMED>(rhs_lane[t] + k1 * rhs_kstep);
     }
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
@@ -216,7 +223,7 @@ void mmt4d_gemv_resident_lhs_kernel(const GemvArgs a) {
     const bool loaded = tile_rows_loaded(u);
 #pragma unroll
     for (int s = 0; s < UNROLL; ++s)
-      if (loaded) dst[s] = __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4i32*)(p + s * rhs_step_bytes)));
+      if (loaded) dst[s] = load_rhs<true>(p + s * rhs_step_bytes);
   };
   fetch(0, r[0]);
   uint4* own_lhs = gemv_lds + (wave * UNROLL) * 64 + lane;
@@ -301,7 +308,7 @@ __device__ __forceinline__ uint4 lhs_bytes_even_then_odd(uint4 v) {
 // TN rhs tiles per workgroup share each lhs operand: with 16 lhs rows the lhs
 // is twice the bytes of one rhs tile per step (int8 against int4), all of it
 // through L2 for every workgroup.
-template <int TN, int UNROLL, int kWaves>
+template <int TN, int UNROLL, int kWaves, bool STREAMED>
 __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_i4_kernel(const GemvArgs a) {
   __shared__ v4i32 partial[kWaves][TN][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -349,7 +356,7 @@ __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_i4_kernel(const GemvAr
     for (int u = 0; u < UNROLL; ++u) {
 #pragma unroll
       for (int t = 0; t < TN; ++t)
-        r[u][t] = __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4i32*)(rhs_lane[t] + (int64_t)(s + u) * 1024)));
+        r[u][t] = load_rhs<STREAMED>(rhs_lane[t] + (int64_t)(s + u) * 1024);
       if (lhs_valid) {
         l0[u] = *(const uint4*)(lhs_lane + (s + u) * lhs_step_bytes);
         l1[u] = *(const uint4*)(lhs_lane + (s + u) * lhs_step_bytes + 16);
@@ -438,7 +445,7 @@ void mmt4d_gemv_i4_resident_lhs_kernel(const GemvArgs a) {
     const bool loaded = tile_rows_loaded(u);
 #pragma unroll
     for (int s = 0; s < UNROLL; ++s)
-      if (loaded) dst[s] = __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4i32*)(p + (int64_t)s * 1024)));
+      if (loaded) dst[s] = load_rhs<true>(p + (int64_t)s * 1024);
   };
 #pragma unroll
   for (int u = 0; u < DEPTH - 1; ++u)
@@ -560,6 +567,14 @@ int compute_units() {
   return cached[device];
 }
 
+// Whether the rhs is streamed past the caches. Weights of more than 64 MiB are: the last-level cache (256 MiB, shared
+// with whatever else the program keeps) is not likely to hold them from one call to the next. Smaller int4 ones are not
+// (1 x 11008 x 4096, 22 MB: 5.98 -> 5.59 us, 14336 x 8192 12.5 -> 11.4). Types of a byte or more from 24 MiB on are
+// (8192 x 2048 bf16 6.9 us streamed, 7.1 not), below they are not (512 x 8192 bf16 8.5 -> 5.7 us).
+bool streamed_rhs(const GemvArgs& g, int rhs_rb, bool i4) {
+  return (int64_t)g.N * g.K * rhs_rb * 16 > ((i4 ? 64ll : 24ll) << 20);
+}
+
 // The resident-lhs kernel, if it fits: more than 4 lhs rows, K in whole 64-byte
 // steps whose number is what one of the instantiations splits over its
 // wavefronts, at least a tile per compute unit and at most MAX_TILES of them.
@@ -602,8 +617,8 @@ hipError_t launch_kind(const GemvArgs& g, hipStream_t stream, const char** name)
   }
   // One rhs tile per workgroup (most workgroups, best balance over the CUs),
   // 4 wavefronts splitting K, 16 KiB of rhs in flight per wavefront.
-  constexpr int TN = 1, UNROLL = 16, WAVES = 4;
-  return launch_kernel<GemvArgs>(mmt4d_gemv_kernel<KIND, TN, UNROLL, WAVES>, (g.N + TN - 1) / TN, 64 * WAVES, 0, stream, g);
+  return launch_kernel<GemvArgs>(streamed_rhs(g, g.rb, false) ? mmt4d_gemv_kernel<KIND, 1, 16, 4, true>
+                                                              : mmt4d_gemv_kernel<KIND, 1, 16, 4, false>, g.N, 256, 0, stream, g);
 }
 
 hipError_t launch_gemv(const Mmt4dArgs& a, hipStream_t stream, const char** name) {
@@ -617,14 +632,15 @@ hipError_t launch_gemv(const Mmt4dArgs& a, hipStream_t stream, const char** name
     // 0.51 against 0.48): the resident-lhs kernel, where its instantiations fit the number of steps (each of 128
     // values of K; the lhs of 64 steps fills 128 KiB of LDS).
     const int units = compute_units();
+    const bool streamed = streamed_rhs(g, g.rb / 2, true);
     constexpr int MAX_TILES = 8;
     if (((g.M << g.log2_M0) > 4 || g.N >= 6 * (int64_t)units) && units > 0 && g.N >= units && (2 * (int64_t)g.N + units - 1) / units / 2 + 1 <= MAX_TILES &&
         (g.steps == 64 || g.steps == 32)) {
       const int lds_bytes = 128 * 1024;  // the lhs operands of 64 steps; the partial sums need less
       // (16 wavefronts x 4 steps with three tiles' loads in flight: 0.65 of the HBM peak at 16 x 28672 x 8192 against
       // 0.62 for the kernel below; 8 wavefronts x 8 steps 0.63, deeper prefetch slower.)
-      void (*kernel)(const GemvArgs) = g.steps == 64 ? mmt4d_gemv_i4_resident_lhs_kernel<16, 4, MAX_TILES>
-                                                     : mmt4d_gemv_i4_resident_lhs_kernel<8, 4, MAX_TILES>;
+      void (*kernel)(const GemvArgs) =
+          g.steps == 64 ? mmt4d_gemv_i4_resident_lhs_kernel<16, 4, MAX_TILES> : mmt4d_gemv_i4_resident_lhs_kernel<8, 4, MAX_TILES>;
       const hipError_t attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
       if (attr != hipSuccess) return attr;
       *name = "mmt4d_gemv_resident_lhs";
@@ -632,8 +648,15 @@ hipError_t launch_gemv(const Mmt4dArgs& a, hipStream_t stream, const char** name
     }
     // More than 4 lhs rows: two rhs tiles per workgroup (measured on 16 rows x
     // 65536 x 8192: 4.5 TB/s with one, 5.9 with two, 4.9 with four).
-    if ((g.M << g.log2_M0) > 4) return launch_kernel<GemvArgs>(mmt4d_gemv_i4_kernel<2, 8, 4>, (g.N + 1) / 2, 256, 0, stream, g);
-    return launch_kernel<GemvArgs>(mmt4d_gemv_i4_kernel<1, 8, 4>, g.N, 256, 0, stream, g);
+    // No more tiles than compute units and a long K: a workgroup has a unit to itself, 16 wavefronts (16 x 512 x 12288 9.1
+    // -> 4.4 us, 16 x 4096 x 4096 4.55 -> 4.3; with less K, and for the other types, 4 wavefronts do as well).
+    if (g.N <= units && g.steps >= 32)
+      return launch_kernel<GemvArgs>(mmt4d_gemv_i4_kernel<1, 4, 16, false>, g.N, 1024, 0, stream, g);
+    if ((g.M << g.log2_M0) > 4)
+      return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<2, 8, 4, true> : mmt4d_gemv_i4_kernel<2, 8, 4, false>,
+                                     (g.N + 1) / 2, 256, 0, stream, g);
+    return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<1, 8, 4, true> : mmt4d_gemv_i4_kernel<1, 8, 4, false>,
+                                   g.N, 256, 0, stream, g);
   }
   if (kind == kI8) return launch_kind<kI8>(g, stream, name);
   if (kind == kF16) return launch_kind<kF16>(g, stream, name);

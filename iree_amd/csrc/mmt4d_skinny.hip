@@ -266,16 +266,16 @@ __device__ __forceinline__ float exchange(float v, int lane_xor) { return __shfl
 
 // G: bytes of a row piece; ROWS: lhs rows the kernel keeps accumulators for
 // (a.rows <= ROWS); UNROLL: 1 KiB blocks of the rhs stream a wavefront has in
-// flight; NARROW: the output has the 16-bit type of the operands. One
-// workgroup of four wavefronts per rhs tile row.
-template <int KIND, int G, int ROWS, int UNROLL, bool NARROW>
-__global__ __launch_bounds__(256) void mmt4d_skinny_kernel(const SkinnyArgs a) {
+// flight; STREAMED: the rhs is read past the caches; NARROW: the output has the
+// 16-bit type of the operands. One workgroup per rhs tile row.
+template <int KIND, int G, int ROWS, int WAVES, int UNROLL, bool STREAMED, bool NARROW>
+__global__ __launch_bounds__(64 * WAVES) void mmt4d_skinny_kernel(const SkinnyArgs a) {
   static_assert(!NARROW || KIND == kF16 || KIND == kBF16, "16-bit outputs are floats");
   typedef typename Acc<KIND>::type acc_t;
   // (One-byte pieces of int8: 8-row tiles, two k steps per lane.)
   constexpr bool TWO_KSTEPS = KIND == kI8 && G == 1;
   constexpr int R = TWO_KSTEPS ? 8 : 16 / G;  // rhs rows in a lane's 16 bytes
-  __shared__ acc_t partial[4][ROWS][32];
+  __shared__ acc_t partial[WAVES][ROWS][32];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int32_t M0 = 1 << a.log2_M0, N0 = 1 << a.log2_N0;
@@ -302,12 +302,12 @@ __global__ __launch_bounds__(256) void mmt4d_skinny_kernel(const SkinnyArgs a) {
     for (int r = 0; r < R; ++r) acc[m][r] = 0;
 
   const int64_t blocks = (a.tile_bytes + 1023) >> 10;
-  for (int64_t j0 = wave; j0 < blocks; j0 += 4 * UNROLL) {
+  for (int64_t j0 = wave; j0 < blocks; j0 += WAVES * UNROLL) {
     uint4 v[UNROLL];
     typename LhsPiece<KIND>::type l[UNROLL][ROWS];
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-      const int64_t off = ((j0 + 4 * u) << 10) + 16 * lane;
+      const int64_t off = ((j0 + WAVES * u) << 10) + 16 * lane;
       const bool inside = off < a.tile_bytes;
       v[u] = make_uint4(0, 0, 0, 0);
       if (TWO_KSTEPS && inside && off + 16 > a.tile_bytes) {
@@ -316,10 +316,11 @@ __global__ __launch_bounds__(256) void mmt4d_skinny_kernel(const SkinnyArgs a) {
         v[u].x = half.x;
         v[u].y = half.y;
       } else if (inside) {
-        v[u] = __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4i32*)(rhs_tile + off)));
+        if constexpr (STREAMED) v[u] = __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4i32*)(rhs_tile + off)));
+        else v[u] = *(const uint4*)(rhs_tile + off);
       }
       // The lhs piece of this lane's k step.
-      const int64_t kstep = inside ? ((j0 + 4 * u) << (10 - log2_kstep_bytes)) + kstep_in_block : 0;
+      const int64_t kstep = inside ? ((j0 + WAVES * u) << (10 - log2_kstep_bytes)) + kstep_in_block : 0;
 #pragma unroll
       for (int m = 0; m < ROWS; ++m) {
         if constexpr (TWO_KSTEPS) {
@@ -357,9 +358,8 @@ __global__ __launch_bounds__(256) void mmt4d_skinny_kernel(const SkinnyArgs a) {
   const int m = a.row0 + slab_row;
   if (slab_row < ROWS && m < a.rows) {
     acc_t sum = partial[0][slab_row][j0];
-    sum += partial[1][slab_row][j0];
-    sum += partial[2][slab_row][j0];
-    sum += partial[3][slab_row][j0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) sum += partial[w][slab_row][j0];
     if constexpr (KIND == kI8I4) sum >>= 4;
     const int64_t index = (int64_t)(m >> a.log2_M0) * a.out_stride0 +
                           ((int64_t)blockIdx.x << (a.log2_M0 + a.log2_N0)) + ((m & (M0 - 1)) << a.log2_N0) + j0;
@@ -445,22 +445,34 @@ bool make_args(const Mmt4dArgs& a, bool probe_only, int* kind, int* piece_bytes,
   return true;
 }
 
-template <int KIND, int G, bool NARROW>
-hipError_t launch_piece(const SkinnyArgs& all_rows, hipStream_t stream) {
+template <int KIND, int G, int WAVES, bool STREAMED, bool NARROW>
+hipError_t launch_slabs(const SkinnyArgs& all_rows, hipStream_t stream) {
   // Fewer lhs rows leave registers for more of the rhs stream in flight. More
   // than 8 rows: one launch per slab of 8.
+  constexpr int SHARE = WAVES / 4;
   void (*kernel)(const SkinnyArgs);
   SkinnyArgs s = all_rows;
   for (s.row0 = 0; s.row0 < s.rows; s.row0 += 8) {
     const int left = s.rows - s.row0;
-    if (left <= 1) kernel = mmt4d_skinny_kernel<KIND, G, 1, 16, NARROW>;
-    else if (left <= 2) kernel = mmt4d_skinny_kernel<KIND, G, 2, 16, NARROW>;
-    else if (left <= 4) kernel = mmt4d_skinny_kernel<KIND, G, 4, 8, NARROW>;
-    else kernel = mmt4d_skinny_kernel<KIND, G, 8, 4, NARROW>;
-    const hipError_t e = launch_kernel(kernel, (unsigned)all_rows.N, 256, 0, stream, s);
+    if (left <= 1) kernel = mmt4d_skinny_kernel<KIND, G, 1, WAVES, 16 / SHARE, STREAMED, NARROW>;
+    else if (left <= 2) kernel = mmt4d_skinny_kernel<KIND, G, 2, WAVES, 16 / SHARE, STREAMED, NARROW>;
+    else if (left <= 4) kernel = mmt4d_skinny_kernel<KIND, G, 4, WAVES, 8 / SHARE, STREAMED, NARROW>;
+    else kernel = mmt4d_skinny_kernel<KIND, G, 8, WAVES, 4 / SHARE, STREAMED, NARROW>;
+    const hipError_t e = launch_kernel(kernel, (unsigned)all_rows.N, 64 * WAVES, 0, stream, s);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+template <int KIND, int G, bool NARROW>
+hipError_t launch_piece(const SkinnyArgs& s, hipStream_t stream) {
+  // Weights that the last-level cache (256 MiB) will not hold to the next call are streamed past the caches (1 x 14336 x
+  // 4096 bf16, 112 MiB: 19.4 us, through them 21.3); smaller ones are not (512 x 12288 f16 11.9 -> 9.8 us).
+  if (s.tile_bytes * s.N > (96ll << 20)) return launch_slabs<KIND, G, 4, true, NARROW>(s, stream);
+  // No more tile rows than compute units, and long ones: eight wavefronts (4 x 512 x 8192 bf16 14.4 -> 10.3 us, 1 x 512 x
+  // 4096 5.0 -> 3.9). With shorter ones, or several to a unit, the summing at the end costs more than it gives.
+  if (s.N <= 256 && s.tile_bytes >= 128 * 1024) return launch_slabs<KIND, G, 8, false, NARROW>(s, stream);
+  return launch_slabs<KIND, G, 4, false, NARROW>(s, stream);
 }
 
 template <int KIND, bool NARROW>

@@ -9,7 +9,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <immintrin.h>
 
+#include "host_crew.h"
 #include "uk_internal.h"
 
 #define UK_API extern "C" __attribute__((visibility("default")))
@@ -88,17 +90,69 @@ bool device_accessible(const void* p) {
          attr.type == hipMemoryTypeHost;
 }
 
-// Per-thread device staging buffers for host operands (grow-only, released
-// when the thread exits).
-struct StageBuffer {
-  void* ptr = nullptr;
+// Per-thread device memory that host operands are mirrored in (grow-only, released when the thread exits or goes on to
+// another device).
+struct StageArena {
+  uint8_t* ptr = nullptr;
   size_t capacity = 0;
-  ~StageBuffer() {
+  int device = -1;
+  ~StageArena() {
     // At process teardown the HIP runtime may already be gone: errors are moot.
     if (ptr) (void)hipFree(ptr);
   }
 };
-thread_local StageBuffer tl_stage[3];
+thread_local StageArena tl_arena;
+
+// Per-thread pinned memory that host operands pass through on their way to and from the device: the CPU copies the
+// caller's pages (55 to 80 GB/s) a chunk at a time while the previous chunks are on the bus (50 GB/s each way). The
+// runtime's own path for pageable memory moves 20 to 33 GB/s up and 17 down, in 30 to 100 us for a few KiB. int8 through
+// both: 64 x 256 x 256 47 -> 21 us, 512 x 2048 x 2048 (5 MB up, 4 down) 430 -> 255, 4096 x 2048 x 4096 2731 -> 1458.
+struct HostPipe {
+  static constexpr size_t kSlotBytes = 1 << 20, kFirstBytes = 128 << 10;
+  static constexpr int kSlots = 8;
+  static constexpr size_t kHalfBytes = kSlots / 2 * kSlotBytes;  // a download alternates between halves
+  static constexpr int kFlags = (int)(2 * kHalfBytes / uk::kDownloadPieceBytes);
+  uint8_t* pinned = nullptr;
+  uint32_t* flags = nullptr;  // behind the slots
+  uint32_t generation = 0;
+  hipEvent_t event[kSlots] = {};
+  int device = -1;
+
+  ~HostPipe() { release(); }
+  void release() {
+    for (hipEvent_t& e : event) {
+      if (e) (void)hipEventDestroy(e);
+      e = nullptr;
+    }
+    if (pinned) (void)hipHostFree(pinned);
+    pinned = nullptr;
+  }
+  // False: no pinned memory to be had; the caller copies from pageable memory.
+  bool ready(int current_device) {
+    if (pinned && device == current_device) return true;
+    release();
+    device = current_device;
+    if (hipHostMalloc((void**)&pinned, kSlots * kSlotBytes + kFlags * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      pinned = nullptr;
+      return false;
+    }
+    flags = (uint32_t*)(pinned + kSlots * kSlotBytes);
+    memset(flags, 0, kFlags * sizeof(uint32_t));
+    generation = 0;
+    for (hipEvent_t& e : event) {
+      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        e = nullptr;
+        release();
+        return false;
+      }
+    }
+    return true;
+  }
+  uint8_t* slot(int i) { return pinned + (size_t)i * kSlotBytes; }
+};
+thread_local HostPipe tl_pipe;
 
 // Static staging memory of the allocation-free entry point: one array per
 // device, owned by the code object, resolved to a device address once per
@@ -143,57 +197,57 @@ unsigned char* scratch_for_current_device(int* device_out = nullptr) {
   return (unsigned char*)resolved;
 }
 
-// Where the calling entry point mirrors host operands: the thread's grow-only
-// buffers (may call hipMalloc), or a bump allocator over the device's static
-// scratch (never allocates; fails when the operands do not fit).
+// Where the calling entry point mirrors host operands: the thread's grow-only memory (may call hipMalloc), or the
+// device's static scratch (never allocates; fails when the operands do not fit).
 struct Stager {
-  unsigned char* fixed_base = nullptr;  // non-null: static scratch
-  size_t fixed_used = 0;
   bool no_alloc = false;
   bool copies_issued = false;           // something was enqueued on the stream for this call
+  bool piped = false;                   // contiguous operands go through the thread's pinned memory
+  uk::HostCrew* crew = nullptr;         // helps with those copies, until the end of the call
   ScratchLease lease;                   // held while the static scratch is in use
+  ~Stager() {
+    if (crew) crew->release();
+  }
 };
 
-size_t rounded_for_scratch(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+size_t rounded_for_staging(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 
-bool stage_reserve(Stager& stager, int slot, size_t bytes, void** out) {
+bool stage_reserve(Stager& stager, size_t bytes, uint8_t** out) {
+  int device = -1;
   if (stager.no_alloc) {
-    if (!stager.fixed_base) {
-      int device = -1;
-      unsigned char* base = scratch_for_current_device(&device);
-      if (!base) {
-        report_failure(__FILE__, __LINE__, __func__, "hipGetSymbolAddress(scratch) failed on the current device");
-        return false;
-      }
-      bool expected = false;
-      if (!g_scratch_busy[device].compare_exchange_strong(expected, true, std::memory_order_acq_rel)) {
-        report_failure(__FILE__, __LINE__, __func__,
-                       "static staging memory busy: another iree_uk_mi355x_mmt4d_noalloc_p call with host "
-                       "operands is running on this device");
-        return false;
-      }
-      stager.lease.flag = &g_scratch_busy[device];
-      stager.fixed_base = base;
-    }
-    const size_t rounded = rounded_for_scratch(bytes);
-    if (rounded > kScratchBytes - stager.fixed_used) {
+    if (bytes > kScratchBytes) {
       report_failure(__FILE__, __LINE__, __func__,
                      "host operands exceed IREE_UK_MI355X_NOALLOC_MAX_STAGED_BYTES of static staging memory");
       return false;
     }
-    *out = stager.fixed_base + stager.fixed_used;
-    stager.fixed_used += rounded;
+    unsigned char* base = scratch_for_current_device(&device);
+    if (!base) {
+      report_failure(__FILE__, __LINE__, __func__, "hipGetSymbolAddress(scratch) failed on the current device");
+      return false;
+    }
+    bool expected = false;
+    if (!g_scratch_busy[device].compare_exchange_strong(expected, true, std::memory_order_acq_rel)) {
+      report_failure(__FILE__, __LINE__, __func__,
+                     "static staging memory busy: another iree_uk_mi355x_mmt4d_noalloc_p call with host "
+                     "operands is running on this device");
+      return false;
+    }
+    stager.lease.flag = &g_scratch_busy[device];
+    *out = base;
     return true;
   }
-  StageBuffer& s = tl_stage[slot];
-  if (s.capacity < bytes) {
+  UK_HIP_OK(hipGetDevice(&device));
+  StageArena& s = tl_arena;
+  if (s.capacity < bytes || s.device != device) {
     if (s.ptr) UK_HIP_OK(hipFree(s.ptr));
     s.ptr = nullptr;
     s.capacity = 0;
     size_t cap = bytes + bytes / 4 + 256;
-    UK_HIP_OK(hipMalloc(&s.ptr, cap));
+    UK_HIP_OK(hipMalloc((void**)&s.ptr, cap));
     s.capacity = cap;
+    s.device = device;
   }
+  stager.piped = tl_pipe.ready(device);
   *out = s.ptr;
   return true;
 }
@@ -255,49 +309,212 @@ bool copy_rows(void* dst, const void* src, const RowRegion& r, hipMemcpyKind kin
   return true;
 }
 
-// Makes one operand reachable from the device. For a host operand the region is
-// mirrored at the same layout in a staging buffer; `upload` says whether its
-// current contents are needed on the device.
-struct Staged {
-  const void* host = nullptr;  // non-null iff staged
-  void* dev = nullptr;
+// One operand of a call. For a host operand the region is mirrored at the same layout in device memory; `upload` says
+// whether its current contents are needed there.
+struct Operand {
+  const void* ptr;
+  RowRegion region;
+  bool upload;
+  const void* dev = nullptr;   // where the kernel finds it
+  const void* host = nullptr;  // non-null iff mirrored
+  bool contiguous() const { return region.rows == 1 || region.pitch == region.width; }
 };
 
-bool stage_operand(Stager& stager, int slot, const void* ptr, const RowRegion& region, bool upload,
-                   hipStream_t stream, Staged* st, const void** dev_ptr, int known_on_device = -1) {
-  *dev_ptr = ptr;
-  if (region.span == 0) return true;
-  const bool on_device = known_on_device < 0 ? device_accessible(ptr) : known_on_device != 0;
-  if (tl_async) {
-    // Nothing is staged in asynchronous mode, and a host address must not
-    // reach a kernel: the device would fault.
-    if (!on_device) {
-      report_failure(__FILE__, __LINE__, __func__, "asynchronous mode needs device-accessible operands");
-      return false;
+// Copies between the caller's memory and the pinned memory. `stream_past_caches` (operands that together are larger than
+// what the caches are likely to hold anyway): 42 GB/s on cold pages where memcpy moves 33, both ways.
+__attribute__((target("avx2"))) void copy_past_caches(uint8_t* dst, const uint8_t* src, size_t n) {
+  const size_t head = (size_t)(-(uintptr_t)dst & 31);
+  if (n < 256) {
+    memcpy(dst, src, n);
+    return;
+  }
+  memcpy(dst, src, head);
+  dst += head; src += head; n -= head;
+  for (; n >= 128; n -= 128, dst += 128, src += 128) {
+    _mm_prefetch((const char*)src + 1024, _MM_HINT_NTA);
+    _mm_prefetch((const char*)src + 1088, _MM_HINT_NTA);
+    const __m256i a = _mm256_loadu_si256((const __m256i*)src), b = _mm256_loadu_si256((const __m256i*)(src + 32)),
+                  c = _mm256_loadu_si256((const __m256i*)(src + 64)), d = _mm256_loadu_si256((const __m256i*)(src + 96));
+    _mm256_stream_si256((__m256i*)dst, a);
+    _mm256_stream_si256((__m256i*)(dst + 32), b);
+    _mm256_stream_si256((__m256i*)(dst + 64), c);
+    _mm256_stream_si256((__m256i*)(dst + 96), d);
+  }
+  _mm_sfence();
+  memcpy(dst, src, n);
+}
+
+constexpr size_t kPastCachesBytes = 2 << 20;
+void host_copy(void* dst, const void* src, size_t n, bool stream_past_caches) {
+  static const bool avx2 = __builtin_cpu_supports("avx2");
+  if (stream_past_caches && avx2) copy_past_caches((uint8_t*)dst, (const uint8_t*)src, n);
+  else memcpy(dst, src, n);
+}
+
+// Contiguous operands, mirrored one after the other from `base` on, to the device through the pinned memory: chunks
+// that double from 128 KiB to 1 MiB (the first one is on the bus early, the later ones cost few launches), small
+// operands together in one.
+bool pipe_up(Stager& stager, uint8_t* base, Operand* const* ops, int count, hipStream_t stream) {
+  HostPipe& pipe = tl_pipe;
+  const Operand& last = *ops[count - 1];
+  const size_t total = (size_t)((const uint8_t*)last.dev - base) + (size_t)last.region.span;
+  const bool wraps = total > (HostPipe::kSlots - 1) * HostPipe::kSlotBytes, past_caches = total >= kPastCachesBytes;
+  constexpr size_t kPiece = 64 << 10;  // of a chunk, per helper and turn
+  size_t chunk = HostPipe::kFirstBytes;
+  for (size_t at = 0, n = 0, used = 0; at < total; at += n, ++used) {
+    const int slot = (int)(used % HostPipe::kSlots);
+    if (used >= (size_t)HostPipe::kSlots) UK_HIP_OK(hipEventSynchronize(pipe.event[slot]));
+    n = total - at < chunk ? total - at : chunk;
+    auto fill = [&](size_t from, size_t to) {  // of the mirrored bytes
+      for (int op = 0; op < count; ++op) {
+        const size_t begin = (size_t)((const uint8_t*)ops[op]->dev - base), end = begin + (size_t)ops[op]->region.span;
+        const size_t f = begin > from ? begin : from, t = end < to ? end : to;
+        if (f < t) host_copy(pipe.slot(slot) + (f - at), (const uint8_t*)ops[op]->host + (f - begin), t - f, past_caches);
+      }
+    };
+    if (stager.crew && n > kPiece) {
+      stager.crew->run((uint32_t)((n + kPiece - 1) / kPiece), [&](uint32_t i) {
+        const size_t from = at + i * kPiece;
+        fill(from, from + kPiece < at + n ? from + kPiece : at + n);
+      }, [] {});
+    } else {
+      fill(at, at + n);
     }
-    return true;
+    UK_HIP_OK(uk::launch_upload(pipe.slot(slot), base + at, n, stream));
+    if (wraps) UK_HIP_OK(hipEventRecord(pipe.event[slot], stream));
+    if (chunk < HostPipe::kSlotBytes) chunk *= 2;
   }
-  if (on_device) return true;
-  void* d = nullptr;
-  if (!stage_reserve(stager, slot, (size_t)region.span, &d)) return false;
-  if (upload) {
-    stager.copies_issued = true;
-    if (!copy_rows(d, ptr, region, hipMemcpyHostToDevice, stream)) return false;
-  }
-  st->host = ptr;
-  st->dev = d;
-  *dev_ptr = d;
   return true;
 }
 
-bool finish(hipStream_t stream, const Staged& out, const RowRegion& out_region, bool any_staged) {
-  if (out.host && !copy_rows(const_cast<void*>(out.host), out.dev, out_region,
-                             hipMemcpyDeviceToHost, stream)) {
-    if (!tl_async) (void)hipStreamSynchronize(stream);
+// The way back, results visible on return. The pinned memory is used in halves: while the pieces of one are taken as
+// their flags come in, the other is filled. (Everything that the caller's stream did before has ended with the last flag.)
+bool pipe_down(const Stager& stager, void* host, const void* dev, size_t bytes, hipStream_t stream) {
+  HostPipe& pipe = tl_pipe;
+  constexpr size_t kHalf = HostPipe::kHalfBytes, kPiece = uk::kDownloadPieceBytes;
+  const uint32_t first_generation = pipe.generation + 1;
+  pipe.generation += (uint32_t)((bytes + kHalf - 1) / kHalf);
+  std::atomic<bool> failed{false};
+  hipError_t status = hipSuccess;
+  auto send = [&](size_t at) -> bool {
+    const size_t half = at / kHalf % 2, n = bytes - at < kHalf ? bytes - at : kHalf;
+    UK_HIP_OK(uk::launch_download((const uint8_t*)dev + at, pipe.pinned + half * kHalf, pipe.flags + half * (kHalf / kPiece),
+                                  first_generation + (uint32_t)(at / kHalf), n, stream));
+    return true;
+  };
+  const std::thread::id caller = std::this_thread::get_id();
+  if (!send(0)) return false;
+  for (size_t at = 0; at < bytes && !failed; at += kHalf) {
+    if (at + kHalf < bytes && !send(at + kHalf)) return false;  // (into the half that was taken before this one)
+    const size_t half = at / kHalf % 2, n = bytes - at < kHalf ? bytes - at : kHalf;
+    const uint32_t generation = first_generation + (uint32_t)(at / kHalf);
+    const uint32_t* flags = pipe.flags + half * (kHalf / kPiece);
+    const uint32_t pieces = (uint32_t)((n + kPiece - 1) / kPiece);
+    // A stream that has ended (or failed) without setting its flags will not set them any more.
+    auto check_stream = [&] {
+      const hipError_t e = hipStreamQuery(stream);
+      if (e == hipErrorNotReady) return;
+      if (e == hipSuccess && __atomic_load_n(flags + pieces - 1, __ATOMIC_ACQUIRE) == generation) return;
+      status = e;
+      failed = true;
+    };
+    auto take = [&](uint32_t i) {
+      for (uint32_t spins = 1; __atomic_load_n(flags + i, __ATOMIC_ACQUIRE) != generation && !failed; ++spins) {
+        __builtin_ia32_pause();
+        if (spins % (1u << 16) == 0 && std::this_thread::get_id() == caller) check_stream();
+      }
+      if (failed) return;
+      const size_t from = i * kPiece, len = n - from < kPiece ? n - from : kPiece;
+      host_copy((uint8_t*)host + at + from, pipe.pinned + half * kHalf + from, len, bytes >= kPastCachesBytes);
+    };
+    if (stager.crew) {
+      stager.crew->run(pieces, take, check_stream);
+    } else {
+      for (uint32_t i = 0; i < pieces; ++i) take(i);
+    }
+  }
+  if (failed) {
+    UK_HIP_OK(status);
+    report_failure(__FILE__, __LINE__, __func__, "the copy to host memory ended without its flags");
     return false;
   }
+  return true;
+}
+
+// Makes the operands of a call reachable from the device.
+bool stage_operands(Stager& stager, Operand* const* ops, int count, hipStream_t stream) {
+  Operand* mirrored[3];
+  int mirrors = 0, piped = 0;
+  for (int i = 0; i < count; ++i) {
+    Operand& o = *ops[i];
+    o.dev = o.ptr;
+    if (o.region.span == 0 || device_accessible(o.ptr)) continue;
+    if (tl_async) {
+      // Nothing is staged in asynchronous mode, and a host address must not
+      // reach a kernel: the device would fault.
+      report_failure(__FILE__, __LINE__, __func__, "asynchronous mode needs device-accessible operands");
+      return false;
+    }
+    // (What is uploaded in one piece comes first.)
+    if (o.upload && o.contiguous()) {
+      for (int k = mirrors; k > piped; --k) mirrored[k] = mirrored[k - 1];
+      mirrored[piped++] = &o;
+    } else {
+      mirrored[mirrors] = &o;
+    }
+    ++mirrors;
+  }
+  if (mirrors == 0) return true;
+  // Whether the operands fit is settled before the first byte is copied.
+  Checked need;
+  int64_t total = 0;
+  for (int i = 0; i < mirrors; ++i) total = need.add(total, need.add(mirrored[i]->region.span, 255) & ~(int64_t)255);
+  if (!need.ok) {
+    report_failure(__FILE__, __LINE__, __func__, stager.no_alloc
+                       ? "host operands exceed IREE_UK_MI355X_NOALLOC_MAX_STAGED_BYTES of static staging memory"
+                       : "host operands exceed the address space");
+    return false;
+  }
+  uint8_t* base = nullptr;
+  if (!stage_reserve(stager, (size_t)total, &base)) return false;
+  size_t at = 0;
+  for (int i = 0; i < mirrors; ++i) {
+    Operand& o = *mirrored[i];
+    o.host = o.ptr;
+    o.dev = base + at;
+    at += rounded_for_staging((size_t)o.region.span);
+  }
+  // The helpers are woken for what takes longer than waking them.
+  if (stager.piped && total >= (int64_t)kPastCachesBytes && uk::HostCrew::instance().engage())
+    stager.crew = &uk::HostCrew::instance();
+  int i = 0;
+  if (stager.piped && piped > 0) {
+    stager.copies_issued = true;
+    if (!pipe_up(stager, base, mirrored, piped, stream)) return false;
+    i = piped;
+  }
+  for (; i < mirrors; ++i) {
+    Operand& o = *mirrored[i];
+    if (!o.upload) continue;
+    stager.copies_issued = true;
+    if (!copy_rows(const_cast<void*>(o.dev), o.host, o.region, hipMemcpyHostToDevice, stream)) return false;
+  }
+  return true;
+}
+
+bool finish(const Stager& stager, hipStream_t stream, const Operand& out) {
+  if (out.host) {
+    if (stager.piped && out.contiguous()) {
+      if (pipe_down(stager, const_cast<void*>(out.host), out.dev, (size_t)out.region.span, stream)) return true;
+      (void)hipStreamSynchronize(stream);
+      return false;
+    }
+    if (!copy_rows(const_cast<void*>(out.host), out.dev, out.region, hipMemcpyDeviceToHost, stream)) {
+      (void)hipStreamSynchronize(stream);
+      return false;
+    }
+  }
   if (!tl_async) UK_HIP_OK(hipStreamSynchronize(stream));
-  (void)any_staged;
   return true;
 }
 
@@ -408,40 +625,19 @@ void mmt4d_impl(const iree_uk_mmt4d_params_t* p, Stager& stager) {
   const void* out = offset_pointer(p->out_buffer, out_offset_bytes);
 
   hipStream_t stream = tl_stream;
-  Staged s_lhs, s_rhs, s_out;
-  const void *d_lhs, *d_rhs, *d_out;
   // A host operand whose rows overlap is staged as one span.
   auto as_copied = [](const RowRegion& r) { return r.rows > 1 && r.pitch < r.width ? as_one_span(r) : r; };
-  const RowRegion lhs_copy = as_copied(lhs_region), rhs_copy = as_copied(rhs_region);
-  int lhs_dev = -1, rhs_dev = -1, out_dev = -1;
-  if (stager.no_alloc && !tl_async) {
-    // Whether the host operands fit the static memory is settled before the
-    // first byte is copied.
-    lhs_dev = lhs_copy.span == 0 || device_accessible(lhs);
-    rhs_dev = rhs_copy.span == 0 || device_accessible(rhs);
-    out_dev = out_region.span == 0 || device_accessible(out);
-    Checked need;
-    int64_t total = 0;
-    if (!lhs_dev) total = need.add(total, need.add(lhs_copy.span, 255) & ~(int64_t)255);
-    if (!rhs_dev) total = need.add(total, need.add(rhs_copy.span, 255) & ~(int64_t)255);
-    if (!out_dev) total = need.add(total, need.add(out_region.span, 255) & ~(int64_t)255);
-    if (!need.ok || total > (int64_t)kScratchBytes) {
-      report_failure(__FILE__, __LINE__, __func__,
-                     "host operands exceed IREE_UK_MI355X_NOALLOC_MAX_STAGED_BYTES of static staging memory");
-      return;
-    }
-  }
-  if (!stage_operand(stager, 0, lhs, lhs_copy, true, stream, &s_lhs, &d_lhs, lhs_dev) ||
-      !stage_operand(stager, 1, rhs, rhs_copy, true, stream, &s_rhs, &d_rhs, rhs_dev) ||
-      !stage_operand(stager, 2, out, out_region, accumulate, stream, &s_out, &d_out, out_dev)) {
+  Operand o_lhs{lhs, as_copied(lhs_region), true}, o_rhs{rhs, as_copied(rhs_region), true}, o_out{out, out_region, accumulate};
+  Operand* const operands[] = {&o_lhs, &o_rhs, &o_out};
+  if (!stage_operands(stager, operands, 3, stream)) {
     abandon(stager, stream);
     return;
   }
 
   uk::Mmt4dArgs a;
-  a.lhs = (const uint8_t*)d_lhs;
-  a.rhs = (const uint8_t*)d_rhs;
-  a.out = (uint8_t*)const_cast<void*>(d_out);
+  a.lhs = (const uint8_t*)o_lhs.dev;
+  a.rhs = (const uint8_t*)o_rhs.dev;
+  a.out = (uint8_t*)const_cast<void*>(o_out.dev);
   a.lhs_stride0 = p->lhs_stride0;
   a.rhs_stride0 = p->rhs_stride0;
   a.out_stride0 = p->out_stride0;
@@ -472,7 +668,7 @@ void mmt4d_impl(const iree_uk_mmt4d_params_t* p, Stager& stager) {
         return;
       }
     }
-    finish(stream, s_out, out_region, s_lhs.host || s_rhs.host || s_out.host);
+    finish(stager, stream, o_out);
     return;
   }
 
@@ -482,7 +678,7 @@ void mmt4d_impl(const iree_uk_mmt4d_params_t* p, Stager& stager) {
     abandon(stager, stream);
     return;
   }
-  finish(stream, s_out, out_region, s_lhs.host || s_rhs.host || s_out.host);
+  finish(stager, stream, o_out);
 }
 
 }  // namespace
@@ -583,22 +779,21 @@ UK_API void iree_uk_pack_p(const iree_uk_pack_params_t* p) {
   const void* out = offset_pointer(p->out_buffer, out_offset_bytes);
 
   hipStream_t stream = tl_stream;
-  Staged s_in, s_out;
-  const void *d_in, *d_out;
   // A host input whose rows overlap or interleave (stride0 < row width) is
   // staged as one span.
   RowRegion in_copy = in_region;
   if (in_copy.rows > 1 && in_copy.pitch < in_copy.width) in_copy = as_one_span(in_region);
   Stager stager;
-  if (!stage_operand(stager, 0, in, in_copy, true, stream, &s_in, &d_in) ||
-      !stage_operand(stager, 2, out, out_region, false, stream, &s_out, &d_out)) {
+  Operand o_in{in, in_copy, true}, o_out{out, out_region, false};
+  Operand* const operands[] = {&o_in, &o_out};
+  if (!stage_operands(stager, operands, 2, stream)) {
     abandon(stager, stream);
     return;
   }
 
   uk::PackArgs a;
-  a.in = (const uint8_t*)d_in;
-  a.out = (uint8_t*)const_cast<void*>(d_out);
+  a.in = (const uint8_t*)o_in.dev;
+  a.out = (uint8_t*)const_cast<void*>(o_out.dev);
   a.in_stride0 = p->in_stride0; a.in_stride1 = p->in_stride1;
   a.out_stride0 = p->out_stride0;
   a.in_size0 = p->in_size0; a.in_size1 = p->in_size1;
@@ -611,7 +806,7 @@ UK_API void iree_uk_pack_p(const iree_uk_pack_params_t* p) {
     abandon(stager, stream);
     return;
   }
-  finish(stream, s_out, out_region, s_in.host || s_out.host);
+  finish(stager, stream, o_out);
 }
 
 UK_API void iree_uk_pack(const void* in_buffer, iree_uk_index_t in_offset, iree_uk_index_t in_stride0,
@@ -681,20 +876,19 @@ UK_API void iree_uk_unpack_p(const iree_uk_unpack_params_t* p) {
   const void* out = offset_pointer(p->out_buffer, out_offset_bytes);
 
   hipStream_t stream = tl_stream;
-  Staged s_in, s_out;
-  const void *d_in, *d_out;
   Stager stager;
   // With an inner output stride the bytes between elements must survive the
   // round trip through the staging buffer, so the rows are uploaded first.
-  if (!stage_operand(stager, 0, in, in_region, true, stream, &s_in, &d_in) ||
-      !stage_operand(stager, 2, out, out_region, p->out_stride1 != 1, stream, &s_out, &d_out)) {
+  Operand o_in{in, in_region, true}, o_out{out, out_region, p->out_stride1 != 1};
+  Operand* const operands[] = {&o_in, &o_out};
+  if (!stage_operands(stager, operands, 2, stream)) {
     abandon(stager, stream);
     return;
   }
 
   uk::UnpackArgs a;
-  a.in = (const uint8_t*)d_in;
-  a.out = (uint8_t*)const_cast<void*>(d_out);
+  a.in = (const uint8_t*)o_in.dev;
+  a.out = (uint8_t*)const_cast<void*>(o_out.dev);
   a.in_stride0 = p->in_stride0;
   a.out_stride0 = p->out_stride0; a.out_stride1 = p->out_stride1;
   a.in_size0 = p->in_size0; a.in_size1 = p->in_size1;
@@ -706,7 +900,7 @@ UK_API void iree_uk_unpack_p(const iree_uk_unpack_params_t* p) {
     abandon(stager, stream);
     return;
   }
-  finish(stream, s_out, out_region, s_in.host || s_out.host);
+  finish(stager, stream, o_out);
 }
 
 UK_API void iree_uk_unpack(const void* in_buffer, iree_uk_index_t in_offset,

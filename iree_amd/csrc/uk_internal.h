@@ -81,6 +81,14 @@ hipError_t launch_mmt4d_generic(const Mmt4dArgs& a, hipStream_t stream, const ch
 hipError_t launch_pack(const PackArgs& a, hipStream_t stream, const char** name);
 hipError_t launch_unpack(const UnpackArgs& a, hipStream_t stream, const char** name);
 
+// Copies between pinned host memory and the device as kernels on the stream (host_copy.hip), 16 bytes at a time: both
+// sides are 16-byte aligned and may be touched up to the next multiple of 16 bytes. A download sets flag b to
+// `generation` when piece b of kDownloadPieceBytes is visible to the host.
+constexpr int kDownloadPieceBytes = 32 * 1024;
+hipError_t launch_upload(const void* pinned, void* dst, size_t bytes, hipStream_t stream);
+hipError_t launch_download(const void* src, void* pinned, uint32_t* flags, uint32_t generation, size_t bytes,
+                           hipStream_t stream);
+
 // Bit widths of the (lhs, rhs, out) element types of an mmt4d type flag;
 // returns false for an unknown flag.
 inline bool mmt4d_type_bits(uint32_t flags, int* lhs, int* rhs, int* out) {

@@ -191,11 +191,12 @@ __device__ __forceinline__ uint4 load_tiled(const uint8_t* p) {
   else return *(const uint4*)p;
 }
 
-// A whole vector of the tiled side (pack).
+// A whole vector of the tiled side (pack). (The no-op keeps a vector instruction that overwrites the stored registers one
+// wait state away: the compiler looks after that hazard of wide stores, but not behind inline assembly.)
 template <int POLICY>
 __device__ __forceinline__ void store_tiled(uint4 vec, uint8_t* p) {
   const v4i32 v = __builtin_bit_cast(v4i32, vec);
-  if constexpr (POLICY == kKeep) asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
+  if constexpr (POLICY == kKeep) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" : : "v"(p), "v"(v) : "memory");
   else __builtin_nontemporal_store(v, (v4i32*)p);
 }
 

@@ -110,6 +110,9 @@ thread_local StageArena tl_arena;
 struct HostPipe {
   static constexpr size_t kSlotBytes = 1 << 20, kFirstBytes = 128 << 10;
   static constexpr int kSlots = 8;
+  // What an upload moves before it comes back to its first slot: 1, 2 and 4 times kFirstBytes, then whole slots.
+  static constexpr size_t kUnwrappedBytes = 7 * kFirstBytes + (kSlots - 3) * kSlotBytes;
+  static_assert(8 * kFirstBytes == kSlotBytes, "kUnwrappedBytes counts three doublings");
   static constexpr size_t kHalfBytes = kSlots / 2 * kSlotBytes;  // a download alternates between halves
   static constexpr int kFlags = (int)(2 * kHalfBytes / uk::kDownloadPieceBytes);
   uint8_t* pinned = nullptr;
@@ -358,7 +361,7 @@ bool pipe_up(Stager& stager, uint8_t* base, Operand* const* ops, int count, hipS
   HostPipe& pipe = tl_pipe;
   const Operand& last = *ops[count - 1];
   const size_t total = (size_t)((const uint8_t*)last.dev - base) + (size_t)last.region.span;
-  const bool wraps = total > (HostPipe::kSlots - 1) * HostPipe::kSlotBytes, past_caches = total >= kPastCachesBytes;
+  const bool wraps = total > HostPipe::kUnwrappedBytes, past_caches = total >= kPastCachesBytes;
   constexpr size_t kPiece = 64 << 10;  // of a chunk, per helper and turn
   size_t chunk = HostPipe::kFirstBytes;
   for (size_t at = 0, n = 0, used = 0; at < total; at += n, ++used) {

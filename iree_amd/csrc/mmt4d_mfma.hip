@@ -31,7 +31,7 @@ double block_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
   const bool direct = mfma_direct_covers(m, gather, rhs_i4);
   if (gather == 16 && (kind == kF16 || kind == kBF16) && direct && split_k_covers(m)) return 4.5 + 0.235 * m.chunks;
   const TileChoice* t;
-  choose_tile(m, rhs_i4, direct, &t);
+  choose_tile(m, kind, rhs_i4, gather, direct, &t);
   const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
   const int64_t tiles = ((rows + 64 * t->am - 1) / (64 * t->am)) * ((cols + 64 * t->bn - 1) / (64 * t->bn));
   double per_chunk = t->us_per_chunk;
@@ -178,9 +178,11 @@ const char* class_name(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
     if (kind != kI8 && split_k_covers(m)) return "mmt4d_mfma_128x64_split_k";
   }
   static const char* const kNames[] = {"mmt4d_mfma_256x256", "mmt4d_mfma_256x128", "mmt4d_mfma_128x128",
-                                       "mmt4d_mfma_128x64",  "mmt4d_mfma_64x64",   "mmt4d_mfma_64x128"};
+                                       "mmt4d_mfma_128x64",  "mmt4d_mfma_64x64",   "mmt4d_mfma_64x128",
+                                       "mmt4d_mfma_192x192", "mmt4d_mfma_128x192", "mmt4d_mfma_192x128",
+                                       "mmt4d_mfma_256x192", "mmt4d_mfma_192x256"};
   const TileChoice* tile;
-  return kNames[choose_tile(m, rhs_i4, direct, &tile)];
+  return kNames[choose_tile(m, kind, rhs_i4, gather, direct, &tile)];
 }
 
 hipError_t launch_wave_k(const Plan& plan, hipStream_t stream, const char** name) {

@@ -94,20 +94,14 @@ hipError_t launch_wave_k_f32(const MfmaArgs& m, int gather, int shape, bool stre
 hipError_t launch_wave_k_f16_narrow(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);
 hipError_t launch_wave_k_bf16_narrow(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);
 
-// The block tiles of the block kernels, and which of them a problem takes. The estimate is
-//   (workgroups per compute unit, rounded up) x (tile area) / (tile efficiency),
-// with the efficiencies measured at saturation on bf16 16x16x8 operands
-// (TFLOP/s at 2048 x 14336 x 4096: 256x256 1003, 256x128 905, 128x128 851,
-// 128x64 607, 64x64 529). It reproduces the measured best tile on every shape
-// tried (128 .. 4096 rows against 14336 columns, 1024^2 .. 4096^2 squares).
-// Larger tiles move fewer operand bytes per multiply through L2 -> LDS and run
-// the matrix pipe longer between barriers, smaller ones spread a problem over
-// more compute units.
+// The block tiles of the block kernels. Larger ones move fewer operand bytes per multiply through L2 -> LDS and run the
+// matrix pipe longer between barriers, smaller ones spread a problem over more compute units; those with a side of 192
+// are there for the problems that leave a last round of 128- or 256-wide tiles nearly empty (bf16 752 x 10928 x 2272 has
+// 516 tiles of 128x128 for 256 compute units: 56 us, and 228 of 192x192: 39 us).
 struct TileChoice {
   int am, bn;
-  float efficiency;
-  bool direct_only;   // no register-staged instantiation of this shape
-  float us_per_chunk; // one workgroup per compute unit, 64 bytes of K per row (bf16 and int8, direct-to-LDS kernel)
+  bool direct_only;    // no register-staged instantiation of this shape
+  float us_per_chunk;  // one workgroup per compute unit, 64 bytes of K per row (bf16 and int8): see block_cost
 };
 
 // The 128x64 tile with K split over its wavefronts (mmt4d_mfma_split_k_kernel): 65 to 128 lhs rows, one row of tiles.
@@ -120,24 +114,43 @@ inline bool split_k_covers(const MfmaArgs& m) {
   return rows > 64 && rows <= 128 && cols <= 256 * 64 && row_bytes % 128 == 0 && row_bytes >= 8192;
 }
 
-inline int choose_tile(const MfmaArgs& m, bool rhs_i4, bool direct, const TileChoice** chosen) {
-  static const TileChoice kTiles[] = {
-      {4, 4, 1003.f, false, 0.50f}, {4, 2, 905.f, true, 0.31f}, {2, 2, 851.f, false, 0.25f},
-      {2, 1, 607.f, true, 0.168f}, {1, 1, 529.f, false, 0.122f}, {1, 2, 600.f, true, 0.19f}};
+// The tile that a problem takes: the least time for 64 bytes of K per row over all of its workgroups, from the time that
+// one workgroup per compute unit takes and, where two fit a compute unit (LDS: up to 128x128), two beside each other.
+// Microseconds on the direct-to-LDS kernel, fitted to 24 shapes (M 160..4096, N 464..13952, K 700..8192) with every tile
+// for bf16 / f16 16x16x16, bf16 8x8x4, int8 8x8x4 and 16x16x64, f16 16x16x1 and int8 16x16x2 (2-byte pieces: fragments
+// come in pairs, which an odd number of them does not have), int4 16x16x32. The tile picked is 0.1 to 1.3 % slower in the
+// mean than the best one; without the 192-wide ones and one efficiency per tile it was 4 to 7 %. f32 is bound by the
+// matrix pipe whatever the tile, which leaves the number of rounds (in units of a 128x128 tile; the large tiles, which
+// move fewer bytes, are favoured by 10 %).
+inline int choose_tile(const MfmaArgs& m, int kind, bool rhs_i4, int gather, bool direct, const TileChoice** chosen) {
+  static const TileChoice kTiles[] = {{4, 4, false, 0.50f}, {4, 2, true, 0.31f},  {2, 2, false, 0.25f}, {2, 1, true, 0.168f},
+                                      {1, 1, false, 0.122f}, {1, 2, true, 0.19f}, {3, 3, true, 0.34f},  {2, 3, true, 0.25f},
+                                      {3, 2, true, 0.25f},   {4, 3, true, 0.40f}, {3, 4, true, 0.40f}};
+  constexpr int kCount = sizeof kTiles / sizeof kTiles[0];
+  // Per class of operands and tile, 0: no such instantiation.
+  enum { kSixteenBit, kInt8, kTwoBytePieces, kInt4, kFloat32 };
+  static const float kOne[][kCount] = {{.51f, .33f, .222f, .148f, .129f, 0, .342f, .25f, .25f, .40f, .405f},
+                                       {.50f, .35f, .249f, .170f, .125f, 0, .352f, .28f, .28f, .40f, .405f},
+                                       {.61f, .40f, .285f, .251f, .25f, 0, 0, 0, 0, .52f, .523f},
+                                       {.62f, .324f, .237f, 0, .129f, .172f, 0, 0, .26f, 0, 0},
+                                       {3.45f, 1.87f, 1.0f, .53f, .27f, 0, 0, 0, 0, 0, 0}};
+  static const float kTwo[][kCount] = {{0, 0, .345f, .31f, .195f}, {0, 0, .44f, .345f, .23f}, {0, 0, .48f, .52f, .35f},
+                                       {0, 0, .345f, 0, .195f, .263f}, {0, 0, 2.0f, 1.06f, .54f}};
+  const int what = kind == kF32 ? kFloat32 : rhs_i4 ? kInt4 : gather == 2 ? kTwoBytePieces : kind == kI8 ? kInt8 : kSixteenBit;
   const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
   int best = -1;
   double best_cost = 0;
-  for (int i = 0; i < (int)(sizeof kTiles / sizeof kTiles[0]); ++i) {
+  for (int i = 0; i < kCount; ++i) {
     const TileChoice& t = kTiles[i];
-    if (t.direct_only && !direct) continue;
-    if (rhs_i4 && t.bn < 2 && t.direct_only) continue;  // the int4 direct path needs a rhs fragment per wavefront
-    if (!rhs_i4 && t.am == 1 && t.bn == 2) continue;    // 64x128 exists for the int4 rhs only (in place of 128x64)
+    if (kOne[what][i] == 0 || (t.direct_only && !direct)) continue;
+    if (gather == 1 && (t.am == 3 || t.bn == 3)) continue;
     // The int4 64x64 tile exists only register-staged, at less than half the
     // rate of the direct 64x128 one on the same problem.
     if (rhs_i4 && direct && t.am == 1 && t.bn == 1) continue;
     const int64_t br = 64 * t.am, bc = 64 * t.bn;
-    const int64_t workgroups = ((rows + br - 1) / br) * ((cols + bc - 1) / bc);
-    const double cost = (double)((workgroups + 255) / 256) * (double)(br * bc) / t.efficiency;
+    const int64_t rounds = (((rows + br - 1) / br) * ((cols + bc - 1) / bc) + 255) / 256;
+    const double one = kOne[what][i], two = kTwo[what][i];
+    const double cost = two > 0 ? (rounds & 1) * one + (rounds >> 1) * two : rounds * one;
     if (best < 0 || cost < best_cost) {
       best = i;
       best_cost = cost;
@@ -689,7 +702,7 @@ __device__ __forceinline__ void wait_loads_but() {
 // an accumulating call, the destination read in the tail; 3 = accumulating call with the destination read and
 // added during the main loop (needs enough steps), tail as in 1.
 template <int KIND, bool RHS_I4, bool NARROW, int G, int AM, int BN, int STAGES, int STAGGER = 0>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, AM * BN >= 16 ? 1 : (AM * BN >= 4 ? 2 : 4))))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, AM * BN >= 9 ? 1 : (AM * BN >= 4 ? 2 : 4))))
 void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   typedef typename AccType<KIND>::type acc_t;
   static_assert(!RHS_I4 || (G == 16 && BN >= 2), "int4 rhs: 16-byte pieces, at least one fragment per wavefront");
@@ -1882,8 +1895,9 @@ hipError_t launch_variant(const MfmaArgs& m, hipStream_t stream, const char** na
       return launch_split_k<KIND, NARROW>(m, stream);
     }
   }
+  constexpr bool kWide192 = KIND != kF32 && G != 1;
   const TileChoice* tile;
-  switch (choose_tile(m, RHS_I4, direct, &tile)) {
+  switch (choose_tile(m, KIND, RHS_I4, G, direct, &tile)) {
     case 0:
       *name = "mmt4d_mfma_256x256";
 #ifndef UK_STAGES_256
@@ -1898,6 +1912,27 @@ hipError_t launch_variant(const MfmaArgs& m, hipStream_t stream, const char** na
       *name = "mmt4d_mfma_128x128";
       if (direct) return launch_direct<KIND, RHS_I4, NARROW, G, 2, 2, 4>(m, stream);
       return launch_staged<KIND, RHS_I4, NARROW, G, 2, 2, 2>(m, stream);
+    // (The conditions are choose_tile's: these shapes are not instantiated where it does not take them.)
+    case 6:
+      *name = "mmt4d_mfma_192x192";
+      if constexpr (kWide192 && G != 2 && !RHS_I4) return launch_direct<KIND, RHS_I4, NARROW, G, 3, 3, 4>(m, stream);
+      return hipErrorInvalidValue;
+    case 7:
+      *name = "mmt4d_mfma_128x192";
+      if constexpr (kWide192 && G != 2 && !RHS_I4) return launch_direct<KIND, RHS_I4, NARROW, G, 2, 3, 4>(m, stream);
+      return hipErrorInvalidValue;
+    case 8:
+      *name = "mmt4d_mfma_192x128";
+      if constexpr (kWide192 && G != 2) return launch_direct<KIND, RHS_I4, NARROW, G, 3, 2, 4>(m, stream);
+      return hipErrorInvalidValue;
+    case 9:
+      *name = "mmt4d_mfma_256x192";
+      if constexpr (kWide192 && !RHS_I4) return launch_direct<KIND, RHS_I4, NARROW, G, 4, 3, 4>(m, stream);
+      return hipErrorInvalidValue;
+    case 10:
+      *name = "mmt4d_mfma_192x256";
+      if constexpr (kWide192 && !RHS_I4) return launch_direct<KIND, RHS_I4, NARROW, G, 3, 4, 4>(m, stream);
+      return hipErrorInvalidValue;
     case 5:
       *name = "mmt4d_mfma_64x128";
       if constexpr (RHS_I4) return launch_direct<KIND, RHS_I4, NARROW, G, 1, 2, 8>(m, stream);

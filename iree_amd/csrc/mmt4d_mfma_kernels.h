@@ -1886,6 +1886,18 @@ hipError_t launch_staged(MfmaArgs m, hipStream_t stream) {
   }
 }
 
+// One workgroup per compute unit at most, and operands that do not stay in the last-level cache (256 MiB, shared with what
+// else the program has) from one launch to the next: what the workgroups have in flight then has to cover the latency of
+// HBM, about 2 us under load, and the 24 KiB of either operand that four 128x128 stages hold ahead amount to 2.5 TB/s. Ten
+// stages, all of the LDS, take bf16 160 x 13952 x 4420 (123 MB) from 49.7 to 35.5 us, 160 x 14336 x 3072 (88 MB) from 35.2
+// to 28.4, int8 160 x 14336 x 8192 (117 MB) from 49.7 to 45.4; below 75 MB they cost 2 to 6 % (int8 192 x 14336 x 5000, 72
+// MB: even). Tiles of 64 columns have rings of eight stages and gained nothing from more.
+inline bool streams_operands(const MfmaArgs& m, int block_rows, int block_cols) {
+  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
+  const int64_t tiles = ((rows + block_rows - 1) / block_rows) * ((cols + block_cols - 1) / block_cols);
+  return tiles <= 256 && (rows * m.lhs_rb + cols * m.rhs_rb) * m.K > (75ll << 20);
+}
+
 template <int KIND, bool RHS_I4, int G, bool NARROW>
 hipError_t launch_variant(const MfmaArgs& m, hipStream_t stream, const char** name) {
   const bool direct = direct_covers<RHS_I4, G>(m);
@@ -1910,6 +1922,9 @@ hipError_t launch_variant(const MfmaArgs& m, hipStream_t stream, const char** na
       return launch_direct<KIND, RHS_I4, NARROW, G, 4, 2, 4>(m, stream);
     case 2:
       *name = "mmt4d_mfma_128x128";
+      if constexpr (!RHS_I4 && KIND != kF32) {
+        if (direct && streams_operands(m, 128, 128)) return launch_direct<KIND, RHS_I4, NARROW, G, 2, 2, 10>(m, stream);
+      }
       if (direct) return launch_direct<KIND, RHS_I4, NARROW, G, 2, 2, 4>(m, stream);
       return launch_staged<KIND, RHS_I4, NARROW, G, 2, 2, 2>(m, stream);
     // (The conditions are choose_tile's: these shapes are not instantiated where it does not take them.)

@@ -5,7 +5,7 @@
 // workgroup barrier, about 150 ns a chunk whatever the tile, and a problem with
 // fewer tiles than compute units has nothing to hide that behind. Here a
 // workgroup of 8 wavefronts owns a (16*FA) x (16*FB) tile and every wavefront
-// multiplies the WHOLE tile over its own contiguous share of K: operands go from
+// multiplies the WHOLE tile over its own share of K: operands go from
 // global memory straight to the MFMA's registers, a batch of UNROLL 64-byte
 // steps in flight while the previous batch is multiplied, with no LDS and no
 // barrier until the partial tiles are summed through LDS at the end, in

@@ -3,7 +3,7 @@ that they do not divide and that the choice of tile gives to them, with K from o
 inside one, strided and accumulating.
 
 Integers are compared bit for bit with a float64 product, floats within 1e-3 of max(|ref|, rms(ref)): sums of at most
-260 products of unit-scale values in 32 bits differ by about 1e-6 of that in any order, 16-bit results by one unit in
+3100 products of unit-scale values in 32 bits differ by about 1e-6 of that in any order, 16-bit results by one unit in
 their last place besides.
 """
 import pytest
@@ -34,3 +34,11 @@ def test_ragged(gpu_lib, flags, M0, N0, K0, have):  # noqa: F811
             pad = 32 // e if K % 2 else 0
             run_case(gpu_lib, flags, rows // M0, cols // N0, K, M0, N0, K0, "mmt4d_mfma_" + tile, lhs_pad=pad, rhs_pad=2 * pad,
                      out_pad=4 if n % 2 else 0, offsets=(pad, 2 * pad, 4 if n % 2 else 0), accumulate=K == 4 * whole, seed=n)
+
+
+@pytest.mark.parametrize("flags,M0,N0,K0", [(S8, 8, 8, 4), (BF16, 16, 16, 16), (F16, 16, 16, 1), (abi.MMT4D_TYPE_BF16BF16BF16, 16, 16, 2)])
+def test_deep_ring(gpu_lib, flags, M0, N0, K0):  # noqa: F811
+    # Operands of more than 75 MiB on at most 256 tiles of 128x128: a ring of ten stages. K ends inside a chunk.
+    e = 1 if flags == S8 else 2
+    cols, row_bytes = 14300 // N0, 6000
+    run_case(gpu_lib, flags, 152 // M0, cols, row_bytes // (K0 * e) + 1, M0, N0, K0, "mmt4d_mfma_128x128", accumulate=True, out_pad=4)

@@ -6,6 +6,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 from iree_amd import abi
 from test_gpu_grid import gpu_lib  # noqa: F401
@@ -51,3 +52,15 @@ def test_several_threads(gpu_lib):  # noqa: F811
         jobs = [pool.submit(product, gpu_lib, 64 + i, 60, 256, i % 2 == 1, i) for i in range(9)]
         for job in jobs:
             job.result()
+
+
+def test_upload_behind_other_work(gpu_lib):  # noqa: F811
+    # 6.7 MiB in nine chunks: the ninth reuses the first slot, whose own upload is still queued behind earlier work on the
+    # caller's stream, and has to wait for it.
+    a = torch.ones(8192, 8192, device="cuda")
+    b = torch.empty_like(a)
+    gpu_lib.iree_uk_mi355x_set_stream(torch.cuda.current_stream().cuda_stream, 0)
+    for _ in range(4):
+        torch.mm(a, a, out=b)
+    product(gpu_lib, 100, 121, 1000, False, 5)
+    torch.cuda.synchronize()

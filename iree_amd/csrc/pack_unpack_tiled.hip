@@ -232,12 +232,13 @@ __device__ __forceinline__ v4i32 place_edge_vec(const TiledArgs& a, int64_t row,
   return v;
 }
 
-// A whole vector of the tiled side (pack). (The no-op keeps a vector instruction that overwrites the stored registers one
-// wait state away: the compiler looks after that hazard of wide stores, but not behind inline assembly.)
+// A whole vector of the tiled side (pack). (The no-op keeps a vector instruction that overwrites the stored registers two
+// wait states away, which is what gfx950 needs behind a store of more than 8 bytes: the compiler looks after that hazard,
+// but not behind inline assembly.)
 template <int POLICY>
 __device__ __forceinline__ void store_tiled(uint4 vec, uint8_t* p) {
   const v4i32 v = __builtin_bit_cast(v4i32, vec);
-  if constexpr (POLICY == kKeep) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" : : "v"(p), "v"(v) : "memory");
+  if constexpr (POLICY == kKeep) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
   else __builtin_nontemporal_store(v, (v4i32*)p);
 }
 

@@ -31,7 +31,9 @@
 //
 // Anything this file does not cover (non power-of-two tiles, unaligned tiled
 // buffers) goes to the generic kernels.
+#include <atomic>
 #include <cstdlib>
+#include <mutex>
 #include <type_traits>
 
 #include "uk_internal.h"
@@ -848,24 +850,55 @@ void host_row_col(const TiledArgs& a, int32_t e, int32_t* row, int32_t* col) {
   *col = (o1l << a.log2_t1) + t1;
 }
 
-// What the host searches below find for a block geometry, kept from one call to the next: the searches take
-// microseconds (choose_pitch) to a millisecond, more than the launch. A few entries per thread, the newest one in
-// the place of whichever shared its slot.
+// What the host searches below find for a block geometry.
 struct LdsLayout {
-  uint64_t key = 0;
   int32_t pitch_bytes, log2_lpr, log2_period, pad_bytes;
 };
 
-template <typename Search>
-const LdsLayout& lds_layout(uint64_t key, Search search) {
-  constexpr int kSlots = 64;
-  thread_local LdsLayout known[kSlots];
-  LdsLayout& l = known[(key * 0x9E3779B97F4A7C15ull) >> 58];
-  if (l.key != key) {
-    search(&l);
-    l.key = key;
+// The searches take microseconds (choose_pitch) to a millisecond, more than the launch, so each is made once in a process:
+// geometries are powers of two within a 16 KiB block, fewer than 3000 over all element sizes and transposes, and fit the
+// table (linear probing; should it ever be full, what is not in it is searched for each time). An entry does not change
+// once its key is there, so a call finds its layouts without a lock.
+struct KnownLayouts {
+  static constexpr uint32_t kLog2Entries = 12, kEntries = 1u << kLog2Entries;
+  struct Entry {
+    std::atomic<uint64_t> key;
+    LdsLayout layout;
+  };
+  Entry entries[kEntries];
+  std::mutex writing;
+
+  // The key's entry, or the empty one that is to take it; null if there is neither.
+  Entry* find(uint64_t key, bool* known) {
+    const uint32_t home = (uint32_t)((key * 0x9E3779B97F4A7C15ull) >> (64 - kLog2Entries));
+    for (uint32_t i = 0; i < kEntries; ++i) {
+      Entry& e = entries[(home + i) % kEntries];
+      const uint64_t k = e.key.load(std::memory_order_acquire);
+      *known = k == key;
+      if (*known || k == 0) return &e;
+    }
+    return nullptr;
   }
-  return l;
+  void add(uint64_t key, const LdsLayout& layout) {
+    std::lock_guard<std::mutex> lock(writing);
+    bool known;
+    Entry* e = find(key, &known);
+    if (!e || known) return;
+    e->layout = layout;
+    e->key.store(key, std::memory_order_release);
+  }
+};
+KnownLayouts known_layouts;
+
+template <typename Search>
+LdsLayout lds_layout(uint64_t key, Search search) {
+  bool known;
+  const KnownLayouts::Entry* e = known_layouts.find(key, &known);
+  if (known) return e->layout;
+  LdsLayout found;
+  search(&found);
+  known_layouts.add(key, found);
+  return found;
 }
 
 // Everything that the searches look at; never 0.
@@ -997,7 +1030,7 @@ bool make_plan(const uint8_t* flat, const uint8_t* tiled, int64_t flat_stride0, 
   if (plan->line_aligned) a.ext_cols = (int32_t)(T1 > 128 / E ? T1 : 128 / E);
   if (plan->line_aligned && tr_outer && a.ext_cols * br * E / 16 > 512) plan->line_aligned = false, a.ext_cols = 0;
   a.pitch_bytes = lds_layout(geometry_key(a, E, 0, piece, a.ext_cols), [&](LdsLayout* found) {
-    found->pitch_bytes = choose_pitch(a, E, piece, a.ext_cols);
+    *found = LdsLayout{choose_pitch(a, E, piece, a.ext_cols), 0, 0, 0};
   }).pitch_bytes;
   a.blocks1 = (int32_t)((size1 + bc - 1) / bc);
   // Blocks must cover every tile of the tiled side, not only the 2-D extent
@@ -1046,7 +1079,7 @@ void search_transposing(const TiledArgs* a, int elem_bytes, int rq, LdsLayout* f
   const int cq = 4 / (elem_bytes * rq);
   const int log2_cg = a->log2_bc + (elem_bytes == 2 ? 1 : 0) - 4;
   LdsLayout& best = *found;
-  best.log2_lpr = 0; best.log2_period = 14; best.pad_bytes = 0;
+  best = LdsLayout{0, 0, 14, 0};
   long best_cost = -1;
   TiledArgs t = *a;
   for (t.log2_lpr = log2_cg < 2 ? log2_cg : 2; t.log2_lpr <= log2_cg; ++t.log2_lpr) {
@@ -1085,7 +1118,7 @@ void search_transposing(const TiledArgs* a, int elem_bytes, int rq, LdsLayout* f
 void search_transposing_wide(const TiledArgs* a, int elem_bytes, LdsLayout* found) {
   const int rq = 4 / elem_bytes, ve = 16 / elem_bytes;
   LdsLayout& best = *found;
-  best.log2_lpr = 0; best.log2_period = 14; best.pad_bytes = 0;
+  best = LdsLayout{0, 0, 14, 0};
   long best_cost = -1;
   TiledArgs t = *a;
   for (t.log2_period = 6; t.log2_period <= 14; ++t.log2_period) {
@@ -1116,7 +1149,7 @@ void search_transposing_wide(const TiledArgs* a, int elem_bytes, LdsLayout* foun
 
 // `rq`: rows per dword of pack_transposing_kernel; 0: pack_transposing_wide_kernel.
 void choose_transposing(TiledArgs* a, int elem_bytes, int rq) {
-  const LdsLayout& l = lds_layout(geometry_key(*a, elem_bytes, 1 + rq, 0, 0), [&](LdsLayout* found) {
+  const LdsLayout l = lds_layout(geometry_key(*a, elem_bytes, 1 + rq, 0, 0), [&](LdsLayout* found) {
     if (rq) search_transposing(a, elem_bytes, rq, found); else search_transposing_wide(a, elem_bytes, found);
   });
   a->log2_lpr = l.log2_lpr; a->log2_period = l.log2_period; a->pad_bytes = l.pad_bytes;

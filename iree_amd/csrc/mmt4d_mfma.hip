@@ -22,23 +22,29 @@ struct Plan {
   MfmaArgs args;
 };
 
-// Estimates in microseconds, fitted to a sweep of M 16..1024 x N 256..16384 x K 256..8192 for every type and row piece
-// (weights that the last-level cache holds, one launch after another): the kernel that they pick is within 2 % of the
-// faster one in the mean. Both write the output at the same rate, which is left out.
+// Estimates in microseconds, to choose between the block kernels and the one that splits K over wavefronts. Both write
+// the output at the same rate, which is left out. Measured over 1094 problems (M 24..512, N 512..28672, K 1024..14336,
+// every type and row piece) with operands from HBM (sets of 640 MB in turn, the condition of weights in a model's layers)
+// and with operands that the last-level cache holds (150 MB), the coefficients fitted to the geometric mean of the two: the
+// kernel picked is 0.3 % slower than the best one in the mean, 5 % and more on 24 problems. Fitted to repeated operands
+// alone they had picked 32x64 tiles for bf16 96 x 14336 x 4096: 27.5 us held and 40.6 from HBM, where the 128x64 tile with
+// K split takes 23.9 and 32.6; int4 96 x 14336 x 4096 19.1 from HBM against 16.3.
 //
-// A block kernel takes a fixed time per 64-byte chunk of K, whatever the number of tiles up to one per compute unit.
+// A block kernel takes a fixed time per 64-byte chunk of K (choose_tile), or what its operands take from memory.
 double block_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
   const bool direct = mfma_direct_covers(m, gather, rhs_i4);
-  if (gather == 16 && (kind == kF16 || kind == kBF16) && direct && split_k_covers(m)) return 4.5 + 0.235 * m.chunks;
-  const TileChoice* t;
-  choose_tile(m, kind, rhs_i4, gather, direct, &t);
   const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
-  const int64_t tiles = ((rows + 64 * t->am - 1) / (64 * t->am)) * ((cols + 64 * t->bn - 1) / (64 * t->bn));
-  double per_chunk = t->us_per_chunk;
-  if (kind == kF32) per_chunk *= 2.3;                                   // bound by the matrix pipe
-  if (gather == 2) per_chunk *= t->am * t->bn == 1 ? 2.1 : 1.55;        // 2-byte pieces: more LDS reads per step
-  if (!direct) per_chunk *= 2.2;                                        // staged through registers
-  return 3.2 + (double)((tiles + 255) / 256) * m.chunks * per_chunk;
+  const double memory_us = (double)(rows * m.lhs_rb + cols * m.rhs_rb) * m.K / 6.0e6;
+  double us_per_chunk, start_us = 3.0;
+  if (gather == 16 && (kind == kF16 || kind == kBF16) && direct && split_k_covers(m)) {
+    us_per_chunk = 0.153;
+    start_us = 6.2;  // (and the summing of the partial tiles)
+  } else {
+    choose_tile(m, kind, rhs_i4, gather, direct, &us_per_chunk);
+    if (!direct) us_per_chunk *= 2.2;  // staged through registers
+  }
+  const double chunks_us = m.chunks * us_per_chunk;
+  return start_us + (chunks_us > memory_us ? chunks_us : memory_us);
 }
 
 // The kernel that splits K over wavefronts is bound by the bytes a workgroup loads; workgroups beyond one per compute
@@ -47,13 +53,13 @@ double wave_k_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather, const W
   const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
   const int64_t tiles = ((rows + 16 * s.fa - 1) / (16 * s.fa)) * ((cols + 16 * s.fb - 1) / (16 * s.fb));
   const double row_kb = 1e-3 * m.K * m.lhs_rb, rhs_share = rhs_i4 ? 0.5 : 1.0;
-  double tile_us = 16 * (s.fa + s.fb * rhs_share) * row_kb / (gather < 16 ? 75 : 115);
-  if (kind == kF32) tile_us = tile_us > 0.0234 * s.fa * s.fb * m.chunks ? tile_us : 0.0234 * s.fa * s.fb * m.chunks;
-  double us = (gather < 16 || rhs_i4 ? 3.1 : 2.8) + 0.04 * s.fa * s.fb + 5e-5 * (rows + cols * rhs_share) * row_kb;
+  double tile_us = 16 * (s.fa + s.fb * rhs_share) * row_kb / (gather < 16 ? 72 : 110);
+  if (kind == kF32) tile_us = tile_us > 0.024 * s.fa * s.fb * m.chunks ? tile_us : 0.024 * s.fa * s.fb * m.chunks;
+  double us = (gather < 16 || rhs_i4 ? 3.1 : 2.5) + 0.04 * s.fa * s.fb + 4.75e-5 * (rows + cols * rhs_share) * row_kb;
   if (tiles <= 256) return us + tile_us;
   const double rounds = tiles / 256.0;
   if (tiles > (s.fa * s.fb >= 16 ? 256 : 1024)) us += 1e3 * rounds;
-  return us + (rounds + 0.8) * tile_us + 0.6 * rounds;
+  return us + (rounds + 0.7) * tile_us + 0.66 * rounds;
 }
 
 // Whether the kernel that splits K over wavefronts covers the problem: 16-byte aligned operands whose 16 contiguous
@@ -181,8 +187,8 @@ const char* class_name(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
                                        "mmt4d_mfma_128x64",  "mmt4d_mfma_64x64",   "mmt4d_mfma_64x128",
                                        "mmt4d_mfma_192x192", "mmt4d_mfma_128x192", "mmt4d_mfma_192x128",
                                        "mmt4d_mfma_256x192", "mmt4d_mfma_192x256"};
-  const TileChoice* tile;
-  return kNames[choose_tile(m, kind, rhs_i4, gather, direct, &tile)];
+  double us_per_chunk;
+  return kNames[choose_tile(m, kind, rhs_i4, gather, direct, &us_per_chunk)];
 }
 
 hipError_t launch_wave_k(const Plan& plan, hipStream_t stream, const char** name) {

@@ -100,8 +100,7 @@ hipError_t launch_wave_k_bf16_narrow(const MfmaArgs& m, int gather, int shape, b
 // 516 tiles of 128x128 for 256 compute units: 56 us, and 228 of 192x192: 39 us).
 struct TileChoice {
   int am, bn;
-  bool direct_only;    // no register-staged instantiation of this shape
-  float us_per_chunk;  // one workgroup per compute unit, 64 bytes of K per row (bf16 and int8): see block_cost
+  bool direct_only;  // no register-staged instantiation of this shape
 };
 
 // The 128x64 tile with K split over its wavefronts (mmt4d_mfma_split_k_kernel): 65 to 128 lhs rows, one row of tiles.
@@ -122,10 +121,10 @@ inline bool split_k_covers(const MfmaArgs& m) {
 // mean than the best one; without the 192-wide ones and one efficiency per tile it was 4 to 7 %. f32 is bound by the
 // matrix pipe whatever the tile, which leaves the number of rounds (in units of a 128x128 tile; the large tiles, which
 // move fewer bytes, are favoured by 10 %).
-inline int choose_tile(const MfmaArgs& m, int kind, bool rhs_i4, int gather, bool direct, const TileChoice** chosen) {
-  static const TileChoice kTiles[] = {{4, 4, false, 0.50f}, {4, 2, true, 0.31f},  {2, 2, false, 0.25f}, {2, 1, true, 0.168f},
-                                      {1, 1, false, 0.122f}, {1, 2, true, 0.19f}, {3, 3, true, 0.34f},  {2, 3, true, 0.25f},
-                                      {3, 2, true, 0.25f},   {4, 3, true, 0.40f}, {3, 4, true, 0.40f}};
+// `us_per_chunk`: that least time.
+inline int choose_tile(const MfmaArgs& m, int kind, bool rhs_i4, int gather, bool direct, double* us_per_chunk) {
+  static const TileChoice kTiles[] = {{4, 4, false}, {4, 2, true}, {2, 2, false}, {2, 1, true}, {1, 1, false}, {1, 2, true},
+                                      {3, 3, true},  {2, 3, true}, {3, 2, true},  {4, 3, true}, {3, 4, true}};
   constexpr int kCount = sizeof kTiles / sizeof kTiles[0];
   // Per class of operands and tile, 0: no such instantiation.
   enum { kSixteenBit, kInt8, kTwoBytePieces, kInt4, kFloat32 };
@@ -156,7 +155,7 @@ inline int choose_tile(const MfmaArgs& m, int kind, bool rhs_i4, int gather, boo
       best_cost = cost;
     }
   }
-  *chosen = &kTiles[best];
+  *us_per_chunk = best_cost;
   return best;
 }
 
@@ -1908,8 +1907,8 @@ hipError_t launch_variant(const MfmaArgs& m, hipStream_t stream, const char** na
     }
   }
   constexpr bool kWide192 = KIND != kF32 && G != 1;
-  const TileChoice* tile;
-  switch (choose_tile(m, KIND, RHS_I4, G, direct, &tile)) {
+  double us_per_chunk;
+  switch (choose_tile(m, KIND, RHS_I4, G, direct, &us_per_chunk)) {
     case 0:
       *name = "mmt4d_mfma_256x256";
 #ifndef UK_STAGES_256

@@ -567,13 +567,8 @@ int compute_units() {
   return cached[device];
 }
 
-// Whether the rhs is streamed past the caches. Weights of more than 64 MiB are: the last-level cache (256 MiB, shared
-// with whatever else the program keeps) is not likely to hold them from one call to the next. Smaller int4 ones are not
-// (1 x 11008 x 4096, 22 MB: 5.98 -> 5.59 us, 14336 x 8192 12.5 -> 11.4). Types of a byte or more from 24 MiB on are
-// (8192 x 2048 bf16 6.9 us streamed, 7.1 not), below they are not (512 x 8192 bf16 8.5 -> 5.7 us).
-bool streamed_rhs(const GemvArgs& g, int rhs_rb, bool i4) {
-  return (int64_t)g.N * g.K * rhs_rb * 16 > ((i4 ? 64ll : 24ll) << 20);
-}
+// Whether the rhs is streamed past the caches.
+bool streamed_rhs(const GemvArgs& g, int rhs_rb) { return comes_from_hbm((int64_t)g.N * g.K * rhs_rb * 16); }
 
 // The resident-lhs kernel, if it fits: more than 4 lhs rows, K in whole 64-byte
 // steps whose number is what one of the instantiations splits over its
@@ -617,7 +612,7 @@ hipError_t launch_kind(const GemvArgs& g, hipStream_t stream, const char** name)
   }
   // One rhs tile per workgroup (most workgroups, best balance over the CUs),
   // 4 wavefronts splitting K, 16 KiB of rhs in flight per wavefront.
-  return launch_kernel<GemvArgs>(streamed_rhs(g, g.rb, false) ? mmt4d_gemv_kernel<KIND, 1, 16, 4, true>
+  return launch_kernel<GemvArgs>(streamed_rhs(g, g.rb) ? mmt4d_gemv_kernel<KIND, 1, 16, 4, true>
                                                               : mmt4d_gemv_kernel<KIND, 1, 16, 4, false>, g.N, 256, 0, stream, g);
 }
 
@@ -632,7 +627,7 @@ hipError_t launch_gemv(const Mmt4dArgs& a, hipStream_t stream, const char** name
     // 0.51 against 0.48): the resident-lhs kernel, where its instantiations fit the number of steps (each of 128
     // values of K; the lhs of 64 steps fills 128 KiB of LDS).
     const int units = compute_units();
-    const bool streamed = streamed_rhs(g, g.rb / 2, true);
+    const bool streamed = streamed_rhs(g, g.rb / 2);
     constexpr int MAX_TILES = 8;
     if (((g.M << g.log2_M0) > 4 || g.N >= 6 * (int64_t)units) && units > 0 && g.N >= units && (2 * (int64_t)g.N + units - 1) / units / 2 + 1 <= MAX_TILES &&
         (g.steps == 64 || g.steps == 32)) {

@@ -195,11 +195,11 @@ hipError_t launch_wave_k(const Plan& plan, hipStream_t stream, const char** name
   const MfmaArgs& m = plan.args;
   const WaveKShape& shape = kWaveKShapes[plan.wave_shape];
   *name = class_name(m, plan.kind, plan.rhs_i4, plan.gather);
-  // Weights that one row of tiles reads once and the last-level cache (256 MiB, shared with whatever else the program
-  // keeps) is not likely to hold from one call to the next are streamed past the caches: bf16 64 x 14336 x 4096 (117
-  // MB) 27.9 -> 24.8 us. Smaller ones must not be: 64 x 4096 x 4096 (34 MB) 9.0 -> 12.1 us.
+  // Weights that one row of tiles reads once are streamed past the caches like those of a matrix-vector product: bf16 64 x
+  // 14336 x 4096 (117 MB) from HBM 28.1 -> 24.7 us, read again or just written 20.2 -> 24.3. With several rows of tiles
+  // the caches serve the others: streamed 3 to 20 % slower from HBM too.
   const bool streamed = ((int64_t)m.M << m.log2_M0) <= 16 * shape.fa &&
-                        (((int64_t)m.N * m.K * m.rhs_rb) << m.log2_N0) > (64ll << 20);
+                        comes_from_hbm(((int64_t)m.N * m.K * m.rhs_rb) << m.log2_N0);
   switch (plan.kind) {
     case kI8: return launch_wave_k_i8(m, plan.gather, plan.rhs_i4, plan.wave_shape, streamed, stream);
     case kF16:

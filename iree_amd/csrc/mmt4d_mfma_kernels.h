@@ -1885,16 +1885,16 @@ hipError_t launch_staged(MfmaArgs m, hipStream_t stream) {
   }
 }
 
-// One workgroup per compute unit at most, and operands that do not stay in the last-level cache (256 MiB, shared with what
-// else the program has) from one launch to the next: what the workgroups have in flight then has to cover the latency of
-// HBM, about 2 us under load, and the 24 KiB of either operand that four 128x128 stages hold ahead amount to 2.5 TB/s. Ten
-// stages, all of the LDS, take bf16 160 x 13952 x 4420 (123 MB) from 49.7 to 35.5 us, 160 x 14336 x 3072 (88 MB) from 35.2
-// to 28.4, int8 160 x 14336 x 8192 (117 MB) from 49.7 to 45.4; below 75 MB they cost 2 to 6 % (int8 192 x 14336 x 5000, 72
-// MB: even). Tiles of 64 columns have rings of eight stages and gained nothing from more.
+// One workgroup per compute unit at most, and operands from HBM: what the workgroups have in flight then has to cover its
+// latency, about 2 us under load, and the 24 KiB of either operand that four 128x128 stages hold ahead amount to 2.5 TB/s.
+// Ten stages, all of the LDS, take from HBM bf16 512 x 5120 x 5120 (58 MB) from 56.7 to 48.4 us, 384 x 8192 x 4096 (70 MB)
+// from 48.2 to 41.5, int8 192 x 14336 x 4096 (59 MB) from 28.3 to 25.7; with operands that a cache holds they cost nothing
+// there (0.95 to 1.02, 2-byte pieces 1.02 to 1.06), below 48 MiB up to 10 %. Tiles of 64 columns have rings of eight
+// stages and gained nothing from more.
 inline bool streams_operands(const MfmaArgs& m, int block_rows, int block_cols) {
   const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
   const int64_t tiles = ((rows + block_rows - 1) / block_rows) * ((cols + block_cols - 1) / block_cols);
-  return tiles <= 256 && (rows * m.lhs_rb + cols * m.rhs_rb) * m.K > (75ll << 20);
+  return tiles <= 256 && comes_from_hbm((rows * m.lhs_rb + cols * m.rhs_rb) * m.K);
 }
 
 template <int KIND, bool RHS_I4, int G, bool NARROW>

@@ -466,12 +466,16 @@ hipError_t launch_slabs(const SkinnyArgs& all_rows, hipStream_t stream) {
 
 template <int KIND, int G, bool NARROW>
 hipError_t launch_piece(const SkinnyArgs& s, hipStream_t stream) {
-  // Weights that the last-level cache (256 MiB) will not hold to the next call are streamed past the caches (1 x 14336 x
-  // 4096 bf16, 112 MiB: 19.4 us, through them 21.3); smaller ones are not (512 x 12288 f16 11.9 -> 9.8 us).
-  if (s.tile_bytes * s.N > (96ll << 20)) return launch_slabs<KIND, G, 4, true, NARROW>(s, stream);
+  const int64_t bytes = s.tile_bytes * s.N;
   // No more tile rows than compute units, and long ones: eight wavefronts (4 x 512 x 8192 bf16 14.4 -> 10.3 us, 1 x 512 x
-  // 4096 5.0 -> 3.9). With shorter ones, or several to a unit, the summing at the end costs more than it gives.
+  // 4096 5.0 -> 3.9; against four that stream, 4 x 4096 x 14336 int8 22.5 -> 14.3 with its 59 MB held, 22.4 -> 18.8 from
+  // HBM). With shorter ones, or several to a unit, the summing at the end costs more than it gives.
   if (s.N <= 256 && s.tile_bytes >= 128 * 1024) return launch_slabs<KIND, G, 8, false, NARROW>(s, stream);
+  // One byte or less per rhs element against more than two rows is bound by the vector ALU, which streaming does not help:
+  // 4 x 14336 x 4096 int8 17.6 us, streamed 20.6, from HBM 20.9 both; only beyond what the caches can hold it does (235
+  // MB: 60.8 -> 56.8).
+  const bool alu_bound = (KIND == kI8 || KIND == kI8I4 || KIND == kI16U4 || KIND == kI16I8) && s.rows > 2;
+  if (alu_bound ? bytes > (128ll << 20) : comes_from_hbm(bytes)) return launch_slabs<KIND, G, 4, true, NARROW>(s, stream);
   return launch_slabs<KIND, G, 4, false, NARROW>(s, stream);
 }
 

@@ -57,6 +57,17 @@ hipError_t launch_kernel(void (*kernel)(const Args), unsigned grid, unsigned blo
   return hipLaunchKernel((const void*)kernel, dim3(grid), dim3(block), args, lds_bytes, stream);
 }
 
+// Whether operands of that many bytes, which a call reads once, are taken to come from HBM: the matrix-vector kernels then
+// read the rhs past the caches (non-temporal loads), the block kernels have more of it in flight. The caches do not say
+// what they will hold: the L2s (32 MiB) whatever a program has just used, the last-level cache (256 MiB) what it used
+// since. Measured streamed / through the caches for 1 to 16 rows, the same weights in every call, weights of 150 MB in
+// turn, and of 640 MB in turn (a model's layers):
+//   23 to 50 MB: 1.2 to 1.5, 1.03 to 1.15, 0.92 to 0.99;   52 to 135 MB: 0.95 to 1.1, 1.03 to 1.12, 0.86 to 0.95;
+//   from 235 MB on: 0.9 to 1.07, 0.87 to 0.93, 0.87 to 0.93.
+// Up to 48 MiB the caches give more than they cost, from there on as much as they cost, and streamed weights leave what
+// else the program keeps in them alone.
+inline bool comes_from_hbm(int64_t bytes) { return bytes > (48ll << 20); }
+
 // A launcher enqueues one operation on `stream` and returns the HIP status of
 // the launch. `name` receives a static string naming the kernel variant.
 typedef hipError_t (*Mmt4dLauncher)(const Mmt4dArgs& a, hipStream_t stream, const char** name);

@@ -38,7 +38,7 @@ def test_ragged(gpu_lib, flags, M0, N0, K0, have):  # noqa: F811
 
 @pytest.mark.parametrize("flags,M0,N0,K0", [(S8, 8, 8, 4), (BF16, 16, 16, 16), (F16, 16, 16, 1), (abi.MMT4D_TYPE_BF16BF16BF16, 16, 16, 2)])
 def test_deep_ring(gpu_lib, flags, M0, N0, K0):  # noqa: F811
-    # Operands of more than 75 MiB on at most 256 tiles of 128x128: a ring of ten stages. K ends inside a chunk.
+    # Operands of more than 48 MiB on at most 256 tiles of 128x128: a ring of ten stages. K ends inside a chunk.
     e = 1 if flags == S8 else 2
     cols, row_bytes = 14300 // N0, 6000
     run_case(gpu_lib, flags, 152 // M0, cols, row_bytes // (K0 * e) + 1, M0, N0, K0, "mmt4d_mfma_128x128", accumulate=True, out_pad=4)

@@ -51,3 +51,41 @@ def test_the_kernel_picked_is_among_the_best(recorder, layout, m, n, k, times): 
     assert picked in times, mangled
     mean = {name: math.sqrt(held * hbm) for name, (held, hbm) in times.items()}
     assert mean[picked] <= 1.08 * min(mean.values()), (picked, mean)
+
+
+def streams(mangled):
+    """Whether a matrix-vector kernel, or the one that splits K over wavefronts, reads the rhs past the caches."""
+    m = (re.search(r"mmt4d_gemv_kernelILi\dELi\d+ELi\d+ELi\d+ELb(\d)E", mangled) or
+         re.search(r"mmt4d_gemv_i4_kernelILi\d+ELi\d+ELi\d+ELb(\d)E", mangled) or
+         re.search(r"mmt4d_skinny_kernelILi\dELi\dELi\dELi\dELi\d+ELb(\d)ELb\dE", mangled) or
+         re.search(r"mmt4d_wave_k_kernelILi\dELb\dELb\dELi16ELi\dELi\dELi\dELi\dELb(\d)E", mangled))
+    assert m, mangled
+    return m[1] == "1"
+
+
+# Weights are taken to come from HBM above 48 MiB, whichever kernel reads them.
+@pytest.mark.parametrize("flags,M,M0,N0,K0,n,k,bits", [
+    (abi.MMT4D_TYPE_BF16BF16F32, 1, 1, 16, 8, 6144, 4096, 16), (abi.MMT4D_TYPE_S8S8S32, 1, 1, 16, 64, 12288, 4096, 8),
+    (abi.MMT4D_TYPE_S8S4S32, 1, 4, 16, 32, 12288, 8192, 4), (abi.MMT4D_TYPE_S8S8S32, 1, 1, 16, 2, 12288, 4096, 8),
+    (abi.MMT4D_TYPE_BF16BF16F32, 1, 4, 16, 2, 6144, 4096, 16), (abi.MMT4D_TYPE_F32F32F32, 1, 2, 16, 1, 6144, 2048, 32),
+    (abi.MMT4D_TYPE_BF16BF16F32, 2, 16, 16, 16, 6144, 4096, 16), (abi.MMT4D_TYPE_S8S4S32, 2, 16, 16, 32, 24576, 4096, 4)])
+def test_one_rule_for_weights_from_hbm(recorder, flags, M, M0, N0, K0, n, k, bits):  # noqa: F811
+    assert n * k * bits // 8 <= 48 << 20
+    assert not streams(recorder.mmt4d(flags, M, n // N0, k // K0, M0, N0, K0)[0])
+    n += n // 16
+    assert n * k * bits // 8 > 48 << 20
+    assert streams(recorder.mmt4d(flags, M, n // N0, k // K0, M0, N0, K0)[0])
+
+
+def test_narrow_tiles_bound_by_the_vector_alu_stream_only_what_no_cache_holds(recorder):  # noqa: F811
+    s8 = abi.MMT4D_TYPE_S8S8S32
+    assert not streams(recorder.mmt4d(s8, 1, 14336 // 16, 4096 // 2, 4, 16, 2)[0])
+    assert streams(recorder.mmt4d(s8, 1, 28672 // 16, 8192 // 2, 4, 16, 2)[0])
+    # No more tile rows than compute units: eight wavefronts a tile row, through the caches.
+    assert "ELi8ELi8ELb0E" in recorder.mmt4d(s8, 1, 4096 // 16, 14336 // 2, 2, 16, 2)[0]
+
+
+def test_block_kernels_have_the_deep_ring_for_operands_from_hbm(recorder):  # noqa: F811
+    bf16 = abi.MMT4D_TYPE_BF16BF16F32
+    for n, stages in ((11264, 4), (13312, 10)):  # 46 and 54 MiB with 192 rows
+        assert "ELi2ELi2ELi%dE" % stages in recorder.mmt4d(bf16, 12, n // 16, 2048 // 16, 16, 16, 16)[0]

@@ -171,30 +171,10 @@ bool make_plan(const Mmt4dArgs& a, bool probe_only, Plan* plan) {
   return true;
 }
 
-// What iree_uk_mi355x_last_kernel reports for a problem that is worked off by the kernel that splits K over wavefronts:
-// names go by the problem's class (the block tile that its size calls for, or few of them against a long K), not by the
-// tile of that kernel, so that a caller that watches the names is not told of a different class after every retuning.
-const char* class_name(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
-  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
-  const int64_t row_bytes = (int64_t)m.K * m.lhs_rb;
-  const bool direct = mfma_direct_covers(m, gather, rhs_i4);
-  if (direct && gather == 16 && !rhs_i4 && kind != kF32) {
-    if (((rows + 63) / 64) * ((cols + 63) / 64) <= 128 && row_bytes % 256 == 0 && row_bytes >= 4096)
-      return "mmt4d_mfma_64x64_split_k";
-    if (kind != kI8 && split_k_covers(m)) return "mmt4d_mfma_128x64_split_k";
-  }
-  static const char* const kNames[] = {"mmt4d_mfma_256x256", "mmt4d_mfma_256x128", "mmt4d_mfma_128x128",
-                                       "mmt4d_mfma_128x64",  "mmt4d_mfma_64x64",   "mmt4d_mfma_64x128",
-                                       "mmt4d_mfma_192x192", "mmt4d_mfma_128x192", "mmt4d_mfma_192x128",
-                                       "mmt4d_mfma_256x192", "mmt4d_mfma_192x256"};
-  double us_per_chunk;
-  return kNames[choose_tile(m, kind, rhs_i4, gather, direct, &us_per_chunk)];
-}
-
 hipError_t launch_wave_k(const Plan& plan, hipStream_t stream, const char** name) {
   const MfmaArgs& m = plan.args;
   const WaveKShape& shape = kWaveKShapes[plan.wave_shape];
-  *name = class_name(m, plan.kind, plan.rhs_i4, plan.gather);
+  *name = shape.name;
   // Weights that one row of tiles reads once are streamed past the caches like those of a matrix-vector product: bf16 64 x
   // 14336 x 4096 (117 MB) from HBM 28.1 -> 24.7 us, read again or just written 20.2 -> 24.3. With several rows of tiles
   // the caches serve the others: streamed 3 to 20 % slower from HBM too.

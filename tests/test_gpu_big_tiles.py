@@ -9,6 +9,7 @@ same operands (every value is far below 2^53, so that product is exact); float
 results within |got - ref| <= 1e-3 * max(|ref|, rms(ref)) of it.
 """
 import ctypes as C
+import fnmatch
 
 import numpy as np
 import pytest
@@ -18,6 +19,12 @@ from iree_amd import abi
 from test_gpu_configs import REL_TOL, gpu_lib, mm_params  # noqa: F401
 
 pytestmark = pytest.mark.gpu
+
+
+# The block tile of a few dozen rows against very many columns, without and with 2-byte row pieces; bytes of an operand
+# element where they are not 2.
+SMALLEST = ("mmt4d_mfma_64x64", "mmt4d_mfma_128x128")
+BYTES = {abi.MMT4D_TYPE_S8S8S32: 1, abi.MMT4D_TYPE_F32F32F32: 4}
 
 
 def logical(t, outer, K, T0, K0):
@@ -64,7 +71,8 @@ def run_case(gpu_lib, flags, M, N, K, M0, N0, K0, expect_kernel, lhs_pad=0, rhs_
                   flags | (abi.MMT4D_ACCUMULATE if accumulate else 0), lhs_off=lo, rhs_off=ro, out_off=oo,
                   lhs_stride=lhs_stride, rhs_stride=rhs_stride, out_stride=out_stride)
     gpu_lib.iree_uk_mmt4d_p(C.byref(p))
-    assert gpu_lib.iree_uk_mi355x_last_kernel() == expect_kernel.encode()
+    kernel = gpu_lib.iree_uk_mi355x_last_kernel().decode()
+    assert fnmatch.fnmatchcase(kernel, expect_kernel), (kernel, expect_kernel)
 
     def rows_of(buf, off, n_tiles, stride, width):
         return buf[off:off + n_tiles * stride].view(n_tiles, stride)[:, :width]
@@ -134,7 +142,7 @@ def test_float_types_ragged_256(gpu_lib, flags, M0, N0, K0, K):
 
 @pytest.mark.parametrize("M,N,expect,expect_staged", [(226, 232, "mmt4d_mfma_256x256", "mmt4d_mfma_256x256"),
                                                       (100, 119, "mmt4d_mfma_128x128", "mmt4d_mfma_128x128"),
-                                                      (9, 11, "mmt4d_mfma_64x128", "mmt4d_mfma_64x64")])
+                                                      (9, 11, "mmt4d_mfma_wave_k_16x16", "mmt4d_mfma_64x64")])
 def test_s8s4s32_ragged(gpu_lib, M, N, expect, expect_staged):
     run_case(gpu_lib, abi.MMT4D_TYPE_S8S4S32, M, N, 6, 16, 16, 32, expect, accumulate=True, rhs_pad=64, offsets=(16, 64, 4), seed=M)
     # 8-byte rhs pieces: the register-staged kernel, which has a 64x64 tile.
@@ -163,8 +171,11 @@ def test_narrow_and_8_byte_row_pieces(gpu_lib, flags, M0, N0, K0, K):
     # 256x256 blocks, ragged in both directions, accumulating, padded output rows
     M, N = 3608 // M0 + 1, 3704 // N0 + 1
     run_case(gpu_lib, flags, M, N, K, M0, N0, K0, "mmt4d_mfma_256x256", accumulate=True, out_pad=16, seed=K0 + K)
-    # the smallest block tile, strided operands with offsets (all multiples of 16 bytes)
-    run_case(gpu_lib, flags, 72 // M0, 88 // N0, K, M0, N0, K0, "mmt4d_mfma_64x64", lhs_pad=32, rhs_pad=16,
+    # few tiles (K split over wavefronts) and the smallest block tile (pieces of 2 bytes: 128x128), strided operands with
+    # offsets (all multiples of 16 bytes)
+    few = "mmt4d_mfma_64x64" if K * K0 == 64 and flags == abi.MMT4D_TYPE_S8S8S32 else "mmt4d_mfma_wave_k_16x16"  # (one chunk)
+    run_case(gpu_lib, flags, 72 // M0, 88 // N0, K, M0, N0, K0, few, lhs_pad=32, rhs_pad=16, offsets=(16, 32, 4), seed=K0)
+    run_case(gpu_lib, flags, 40 // M0, 27992 // N0, K, M0, N0, K0, SMALLEST[K0 * BYTES.get(flags, 2) == 2], lhs_pad=32, rhs_pad=16,
              offsets=(16, 32, 4), seed=K0)
 
 
@@ -187,7 +198,7 @@ def test_narrow_row_pieces_fall_back_when_the_direct_kernel_cannot_run(gpu_lib):
     # Less than one 64-byte chunk of K, or rows not 16-byte aligned: the skinny kernel's 8-row slabs, still exact.
     run_case(gpu_lib, abi.MMT4D_TYPE_S8S8S32, 9, 11, 31, 16, 16, 2, "mmt4d_skinny", accumulate=True)
     run_case(gpu_lib, abi.MMT4D_TYPE_S8S8S32, 9, 11, 32, 16, 16, 2, "mmt4d_skinny", lhs_pad=4)
-    run_case(gpu_lib, abi.MMT4D_TYPE_S8S8S32, 9, 11, 33, 16, 16, 2, "mmt4d_mfma_64x64", accumulate=True)
+    run_case(gpu_lib, abi.MMT4D_TYPE_S8S8S32, 9, 11, 33, 16, 16, 2, "mmt4d_mfma_wave_k_16x16", accumulate=True)
 
 
 # K ending inside a 64-byte chunk on the direct-to-LDS kernel: the last chunk overlaps the one before it and the
@@ -214,13 +225,18 @@ def test_direct_kernel_with_K_ending_inside_a_chunk(gpu_lib, flags, M0, N0, K0, 
             run_case(gpu_lib, flags, 120 // M0, n_cols // N0, K, M0, N0, K0, "mmt4d_mfma_128x64", accumulate=True, seed=K)
         else:
             run_case(gpu_lib, flags, 1608 // M0, 1912 // N0, K, M0, N0, K0, "mmt4d_mfma_128x128", seed=K)
-        run_case(gpu_lib, flags, 72 // M0, 88 // N0, K, M0, N0, K0, "mmt4d_mfma_64x64", accumulate=True, seed=K + 100)
+        run_case(gpu_lib, flags, 72 // M0, 88 // N0, K, M0, N0, K0, "mmt4d_mfma_wave_k_16x16", accumulate=True, seed=K + 100)
+        if n < 2:
+            run_case(gpu_lib, flags, 40 // M0, 27992 // N0, K, M0, N0, K0, SMALLEST[K0 * BYTES.get(flags, 2) == 2], accumulate=True,
+                     seed=K + 200)
 
 
-def test_K_tail_overlap_is_zeroed_in_both_operands(gpu_lib):
-    # The chunk that K ends in is loaded overlapping the one before it. An infinity inside the overlap must count
-    # once: were only one operand zeroed there, inf * 0 would turn the outputs into NaN.
-    M, N, K, M0, N0, K0 = 5, 6, 5, 16, 16, 16      # 32-byte row pieces: chunks [k0,k1], [k2,k3], tail k4 -> the last chunk is [k3,k4]
+@pytest.mark.parametrize("M,N,kernel", [(5, 6, b"mmt4d_mfma_wave_k_16x16"), (3, 1000, b"mmt4d_mfma_64x64")])
+def test_K_tail_overlap_is_zeroed_in_both_operands(gpu_lib, M, N, kernel):
+    # A block kernel loads the chunk that K ends in overlapping the one before it. An infinity inside the overlap must
+    # count once: were only one operand zeroed there, inf * 0 would turn the outputs into NaN. (The kernel that splits K
+    # over wavefronts zeroes what lies beyond K instead.)
+    K, M0, N0, K0 = 5, 16, 16, 16      # 32-byte row pieces: chunks [k0,k1], [k2,k3], tail k4 -> the last chunk is [k3,k4]
     g = torch.Generator(device="cuda").manual_seed(1)
     lhs = (torch.rand(M * K * M0 * K0, device="cuda", generator=g) + 0.5).to(torch.float16)
     rhs = (torch.rand(N * K * N0 * K0, device="cuda", generator=g) + 0.5).to(torch.float16)
@@ -229,7 +245,7 @@ def test_K_tail_overlap_is_zeroed_in_both_operands(gpu_lib):
     out = torch.zeros(M * N * M0 * N0, device="cuda")
     p = mm_params(lhs.data_ptr(), rhs.data_ptr(), out.data_ptr(), M, N, K, M0, N0, K0, abi.MMT4D_TYPE_F16F16F32)
     gpu_lib.iree_uk_mmt4d_p(C.byref(p))
-    assert gpu_lib.iree_uk_mi355x_last_kernel() == b"mmt4d_mfma_64x64"
+    assert gpu_lib.iree_uk_mi355x_last_kernel() == kernel
     got = out.view(M, N, M0, N0).permute(0, 2, 1, 3).reshape(M * M0, N * N0)
     assert not bool(torch.isnan(got).any())
     inf = torch.isinf(got)
@@ -242,8 +258,8 @@ def test_K_tail_overlap_is_zeroed_in_both_operands(gpu_lib):
     assert bool(((finite.double() - ref).abs() <= REL_TOL * ref.abs()).all())
 
 
-# Few block tiles against a long K: the 64x64 tile whose wavefronts split K (256 bytes of K per row and step) and sum
-# their partial tiles at the end. Even and odd numbers of steps, ragged tiles, one tile only, accumulation, strides.
+# Few block tiles against a long K: the tiles whose wavefronts split K and sum their partial tiles at the end. Even and odd
+# numbers of batches, ragged tiles, one tile only, accumulation, strides.
 @pytest.mark.parametrize("flags,M0,N0,K0", [(abi.MMT4D_TYPE_S8S8S32, 16, 16, 64), (abi.MMT4D_TYPE_S8S8S32, 8, 8, 16),
                                             (abi.MMT4D_TYPE_S8S8S32, 4, 16, 32), (abi.MMT4D_TYPE_F16F16F32, 16, 16, 16),
                                             (abi.MMT4D_TYPE_BF16BF16F32, 16, 16, 8), (abi.MMT4D_TYPE_BF16BF16F32, 1, 16, 8),
@@ -251,18 +267,18 @@ def test_K_tail_overlap_is_zeroed_in_both_operands(gpu_lib):
 def test_split_k_tile(gpu_lib, flags, M0, N0, K0):
     e = 1 if flags == abi.MMT4D_TYPE_S8S8S32 else 2
     per_step = 256 // (K0 * e)                      # k steps per 256 bytes of a row
-    name = "mmt4d_mfma_64x64_split_k"
+    name = "mmt4d_mfma_wave_k_16x16"
     run_case(gpu_lib, flags, 72 // M0 + 1, 88 // N0, 16 * per_step, M0, N0, K0, name, accumulate=True, out_pad=8, seed=1)
     run_case(gpu_lib, flags, 200 // M0, 300 // N0, 17 * per_step, M0, N0, K0, name, lhs_pad=64 // e, rhs_pad=32 // e,
              offsets=(16 // e, 48 // e, 4), seed=2)
     run_case(gpu_lib, flags, max(1, 16 // M0), 48 // N0, 41 * per_step, M0, N0, K0, name, accumulate=True, seed=3)
-    # K not whole steps of 256 bytes, or too short to matter: the ordinary 64x64 tile
-    run_case(gpu_lib, flags, 72 // M0 + 1, 88 // N0, 16 * per_step + 64 // (K0 * e), M0, N0, K0, "mmt4d_mfma_64x64", seed=4)
-    run_case(gpu_lib, flags, max(1, 48 // M0), 88 // N0, 8 * per_step, M0, N0, K0, "mmt4d_mfma_64x64", seed=5)
+    # K not whole stretches of 256 bytes, and a shorter one
+    run_case(gpu_lib, flags, 72 // M0 + 1, 88 // N0, 16 * per_step + 64 // (K0 * e), M0, N0, K0, name, seed=4)
+    run_case(gpu_lib, flags, max(1, 48 // M0), 88 // N0, 8 * per_step, M0, N0, K0, name, seed=5)
 
 
-# The same with one row of 128x64 tiles (65 .. 128 lhs rows against many rhs rows, f16 / bf16): 128 bytes of K per row
-# and step.
+# One row of 128x64 tiles (up to 128 lhs rows against many rhs rows, f16 / bf16) whose wavefronts split K: 128 bytes of K
+# per row and step.
 @pytest.mark.parametrize("flags,M0,N0,K0", [(abi.MMT4D_TYPE_F16F16F32, 16, 16, 16), (abi.MMT4D_TYPE_BF16BF16F32, 16, 16, 8),
                                             (abi.MMT4D_TYPE_BF16BF16F32, 4, 16, 8), (abi.MMT4D_TYPE_F16F16F16, 16, 16, 8),
                                             (abi.MMT4D_TYPE_BF16BF16BF16, 8, 8, 32), (abi.MMT4D_TYPE_F16F16F32, 2, 4, 16)])
@@ -272,11 +288,16 @@ def test_split_k_tile_128_rows(gpu_lib, flags, M0, N0, K0):
     name = "mmt4d_mfma_128x64_split_k"
     cols = 9000 // N0
     run_case(gpu_lib, flags, 128 // M0, cols, 64 * per_step, M0, N0, K0, name, accumulate=True, out_pad=8, seed=1)
-    run_case(gpu_lib, flags, 100 // M0, cols + 3, 65 * per_step, M0, N0, K0, name, lhs_pad=64 // e, rhs_pad=32 // e,
+    run_case(gpu_lib, flags, 120 // M0, cols + 3, 65 * per_step, M0, N0, K0, name, lhs_pad=64 // e, rhs_pad=32 // e,
              offsets=(16 // e, 48 // e, 4), seed=2)
-    run_case(gpu_lib, flags, 80 // M0, cols, 97 * per_step, M0, N0, K0, name, accumulate=True, seed=3)
-    # 64 rows or fewer, or a K too short to pay for summing the partial tiles: the ordinary tiles
-    run_case(gpu_lib, flags, 64 // M0, cols, 64 * per_step, M0, N0, K0, "mmt4d_mfma_64x64", seed=4)
+    run_case(gpu_lib, flags, 112 // M0, cols, 97 * per_step, M0, N0, K0, name, accumulate=True, seed=3)
+    # Fewer rows: smaller tiles with K split over more wavefronts
+    run_case(gpu_lib, flags, 100 // M0, cols + 3, 65 * per_step, M0, N0, K0,
+             "mmt4d_mfma_wave_k_32x64" if 100 // M0 * M0 <= 96 else name, lhs_pad=64 // e, rhs_pad=32 // e,
+             offsets=(16 // e, 48 // e, 4), seed=2)
+    run_case(gpu_lib, flags, 80 // M0, cols, 97 * per_step, M0, N0, K0, "mmt4d_mfma_wave_k_32x64", accumulate=True, seed=3)
+    run_case(gpu_lib, flags, 64 // M0, cols, 64 * per_step, M0, N0, K0, "mmt4d_mfma_wave_k_64x64", seed=4)
+    # A K too short to pay for summing the partial tiles: the ordinary tile
     run_case(gpu_lib, flags, 128 // M0, cols, 32 * per_step, M0, N0, K0, "mmt4d_mfma_128x64", seed=5)
 
 

@@ -21,8 +21,9 @@ CASES = [
     # flags, M, N, K, M0, N0, K0, kernel the case is meant to reach (prefix)
     (F16, 32, 32, 64, 16, 16, 16, b"mmt4d_mfma_"),
     (BF16, 64, 64, 32, 16, 16, 8, b"mmt4d_mfma_"),
-    (BF16, 4, 4, 512, 16, 16, 8, b"mmt4d_mfma_64x64_split_k"),
-    (BF16, 8, 300, 512, 16, 16, 8, b"mmt4d_mfma_128x64_split_k"),
+    (BF16, 4, 4, 512, 16, 16, 8, b"mmt4d_mfma_wave_k_16x16"),
+    (BF16, 8, 300, 512, 16, 16, 8, b"mmt4d_mfma_wave_k_64x64"),
+    (BF16, 8, 562, 512, 16, 16, 8, b"mmt4d_mfma_128x64_split_k"),
     (F32, 16, 16, 64, 16, 16, 4, b"mmt4d_mfma_"),
     (abi.MMT4D_TYPE_F16F16F16 | SKIP, 16, 16, 64, 16, 16, 16, b"mmt4d_mfma_"),
     (BF16, 1, 100, 300, 16, 16, 8, b"mmt4d_gemv"),

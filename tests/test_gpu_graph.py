@@ -60,7 +60,8 @@ def test_mmt4d_and_pack_in_a_hip_graph(gpu_lib):
 
 def test_kernels_with_large_workgroup_memory_in_a_hip_graph(gpu_lib):
     # The 256x256 tile and the split-K tile use more than 64 KiB of workgroup memory, which is requested per kernel
-    # right before the launch, also while a stream is being captured; the skinny kernel for narrow tiles rides along.
+    # right before the launch, also while a stream is being captured; the kernel that splits K over more wavefronts and
+    # the skinny kernel for narrow tiles ride along.
     g = torch.Generator(device="cuda").manual_seed(2)
 
     def int8(n):
@@ -74,7 +75,9 @@ def test_kernels_with_large_workgroup_memory_in_a_hip_graph(gpu_lib):
         (int8(512 * 16 * 32), int8(512 * 16 * 32), torch.zeros(4096 * 4096, dtype=torch.int32, device="cuda"),
          512, 512, 16, 8, 8, 4, abi.MMT4D_TYPE_S8S8S32, b"mmt4d_mfma_256x256"),
         (bf16(5 * 256 * 128), bf16(7 * 256 * 128), torch.zeros(5 * 7 * 256, device="cuda"),
-         5, 7, 256, 16, 16, 8, abi.MMT4D_TYPE_BF16BF16F32, b"mmt4d_mfma_64x64_split_k"),
+         5, 7, 256, 16, 16, 8, abi.MMT4D_TYPE_BF16BF16F32, b"mmt4d_mfma_wave_k_16x16"),
+        (bf16(8 * 512 * 128), bf16(562 * 512 * 128), torch.zeros(8 * 562 * 256, device="cuda"),
+         8, 562, 512, 16, 16, 8, abi.MMT4D_TYPE_BF16BF16F32, b"mmt4d_mfma_128x64_split_k"),
         (int8(200 * 2), int8(64 * 200 * 32), torch.zeros(64 * 16, dtype=torch.int32, device="cuda"),
          1, 64, 200, 1, 16, 2, abi.MMT4D_TYPE_S8S8S32, b"mmt4d_skinny"),
     ]

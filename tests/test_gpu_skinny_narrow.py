@@ -66,8 +66,8 @@ def test_non_finite_lhs_values_do_not_leak_into_other_k_steps(gpu_lib):
 def test_eight_row_tiles_a_matrix_kernel_can_load_go_there(gpu_lib):
     # More than 4 rows make this kernel VALU bound; 8x16x2 int8 tiles are 16 bytes per k step, which the matrix
     # kernels load directly.
-    run_case(gpu_lib, S8, 1, 40, 64, 8, 16, 2, "mmt4d_mfma_64x64", accumulate=True)
-    run_case(gpu_lib, BF16, 1, 40, 64, 8, 16, 1, "mmt4d_mfma_64x64")
+    run_case(gpu_lib, S8, 1, 40, 64, 8, 16, 2, "mmt4d_mfma_wave_k_16x16", accumulate=True)
+    run_case(gpu_lib, BF16, 1, 40, 64, 8, 16, 1, "mmt4d_mfma_wave_k_16x16")
     # ... unless it cannot (lhs rows only 8-byte aligned)
     run_case(gpu_lib, S8, 1, 40, 64, 8, 16, 2, "mmt4d_skinny", offsets=(8, 0, 0))
 

@@ -35,8 +35,8 @@ def test_edges_of_tiles_and_of_K(gpu_lib, flags, M0, N0, K0):  # noqa: F811
         if i4 and K0 == 32:
             K |= 1
         elif not i4 and K * row_piece % 256 == 0:
-            K += 1  # (whole 256-byte stretches of a long K are another class to the names)
+            K += 1
         pad = 32 // e if n % 2 else 0
         run_case(gpu_lib, flags, -(-rows // M0), -(-cols // N0), K, M0, N0, K0,
-                 "mmt4d_mfma_64x128" if i4 and K0 == 64 else "mmt4d_mfma_64x64", lhs_pad=pad, rhs_pad=pad,
+                 "mmt4d_mfma_wave_k_*" if 0 < n < 6 else "mmt4d_mfma_*", lhs_pad=pad, rhs_pad=pad,
                  out_pad=4 if n % 2 else 0, offsets=(pad, pad, 4 if n % 2 else 0), accumulate=n % 3 == 1, seed=n)

@@ -1,6 +1,7 @@
 """The mmt4d kernel that splits K over the wavefronts of a workgroup (mmt4d_wave_k_kernels.h): every type, row piece size
-and output type it is instantiated for, at sizes that its tiles (16 to 64 rows and columns) do not divide, with K from
-less than a batch of steps per wavefront to many, ending on a step and inside one, strided and accumulating.
+and output type it is instantiated for, on every tile that the host takes for them (16 to 64 rows and columns), at sizes
+that the tiles do not divide, with K from less than a batch of steps per wavefront to many, ending on a step and inside one,
+strided and accumulating; and with weights that are read past the caches.
 
 Integers are compared bit for bit with a float64 product, floats within 1e-3 of max(|ref|, rms(ref)): sums of at most
 5000 products of unit-scale values in 32 bits differ by about 1e-6 of that in any order, 16-bit results by one unit in
@@ -40,3 +41,42 @@ def test_edges_of_tiles_and_of_K(gpu_lib, flags, M0, N0, K0):  # noqa: F811
         run_case(gpu_lib, flags, -(-rows // M0), -(-cols // N0), K, M0, N0, K0,
                  "mmt4d_mfma_wave_k_*" if 0 < n < 6 else "mmt4d_mfma_*", lhs_pad=pad, rhs_pad=pad,
                  out_pad=4 if n % 2 else 0, offsets=(pad, pad, 4 if n % 2 else 0), accumulate=n % 3 == 1, seed=n)
+
+
+# Per tile, sizes at which the host takes it for every layout, the shorter K ending inside a step of some wavefront's first
+# batch; int8 in narrow pieces reaches 64x64 at other sizes, f32 (bound by the matrix pipe) at none.
+TILES = [("16x16", 20, 24, 300), ("16x16", 24, 72, 5000), ("16x32", 20, 3000, 300), ("16x32", 40, 1500, 5000),
+         ("32x32", 40, 3000, 300), ("32x32", 100, 1500, 5000), ("32x64", 72, 3000, 800), ("32x64", 72, 5000, 5000),
+         ("64x32", 820, 600, 1100), ("64x64", 330, 1500, 4500), ("64x64", 264, 2000, 5000)]
+NARROW_INT8 = {(8, 8, 4): (623, 852, 6489), (2, 16, 8): (424, 1183, 6935)}
+
+
+@pytest.mark.parametrize("flags,M0,N0,K0", LAYOUTS)
+def test_every_tile(gpu_lib, flags, M0, N0, K0):  # noqa: F811
+    e = {abi.MMT4D_TYPE_S8S8S32: 1, abi.MMT4D_TYPE_S8S4S32: 1, abi.MMT4D_TYPE_F32F32F32: 4}.get(flags, 2)
+    for n, (tile, rows, cols, row_bytes) in enumerate(TILES):
+        if tile == "64x64":
+            if flags == abi.MMT4D_TYPE_F32F32F32:
+                continue
+            if flags == abi.MMT4D_TYPE_S8S8S32:
+                rows, cols, row_bytes = NARROW_INT8.get((M0, N0, K0), (rows, cols, row_bytes))
+        K = -(-row_bytes // (K0 * e))
+        if flags == abi.MMT4D_TYPE_S8S4S32 and K0 == 32:
+            K |= 1  # half a step
+        pad = 32 // e if n % 2 else 0
+        run_case(gpu_lib, flags, -(-rows // M0), -(-cols // N0), K, M0, N0, K0, "mmt4d_mfma_wave_k_" + tile, lhs_pad=pad,
+                 rhs_pad=pad, out_pad=4 if n % 2 else 0, offsets=(pad, pad, 4 if n % 2 else 0), accumulate=n % 3 == 0, seed=n)
+
+
+# One row of tiles and more than 48 MiB of weights (row pieces of 16 bytes and more): non-temporal loads.
+@pytest.mark.parametrize("flags,M0,N0,K0", [l for l in LAYOUTS if l[3] * {abi.MMT4D_TYPE_F32F32F32: 4}.get(l[0], 1) >= 16])
+def test_weights_from_hbm(gpu_lib, flags, M0, N0, K0):  # noqa: F811
+    i4 = flags == abi.MMT4D_TYPE_S8S4S32
+    e = {abi.MMT4D_TYPE_S8S8S32: 1, abi.MMT4D_TYPE_S8S4S32: 1, abi.MMT4D_TYPE_F32F32F32: 4}.get(flags, 2)
+    problems = [("32x64", 24, 28000, 4200), ("64x64", 48, 13000, 8300)] if i4 else \
+        [("32x32", 24, 7000, 8000), ("32x64", 24, 13000, 4200), ("64x64", 64, 13000, 4200)]
+    for n, (tile, rows, cols, row_bytes) in enumerate(problems):
+        if tile == "64x64" and flags == abi.MMT4D_TYPE_F32F32F32:
+            continue
+        K = -(-row_bytes // (K0 * e)) | 1
+        run_case(gpu_lib, flags, -(-rows // M0), -(-cols // N0), K, M0, N0, K0, "mmt4d_mfma_wave_k_" + tile, accumulate=n == 0, seed=n)

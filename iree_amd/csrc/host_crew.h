@@ -4,8 +4,11 @@
 //
 // The crew is started by the first call that is large enough to use it and ends
 // with the library. One call has it at a time, another that comes meanwhile does
-// without. The helpers sleep between calls and poll while a call has them, so a
-// process with fewer than four CPUs has no crew.
+// without. The helpers sleep between calls. While a call has them they poll for
+// their next piece, 0.2 ms at most: waking takes 30 to 60 us, which is what a
+// product between the copies often takes, and a longer one (or work that the
+// caller's stream had before) costs no CPU time. A process with fewer than four
+// CPUs has no crew.
 #ifndef IREE_AMD_CSRC_HOST_CREW_H_
 #define IREE_AMD_CSRC_HOST_CREW_H_
 
@@ -14,6 +17,7 @@
 #include <unistd.h>
 
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstdint>
 #include <mutex>
@@ -43,6 +47,7 @@ class HostCrew {
     {
       std::lock_guard<std::mutex> lock(mutex_);
       engaged_.store(true, std::memory_order_relaxed);
+      ++engagements_;
     }
     wake_.notify_all();
     return true;
@@ -61,6 +66,11 @@ class HostCrew {
     count_ = count;
     next_.store(0, std::memory_order_relaxed);
     open_.store(true);
+    // A helper counts itself asleep before it looks for open work a last time: either it sees this work or it is woken.
+    if (asleep_.load() != 0) {
+      { std::lock_guard<std::mutex> lock(mutex_); }
+      wake_.notify_all();
+    }
     for (uint32_t i; (i = next_.fetch_add(1, std::memory_order_relaxed)) < count;) work(i);
     // A helper announces itself before it looks whether the work is still open: once none is announced after it has
     // been closed, none reads the fields above any more.
@@ -104,23 +114,34 @@ class HostCrew {
     pthread_sigmask(SIG_SETMASK, &before, nullptr);
   }
 
+  bool work_waits() const { return open_.load() && next_.load(std::memory_order_relaxed) < count_.load(std::memory_order_relaxed); }
+
   void help() {
+    typedef std::chrono::steady_clock clock;
+    constexpr std::chrono::microseconds kPolling(200);
+    uint32_t seen = 0;  // engagements
     for (;;) {
       {
         std::unique_lock<std::mutex> lock(mutex_);
-        wake_.wait(lock, [this] { return stop_.load() || engaged_.load(std::memory_order_relaxed); });
+        asleep_.fetch_add(1);
+        wake_.wait(lock, [&] { return stop_.load() || engagements_ != seen || work_waits(); });
+        asleep_.fetch_sub(1);
         if (stop_.load()) return;
+        seen = engagements_;
       }
-      while (engaged_.load(std::memory_order_relaxed) && !stop_.load(std::memory_order_relaxed)) {
-        if (open_.load(std::memory_order_relaxed) && next_.load(std::memory_order_relaxed) < count_.load(std::memory_order_relaxed)) {
+      clock::time_point idle_since = clock::now();
+      for (uint32_t spins = 1; engaged_.load(std::memory_order_relaxed) && !stop_.load(std::memory_order_relaxed); ++spins) {
+        if (work_waits()) {
           active_.fetch_add(1);
           if (open_.load()) {
             const uint32_t count = count_.load(std::memory_order_relaxed);
             for (uint32_t i; (i = next_.fetch_add(1, std::memory_order_relaxed)) < count;) call_(context_, i);
           }
           active_.fetch_sub(1);
+          idle_since = clock::now();
         } else {
           __builtin_ia32_pause();
+          if (spins % 64 == 0 && clock::now() - idle_since > kPolling) break;
         }
       }
     }
@@ -131,8 +152,9 @@ class HostCrew {
   std::thread helpers_[2];
   std::mutex mutex_;
   std::condition_variable wake_;
+  uint32_t engagements_ = 0;  // (under mutex_)
   std::atomic<bool> stop_{false}, engaged_{false}, open_{false};
-  std::atomic<uint32_t> next_{0}, active_{0}, count_{0};
+  std::atomic<uint32_t> next_{0}, active_{0}, count_{0}, asleep_{0};
   void (*call_)(void*, uint32_t) = nullptr;
   void* context_ = nullptr;
 };

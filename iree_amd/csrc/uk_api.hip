@@ -5,7 +5,9 @@
 // (mmt4d.c:12-48, pack.c:51-103, unpack.c:31-81) and are always on here: a
 // rejected call costs microseconds next to a kernel launch, and an out-of-range
 // parameter reaching a GPU kernel can fault the device rather than one process.
+#include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -421,6 +423,22 @@ bool pipe_down(const Stager& stager, void* host, const void* dev, size_t bytes, 
       status = e;
       failed = true;
     };
+    if (at == 0) {
+      // The first piece comes when everything that the stream had before has ended, the product among it. That is polled
+      // for while it may be a matter of microseconds; then the thread sleeps between looks, a sixteenth of what it has
+      // waited (half a millisecond at most), and the helpers sleep.
+      typedef std::chrono::steady_clock clock;
+      const clock::time_point start = clock::now();
+      for (uint32_t spins = 1; __atomic_load_n(flags, __ATOMIC_ACQUIRE) != generation && !failed; ++spins) {
+        __builtin_ia32_pause();
+        if (spins % 1024 != 0) continue;
+        const clock::duration waited = clock::now() - start;
+        if (waited < std::chrono::microseconds(500)) continue;
+        check_stream();
+        std::this_thread::sleep_for(std::min<clock::duration>(waited / 16, std::chrono::microseconds(500)));
+        spins = 1023;  // (one look per sleep)
+      }
+    }
     auto take = [&](uint32_t i) {
       for (uint32_t spins = 1; __atomic_load_n(flags + i, __ATOMIC_ACQUIRE) != generation && !failed; ++spins) {
         __builtin_ia32_pause();

@@ -20,7 +20,7 @@ def _run(cmd):
 
 
 def build(out_dir):
-    flags = [f for f in hip_build.COMMON_FLAGS if f != "-O3"] + ["-O1", "--offload-host-only"]
+    flags = [f for f in hip_build.COMMON_FLAGS if f != "-O3"] + ["-O1", "--offload-host-only", "-I" + hip_build.CSRC]
 
     def host_object(src):
         obj = os.path.join(out_dir, os.path.basename(src) + ".o")

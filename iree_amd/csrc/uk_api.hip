@@ -109,18 +109,22 @@ thread_local StageArena tl_arena;
 // caller's pages (55 to 80 GB/s) a chunk at a time while the previous chunks are on the bus (50 GB/s each way). The
 // runtime's own path for pageable memory moves 20 to 33 GB/s up and 17 down, in 30 to 100 us for a few KiB. int8 through
 // both: 64 x 256 x 256 47 -> 21 us, 512 x 2048 x 2048 (5 MB up, 4 down) 430 -> 255, 4096 x 2048 x 4096 2731 -> 1458.
+//
+// It is as large as the largest call of the thread so far needs, 64 KiB to 8 MiB. Operands that together fit go up from
+// their place in it; larger ones through its eight slots in turn, each of them guarded by an event.
 struct HostPipe {
   static constexpr size_t kSlotBytes = 1 << 20, kFirstBytes = 128 << 10;
   static constexpr int kSlots = 8;
-  // What an upload moves before it comes back to its first slot: 1, 2 and 4 times kFirstBytes, then whole slots.
-  static constexpr size_t kUnwrappedBytes = 7 * kFirstBytes + (kSlots - 3) * kSlotBytes;
-  static_assert(8 * kFirstBytes == kSlotBytes, "kUnwrappedBytes counts three doublings");
-  static constexpr size_t kHalfBytes = kSlots / 2 * kSlotBytes;  // a download alternates between halves
-  static constexpr int kFlags = (int)(2 * kHalfBytes / uk::kDownloadPieceBytes);
-  uint8_t* pinned = nullptr;
-  uint32_t* flags = nullptr;  // behind the slots
+  static constexpr size_t kMostBytes = kSlots * kSlotBytes, kLeastBytes = 64 << 10;
+  static constexpr size_t kHalfBytes = kMostBytes / 2;  // a download of more than this alternates between halves
+  static constexpr int kFlags = (int)(kMostBytes / uk::kDownloadPieceBytes);
+  static constexpr size_t kFlagBytes = 4096;
+  static_assert(kFlags * sizeof(uint32_t) <= kFlagBytes, "room for the flags");
+  uint32_t* flags = nullptr;  // at the start of the allocation
+  uint8_t* pinned = nullptr;  // behind them
+  size_t capacity = 0;
   uint32_t generation = 0;
-  hipEvent_t event[kSlots] = {};
+  hipEvent_t event[kSlots] = {};  // exist where a call has needed them
   int device = -1;
 
   ~HostPipe() { release(); }
@@ -129,23 +133,32 @@ struct HostPipe {
       if (e) (void)hipEventDestroy(e);
       e = nullptr;
     }
-    if (pinned) (void)hipHostFree(pinned);
+    if (flags) (void)hipHostFree(flags);
+    flags = nullptr;
     pinned = nullptr;
+    capacity = 0;
   }
-  // False: no pinned memory to be had; the caller copies from pageable memory.
-  bool ready(int current_device) {
-    if (pinned && device == current_device) return true;
-    release();
-    device = current_device;
-    if (hipHostMalloc((void**)&pinned, kSlots * kSlotBytes + kFlags * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
-      (void)hipGetLastError();
-      pinned = nullptr;
-      return false;
+  // For a call that mirrors `bytes` in all. False: no pinned memory to be had; the caller copies from pageable memory.
+  bool ready(int current_device, size_t bytes) {
+    const bool slots = bytes > kMostBytes;
+    if (!pinned || device != current_device || capacity < (slots ? kMostBytes : bytes)) {
+      release();
+      device = current_device;
+      size_t size = kLeastBytes;
+      while (size < kMostBytes && size < bytes) size *= 2;
+      void* block = nullptr;
+      if (hipHostMalloc(&block, kFlagBytes + size, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+      }
+      flags = (uint32_t*)block;
+      pinned = (uint8_t*)block + kFlagBytes;
+      capacity = size;
+      memset(flags, 0, kFlagBytes);
+      generation = 0;
     }
-    flags = (uint32_t*)(pinned + kSlots * kSlotBytes);
-    memset(flags, 0, kFlags * sizeof(uint32_t));
-    generation = 0;
     for (hipEvent_t& e : event) {
+      if (!slots || e) continue;
       if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
         (void)hipGetLastError();
         e = nullptr;
@@ -155,7 +168,6 @@ struct HostPipe {
     }
     return true;
   }
-  uint8_t* slot(int i) { return pinned + (size_t)i * kSlotBytes; }
 };
 thread_local HostPipe tl_pipe;
 
@@ -252,7 +264,7 @@ bool stage_reserve(Stager& stager, size_t bytes, uint8_t** out) {
     s.capacity = cap;
     s.device = device;
   }
-  stager.piped = tl_pipe.ready(device);
+  stager.piped = tl_pipe.ready(device, bytes);
   *out = s.ptr;
   return true;
 }
@@ -363,18 +375,19 @@ bool pipe_up(Stager& stager, uint8_t* base, Operand* const* ops, int count, hipS
   HostPipe& pipe = tl_pipe;
   const Operand& last = *ops[count - 1];
   const size_t total = (size_t)((const uint8_t*)last.dev - base) + (size_t)last.region.span;
-  const bool wraps = total > HostPipe::kUnwrappedBytes, past_caches = total >= kPastCachesBytes;
+  const bool slots = total > HostPipe::kMostBytes, past_caches = total >= kPastCachesBytes;
   constexpr size_t kPiece = 64 << 10;  // of a chunk, per helper and turn
   size_t chunk = HostPipe::kFirstBytes;
   for (size_t at = 0, n = 0, used = 0; at < total; at += n, ++used) {
     const int slot = (int)(used % HostPipe::kSlots);
-    if (used >= (size_t)HostPipe::kSlots) UK_HIP_OK(hipEventSynchronize(pipe.event[slot]));
+    if (slots && used >= (size_t)HostPipe::kSlots) UK_HIP_OK(hipEventSynchronize(pipe.event[slot]));
     n = total - at < chunk ? total - at : chunk;
+    uint8_t* const place = pipe.pinned + (slots ? (size_t)slot * HostPipe::kSlotBytes : at);
     auto fill = [&](size_t from, size_t to) {  // of the mirrored bytes
       for (int op = 0; op < count; ++op) {
         const size_t begin = (size_t)((const uint8_t*)ops[op]->dev - base), end = begin + (size_t)ops[op]->region.span;
         const size_t f = begin > from ? begin : from, t = end < to ? end : to;
-        if (f < t) host_copy(pipe.slot(slot) + (f - at), (const uint8_t*)ops[op]->host + (f - begin), t - f, past_caches);
+        if (f < t) host_copy(place + (f - at), (const uint8_t*)ops[op]->host + (f - begin), t - f, past_caches);
       }
     };
     if (stager.crew && n > kPiece) {
@@ -385,8 +398,8 @@ bool pipe_up(Stager& stager, uint8_t* base, Operand* const* ops, int count, hipS
     } else {
       fill(at, at + n);
     }
-    UK_HIP_OK(uk::launch_upload(pipe.slot(slot), base + at, n, stream));
-    if (wraps) UK_HIP_OK(hipEventRecord(pipe.event[slot], stream));
+    UK_HIP_OK(uk::launch_upload(place, base + at, n, stream));
+    if (slots) UK_HIP_OK(hipEventRecord(pipe.event[slot], stream));
     if (chunk < HostPipe::kSlotBytes) chunk *= 2;
   }
   return true;

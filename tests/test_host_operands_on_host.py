@@ -66,3 +66,24 @@ def test_a_long_product_does_not_keep_cpus_busy(recorder):  # noqa: F811
         recorder.lib.recorded_set_kernel_ms(0)
     assert wall >= 0.4
     assert cpu < 0.2, (wall, cpu)
+
+
+def test_pinned_memory_follows_the_calls(recorder):  # noqa: F811
+    lib = recorder.lib
+    lib.recorded_pinned_bytes.restype = lib.recorded_events.restype = C.c_longlong
+    before = lib.recorded_pinned_bytes(), lib.recorded_events()
+    seen = []
+
+    def calls():
+        for M, N, K in ((1, 1, 1), (8, 9, 256), (1, 1, 1), (64, 64, 256), (90, 200, 900), (128, 64, 33)):
+            product(recorder, M, N, K, 7)
+            seen.append((lib.recorded_pinned_bytes() - before[0], lib.recorded_events() - before[1]))
+
+    t = threading.Thread(target=calls)
+    t.start()
+    t.join()
+    kib, flags = 1 << 10, 4096
+    # (0.2 MB in all; less; 5 MB; 26 MB, more than fits; less)
+    assert seen == [(64 * kib + flags, 0), (256 * kib + flags, 0), (256 * kib + flags, 0), (8192 * kib + flags, 0),
+                    (8192 * kib + flags, 8), (8192 * kib + flags, 8)], seen
+    assert (lib.recorded_pinned_bytes(), lib.recorded_events()) == before  # given back with the thread

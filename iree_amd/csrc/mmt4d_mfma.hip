@@ -23,10 +23,10 @@ struct Plan {
 };
 
 // Estimates in microseconds, to choose between the block kernels and the one that splits K over wavefronts. Both write
-// the output at the same rate, which is left out. Measured over 1094 problems (M 24..512, N 512..28672, K 1024..14336,
-// every type and row piece) with operands from HBM (sets of 640 MB in turn, the condition of weights in a model's layers)
-// and with operands that the last-level cache holds (150 MB), the coefficients fitted to the geometric mean of the two: the
-// kernel picked is 0.3 % slower than the best one in the mean, 5 % and more on 24 problems. Fitted to repeated operands
+// the output at the same rate, which is left out. Measured over 9164 problems (M 8..1100, N 64..28672, K 64..14336, every
+// type and row piece) with operands from HBM (sets of 640 MB in turn, the condition of weights in a model's layers) and
+// with operands that the last-level cache holds (150 MB), the coefficients fitted to the geometric mean of the two: the
+// kernel picked is 0.7 % slower than the best one in the mean, 5 % and more on one problem in 25. Fitted to repeated operands
 // alone they had picked 32x64 tiles for bf16 96 x 14336 x 4096: 27.5 us held and 40.6 from HBM, where the 128x64 tile with
 // K split takes 23.9 and 32.6; int4 96 x 14336 x 4096 19.1 from HBM against 16.3.
 //
@@ -34,14 +34,15 @@ struct Plan {
 double block_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
   const bool direct = mfma_direct_covers(m, gather, rhs_i4);
   const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
-  const double memory_us = (double)(rows * m.lhs_rb + cols * m.rhs_rb) * m.K / 6.0e6;
-  double us_per_chunk, start_us = 3.0;
+  const double memory_us = (double)(rows * m.lhs_rb + cols * m.rhs_rb) * m.K / 6.95e6;
+  double us_per_chunk, start_us = 3.32;
   if (gather == 16 && (kind == kF16 || kind == kBF16) && direct && split_k_covers(m)) {
-    us_per_chunk = 0.153;
-    start_us = 6.2;  // (and the summing of the partial tiles)
+    us_per_chunk = 0.163;
+    start_us = 6.6;  // (and the summing of the partial tiles)
   } else {
     choose_tile(m, kind, rhs_i4, gather, direct, &us_per_chunk);
-    if (!direct) us_per_chunk *= 2.2;  // staged through registers
+    if (!direct) us_per_chunk *= 2.2;       // staged through registers
+    if (gather == 2) us_per_chunk *= 1.2;    // (the tiles that few rows take: wide ones, from HBM)
   }
   const double chunks_us = m.chunks * us_per_chunk;
   return start_us + (chunks_us > memory_us ? chunks_us : memory_us);
@@ -53,13 +54,14 @@ double wave_k_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather, const W
   const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
   const int64_t tiles = ((rows + 16 * s.fa - 1) / (16 * s.fa)) * ((cols + 16 * s.fb - 1) / (16 * s.fb));
   const double row_kb = 1e-3 * m.K * m.lhs_rb, rhs_share = rhs_i4 ? 0.5 : 1.0;
-  double tile_us = 16 * (s.fa + s.fb * rhs_share) * row_kb / (gather < 16 ? 72 : 110);
-  if (kind == kF32) tile_us = tile_us > 0.024 * s.fa * s.fb * m.chunks ? tile_us : 0.024 * s.fa * s.fb * m.chunks;
-  double us = (gather < 16 || rhs_i4 ? 3.1 : 2.5) + 0.04 * s.fa * s.fb + 4.75e-5 * (rows + cols * rhs_share) * row_kb;
+  const bool narrow = gather < 16;  // row pieces, which pass through LDS
+  double tile_us = 16 * (s.fa + s.fb * rhs_share) * row_kb / (narrow ? 69.5 : 89.2);
+  if (kind == kF32) tile_us = tile_us > 0.0224 * s.fa * s.fb * m.chunks ? tile_us : 0.0224 * s.fa * s.fb * m.chunks;
+  double us = (narrow || rhs_i4 ? 3.07 : 2.53) + 0.057 * s.fa * s.fb + 4.12e-5 * (rows + cols * rhs_share) * row_kb;
   if (tiles <= 256) return us + tile_us;
   const double rounds = tiles / 256.0;
   if (tiles > (s.fa * s.fb >= 16 ? 256 : 1024)) us += 1e3 * rounds;
-  return us + (rounds + 0.7) * tile_us + 0.66 * rounds;
+  return us + (rounds + (narrow ? 0.988 : 0.893)) * tile_us + (narrow ? 0.552 : 0.43) * rounds;
 }
 
 // Whether the kernel that splits K over wavefronts covers the problem: 16-byte aligned operands whose 16 contiguous

@@ -48,6 +48,7 @@ class HostCrew {
       std::lock_guard<std::mutex> lock(mutex_);
       engaged_.store(true, std::memory_order_relaxed);
       ++engagements_;
+      dozing_.store(0);
     }
     wake_.notify_all();
     return true;
@@ -66,8 +67,9 @@ class HostCrew {
     count_ = count;
     next_.store(0, std::memory_order_relaxed);
     open_.store(true);
-    // A helper counts itself asleep before it looks for open work a last time: either it sees this work or it is woken.
-    if (asleep_.load() != 0) {
+    // A helper that polled in vain says so before it looks for open work a last time: either it sees this work or it is
+    // woken, once. (Not those that `engage` has just woken: a wake-up costs microseconds a time.)
+    if (dozing_.load() != 0 && dozing_.exchange(0) != 0) {
       { std::lock_guard<std::mutex> lock(mutex_); }
       wake_.notify_all();
     }
@@ -120,15 +122,15 @@ class HostCrew {
     typedef std::chrono::steady_clock clock;
     constexpr std::chrono::microseconds kPolling(200);
     uint32_t seen = 0;  // engagements
-    for (;;) {
+    for (bool dozes = false;;) {
       {
         std::unique_lock<std::mutex> lock(mutex_);
-        asleep_.fetch_add(1);
+        if (dozes) dozing_.fetch_add(1);
         wake_.wait(lock, [&] { return stop_.load() || engagements_ != seen || work_waits(); });
-        asleep_.fetch_sub(1);
         if (stop_.load()) return;
         seen = engagements_;
       }
+      dozes = false;
       clock::time_point idle_since = clock::now();
       for (uint32_t spins = 1; engaged_.load(std::memory_order_relaxed) && !stop_.load(std::memory_order_relaxed); ++spins) {
         if (work_waits()) {
@@ -141,7 +143,10 @@ class HostCrew {
           idle_since = clock::now();
         } else {
           __builtin_ia32_pause();
-          if (spins % 64 == 0 && clock::now() - idle_since > kPolling) break;
+          if (spins % 64 == 0 && clock::now() - idle_since > kPolling) {
+            dozes = true;
+            break;
+          }
         }
       }
     }
@@ -154,7 +159,7 @@ class HostCrew {
   std::condition_variable wake_;
   uint32_t engagements_ = 0;  // (under mutex_)
   std::atomic<bool> stop_{false}, engaged_{false}, open_{false};
-  std::atomic<uint32_t> next_{0}, active_{0}, count_{0}, asleep_{0};
+  std::atomic<uint32_t> next_{0}, active_{0}, count_{0}, dozing_{0};
   void (*call_)(void*, uint32_t) = nullptr;
   void* context_ = nullptr;
 };

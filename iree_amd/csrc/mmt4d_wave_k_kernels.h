@@ -10,8 +10,9 @@
 // steps in flight while the previous batch is multiplied, with no LDS and no
 // barrier until the partial tiles are summed through LDS at the end, in
 // wavefront order (results do not depend on scheduling). A workgroup thus has
-// 128 to 256 KiB of loads in flight and is bound by what a compute unit's load
-// path moves, 64 bytes per cycle, i.e. by (16*FA + 16*FB) * 64 bytes per step.
+// 128 to 256 KiB of loads in flight and, where the caches hold the operands, is
+// bound by what a compute unit's load path moves: (16*FA + 16*FB) * 64 bytes per
+// step at 70 to 90 bytes a nanosecond.
 //
 // Operand registers. Fragments are 16 rows x 64 bytes of K
 // (v_mfma_i32_16x16x64_i8, v_mfma_f32_16x16x32_{f16,bf16}, four

@@ -164,7 +164,6 @@ bool make_plan(const Mmt4dArgs& a, bool probe_only, Plan* plan) {
   if (!wave_k_covers(m, gather, i4)) return true;
   double best = block_cost(m, kind, i4, gather);
   for (int s = 0; s < (int)(sizeof kWaveKShapes / sizeof kWaveKShapes[0]); ++s) {
-    if (kind == kF32 && kWaveKShapes[s].fa * kWaveKShapes[s].fb >= 16) continue;  // (not instantiated)
     const double cost = wave_k_cost(m, kind, i4, gather, kWaveKShapes[s]);
     if (cost < best) {
       best = cost;

@@ -87,9 +87,8 @@ struct WaveKShape {
   int fa, fb;  // 16-row fragments of the lhs and of the rhs
   const char* name;
 };
-constexpr WaveKShape kWaveKShapes[] = {{1, 1, "mmt4d_mfma_wave_k_16x16"}, {1, 2, "mmt4d_mfma_wave_k_16x32"},
-                                       {2, 2, "mmt4d_mfma_wave_k_32x32"}, {2, 4, "mmt4d_mfma_wave_k_32x64"},
-                                       {4, 4, "mmt4d_mfma_wave_k_64x64"}};
+constexpr WaveKShape kWaveKShapes[] = {{1, 1, "mmt4d_mfma_wave_k_16x16"}, {1, 2, "mmt4d_mfma_wave_k_16x32"}, {2, 2, "mmt4d_mfma_wave_k_32x32"},
+                                       {2, 4, "mmt4d_mfma_wave_k_32x64"}, {4, 2, "mmt4d_mfma_wave_k_64x32"}, {4, 4, "mmt4d_mfma_wave_k_64x64"}};
 hipError_t launch_wave_k_i8(const MfmaArgs& m, int gather, bool rhs_i4, int shape, bool streamed, hipStream_t stream);
 hipError_t launch_wave_k_f16(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);
 hipError_t launch_wave_k_bf16(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);

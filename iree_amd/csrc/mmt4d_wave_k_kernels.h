@@ -360,10 +360,8 @@ hipError_t launch_wave_k_piece(const MfmaArgs& m, int shape, bool streamed, hipS
     case 1: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 2, 8, 2>(m, streamed, stream);
     case 2: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 2, 2, 8, 2>(m, streamed, stream);
     case 3: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 2, 4, 8, 1>(m, streamed, stream);
-    case 4:
-      // (f32 is bound by the matrix pipe, which 64x64 block tiles keep busier.)
-      if constexpr (KIND != kF32) return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 4, 4, 8, 1>(m, streamed, stream);
-      return hipErrorInvalidValue;
+    case 4: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 4, 2, 8, 1>(m, streamed, stream);
+    case 5: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 4, 4, 8, 1>(m, streamed, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -47,7 +47,7 @@ def test_mmt4d(recorder):  # noqa: F811
         assert name == want == name_of(symbol), (symbol, name)
         seen.add(name)
     tiles = ["256x256", "256x128", "128x128", "128x64", "64x64", "64x128", "192x192", "128x192", "192x128", "256x192", "192x256",
-             "128x64_split_k"] + ["wave_k_" + t for t in ("16x16", "16x32", "32x32", "32x64", "64x64")]
+             "128x64_split_k"] + ["wave_k_" + t for t in ("16x16", "16x32", "32x32", "32x64", "64x32", "64x64")]
     missing = {"mmt4d_" + n for n in ["gemv", "gemv_resident_lhs", "skinny", "generic"] + ["mfma_" + t for t in tiles]} - seen
     assert not missing
 

@@ -66,6 +66,19 @@ def test_every_tile(gpu_lib, flags, M0, N0, K0):  # noqa: F811
     assert {"mmt4d_mfma_wave_k_" + t for t in tiles} <= seen, seen
 
 
+# At most 256 tiles of 64x32, one for a compute unit, where there are more than 256 of 32x64.
+@pytest.mark.parametrize("flags,M0,N0,K0", LAYOUTS)
+def test_tiles_of_64x32_fill_the_units_once(gpu_lib, flags, M0, N0, K0):  # noqa: F811
+    e = {abi.MMT4D_TYPE_S8S8S32: 1, abi.MMT4D_TYPE_S8S4S32: 1, abi.MMT4D_TYPE_F32F32F32: 4}.get(flags, 2)
+    for n, (rows, cols, row_bytes) in enumerate([(190, 2700, 600), (304, 1620, 2100), (614, 790, 4300)]):
+        K = -(-row_bytes // (K0 * e))
+        if flags == abi.MMT4D_TYPE_S8S4S32 and K0 == 32:
+            K |= 1
+        pad = 32 // e if n % 2 else 0
+        run_case(gpu_lib, flags, -(-rows // M0), -(-cols // N0), K, M0, N0, K0, "mmt4d_mfma_wave_k_64x32", lhs_pad=pad,
+                 rhs_pad=pad, out_pad=4 if n % 2 else 0, offsets=(pad, pad, 4 if n % 2 else 0), accumulate=n % 3 == 0, seed=n)
+
+
 # One row of tiles and more than 48 MiB of weights (row pieces of 16 bytes and more): non-temporal loads.
 @pytest.mark.parametrize("flags,M0,N0,K0", [l for l in LAYOUTS if l[3] * {abi.MMT4D_TYPE_F32F32F32: 4}.get(l[0], 1) >= 16])
 def test_weights_from_hbm(gpu_lib, flags, M0, N0, K0):  # noqa: F811

@@ -31,6 +31,7 @@ TIMES = [
     ("s8, 4-byte pieces", 128, 2048, 2048, {"32x32": (5.6, 5.9), "16x32": (6.1, 6.4), "32x64": (6.5, 6.9), "block": (7.8, 7.9)}),
     ("bf16, 8-byte pieces", 32, 14336, 4096, {"32x64": (20.5, 25.2), "block": (19.9, 26.0), "64x64": (21.8, 26.6)}),
     ("s8, 2-byte pieces", 256, 11008, 2048, {"block": (15.5, 17.6), "64x64": (21.2, 23.8), "64x32": (28.1, 31.4)}),
+    ("s8, 2-byte pieces", 304, 1632, 272, {"64x32": (4.0, 4.1), "64x64": (4.7, 4.9), "block": (4.8, 5.0)}),
     ("s8, 4-byte pieces", 16, 20000, 3000, {"16x32": (12.4, 15.2), "16x16": (13.3, 17.0), "block": (14.5, 17.4)}),
     ("s8, 2-byte pieces", 96, 10112, 10112, {"32x64": (31.5, 39.0), "block": (44.3, 44.6), "64x64": (42.0, 48.4)}),
     ("bf16, 4-byte pieces", 16, 10112, 10112, {"32x64": (41.7, 41.7), "16x32": (47.6, 47.6), "16x16": (45.1, 45.0), "block": (48.3, 48.1)}),

@@ -42,6 +42,10 @@ double block_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
   } else {
     choose_tile(m, kind, rhs_i4, gather, direct, &us_per_chunk);
     if (!direct) us_per_chunk *= 2.2;       // staged through registers
+    // Few rows and more 64x64 tiles than units: the unit's second tile, row pieces of 4 and 8 bytes, is dearer than the
+    // table's (from 16-byte pieces, many rows): bf16 16 x 20720 x 7396, 16x16x2 tiles, 0.28 us and not 0.195. Without the
+    // factor the block kernel was taken, 68 us, where a wave-K tile takes 60.
+    if ((gather == 4 || gather == 8) && (kind == kF16 || kind == kBF16) && rows <= 16 && cols > 64 * 256) us_per_chunk *= 1.3;
     if (gather == 2) us_per_chunk *= 1.2;    // (the tiles that few rows take: wide ones, from HBM)
   }
   const double chunks_us = m.chunks * us_per_chunk;

@@ -35,6 +35,7 @@ TIMES = [
     ("s8, 4-byte pieces", 16, 20000, 3000, {"16x32": (12.4, 15.2), "16x16": (13.3, 17.0), "block": (14.5, 17.4)}),
     ("s8, 2-byte pieces", 96, 10112, 10112, {"32x64": (31.5, 39.0), "block": (44.3, 44.6), "64x64": (42.0, 48.4)}),
     ("bf16, 4-byte pieces", 16, 10112, 10112, {"32x64": (41.7, 41.7), "16x32": (47.6, 47.6), "16x16": (45.1, 45.0), "block": (48.3, 48.1)}),
+    ("bf16, 4-byte pieces", 16, 20000, 3000, {"16x32": (20.8, 25.9), "16x16": (20.6, 28.0), "block": (24.4, 29.5)}),
     ("f32", 64, 2048, 2048, {"16x32": (10.2, 10.8), "16x16": (12.2, 13.0), "32x32": (15.9, 16.7), "block": (37.4, 37.5)}),
 ]
 

@@ -16,9 +16,8 @@
 //     least one full chunk of K (a K that ends inside a chunk is handled by
 //     overlapping the last chunk with the one before it).
 //   mmt4d_mfma_kernel (everything else the plan admits: 4-byte aligned
-//     operands, narrow tiles, less than a chunk of K, an int4 rhs whose K ends
-//     inside a chunk): global -> registers (issued two chunks
-//     ahead) -> LDS -> registers (read one chunk ahead) -> MFMA.
+//     operands, narrow tiles, less than a chunk of K, an int4 rhs of 8-byte row
+//     pieces): global -> registers (issued two chunks ahead) -> LDS -> registers (read one chunk ahead) -> MFMA.
 // In both, LDS holds the operands fragment-major, so that a wavefront fetches
 // a 32-row x 32-byte MFMA operand with conflict-free reads that are linear in
 // the lane number.
@@ -635,9 +634,8 @@ __global__ __launch_bounds__(256, MIN_BLOCKS) void mmt4d_mfma_kernel(const MfmaA
 // (global_load_lds_dwordx4: lane l of a wavefront writes its 16 bytes at
 // M0 + 16*l), through a ring of 4 LDS stages filled three chunks ahead of the
 // MFMAs. It needs no register prefetch buffers, no LDS writes and no
-// data-dependent waits other than one counter wait per chunk. It covers the
-// int8/f16/bf16 rhs (no nibble widening on the way) and K that ends on a chunk
-// boundary; everything else uses the kernel above.
+// data-dependent waits other than one counter wait per chunk. (direct_covers
+// says what it takes; everything else uses the kernel above.)
 //
 // Every load moves 16 contiguous bytes per lane, also for the 4-byte row
 // pieces of e.g. the 8x8x4 int8 tiles (G == 4), where 16 contiguous bytes are
@@ -898,14 +896,16 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
 
-  // K may end inside the last chunk (not with an int4 rhs). That chunk is then
+  // K may end inside the last chunk. That chunk is then
   // loaded from where a full chunk ends at K, so it overlaps the chunk before
   // it and every load stays inside the operands, and the overlap, i.e. the
   // first `cut_bytes` of its 64 bytes per row, is zeroed in the fragments of
-  // both operands (0 * 0 adds nothing, whatever the data).
+  // both operands (0 * 0 adds nothing, whatever the data; with an int4 rhs, where 0 * anything
+  // does, in the lhs alone). int4 with an odd number of k steps of 32 went to the register-staged kernel
+  // before: 1360 x 1712 x 1440 23.1 -> 11.6 us, 2512 x 4352 x 1504 51.2 -> 26.1.
   const int chunks = a.chunks;
   const int last_chunk = chunks - 1;
-  const int32_t cut_bytes = RHS_I4 ? 0 : (int32_t)((64 - (((int64_t)a.K << a.log2_lhs_rb) & 63)) & 63);
+  const int32_t cut_bytes = (int32_t)((64 - (((int64_t)a.K << a.log2_lhs_rb) & 63)) & 63);
   const int64_t lhs_last_base = a.K * lhs_kstep - lhs_chunk_bytes;
   const int64_t rhs_last_base = a.K * rhs_kstep - rhs_chunk_bytes;
   const int64_t lhs_last_advance = lhs_last_base - (last_chunk - 1) * lhs_chunk_bytes;
@@ -1025,6 +1025,36 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   const uint32_t own_half = (lane & 1) ? 0x07060302u : 0x05040100u;
   constexpr int KK16 = ROWS16 ? 32 : 64;
 
+  // Zeroes what the last chunk shares with the one before it. Lane half h of K-step kk holds bytes 32*kk + 16*h .. + 15 of
+  // the chunk's 64 bytes per row, in ascending order of k in every layout above; with an int4 rhs bytes 16*kk + 32*h .. + 15.
+  auto cut_fragments = [&](uint4 (*fa)[2], uint4 (*fb)[2]) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int first_byte = RHS_I4 ? 16 * kk + 32 * (lane >> 5) : 32 * kk + 16 * (lane >> 5);
+      const int cut = min(max(cut_bytes - first_byte, 0), 16);
+      uint32_t keep[4];
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        keep[w] = cut >= 4 * w + 4 ? 0u : (cut <= 4 * w ? 0xFFFFFFFFu : 0xFFFFFFFFu << (8 * (cut - 4 * w)));
+#pragma unroll
+      for (int i = 0; i < AM; ++i) {
+        fa[i][kk].x &= keep[0]; fa[i][kk].y &= keep[1]; fa[i][kk].z &= keep[2]; fa[i][kk].w &= keep[3];
+      }
+      if constexpr (!RHS_I4) {
+#pragma unroll
+        for (int j = 0; j < BN; ++j) {
+          fb[j][kk].x &= keep[0]; fb[j][kk].y &= keep[1]; fb[j][kk].z &= keep[2]; fb[j][kk].w &= keep[3];
+        }
+      }
+    }
+  };
+  // Where that happens: behind the loop, in front of the last chunk's step, or in the step that reads its fragments. A
+  // branch in every step costs the smaller tiles (int8 1024^3 in 64x64 tiles 5.86 -> 5.35 us without it, f16 384 x 2912 x
+  // 2848 in 128x64 tiles 17.2 -> 14.8) and all int4 ones (128x128 and 64x128 11 to 14 %). The larger tiles hide it, and
+  // lose more by the further step that the code then has behind the loop, run once and fetched from memory (192x192
+  // tiles 1 us of 16).
+  constexpr bool CUT_BEHIND_LOOP = RHS_I4 || AM * BN <= 4;
+
   // One pipeline step for the chunk whose fragments are in `cur`:
   //   a few MFMAs first (they only need registers, and keep the matrix pipe
   //   fed across the barrier); wait until this wavefront's loads of the next
@@ -1112,7 +1142,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     // The fragments read during this step are those of chunk load_chunk - AHEAD + 1.
     // (The variants with the staggered tail are launched for K in whole chunks only: nothing to cut there, and the
     // masking, which the compiler makes unconditional, 64 instructions per step, is left out.)
-    const bool cut_next = STAGGER == 0 && cut_bytes != 0 && load_chunk - AHEAD + 1 == last_chunk;
+    const bool cut_next = !CUT_BEHIND_LOOP && STAGGER == 0 && cut_bytes != 0 && load_chunk - AHEAD + 1 == last_chunk;
     const uint8_t* read_a = ring_bytes + read_stage_off + frag_a_off + pair_a_lane;
     const uint8_t* read_a_kk1 = read_a + lhs_kk1_step;  // (used where the lhs has 16-byte pieces)
     const uint8_t* read_b = ring_bytes + read_stage_off + frag_b_off + pair_b_lane;
@@ -1196,28 +1226,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (!RHS_I4) {
-      if (cut_next) {
-        // Lane half h of K-step kk holds bytes 32*kk + 16*h .. + 15 of the chunk's
-        // 64 bytes per row, in ascending order of k in every layout above.
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          const int cut = min(max(cut_bytes - 32 * kk - 16 * (lane >> 5), 0), 16);
-          uint32_t keep[4];
-#pragma unroll
-          for (int w = 0; w < 4; ++w)
-            keep[w] = cut >= 4 * w + 4 ? 0u : (cut <= 4 * w ? 0xFFFFFFFFu : 0xFFFFFFFFu << (8 * (cut - 4 * w)));
-#pragma unroll
-          for (int i = 0; i < AM; ++i) {
-            nxt_a[i][kk].x &= keep[0]; nxt_a[i][kk].y &= keep[1]; nxt_a[i][kk].z &= keep[2]; nxt_a[i][kk].w &= keep[3];
-          }
-#pragma unroll
-          for (int j = 0; j < BN; ++j) {
-            nxt_b[j][kk].x &= keep[0]; nxt_b[j][kk].y &= keep[1]; nxt_b[j][kk].z &= keep[2]; nxt_b[j][kk].w &= keep[3];
-          }
-        }
-      }
-    }
+    if (cut_next) cut_fragments(nxt_a, nxt_b);
   };
   auto step = [&](const uint4 (*cur_a)[2], const uint4 (*cur_b)[2], uint4 (*nxt_a)[2], uint4 (*nxt_b)[2],
                   bool held_loads_behind = false) {
@@ -1558,11 +1567,30 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     tail(pa, pb);
     return;
   }
-  for (; kc + 1 < chunks; kc += 2) {
+  if constexpr (CUT_BEHIND_LOOP) {
+    for (; kc + 2 < chunks; kc += 2) {
+      step(pa, pb, qa, qb);
+      step(qa, qb, pa, pb);
+    }
+    if (kc + 1 < chunks) {
+      step(pa, pb, qa, qb);
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+        for (int i = 0; i < AM; ++i) pa[i][kk] = qa[i][kk];
+#pragma unroll
+        for (int j = 0; j < BN; ++j) pb[j][kk] = qb[j][kk];
+      }
+    }
+    if (cut_bytes != 0) cut_fragments(pa, pb);
     step(pa, pb, qa, qb);
-    step(qa, qb, pa, pb);
+  } else {
+    for (; kc + 1 < chunks; kc += 2) {
+      step(pa, pb, qa, qb);
+      step(qa, qb, pa, pb);
+    }
+    if (kc < chunks) step(pa, pb, qa, qb);
   }
-  if (kc < chunks) step(pa, pb, qa, qb);
   // No load may still be writing LDS when the workgroup's allocation is freed.
   wait_loads_but<0>();
   UK_TIMELINE(tl_loop_end = __builtin_amdgcn_s_memrealtime();)
@@ -1809,9 +1837,9 @@ void mmt4d_mfma_split_k_kernel(const MfmaArgs a) {
 // of 32 nibbles), and K is long enough.
 template <bool RHS_I4, int G>
 bool direct_covers(const MfmaArgs& m) {
-  // K ending inside a chunk: not with an int4 rhs, and one full chunk at least.
+  // K ending inside a chunk: one full chunk at least.
   const int64_t row_bytes = (int64_t)m.K * m.lhs_rb;
-  if (row_bytes % 64 != 0 && (RHS_I4 || row_bytes < 64)) return false;
+  if (row_bytes % 64 != 0 && row_bytes < 64) return false;
   if (RHS_I4) return m.rhs_rb >= 16 && (uintptr_t)m.rhs % 16 == 0 && m.rhs_stride_bytes % 16 == 0;
   if (G == 16) return true;
   // One-byte pieces: tiles of 8 or 16 rows (a 16-byte piece is one or two k steps of a whole tile).

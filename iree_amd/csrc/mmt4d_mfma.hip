@@ -13,6 +13,8 @@ int log2_exact(int64_t v) {
   return l;
 }
 
+const WaveKShape& wave_k_shape(int kind, int s) { return kind == kF32 ? kWaveKShapesF32[s] : kWaveKShapes[s]; }
+
 struct Plan {
   int kind;
   bool rhs_i4;
@@ -23,22 +25,55 @@ struct Plan {
 };
 
 // Estimates in microseconds, to choose between the block kernels and the one that splits K over wavefronts. Both write
-// the output at the same rate, which is left out. Measured over 9164 problems (M 8..1100, N 64..28672, K 64..14336, every
+// the output at the same rate, which is left out. Measured over 741 problems (M 8..1100, N 64..28672, K 64..14336, every
 // type and row piece) with operands from HBM (sets of 640 MB in turn, the condition of weights in a model's layers) and
 // with operands that the last-level cache holds (150 MB), the coefficients fitted to the geometric mean of the two: the
-// kernel picked is 0.7 % slower than the best one in the mean, 5 % and more on one problem in 25. Fitted to repeated operands
-// alone they had picked 32x64 tiles for bf16 96 x 14336 x 4096: 27.5 us held and 40.6 from HBM, where the 128x64 tile with
+// kernel picked is 0.5 % slower than the best one in the mean, 5 % and more on one problem in 31. Fitted to repeated operands
+// alone they would pick 32x64 tiles for bf16 96 x 14336 x 4096: 27.5 us held and 40.6 from HBM, where the 128x64 tile with
 // K split takes 23.9 and 32.6; int4 96 x 14336 x 4096 19.1 from HBM against 16.3.
 //
+// f32: measured over 210 problems (M 17..4096, N 64..14336, K 64..8192, up to 8.6 GFLOP, 16- and 4-byte row pieces) with every
+// tile, operands held: the terms below are off by 7 % (rms), the kernel picked is 0.5 % slower than the best one in the
+// mean. The time to write the output is in both, per round of tiles.
+double block_cost_f32(const MfmaArgs& m, int gather, bool direct) {
+  // Microseconds per chunk of kBlockTiles' first five: one workgroup per compute unit, two beside each other.
+  static const double kOne[] = {3.45, 1.83, .94, .494, .272}, kTwo[] = {6.9, 3.66, 1.763, .988, .47};
+  double us_per_chunk;
+  const int tile = choose_tile(m, kF32, false, gather, direct, &us_per_chunk);
+  const TileChoice& t = kBlockTiles[tile];
+  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0, br = 64 * t.am, bc = 64 * t.bn;
+  const int64_t rounds = (((rows + br - 1) / br) * ((cols + bc - 1) / bc) + 255) / 256;
+  us_per_chunk = (rounds & 1) * kOne[tile] + (rounds >> 1) * kTwo[tile];
+  if (!direct) us_per_chunk *= 2.2;  // staged through registers
+  const double chunks_us = m.chunks * us_per_chunk + 1.2 * t.am * t.bn * rounds;
+  const double memory_us = (double)(rows * m.lhs_rb + cols * m.rhs_rb) * m.K / 6.95e6;
+  return 2.0 + (chunks_us > memory_us ? chunks_us : memory_us);
+}
+
+double wave_k_cost_f32(const MfmaArgs& m, const WaveKShape& s, int64_t tiles, bool staged) {
+  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
+  const double megabytes = 1e-6 * (double)(rows * m.lhs_rb + cols * m.rhs_rb) * m.K;
+  const int fragments = s.fa * s.fb;
+  // (K below what was measured: the output is all there is, which the block kernels write as fast.)
+  if (m.chunks < 4 && tiles > 256) return 1e30;
+  // A chunk's multiplies at the pipe's rate, or its loads. Workgroups beside each other start and end beside each other too.
+  const double multiplies = (staged ? 0.02 : 0.0142) * fragments, loads = (staged ? 0.0159 : 0.0107) * (s.fa + s.fb);
+  const double us = 1.9 + (tiles > 256 ? tiles / 256.0 : 1.0) * (0.7 + 0.125 * fragments) +
+                    (tiles + 255) / 256 * m.chunks * (multiplies > loads ? multiplies : loads) + 0.035 * megabytes;
+  const double memory_us = 2.0 + megabytes / 6.95;
+  return us > memory_us ? us : memory_us;
+}
+
 // A block kernel takes a fixed time per 64-byte chunk of K (choose_tile), or what its operands take from memory.
 double block_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
   const bool direct = mfma_direct_covers(m, gather, rhs_i4);
+  if (kind == kF32) return block_cost_f32(m, gather, direct);
   const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
   const double memory_us = (double)(rows * m.lhs_rb + cols * m.rhs_rb) * m.K / 6.95e6;
-  double us_per_chunk, start_us = 3.32;
+  double us_per_chunk, start_us = 3.52;
   if (gather == 16 && (kind == kF16 || kind == kBF16) && direct && split_k_covers(m)) {
     us_per_chunk = 0.163;
-    start_us = 6.6;  // (and the summing of the partial tiles)
+    start_us = 6.8;  // (and the summing of the partial tiles)
   } else {
     choose_tile(m, kind, rhs_i4, gather, direct, &us_per_chunk);
     if (!direct) us_per_chunk *= 2.2;       // staged through registers
@@ -56,16 +91,17 @@ double block_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
 // unit run beside each other where their registers and LDS allow it (not those of the 64x64 tile).
 double wave_k_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather, const WaveKShape& s) {
   const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
-  const int64_t tiles = ((rows + 16 * s.fa - 1) / (16 * s.fa)) * ((cols + 16 * s.fb - 1) / (16 * s.fb));
+  // (In fragments, of which there are fewer than 2^31 either way: divisions of 32 bits.)
+  const int64_t tiles = (int64_t)(((uint32_t)((rows + 15) / 16) + s.fa - 1) / s.fa) * (((uint32_t)((cols + 15) / 16) + s.fb - 1) / s.fb);
   const double row_kb = 1e-3 * m.K * m.lhs_rb, rhs_share = rhs_i4 ? 0.5 : 1.0;
-  const bool narrow = gather < 16;  // row pieces, which pass through LDS
-  double tile_us = 16 * (s.fa + s.fb * rhs_share) * row_kb / (narrow ? 69.5 : 89.2);
-  if (kind == kF32) tile_us = tile_us > 0.0224 * s.fa * s.fb * m.chunks ? tile_us : 0.0224 * s.fa * s.fb * m.chunks;
-  double us = (narrow || rhs_i4 ? 3.07 : 2.53) + 0.057 * s.fa * s.fb + 4.12e-5 * (rows + cols * rhs_share) * row_kb;
+  const bool narrow = gather < 16 && !wave_k_loads_pieces(m, kind, gather, s.fa, s.fb);  // row pieces that pass through LDS
+  if (kind == kF32) return wave_k_cost_f32(m, s, tiles, narrow);
+  const double tile_us = 16 * (s.fa + s.fb * rhs_share) * row_kb / (narrow ? 81.4 : 92.5);
+  double us = (narrow || rhs_i4 ? 3.03 : 2.63) + 0.067 * s.fa * s.fb + 4.6e-5 * (rows + cols * rhs_share) * row_kb;
   if (tiles <= 256) return us + tile_us;
   const double rounds = tiles / 256.0;
   if (tiles > (s.fa * s.fb >= 16 ? 256 : 1024)) us += 1e3 * rounds;
-  return us + (rounds + (narrow ? 0.988 : 0.893)) * tile_us + (narrow ? 0.552 : 0.43) * rounds;
+  return us + (rounds + (narrow ? 0.941 : 0.922)) * tile_us + (narrow ? 0.467 : 0.402) * rounds;
 }
 
 // Whether the kernel that splits K over wavefronts covers the problem: 16-byte aligned operands whose 16 contiguous
@@ -78,8 +114,8 @@ bool wave_k_covers(const MfmaArgs& m, int gather, bool rhs_i4) {
 }
 
 // Fills `plan` if the problem is covered. With `probe_only` only type and tile
-// shape are looked at.
-bool make_plan(const Mmt4dArgs& a, bool probe_only, Plan* plan) {
+// shape are looked at; without `choose` the kernel is left open.
+bool make_plan(const Mmt4dArgs& a, bool probe_only, bool choose, Plan* plan) {
   int kind, elem_bytes;
   bool i4 = false, narrow = false;
   // With a 16-bit output the reference rounds the accumulator after every
@@ -165,10 +201,11 @@ bool make_plan(const Mmt4dArgs& a, bool probe_only, Plan* plan) {
   if (((uintptr_t)a.rhs % rhs_align) || (a.N > 1 && rhs_stride_bytes % rhs_align)) return false;
   if ((gather == 1 || gather == 2 || gather == 8) && !mfma_direct_covers(m, gather, i4)) return false;
   plan->wave_shape = -1;
-  if (!wave_k_covers(m, gather, i4)) return true;
+  if (!choose || !wave_k_covers(m, gather, i4)) return true;
   double best = block_cost(m, kind, i4, gather);
-  for (int s = 0; s < (int)(sizeof kWaveKShapes / sizeof kWaveKShapes[0]); ++s) {
-    const double cost = wave_k_cost(m, kind, i4, gather, kWaveKShapes[s]);
+  const int shapes = kind == kF32 ? sizeof kWaveKShapesF32 / sizeof(WaveKShape) : sizeof kWaveKShapes / sizeof(WaveKShape);
+  for (int s = 0; s < shapes; ++s) {
+    const double cost = wave_k_cost(m, kind, i4, gather, wave_k_shape(kind, s));
     if (cost < best) {
       best = cost;
       plan->wave_shape = s;
@@ -179,7 +216,7 @@ bool make_plan(const Mmt4dArgs& a, bool probe_only, Plan* plan) {
 
 hipError_t launch_wave_k(const Plan& plan, hipStream_t stream, const char** name) {
   const MfmaArgs& m = plan.args;
-  const WaveKShape& shape = kWaveKShapes[plan.wave_shape];
+  const WaveKShape& shape = wave_k_shape(plan.kind, plan.wave_shape);
   *name = shape.name;
   // Weights that one row of tiles reads once are streamed past the caches like those of a matrix-vector product: bf16 64 x
   // 14336 x 4096 (117 MB) from HBM 28.1 -> 24.7 us, read again or just written 20.2 -> 24.3. With several rows of tiles
@@ -200,7 +237,7 @@ hipError_t launch_wave_k(const Plan& plan, hipStream_t stream, const char** name
 
 hipError_t launch_mfma(const Mmt4dArgs& a, hipStream_t stream, const char** name) {
   Plan plan;
-  if (!make_plan(a, false, &plan)) return hipErrorInvalidValue;
+  if (!make_plan(a, false, true, &plan)) return hipErrorInvalidValue;
   if (plan.wave_shape >= 0) return launch_wave_k(plan, stream, name);
   const MfmaArgs& m = plan.args;
   switch (plan.kind) {
@@ -215,7 +252,7 @@ hipError_t launch_mfma(const Mmt4dArgs& a, hipStream_t stream, const char** name
 
 Mmt4dLauncher select_mmt4d_mfma(const Mmt4dArgs& a, bool probe_only) {
   Plan plan;
-  return make_plan(a, probe_only, &plan) ? launch_mfma : nullptr;
+  return make_plan(a, probe_only, false, &plan) ? launch_mfma : nullptr;
 }
 
 }  // namespace uk

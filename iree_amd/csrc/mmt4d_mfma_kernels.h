@@ -88,6 +88,28 @@ struct WaveKShape {
 };
 constexpr WaveKShape kWaveKShapes[] = {{1, 1, "mmt4d_mfma_wave_k_16x16"}, {1, 2, "mmt4d_mfma_wave_k_16x32"}, {2, 2, "mmt4d_mfma_wave_k_32x32"},
                                        {2, 4, "mmt4d_mfma_wave_k_32x64"}, {4, 2, "mmt4d_mfma_wave_k_64x32"}, {4, 4, "mmt4d_mfma_wave_k_64x64"}};
+// f32 is bound by the matrix pipe whatever the tile, and what counts is how evenly the tiles fill the compute units: there is
+// one for every size up to 20 fragments (what the LDS holds of partial sums) that has a use. 80 x 10240 x 3648 takes 108 us
+// in 32x32 tiles and 55 in 80x48 ones (a library product 64), 2704 x 208 x 4032 69 in 64x64 and 41 in 32x80.
+constexpr WaveKShape kWaveKShapesF32[] = {
+    {1, 1, "mmt4d_mfma_wave_k_16x16"}, {1, 2, "mmt4d_mfma_wave_k_16x32"}, {2, 2, "mmt4d_mfma_wave_k_32x32"},
+    {2, 3, "mmt4d_mfma_wave_k_32x48"}, {3, 2, "mmt4d_mfma_wave_k_48x32"}, {2, 4, "mmt4d_mfma_wave_k_32x64"},
+    {4, 2, "mmt4d_mfma_wave_k_64x32"}, {3, 3, "mmt4d_mfma_wave_k_48x48"}, {2, 5, "mmt4d_mfma_wave_k_32x80"},
+    {5, 2, "mmt4d_mfma_wave_k_80x32"}, {3, 4, "mmt4d_mfma_wave_k_48x64"}, {4, 3, "mmt4d_mfma_wave_k_64x48"},
+    {3, 5, "mmt4d_mfma_wave_k_48x80"}, {5, 3, "mmt4d_mfma_wave_k_80x48"}, {4, 4, "mmt4d_mfma_wave_k_64x64"},
+    {4, 5, "mmt4d_mfma_wave_k_64x80"}, {5, 4, "mmt4d_mfma_wave_k_80x64"}};
+// Whether it loads the 4-byte row pieces of a tile of fa x fb fragments one at a time rather than through LDS. An instruction
+// then covers 16 rows at four k steps, contiguous with 16-row tiles (bf16 16x16x2, 512 x 2048 x 8192 29.1 -> 23.9 us, 64 x
+// 432 x 3712 5.44 -> 4.37; f32 16x16x1, 288 x 1584 x 4064 46.7 -> 41.2), and not where lhs tiles of 4 rows and a second row
+// of them break it up (bf16 4x16x2, 512 x 2048 x 8192 35.4 -> 38.4). 8x8 tiles: int8 gains from 8 fragments on (8x8x4, 512 x
+// 2048 x 2048 8.09 -> 7.29, one fragment, 32 x 1680 x 6784, 5.8 -> 6.9), bf16 loses 3 to 5 %; f32, bound by the matrix
+// pipe, gains with any tile (8x8x1, 128 x 4096 x 2048 26.5 -> 21.8).
+inline bool wave_k_loads_pieces(const MfmaArgs& m, int kind, int gather, int fa, int fb) {
+  if (gather != 4) return false;
+  if (kind == kF32) return true;
+  if (kind == kI8 && fa * fb != 2 && fa * fb != 4) return fa * fb >= 8;
+  return m.log2_N0 == 4 && (m.log2_M0 >= 3 || m.M == 1);
+}
 hipError_t launch_wave_k_i8(const MfmaArgs& m, int gather, bool rhs_i4, int shape, bool streamed, hipStream_t stream);
 hipError_t launch_wave_k_f16(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);
 hipError_t launch_wave_k_bf16(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);
@@ -123,10 +145,10 @@ inline bool split_k_covers(const MfmaArgs& m) {
 // matrix pipe whatever the tile, which leaves the number of rounds (in units of a 128x128 tile; the large tiles, which
 // move fewer bytes, are favoured by 10 %).
 // `us_per_chunk`: that least time.
-inline int choose_tile(const MfmaArgs& m, int kind, bool rhs_i4, int gather, bool direct, double* us_per_chunk) {
-  static const TileChoice kTiles[] = {{4, 4, false}, {4, 2, true}, {2, 2, false}, {2, 1, true}, {1, 1, false}, {1, 2, true},
+constexpr TileChoice kBlockTiles[] = {{4, 4, false}, {4, 2, true}, {2, 2, false}, {2, 1, true}, {1, 1, false}, {1, 2, true},
                                       {3, 3, true},  {2, 3, true}, {3, 2, true},  {4, 3, true}, {3, 4, true}};
-  constexpr int kCount = sizeof kTiles / sizeof kTiles[0];
+inline int choose_tile(const MfmaArgs& m, int kind, bool rhs_i4, int gather, bool direct, double* us_per_chunk) {
+  constexpr int kCount = sizeof kBlockTiles / sizeof kBlockTiles[0];
   // Per class of operands and tile, 0: no such instantiation.
   enum { kSixteenBit, kInt8, kTwoBytePieces, kInt4, kFloat32 };
   static const float kOne[][kCount] = {{.51f, .33f, .222f, .148f, .129f, 0, .342f, .25f, .25f, .40f, .405f},
@@ -141,7 +163,7 @@ inline int choose_tile(const MfmaArgs& m, int kind, bool rhs_i4, int gather, boo
   int best = -1;
   double best_cost = 0;
   for (int i = 0; i < kCount; ++i) {
-    const TileChoice& t = kTiles[i];
+    const TileChoice& t = kBlockTiles[i];
     if (kOne[what][i] == 0 || (t.direct_only && !direct)) continue;
     if (gather == 1 && (t.am == 3 || t.bn == 3)) continue;
     // The int4 64x64 tile exists only register-staged, at less than half the

@@ -20,18 +20,19 @@
 // are is free as long as lhs and rhs agree. A load is 16 contiguous bytes per
 // lane and covers one fragment's step, 1 KiB. G = bytes of a row piece:
 //   16 (or more): lane 16*q + r loads 16-byte column q of row r: the operand.
-//   8, 4, 2: 16 contiguous bytes are 16 / G rows of one k step. They pass through
+//   4, as pieces: lane 16*q + r loads the pieces of k steps 4*d + q of row r, d = 0 .. 3, one at a time: 256 contiguous
+//     bytes an instruction with 16-row tiles. (wave_k_loads_pieces says when.)
+//   8, 4, 2, staged: 16 contiguous bytes are 16 / G rows of one k step. They pass through
 //     1 KiB of LDS that only this wavefront uses (no barrier), as [k][16 rows][G
 //     bytes], and come back as the pieces of k steps 4*d + q of row r (8, 4: reads
 //     linear in the lane number) resp. 16*d + 4*q + {0..3} (2: the transposing
-//     read ds_read_b64_tr_b16). Loaded piece by piece instead, without LDS, an
-//     instruction covers short stretches of several tiles, and where these lie a
-//     multiple of 64 KiB apart (int8 8x8x4 at K = 8192) everything took 5 times as long.
+//     read ds_read_b64_tr_b16). (8-byte pieces one at a time: 3 to 15 % slower; the
+//     instruction moves half of what the others do.)
 //   int4 rhs (K0 = 32 or 64): a step is 128 values of K; a lane's 16 bytes are 32
 //     nibbles, widened to two int8 operands of 16x the values, against two
 //     16-byte pieces of the lhs; the sums are shifted right by 4 at the end.
-// K may end inside a step: the last steps are loaded with a check per piece, and
-// what lies beyond K is zero in both operands.
+// K may end inside a step: what lies beyond K in the last one is zeroed in both
+// operands.
 #ifndef IREE_AMD_CSRC_MMT4D_WAVE_K_KERNELS_H_
 #define IREE_AMD_CSRC_MMT4D_WAVE_K_KERNELS_H_
 
@@ -78,38 +79,90 @@ __device__ __forceinline__ uint2 lds_read_transposed_b16(const uint8_t* p) {
   return __builtin_bit_cast(uint2, v);
 }
 
+// Operand memory, said to be global: the base comes from scalar registers by way of an integer (uniform_pointer), and from a
+// pointer that may lead anywhere the compiler makes flat loads. Those may return in any order and count as LDS accesses too,
+// so that the only wait it can put in front of a batch's MFMAs is for every load in flight, the next batch's among them, and
+// nothing is prefetched. Nor may the loads' addresses be made on the vector unit, in 64 bits (see load): those additions and
+// f32 MFMAs get in each other's way. f32 288 x 1584 x 8128 in 32x64 tiles: flat loads 103 us, global ones with additions in
+// front of them 109, with a scalar base and a 32-bit offset 60. bf16 and int8, bound by the loads, 1 to 5 %.
+typedef const __attribute__((address_space(1))) uint8_t* global_bytes_t;
+typedef const __attribute__((address_space(1))) v4i32* global_v4i32_t;
+typedef const __attribute__((address_space(1))) uint32_t* global_u32_t;
+
 // One operand of a workgroup's tile: F fragments, pieces of G bytes. WIDE: the int8 operand that meets an int4 one,
 // two 16-byte pieces per fragment and step.
-template <int G, int F, bool WIDE>
+// PIECES: 4-byte pieces are loaded one at a time.
+template <int G, int F, bool WIDE, bool PIECES>
 struct Operand {
   static constexpr int RAW = WIDE ? 2 * F : F;  // 16-byte registers that hold what one step loads
-  const uint8_t* base;   // uniform: the tile's first row of tiles, k = 0
+  global_bytes_t base;   // uniform: the tile's first row of tiles, k = 0
   uint32_t off[F];       // per lane, from base, at step 0
   uint32_t step_bytes;   // from one step to the next
+  uint32_t kstep_bytes;  // from one k step to the next
   int32_t k_lane;        // k step (within a step) of what this lane loads
-  uint32_t lds_slot;     // G < 16: where in a fragment's 1 KiB the lane's 16 bytes go
+  uint32_t lds_slot;     // staged: where in a fragment's 1 KiB the lane's 16 bytes go
 
-  // What step `s` holds. CHECKED: pieces from k step `K` on read as zero (`k0` = the step's first k step).
+  // What step `s` holds. CHECKED: a lane whose k step (`k0` = the step's first) is not below `K` loads that of K - 1 instead,
+  // for zero_beyond to clear: no branches, and nothing that waits for a load in front of the next one.
   // STREAMED: the caller reads every byte once (non-temporal loads).
   template <bool CHECKED, bool STREAMED>
-  __device__ __forceinline__ void load(int32_t s, int32_t k0, int32_t K, uint4 (&raw)[RAW]) const {
-    const uint8_t* p = base + (uint64_t)(uint32_t)s * step_bytes;
+  __device__ __forceinline__ void load(int32_t s, int32_t k0, int32_t K, uint4 (&raw)[RAW]) {
+    // (The empty statements keep base and offset apart up to the load: where the compiler widens the offset to 64 bits ahead
+    // of the loop, or adds the bases of a step's pieces to it, every load has 64-bit additions in front of it.)
+    global_bytes_t at[PIECES ? 4 : 1];
+#pragma unroll
+    for (int d = 0; d < (PIECES ? 4 : 1); ++d) {
+      at[d] = base + (uint64_t)(uint32_t)s * step_bytes + d * (uint64_t)(step_bytes / 4);
+      asm volatile("" : "+s"(at[d]));
+    }
+    int32_t back[PIECES ? 4 : 1];  // bytes (the k steps that a step has are a power of two)
+    if constexpr (CHECKED) {
+#pragma unroll
+      for (int d = 0; d < (PIECES ? 4 : 1); ++d)
+        back[d] = max(k0 + k_lane + 4 * d - (K - 1), 0) * (int32_t)kstep_bytes;
+    }
 #pragma unroll
     for (int f = 0; f < F; ++f) {
+      asm volatile("" : "+v"(off[f]));
 #pragma unroll
       for (int w = 0; w < RAW / F; ++w) {
         uint4& to = raw[(RAW / F) * f + w];
-        if (CHECKED) to = make_uint4(0, 0, 0, 0);
-        if (!CHECKED || k0 + k_lane < K) {
-          const v4i32* from = (const v4i32*)(p + off[f] + 16 * w);
+        if constexpr (PIECES) {
+          uint32_t piece[4];
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {
+            global_u32_t from = (global_u32_t)(at[d] + off[f]);
+            if constexpr (CHECKED) from = (global_u32_t)((global_bytes_t)from - back[d]);
+            if constexpr (STREAMED) piece[d] = __builtin_nontemporal_load(from);
+            else piece[d] = *from;
+          }
+          to = make_uint4(piece[0], piece[1], piece[2], piece[3]);
+        } else {
+          global_v4i32_t from = (global_v4i32_t)(at[0] + off[f] + 16 * w);
+          if constexpr (CHECKED) from = (global_v4i32_t)((global_bytes_t)from - back[0]);
           if constexpr (STREAMED) to = __builtin_bit_cast(uint4, __builtin_nontemporal_load(from));
           else to = __builtin_bit_cast(uint4, *from);
         }
       }
     }
   }
+  // Clears what a checked load brought from k steps that are not below K.
+  __device__ __forceinline__ void zero_beyond(int32_t k0, int32_t K, uint4 (&raw)[RAW]) const {
+#pragma unroll
+    for (int i = 0; i < RAW; ++i) {
+      if constexpr (PIECES) {
+        raw[i].x = k0 + k_lane < K ? raw[i].x : 0u;
+        raw[i].y = k0 + k_lane + 4 < K ? raw[i].y : 0u;
+        raw[i].z = k0 + k_lane + 8 < K ? raw[i].z : 0u;
+        raw[i].w = k0 + k_lane + 12 < K ? raw[i].w : 0u;
+      } else {
+        const bool below = k0 + k_lane < K;
+        raw[i] = make_uint4(below ? raw[i].x : 0u, below ? raw[i].y : 0u, below ? raw[i].z : 0u, below ? raw[i].w : 0u);
+      }
+    }
+  }
 
-  // G < 16: the loaded 16 bytes of every fragment into the wavefront's LDS, and fragment f back out of it.
+  // Staged: the loaded 16 bytes of every fragment into the wavefront's LDS, and fragment f back out of it.
   __device__ __forceinline__ void to_lds(const uint4 (&raw)[RAW], uint8_t* lds) const {
 #pragma unroll
     for (int f = 0; f < F; ++f) *(uint4*)(lds + 1024 * f + lds_slot) = raw[f];
@@ -129,13 +182,15 @@ struct Operand {
   }
 };
 
-template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int UNROLL, bool STREAMED>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, FA * FB >= 16 ? 2 : 4)))
+template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int UNROLL, bool STREAMED, bool PIECES>
+__global__ __launch_bounds__(64 * WAVES)
+__attribute__((amdgpu_waves_per_eu(2, FA * FB >= 16 ? 2 : 4)))
 void mmt4d_wave_k_kernel(const MfmaArgs a) {
   typedef typename Acc16<KIND>::type acc_t;
-  typedef Operand<G, FA, RHS_I4> lhs_t;
-  typedef Operand<G, FB, false> rhs_t;
-  constexpr bool STAGED = G < 16;  // operands pass through LDS
+  typedef Operand<G, FA, RHS_I4, PIECES> lhs_t;
+  typedef Operand<G, FB, false, PIECES> rhs_t;
+  static_assert(!PIECES || G == 4, "4-byte pieces");
+  constexpr bool STAGED = G < 16 && !PIECES;  // operands pass through LDS
   static_assert(!RHS_I4 || (KIND == kI8 && G == 16), "int4 rhs");
   // The wavefronts' staging of narrow row pieces, [WAVES][UNROLL][FA + FB][1 KiB]; then [WAVES][FA * FB][64] partial sums.
   extern __shared__ uint4 ring[];
@@ -152,11 +207,17 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
                     int log2_rb, int32_t lane_bytes) {
     const int64_t kstep = (int64_t)rb << log2_t0;
     const int32_t first_tile = (int32_t)(first >> log2_t0);
-    op.base = uniform_pointer(base + first_tile * stride);
+    op.base = (global_bytes_t)uniform_pointer(base + first_tile * stride);
     op.step_bytes = (uint32_t)(4 * lane_bytes) << log2_t0;
+    op.kstep_bytes = (uint32_t)kstep;
     int32_t row;  // of the fragment
     int64_t lane_off;
-    if constexpr (G == 16) {
+    if constexpr (PIECES) {
+      row = r;
+      op.k_lane = q;
+      lane_off = q * kstep;
+      op.lds_slot = 0;
+    } else if constexpr (G == 16) {
       row = r;
       op.k_lane = (lane_bytes * q) >> log2_rb;
       lane_off = op.k_lane * kstep + ((lane_bytes * q) & (rb - 1));
@@ -188,7 +249,6 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
   for (int i = 0; i < FA; ++i)
 #pragma unroll
     for (int j = 0; j < FB; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
-
   // Batches of UNROLL steps, whose loads are in flight together, are dealt out to the wavefronts in turn: at any time
   // the workgroup reads one contiguous stretch of every row panel. (A contiguous share of K per wavefront puts all
   // loads of a launch at the same few offsets modulo the share: 5 to 10 % slower.)
@@ -214,9 +274,16 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       const int32_t s = all_batches * UNROLL + u;
-      const int32_t K = s < steps ? a.K : 0;
-      rhs.template load<true, false>(s, s * ksteps_per_step, K, to.r[u]);
-      lhs.template load<true, false>(s, s * ksteps_per_step, K, to.l[u]);
+      rhs.template load<true, false>(s, s * ksteps_per_step, a.K, to.r[u]);
+      lhs.template load<true, false>(s, s * ksteps_per_step, a.K, to.l[u]);
+    }
+  };
+  auto zero_rest = [&](Batch& of) {
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const int32_t k0 = (all_batches * UNROLL + u) * ksteps_per_step;
+      rhs.zero_beyond(k0, a.K, of.r[u]);
+      lhs.zero_beyond(k0, a.K, of.l[u]);
     }
   };
   auto multiply = [&](const Batch& from) {
@@ -278,14 +345,21 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
         multiply(p);
         if (has_rest) fetch_rest(p);
         multiply(n);
-        if (has_rest) multiply(p);
+        if (has_rest) {
+          zero_rest(p);
+          multiply(p);
+        }
       } else {
         if (has_rest) fetch_rest(n);
         multiply(p);
-        if (has_rest) multiply(n);
+        if (has_rest) {
+          zero_rest(n);
+          multiply(n);
+        }
       }
     } else if (has_rest) {
       fetch_rest(p);
+      zero_rest(p);
       multiply(p);
     }
   }
@@ -334,15 +408,16 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
   }
 }
 
-template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int UNROLL>
-hipError_t launch_wave_k_tile(MfmaArgs m, bool streamed, hipStream_t stream) {
+template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int UNROLL, bool PIECES>
+hipError_t launch_wave_k_loads(MfmaArgs m, bool streamed, hipStream_t stream) {
   unsigned grid;
   set_tile_grid(&m, 16 * FA, 16 * FB, &grid);
-  constexpr int staging_kib = G < 16 ? WAVES * UNROLL * (FA + FB) : 0, partial_kib = WAVES * FA * FB;
+  constexpr int staging_kib = G < 16 && !PIECES ? WAVES * UNROLL * (FA + FB) : 0, partial_kib = WAVES * FA * FB;
   constexpr int lds_bytes = 1024 * (staging_kib > partial_kib ? staging_kib : partial_kib);
-  auto kernel = mmt4d_wave_k_kernel<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, false>;
+  static_assert(lds_bytes <= 160 * 1024, "partial sums do not fit the LDS");
+  auto kernel = mmt4d_wave_k_kernel<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, false, PIECES>;
   if constexpr (G == 16) {
-    if (streamed) kernel = mmt4d_wave_k_kernel<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, true>;
+    if (streamed) kernel = mmt4d_wave_k_kernel<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, true, PIECES>;
   }
   if (lds_bytes > 65536) {
     const hipError_t attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
@@ -351,14 +426,28 @@ hipError_t launch_wave_k_tile(MfmaArgs m, bool streamed, hipStream_t stream) {
   return launch_kernel<MfmaArgs>(kernel, grid, 64 * WAVES, lds_bytes, stream, m);
 }
 
+template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int UNROLL>
+hipError_t launch_wave_k_tile(const MfmaArgs& m, bool streamed, hipStream_t stream) {
+  if constexpr (G != 4) {
+    return launch_wave_k_loads<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, false>(m, streamed, stream);
+  } else if constexpr (KIND == kF32) {
+    return launch_wave_k_loads<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, true>(m, streamed, stream);
+  } else {
+    return wave_k_loads_pieces(m, KIND, G, FA, FB)
+               ? launch_wave_k_loads<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, true>(m, streamed, stream)
+               : launch_wave_k_loads<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, false>(m, streamed, stream);
+  }
+}
+
+// One 64-byte step of K in flight ahead of the one that is multiplied, for each of eight wavefronts. (What is left of K
+// after whole batches is one wavefront's work, and longer batches leave more: four and two steps a batch for the tiles of one
+// and of two to four fragments took 3 to 12 % longer near where these tiles are the best, 2 % less nowhere.)
 template <int KIND, bool RHS_I4, bool NARROW, int G>
 hipError_t launch_wave_k_piece(const MfmaArgs& m, int shape, bool streamed, hipStream_t stream) {
-  // (8 wavefronts; steps in flight per wavefront such that two batches of the small tiles fit 128 registers, which
-  // leaves room for a second workgroup on the compute unit: 128 x 4096 x 4096 bf16 in 32x32 tiles 15.6 -> 13.7 us.)
   switch (shape) {
-    case 0: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 1, 8, 4>(m, streamed, stream);
-    case 1: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 2, 8, 2>(m, streamed, stream);
-    case 2: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 2, 2, 8, 2>(m, streamed, stream);
+    case 0: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 1, 8, 1>(m, streamed, stream);
+    case 1: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 2, 8, 1>(m, streamed, stream);
+    case 2: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 2, 2, 8, 1>(m, streamed, stream);
     case 3: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 2, 4, 8, 1>(m, streamed, stream);
     case 4: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 4, 2, 8, 1>(m, streamed, stream);
     case 5: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 4, 4, 8, 1>(m, streamed, stream);

@@ -66,94 +66,107 @@ __device__ __forceinline__ uint4 load_rhs(const uint8_t* p) {
   else return *(const uint4*)p;
 }
 
-// TN: rhs tiles per workgroup. UNROLL: K-steps whose loads are in flight together.
-template <int KIND, int TN, int UNROLL, int kWaves, bool STREAMED>
+// UNROLL: K-steps whose loads a wavefront has in flight: a ring of operand registers, each loaded again as soon as it is
+// multiplied. A share's last steps, of any number, are one batch of loads too.
+// SPLIT: workgroups per rhs tile, 16 / SPLIT of its rows each, against at most as many lhs rows. Rows 0 .. 16 / SPLIT - 1
+// of both operands are then those rows at the first 64 bytes of a K-step of 64 * SPLIT, the next rows the same rows at the
+// next 64 bytes: of the product the SPLIT blocks on the diagonal count, and are summed at the end.
+template <int KIND, int UNROLL, int kWaves, int SPLIT, bool STREAMED>
 __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_kernel(const GemvArgs a) {
   typedef typename Acc<KIND>::type acc_t;
-  __shared__ acc_t partial[kWaves][TN][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = lane & 15, g = lane >> 4;
+  constexpr int ROWS = 16 / SPLIT;
+  __shared__ acc_t partial[kWaves][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = lane & (ROWS - 1), g = lane >> 4;
+  const int k_part = (lane & 15) / ROWS;  // which 64 bytes of the K-step
   const int32_t M0 = 1 << a.log2_M0;
-  const int32_t lhs_rows = a.M << a.log2_M0;  // <= 16
+  const int32_t lhs_rows = a.M << a.log2_M0;  // <= ROWS
 
   // Per-lane byte offset of its 16-byte operand column inside one K-step, as a
-  // function of the step: k1 = (64*step + 16*g) >> log2_rb.
-  const int32_t ksteps_per_step = 64 >> a.log2_rb;
-  const int32_t k1_lane = (16 * g) >> a.log2_rb;
+  // function of the step: k1 = (64*SPLIT*step + 64*k_part + 16*g) >> log2_rb.
+  const int32_t ksteps_per_step = (64 * SPLIT) >> a.log2_rb;
+  const int32_t k1_lane = (64 * k_part + 16 * g) >> a.log2_rb;
   const int32_t within = (16 * g) & (a.rb - 1);
   const int64_t rhs_kstep = (int64_t)a.rb * 16;
   const int64_t lhs_kstep = (int64_t)a.rb << a.log2_M0;
+  constexpr int32_t rhs_step = 1024 * SPLIT;  // bytes of a K-step
+  const int64_t lhs_step = (int64_t)(64 * SPLIT) << a.log2_M0;
 
-  const bool lhs_valid = row < lhs_rows;
-  const uint8_t* lhs_lane = a.lhs + (int64_t)(row >> a.log2_M0) * a.lhs_stride_bytes +
-                            (int64_t)(row & (M0 - 1)) * a.rb + k1_lane * lhs_kstep + within;
-  const int64_t tile0 = (int64_t)blockIdx.x * TN;
-  const uint8_t* rhs_lane[TN];
-#pragma unroll
-  for (int t = 0; t < TN; ++t) {
-    const int64_t tile = tile0 + t < a.N ? tile0 + t : a.N - 1;  // clamp: computed, not stored
-    rhs_lane[t] = a.rhs + tile * a.rhs_stride_bytes + (int64_t)row * a.rb + k1_lane * rhs_kstep + within;
+  // This wavefront's share of the whole K-steps.
+  const int32_t full_steps = a.K / ksteps_per_step;
+  const int32_t share = full_steps / kWaves, longer = full_steps % kWaves;
+  const int32_t s_begin = wave * share + min(wave, longer);
+  int32_t left = share + (wave < longer);
+
+  // (Lanes of lhs rows that do not exist load the last one's: a row reaches its own row of the result only.)
+  const int lhs_row = min(row, lhs_rows - 1);
+  const int64_t tile = blockIdx.x / SPLIT;
+  const int rhs_row0 = (blockIdx.x % SPLIT) * ROWS;
+  const uint8_t* lhs = a.lhs + (int64_t)(lhs_row >> a.log2_M0) * a.lhs_stride_bytes + (int64_t)(lhs_row & (M0 - 1)) * a.rb +
+                       k1_lane * lhs_kstep + within;
+  const uint8_t* rhs = a.rhs + tile * a.rhs_stride_bytes + (int64_t)(rhs_row0 + row) * a.rb + k1_lane * rhs_kstep + within;
+
+  // K may end inside a step: its lanes beyond K hold zeros. The last wavefront multiplies it, at the end.
+  const bool has_rest = wave == kWaves - 1 && full_steps * ksteps_per_step < a.K;
+  uint4 rest_l = make_uint4(0, 0, 0, 0), rest_r = rest_l;
+  if (has_rest && full_steps * ksteps_per_step + k1_lane < a.K) {
+    rest_l = *(const uint4*)(lhs + full_steps * lhs_step);
+    rest_r = *(const uint4*)(rhs + (int64_t)full_steps * rhs_step);
   }
 
-  acc_t acc[TN];
+  acc_t acc = acc_t{0, 0, 0, 0};
+  uint4 l[UNROLL], r[UNROLL];
+  lhs += s_begin * lhs_step;
+  rhs += (int64_t)s_begin * rhs_step;
+  auto load = [&](int u) {
+    l[u] = *(const uint4*)(lhs + u * lhs_step);
+    r[u] = load_rhs<STREAMED>(rhs + u * rhs_step);
+  };
+  auto next_batch = [&] {
+    left -= UNROLL;
+    lhs += UNROLL * lhs_step;
+    rhs += UNROLL * rhs_step;
+  };
+  if (left >= UNROLL) {
 #pragma unroll
-  for (int t = 0; t < TN; ++t) acc[t] = acc_t{0, 0, 0, 0};
-
-  // This wavefront's share of the K-steps.
-  const int32_t per_wave = (a.steps + kWaves - 1) / kWaves;
-  const int32_t s_begin = wave * per_wave;
-  const int32_t s_end = min(s_begin + per_wave, a.steps);
-  // Steps whose k steps all lie below K need no checks.
-  const int32_t full_steps = a.K / ksteps_per_step;
-
-  int32_t s = s_begin;
-  for (; s + UNROLL <= min(s_end, full_steps); s += UNROLL) {
-    uint4 l[UNROLL], r[UNROLL][TN];
+    for (int u = 0; u < UNROLL; ++u) load(u);
+    next_batch();
+    while (left >= UNROLL) {
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        acc = mfma16<KIND>(r[u], l[u], acc);
+        load(u);
+        __builtin_amdgcn_sched_barrier(0);  // (no load moves in front of the multiplication of what its registers hold)
+      }
+      next_batch();
+    }
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-      const int64_t k1 = (int64_t)(s + u) * ksteps_per_step;
-      l[u] = make_uint4(0, 0, 0, 0);
-      if (lhs_valid) l[u] = *(const uint4*)(lhs_lane + k1 * lhs_kstep);
-#pragma unroll
-      for (int t = 0; t < TN; ++t) r[u][t] = load_rhs<STREAMED>(rhs_lane[t] + k1 * rhs_kstep);
+      acc = mfma16<KIND>(r[u], l[u], acc);
+      if (u < left) load(u);
     }
+  } else {
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u)
-#pragma unroll
-      for (int t = 0; t < TN; ++t) acc[t] = mfma16<KIND>(r[u][t], l[u], acc[t]);
+    for (int u = 0; u < UNROLL - 1; ++u)
+      if (u < left) load(u);
   }
-  for (; s < s_end; ++s) {
-    const int64_t k1 = (int64_t)s * ksteps_per_step;
-    const bool in_k = k1 + k1_lane < a.K;
-    uint4 l = make_uint4(0, 0, 0, 0);
-    if (lhs_valid && in_k) l = *(const uint4*)(lhs_lane + k1 * lhs_kstep);
 #pragma unroll
-    for (int t = 0; t < TN; ++t) {
-      uint4 r = make_uint4(0, 0, 0, 0);
-      if (in_k) r = *(const uint4*)(rhs_lane[t] + k1 * rhs_kstep);
-      acc[t] = mfma16<KIND>(r, l, acc[t]);
-    }
-  }
+  for (int u = 0; u < UNROLL - 1; ++u)
+    if (u < left) acc = mfma16<KIND>(r[u], l[u], acc);
+  if (has_rest) acc = mfma16<KIND>(rest_r, rest_l, acc);
 
-#pragma unroll
-  for (int t = 0; t < TN; ++t) partial[wave][t][lane] = acc[t];
+  partial[wave][lane] = acc;
   __syncthreads();
-  if (wave != 0) return;
-  // Lane l holds lhs row l & 15 and rhs rows 4*(l >> 4) + {0..3} of each tile:
-  // four consecutive j0 of output row i0.
-  if (!lhs_valid) return;
+  // Lane l holds row l & 15 of the lhs operand and rows 4*(l >> 4) + {0..3} of the rhs operand: four consecutive j0 of
+  // output row i0.
+  if (wave != 0 || (lane & 15) >= lhs_rows || g >= 4 / SPLIT) return;
+  acc = partial[0][lane];
 #pragma unroll
-  for (int t = 0; t < TN; ++t) {
-    if (tile0 + t >= a.N) continue;
-    acc_t v = partial[0][t][lane];
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w) v += partial[w][t][lane];
-    acc_t* dst = (acc_t*)(a.out + 4 * ((int64_t)(row >> a.log2_M0) * a.out_stride0 +
-                                       (tile0 + t) * ((int64_t)M0 * 16) +
-                                       (int64_t)(row & (M0 - 1)) * 16 + 4 * g));
-    if (a.accumulate) v += *dst;
-    *dst = v;
-  }
+  for (int i = 1; i < kWaves * SPLIT; ++i) acc += partial[i / SPLIT][lane + (i % SPLIT) * (64 / SPLIT + ROWS)];
+  acc_t* dst = (acc_t*)(a.out + 4 * ((int64_t)(row >> a.log2_M0) * a.out_stride0 + tile * ((int64_t)M0 * 16) +
+                                     (int64_t)(row & (M0 - 1)) * 16 + rhs_row0 + 4 * g));
+  if (a.accumulate) acc += *dst;
+  *dst = acc;
 }
 
 // The same product for more than 4 lhs rows, where the lhs operand of a K-step
@@ -603,6 +616,12 @@ bool launch_resident_lhs(const GemvArgs& g, hipStream_t stream, hipError_t* stat
   }
 }
 
+template <int KIND, int SPLIT>
+hipError_t launch_split(const GemvArgs& g, hipStream_t stream) {
+  return launch_kernel<GemvArgs>(streamed_rhs(g, g.rb) ? mmt4d_gemv_kernel<KIND, 8, 4, SPLIT, true>
+                                                       : mmt4d_gemv_kernel<KIND, 8, 4, SPLIT, false>, g.N * SPLIT, 256, 0, stream, g);
+}
+
 template <int KIND>
 hipError_t launch_kind(const GemvArgs& g, hipStream_t stream, const char** name) {
   hipError_t status;
@@ -610,10 +629,15 @@ hipError_t launch_kind(const GemvArgs& g, hipStream_t stream, const char** name)
     *name = "mmt4d_gemv_resident_lhs";
     return status;
   }
-  // One rhs tile per workgroup (most workgroups, best balance over the CUs),
-  // 4 wavefronts splitting K, 16 KiB of rhs in flight per wavefront.
-  return launch_kernel<GemvArgs>(streamed_rhs(g, g.rb) ? mmt4d_gemv_kernel<KIND, 1, 16, 4, true>
-                                                              : mmt4d_gemv_kernel<KIND, 1, 16, 4, false>, g.N, 256, 0, stream, g);
+  // Four wavefronts splitting K, eight loads of 1 KiB of rhs in flight in each: 4 to 20 % ahead of 16 loads or of 8 and 16
+  // wavefronts over 130 problems of 16 to 1800 tiles. Tiles are split where there are too few to occupy the units, whose
+  // loads then limit (at most 60 GB/s of rhs each: 8 x 544 x 11264 f16 7.6 -> 5.7 us with two to a tile, 1 x 400 x 13744 8.1
+  // -> 5.5 -> 4.6 with four), and where few more tiles than units give some units two (1 x 4752 x 13584 bf16 26.5 -> 23.1 us
+  // with two); with 139 to 248 tiles halves lose up to 18 %, with 400 and more up to 4 %.
+  const int units = compute_units(), rows = g.M << g.log2_M0;
+  if (rows <= 4 && g.N <= units * 3 / 16) return launch_split<KIND, 4>(g, stream);
+  if (rows <= 8 && (g.N <= units / 2 || (g.N > units && g.N <= units * 3 / 2))) return launch_split<KIND, 2>(g, stream);
+  return launch_split<KIND, 1>(g, stream);
 }
 
 hipError_t launch_gemv(const Mmt4dArgs& a, hipStream_t stream, const char** name) {

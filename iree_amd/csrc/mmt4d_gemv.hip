@@ -36,7 +36,7 @@ struct GemvArgs {
   int32_t M, N, K;
   int32_t log2_M0;
   int32_t rb, log2_rb;  // bytes of one (k, row) piece
-  int32_t steps;        // MFMA K-steps: ceil(K * rb / 64)
+  int32_t steps;        // MFMA K-steps: ceil(K * rb / 64); int4: whole ones of 128 values
   int32_t accumulate;
 };
 
@@ -320,34 +320,41 @@ __device__ __forceinline__ uint4 lhs_bytes_even_then_odd(uint4 v) {
 // until the end; K * K0 < 131072 keeps that inside int32.
 // TN rhs tiles per workgroup share each lhs operand: with 16 lhs rows the lhs
 // is twice the bytes of one rhs tile per step (int8 against int4), all of it
-// through L2 for every workgroup.
-template <int TN, int UNROLL, int kWaves, bool STREAMED>
+// through L2 for every workgroup. The ring of UNROLL loads and SPLIT as in mmt4d_gemv_kernel.
+template <int TN, int UNROLL, int kWaves, int SPLIT, bool STREAMED>
 __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_i4_kernel(const GemvArgs a) {
+  static_assert(TN == 1 || SPLIT == 1, "several tiles to a workgroup or several workgroups to a tile");
+  constexpr int ROWS = 16 / SPLIT;
   __shared__ v4i32 partial[kWaves][TN][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = lane & (ROWS - 1), g = lane >> 4;
+  const int k_part = (lane & 15) / ROWS;  // which 128 values of the K-step
   const int32_t M0 = 1 << a.log2_M0;
-  const int32_t lhs_rows = a.M << a.log2_M0;  // <= 16
+  const int32_t lhs_rows = a.M << a.log2_M0;  // <= ROWS
   // a.rb / a.log2_rb describe the lhs row piece (K0 bytes); the rhs piece is half of it.
   const int32_t rhs_rb = a.rb >> 1, log2_rhs_rb = a.log2_rb - 1;
   const int64_t lhs_kstep = (int64_t)a.rb << a.log2_M0;
-  const bool lhs_valid = row < lhs_rows;
-  const uint8_t* lhs_lane = a.lhs + (int64_t)(row >> a.log2_M0) * a.lhs_stride_bytes +
-                            (int64_t)(row & (M0 - 1)) * a.rb + ((32 * g) >> a.log2_rb) * lhs_kstep +
-                            ((32 * g) & (a.rb - 1));
-  const int64_t lhs_step_bytes = (int64_t)128 << a.log2_M0;
-  const int64_t tile0 = (int64_t)blockIdx.x * TN;
-  const uint8_t* rhs_lane[TN];
+  constexpr int32_t rhs_step = 1024 * SPLIT;  // bytes of a K-step of 128 * SPLIT values
+  const int64_t lhs_step = (int64_t)(128 * SPLIT) << a.log2_M0;
+
+  const int32_t columns = (int32_t)(((int64_t)a.K * a.rb) >> 5);  // of 32 values of K, one a lane
+  const int32_t full_steps = columns / (4 * SPLIT);
+  const int32_t share = full_steps / kWaves, longer = full_steps % kWaves;
+  const int32_t s_begin = wave * share + min(wave, longer);
+  int32_t left = share + (wave < longer);
+
+  const int lhs_row = min(row, lhs_rows - 1);  // (rows that do not exist, see mmt4d_gemv_kernel)
+  const uint8_t* lhs = a.lhs + (int64_t)(lhs_row >> a.log2_M0) * a.lhs_stride_bytes + (int64_t)(lhs_row & (M0 - 1)) * a.rb +
+                       ((128 * k_part + 32 * g) >> a.log2_rb) * lhs_kstep + ((32 * g) & (a.rb - 1));
+  const int64_t tile0 = SPLIT > 1 ? blockIdx.x / SPLIT : (int64_t)blockIdx.x * TN;
+  const int rhs_row0 = (blockIdx.x % SPLIT) * ROWS;
+  const uint8_t* rhs[TN];
 #pragma unroll
   for (int t = 0; t < TN; ++t) {
     const int64_t tile = tile0 + t < a.N ? tile0 + t : a.N - 1;  // clamp: computed, not stored
-    rhs_lane[t] = a.rhs + tile * a.rhs_stride_bytes + (int64_t)row * rhs_rb +
-                  ((16 * g) >> log2_rhs_rb) * ((int64_t)rhs_rb * 16) + ((16 * g) & (rhs_rb - 1));
+    rhs[t] = a.rhs + tile * a.rhs_stride_bytes + (int64_t)(rhs_row0 + row) * rhs_rb + k_part * 1024 +
+             ((16 * g) >> log2_rhs_rb) * ((int64_t)rhs_rb * 16) + ((16 * g) & (rhs_rb - 1));
   }
-
-  const int32_t per_wave = (a.steps + kWaves - 1) / kWaves;
-  const int32_t s_begin = wave * per_wave;
-  const int32_t s_end = min(s_begin + per_wave, a.steps);
 
   v4i32 acc[TN];
 #pragma unroll
@@ -358,51 +365,81 @@ __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_i4_kernel(const GemvAr
     acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i32, widen_i4_times16(r.z, r.w)),
                                                    __builtin_bit_cast(v4i32, l1), acc[t], 0, 0, 0);
   };
-  int32_t s = s_begin;
-  // (Lanes of lhs rows that do not exist never load: their operands stay zero, set once.)
-  uint4 l0[UNROLL], l1[UNROLL];
+
+  // K may end inside a step: its lanes beyond K hold zeros. The last wavefront multiplies it, at the end.
+  const bool has_rest = wave == kWaves - 1 && full_steps * (4 * SPLIT) < columns;
+  uint4 rest_l0 = make_uint4(0, 0, 0, 0), rest_l1 = rest_l0, rest_r[TN];
 #pragma unroll
-  for (int u = 0; u < UNROLL; ++u) l0[u] = l1[u] = make_uint4(0, 0, 0, 0);
-  for (; s + UNROLL <= s_end; s += UNROLL) {
-    uint4 r[UNROLL][TN];
+  for (int t = 0; t < TN; ++t) rest_r[t] = rest_l0;
+  if (has_rest && full_steps * (4 * SPLIT) + 4 * k_part + g < columns) {
+    rest_l0 = *(const uint4*)(lhs + full_steps * lhs_step);
+    rest_l1 = *(const uint4*)(lhs + full_steps * lhs_step + 16);
+#pragma unroll
+    for (int t = 0; t < TN; ++t) rest_r[t] = *(const uint4*)(rhs[t] + (int64_t)full_steps * rhs_step);
+  }
+
+  uint4 l0[UNROLL], l1[UNROLL], r[UNROLL][TN];
+  auto advance = [&](int32_t steps) {
+    lhs += steps * lhs_step;
+#pragma unroll
+    for (int t = 0; t < TN; ++t) rhs[t] += (int64_t)steps * rhs_step;
+  };
+  auto load = [&](int u) {
+    l0[u] = *(const uint4*)(lhs + u * lhs_step);
+    l1[u] = *(const uint4*)(lhs + u * lhs_step + 16);
+#pragma unroll
+    for (int t = 0; t < TN; ++t) r[u][t] = load_rhs<STREAMED>(rhs[t] + u * rhs_step);
+  };
+  auto multiply_step = [&](int u) {
+#pragma unroll
+    for (int t = 0; t < TN; ++t) multiply(t, r[u][t], l0[u], l1[u]);
+  };
+  advance(s_begin);
+  if (left >= UNROLL) {
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) load(u);
+    left -= UNROLL;
+    advance(UNROLL);
+    while (left >= UNROLL) {
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        multiply_step(u);
+        load(u);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      left -= UNROLL;
+      advance(UNROLL);
+    }
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-#pragma unroll
-      for (int t = 0; t < TN; ++t)
-        r[u][t] = load_rhs<STREAMED>(rhs_lane[t] + (int64_t)(s + u) * 1024);
-      if (lhs_valid) {
-        l0[u] = *(const uint4*)(lhs_lane + (s + u) * lhs_step_bytes);
-        l1[u] = *(const uint4*)(lhs_lane + (s + u) * lhs_step_bytes + 16);
-      }
+      multiply_step(u);
+      if (u < left) load(u);
     }
+  } else {
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u)
-#pragma unroll
-      for (int t = 0; t < TN; ++t) multiply(t, r[u][t], l0[u], l1[u]);
+    for (int u = 0; u < UNROLL - 1; ++u)
+      if (u < left) load(u);
   }
-  for (; s < s_end; ++s) {
-    uint4 l0 = make_uint4(0, 0, 0, 0), l1 = l0;
-    if (lhs_valid) {
-      l0 = *(const uint4*)(lhs_lane + s * lhs_step_bytes);
-      l1 = *(const uint4*)(lhs_lane + s * lhs_step_bytes + 16);
-    }
 #pragma unroll
-    for (int t = 0; t < TN; ++t) multiply(t, *(const uint4*)(rhs_lane[t] + (int64_t)s * 1024), l0, l1);
-  }
+  for (int u = 0; u < UNROLL - 1; ++u)
+    if (u < left) multiply_step(u);
+  if (has_rest)
+#pragma unroll
+    for (int t = 0; t < TN; ++t) multiply(t, rest_r[t], rest_l0, rest_l1);
 
 #pragma unroll
   for (int t = 0; t < TN; ++t) partial[wave][t][lane] = acc[t];
   __syncthreads();
-  if (wave != 0 || !lhs_valid) return;
+  if (wave != 0 || (lane & 15) >= lhs_rows || g >= 4 / SPLIT) return;
 #pragma unroll
   for (int t = 0; t < TN; ++t) {
     if (tile0 + t >= a.N) continue;
     v4i32 v = partial[0][t][lane];
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) v += partial[w][t][lane];
+    for (int i = 1; i < kWaves * SPLIT; ++i) v += partial[i / SPLIT][t][lane + (i % SPLIT) * (64 / SPLIT + ROWS)];
     v = v4i32{v.x >> 4, v.y >> 4, v.z >> 4, v.w >> 4};
     v4i32* dst = (v4i32*)(a.out + 4 * ((int64_t)(row >> a.log2_M0) * a.out_stride0 + (tile0 + t) * ((int64_t)M0 * 16) +
-                                       (int64_t)(row & (M0 - 1)) * 16 + 4 * g));
+                                       (int64_t)(row & (M0 - 1)) * 16 + rhs_row0 + 4 * g));
     if (a.accumulate) v += *dst;
     *dst = v;
   }
@@ -549,8 +586,8 @@ bool make_args(const Mmt4dArgs& a, bool probe_only, int* kind, GemvArgs* g) {
   if (a.N < 16) return false;
   const int64_t lhs_stride_bytes = a.lhs_stride0 * elem_bytes;
   const int64_t rhs_stride_bytes = i4 ? a.rhs_stride0 / 2 : a.rhs_stride0 * elem_bytes;
-  // int4: whole steps of 128 K values only, and the 16x-scaled sums must fit int32.
-  if (i4 && (((int64_t)a.K * a.K0) % 128 != 0 || (int64_t)a.K * a.K0 >= 131072)) return false;
+  // int4: a whole step of 128 K values at least, and the 16x-scaled sums must fit int32.
+  if (i4 && ((int64_t)a.K * a.K0 < 128 || (int64_t)a.K * a.K0 >= 131072)) return false;
   if ((uintptr_t)a.lhs % 16 || (a.M > 1 && lhs_stride_bytes % 16)) return false;
   if ((uintptr_t)a.rhs % 16 || rhs_stride_bytes % 16) return false;
   if ((uintptr_t)a.out % 16 || (a.M > 1 && a.out_stride0 % 4)) return false;
@@ -654,7 +691,7 @@ hipError_t launch_gemv(const Mmt4dArgs& a, hipStream_t stream, const char** name
     const bool streamed = streamed_rhs(g, g.rb / 2);
     constexpr int MAX_TILES = 8;
     if (((g.M << g.log2_M0) > 4 || g.N >= 6 * (int64_t)units) && units > 0 && g.N >= units && (2 * (int64_t)g.N + units - 1) / units / 2 + 1 <= MAX_TILES &&
-        (g.steps == 64 || g.steps == 32)) {
+        (int64_t)g.K * g.rb % 128 == 0 && (g.steps == 64 || g.steps == 32)) {
       const int lds_bytes = 128 * 1024;  // the lhs operands of 64 steps; the partial sums need less
       // (16 wavefronts x 4 steps with three tiles' loads in flight: 0.65 of the HBM peak at 16 x 28672 x 8192 against
       // 0.62 for the kernel below; 8 wavefronts x 8 steps 0.63, deeper prefetch slower.)
@@ -665,16 +702,26 @@ hipError_t launch_gemv(const Mmt4dArgs& a, hipStream_t stream, const char** name
       *name = "mmt4d_gemv_resident_lhs";
       return launch_kernel(kernel, units, g.steps == 64 ? 1024 : 512, lds_bytes, stream, g);
     }
-    // More than 4 lhs rows: two rhs tiles per workgroup (measured on 16 rows x
-    // 65536 x 8192: 4.5 TB/s with one, 5.9 with two, 4.9 with four).
-    // No more tiles than compute units and a long K: a workgroup has a unit to itself, 16 wavefronts (16 x 512 x 12288 9.1
-    // -> 4.4 us, 16 x 4096 x 4096 4.55 -> 4.3; with less K, and for the other types, 4 wavefronts do as well).
-    if (g.N <= units && g.steps >= 32)
-      return launch_kernel<GemvArgs>(mmt4d_gemv_i4_kernel<1, 4, 16, false>, g.N, 1024, 0, stream, g);
-    if ((g.M << g.log2_M0) > 4)
-      return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<2, 8, 4, true> : mmt4d_gemv_i4_kernel<2, 8, 4, false>,
+    // Otherwise four wavefronts with six steps' loads in flight, or four steps' where that is all a wavefront has (1 x 25168
+    // x 640 3.8 -> 3.4 us; four elsewhere up to 3 % behind). Too few tiles to occupy the units, or few more tiles than
+    // units: two workgroups to a tile (1 x 1008 x 12672 4.5 -> 3.7, 1 x 4272 x 5504 5.1 -> 4.5). More than 8 lhs rows,
+    // whose operands are as much as four tiles': two tiles to a workgroup (16 x 21856 x 6144 18.8 -> 15.1, 16 x 7520 x
+    // 12544 9.8 -> 9.0), from HBM with up to four tiles a unit four (16 x 9216 x 14336 19.6 -> 17.2; 16 x 21280 x 8832
+    // 20.0, with four 21.4). From HBM two tiles with fewer rows as well where a unit has more than three (1 x 21280 x 8832
+    // 18.3 -> 16.3, 1 x 14336 x 6912 10.5 -> 9.8; 1 x 11008 x 11008 12.9, with two 13.4).
+    const int rows = g.M << g.log2_M0;
+    if (rows > 8 && streamed && g.N > units && g.N <= 4 * (int64_t)units)
+      return launch_kernel<GemvArgs>(mmt4d_gemv_i4_kernel<4, 3, 4, 1, true>, (g.N + 3) / 4, 256, 0, stream, g);
+    if ((rows > 8 && g.N > units) || (streamed && g.N > 3 * (int64_t)units))
+      return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<2, 4, 4, 1, true> : mmt4d_gemv_i4_kernel<2, 4, 4, 1, false>,
                                      (g.N + 1) / 2, 256, 0, stream, g);
-    return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<1, 8, 4, true> : mmt4d_gemv_i4_kernel<1, 8, 4, false>,
+    if (rows <= 8 && (g.N <= units / 2 || (g.N > units && g.N <= units * 3 / 2)))
+      return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<1, 8, 4, 2, true> : mmt4d_gemv_i4_kernel<1, 8, 4, 2, false>,
+                                     g.N * 2, 256, 0, stream, g);
+    if (g.steps <= 16)
+      return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<1, 4, 4, 1, true> : mmt4d_gemv_i4_kernel<1, 4, 4, 1, false>,
+                                     g.N, 256, 0, stream, g);
+    return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<1, 6, 4, 1, true> : mmt4d_gemv_i4_kernel<1, 6, 4, 1, false>,
                                    g.N, 256, 0, stream, g);
   }
   if (kind == kI8) return launch_kind<kI8>(g, stream, name);

@@ -30,3 +30,17 @@ def test_shares(gpu_lib, flags, K0, M, M0):  # noqa: F811
                      out_pad=4 if n % 2 else 0, offsets=(pad, 2 * pad, 4 if n % 2 else 0), accumulate=n % 3 == 1, seed=n)
     for N in tiles:
         run_case(gpu_lib, flags, M, N, 2304 // (K0 * e) + 1, M0, 16, K0, "mmt4d_gemv", seed=N)
+
+
+@pytest.mark.parametrize("K0", [32, 64])
+@pytest.mark.parametrize("M,M0", [(1, 1), (7, 1), (2, 4), (9, 1), (1, 16)])
+def test_int4_shares(gpu_lib, K0, M, M0):  # noqa: F811
+    # (a step is 128 values; the ring is 4, 6 or 8 steps long; 1030 tiles of 58 KB and more come from HBM)
+    for n, values in enumerate([128, 160, 192, 256, 480, 1920, 2048, 2080, 2112, 3072, 3104, 4000, 4128, 6336, 12000]):
+        for N in {[16, 128, 129, 255, 257, 384, 385][(n + M) % 7], 771 + n if values < 4000 else 31}:
+            pad = 32 if n % 2 else 0
+            run_case(gpu_lib, abi.MMT4D_TYPE_S8S4S32, M, N, values // K0, M0, 16, K0, "mmt4d_gemv*", lhs_pad=pad,
+                     rhs_pad=2 * pad, out_pad=4 if n % 2 else 0, offsets=(pad, 2 * pad, 4 if n % 2 else 0),
+                     accumulate=n % 3 == 1, seed=n)
+    for N in (770, 1025, 1030):
+        run_case(gpu_lib, abi.MMT4D_TYPE_S8S4S32, M, N, 8320 // K0, M0, 16, K0, "mmt4d_gemv", seed=N)

@@ -92,11 +92,10 @@ __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_kernel(const GemvArgs 
   constexpr int32_t rhs_step = 1024 * SPLIT;  // bytes of a K-step
   const int64_t lhs_step = (int64_t)(64 * SPLIT) << a.log2_M0;
 
-  // This wavefront's share of the whole K-steps.
-  const int32_t full_steps = a.K / ksteps_per_step;
-  const int32_t share = full_steps / kWaves, longer = full_steps % kWaves;
-  const int32_t s_begin = wave * share + min(wave, longer);
-  int32_t left = share + (wave < longer);
+  // The whole K-steps are dealt to the wavefronts in turn, so that what a workgroup loads at one time lies together (8192 x
+  // 8192 bf16, one row: 23.5 us with a quarter of K each, 20.5 so; 14336 x 4096 19.3, 18.9).
+  const int32_t full_steps = a.K >> (6 + __builtin_ctz(SPLIT) - a.log2_rb);
+  int32_t left = (full_steps + kWaves - 1 - wave) / kWaves;
 
   // (Lanes of lhs rows that do not exist load the last one's: a row reaches its own row of the result only.)
   const int lhs_row = min(row, lhs_rows - 1);
@@ -116,16 +115,16 @@ __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_kernel(const GemvArgs 
 
   acc_t acc = acc_t{0, 0, 0, 0};
   uint4 l[UNROLL], r[UNROLL];
-  lhs += s_begin * lhs_step;
-  rhs += (int64_t)s_begin * rhs_step;
+  lhs += wave * lhs_step;
+  rhs += wave * rhs_step;
   auto load = [&](int u) {
-    l[u] = *(const uint4*)(lhs + u * lhs_step);
-    r[u] = load_rhs<STREAMED>(rhs + u * rhs_step);
+    l[u] = *(const uint4*)(lhs + u * kWaves * lhs_step);
+    r[u] = load_rhs<STREAMED>(rhs + u * kWaves * rhs_step);
   };
   auto next_batch = [&] {
     left -= UNROLL;
-    lhs += UNROLL * lhs_step;
-    rhs += UNROLL * rhs_step;
+    lhs += UNROLL * kWaves * lhs_step;
+    rhs += UNROLL * kWaves * rhs_step;
   };
   if (left >= UNROLL) {
 #pragma unroll
@@ -339,9 +338,7 @@ __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_i4_kernel(const GemvAr
 
   const int32_t columns = (int32_t)(((int64_t)a.K * a.rb) >> 5);  // of 32 values of K, one a lane
   const int32_t full_steps = columns / (4 * SPLIT);
-  const int32_t share = full_steps / kWaves, longer = full_steps % kWaves;
-  const int32_t s_begin = wave * share + min(wave, longer);
-  int32_t left = share + (wave < longer);
+  int32_t left = (full_steps + kWaves - 1 - wave) / kWaves;  // (dealt in turn)
 
   const int lhs_row = min(row, lhs_rows - 1);  // (rows that do not exist, see mmt4d_gemv_kernel)
   const uint8_t* lhs = a.lhs + (int64_t)(lhs_row >> a.log2_M0) * a.lhs_stride_bytes + (int64_t)(lhs_row & (M0 - 1)) * a.rb +
@@ -382,24 +379,24 @@ __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_i4_kernel(const GemvAr
   auto advance = [&](int32_t steps) {
     lhs += steps * lhs_step;
 #pragma unroll
-    for (int t = 0; t < TN; ++t) rhs[t] += (int64_t)steps * rhs_step;
+    for (int t = 0; t < TN; ++t) rhs[t] += steps * rhs_step;
   };
   auto load = [&](int u) {
-    l0[u] = *(const uint4*)(lhs + u * lhs_step);
-    l1[u] = *(const uint4*)(lhs + u * lhs_step + 16);
+    l0[u] = *(const uint4*)(lhs + u * kWaves * lhs_step);
+    l1[u] = *(const uint4*)(lhs + u * kWaves * lhs_step + 16);
 #pragma unroll
-    for (int t = 0; t < TN; ++t) r[u][t] = load_rhs<STREAMED>(rhs[t] + u * rhs_step);
+    for (int t = 0; t < TN; ++t) r[u][t] = load_rhs<STREAMED>(rhs[t] + u * kWaves * rhs_step);
   };
   auto multiply_step = [&](int u) {
 #pragma unroll
     for (int t = 0; t < TN; ++t) multiply(t, r[u][t], l0[u], l1[u]);
   };
-  advance(s_begin);
+  advance(wave);
   if (left >= UNROLL) {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) load(u);
     left -= UNROLL;
-    advance(UNROLL);
+    advance(UNROLL * kWaves);
     while (left >= UNROLL) {
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
@@ -408,7 +405,7 @@ __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_i4_kernel(const GemvAr
         __builtin_amdgcn_sched_barrier(0);
       }
       left -= UNROLL;
-      advance(UNROLL);
+      advance(UNROLL * kWaves);
     }
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {

@@ -14,7 +14,7 @@
 // k step on the VALU (v_dot4_i32_i8, v_dot2_i32_i16, FMAs on 16-bit floats
 // widened to f32), keeping one accumulator per (lhs row, rhs row). The lhs is small and comes through the
 // caches. At the end the lanes that hold the same rhs rows (they differ in
-// k step) are summed with a butterfly of lane exchanges, the wavefronts of the
+// k step) are summed by exchanges that halve the values in each step, the wavefronts of the
 // workgroup (which split the stream between them) through LDS, both in a
 // fixed order, so results do not depend on scheduling.
 //
@@ -51,6 +51,8 @@
 // again: what the block kernels can load they do faster (the caller prefers
 // them), what they cannot is still far better off here than with one thread
 // per output element.
+#include <type_traits>
+
 #include "uk_device.h"
 #include "uk_internal.h"
 
@@ -261,17 +263,72 @@ __device__ __forceinline__ void multiply_piece(const uint4 v, const typename Lhs
   }
 }
 
-__device__ __forceinline__ int32_t exchange(int32_t v, int lane_xor) { return __shfl_xor(v, lane_xor, 64); }
-__device__ __forceinline__ float exchange(float v, int lane_xor) { return __shfl_xor(v, lane_xor, 64); }
+// The value of lane `lane ^ S`.
+template <int S>
+__device__ __forceinline__ uint32_t exchange(uint32_t v) {
+  if constexpr (S == 1) return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);        // quad_perm [1, 0, 3, 2]
+  else if constexpr (S == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);   // quad_perm [2, 3, 0, 1]
+  else if constexpr (S == 4)  // row_half_mirror is ^ 7, quad_perm [3, 2, 1, 0] ^ 3
+    return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, v, 0x1B, 0xF, 0xF, true), 0x141, 0xF, 0xF, true);
+  else if constexpr (S == 8) return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, true);  // row_ror:8
+  else return __shfl_xor((int)v, S, 64);
+}
+
+// v[i] of the lanes with bit S clear and v[i + HALF] of those with it set are summed over the pair lane, lane ^ S.
+template <int S, typename T>
+__device__ __forceinline__ T sum_pair(T low, T high, bool set) {
+  if constexpr (S >= 16) {
+    // (The instruction swaps the upper lanes of the first operand with the lower ones of the second.)
+    const uint32_t x = __builtin_bit_cast(uint32_t, low), y = __builtin_bit_cast(uint32_t, high);
+    const auto both = S == 32 ? __builtin_amdgcn_permlane32_swap(x, y, false, false) : __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    return __builtin_bit_cast(T, (uint32_t)both[0]) + __builtin_bit_cast(T, (uint32_t)both[1]);
+  } else {
+    const T keep = set ? high : low, send = set ? low : high;
+    return keep + __builtin_bit_cast(T, exchange<S>(__builtin_bit_cast(uint32_t, send)));
+  }
+}
+
+// Sums V values over the lanes that are a multiple of `period` (a power of two) apart, each lane ending with 1 / (64 /
+// period) of them or with one, and calls store(first, values, count). Half as many values in each step, not every value in
+// every step: 32 values, period 2: 31 exchanges, not 160 (4 x 800 x 1280 f16: 1.0 of 6.9 us were these).
+template <int S, int V, typename T, typename Store>
+__device__ __forceinline__ void sum_lanes(const T* v, int lane, int period, int first, const Store& store) {
+  if (S == 0 || S < period) {
+    store(first, v, V);
+    return;
+  }
+  if constexpr (S > 0) {
+    const bool set = lane & S;
+    if constexpr (V > 1) {
+      T half[V / 2];
+#pragma unroll
+      for (int i = 0; i < V / 2; ++i) half[i] = sum_pair<S>(v[i], v[i + V / 2], set);
+      sum_lanes<S / 2, V / 2>(half, lane, period, first + (set ? V / 2 : 0), store);
+    } else {
+      const T sum = v[0] + __builtin_bit_cast(T, exchange<S>(__builtin_bit_cast(uint32_t, v[0])));
+      sum_lanes<S / 2, 1>(&sum, lane, period, first, store);
+    }
+  }
+}
+
+// Bytes of an lhs k step in registers, where one load takes the pieces of all rows.
+template <int BYTES>
+struct alignas(BYTES < 16 ? BYTES : 16) LhsStep { uint32_t dwords[BYTES < 4 ? 1 : BYTES / 4]; };
 
 // G: bytes of a row piece; ROWS: lhs rows the kernel keeps accumulators for
 // (a.rows <= ROWS); UNROLL: 1 KiB blocks of the rhs stream a wavefront has in
-// flight; STREAMED: the rhs is read past the caches; NARROW: the output has the
-// 16-bit type of the operands. One workgroup per rhs tile row.
-template <int KIND, int G, int ROWS, int WAVES, int UNROLL, bool STREAMED, bool NARROW>
+// flight, a ring of registers each loaded again as soon as it is multiplied;
+// STREAMED: the rhs is read past the caches; NARROW: the output has the
+// 16-bit type of the operands; PACKED: there is one lhs tile, of ROWS rows, whose
+// k steps are loaded whole: with a load of 2 to 8 bytes for each of four rows
+// beside 16 bytes of rhs, the loads' issue is the limit (4 x 2432 x 4988 f16
+// 9.6 -> 6.7 us). One workgroup per rhs tile row.
+template <int KIND, int G, int ROWS, int WAVES, int UNROLL, bool STREAMED, bool NARROW, bool PACKED>
 __global__ __launch_bounds__(64 * WAVES) void mmt4d_skinny_kernel(const SkinnyArgs a) {
   static_assert(!NARROW || KIND == kF16 || KIND == kBF16, "16-bit outputs are floats");
+  static_assert(!PACKED || KIND == kI8 || KIND == kI16 || KIND == kF16 || KIND == kBF16 || KIND == kF32, "lhs pieces as long as the rhs's");
   typedef typename Acc<KIND>::type acc_t;
+  typedef typename LhsPiece<KIND>::type piece_t;
   // (One-byte pieces of int8: 8-row tiles, two k steps per lane.)
   constexpr bool TWO_KSTEPS = KIND == kI8 && G == 1;
   constexpr int R = TWO_KSTEPS ? 8 : 16 / G;  // rhs rows in a lane's 16 bytes
@@ -285,73 +342,118 @@ __global__ __launch_bounds__(64 * WAVES) void mmt4d_skinny_kernel(const SkinnyAr
   const int log2_lanes_per_kstep = TWO_KSTEPS ? 0 : log2_kstep_bytes - 4;
   const int32_t kstep_in_block = TWO_KSTEPS ? 2 * lane : lane >> log2_lanes_per_kstep;
   constexpr int LHS_G = KIND == kI16U4 ? 16 : (KIND == kI8I4 || KIND == kI16I8 ? 2 * G : G);  // bytes of an lhs row piece
-  const int32_t lhs_kstep_bytes = LHS_G << a.log2_M0;
+  const int32_t lhs_kstep_bytes = PACKED ? LHS_G * ROWS : LHS_G << a.log2_M0;
 
-  const uint8_t* rhs_tile = a.rhs + (int64_t)blockIdx.x * a.rhs_stride_bytes;
-  const uint8_t* lhs_row[ROWS];
+  const uint8_t* rhs = a.rhs + (int64_t)blockIdx.x * a.rhs_stride_bytes + 16 * lane;
+  const int64_t lhs_lane = (int64_t)kstep_in_block * lhs_kstep_bytes;
+  const int64_t lhs_block = (int64_t)lhs_kstep_bytes << (10 - log2_kstep_bytes);  // bytes of the lhs k steps of a block
+  constexpr int LHS_ROWS = PACKED ? 1 : ROWS;
+  const uint8_t* lhs_row[LHS_ROWS];
 #pragma unroll
-  for (int m = 0; m < ROWS; ++m) {
-    const int row = a.row0 + m < a.rows ? a.row0 + m : a.rows - 1;  // clamp: computed, not stored
-    lhs_row[m] = a.lhs + (int64_t)(row >> a.log2_M0) * a.lhs_stride_bytes + (row & (M0 - 1)) * LHS_G;
+  for (int m = 0; m < LHS_ROWS; ++m) {
+    const int row = PACKED ? 0 : min(a.row0 + m, a.rows - 1);  // clamp: computed, not stored
+    lhs_row[m] = a.lhs + (int64_t)(row >> a.log2_M0) * a.lhs_stride_bytes + (row & (M0 - 1)) * LHS_G + lhs_lane;
   }
 
-  acc_t acc[ROWS][R];
+  acc_t acc[ROWS * R];
 #pragma unroll
-  for (int m = 0; m < ROWS; ++m)
-#pragma unroll
-    for (int r = 0; r < R; ++r) acc[m][r] = 0;
+  for (int i = 0; i < ROWS * R; ++i) acc[i] = 0;
 
-  const int64_t blocks = (a.tile_bytes + 1023) >> 10;
-  for (int64_t j0 = wave; j0 < blocks; j0 += WAVES * UNROLL) {
-    uint4 v[UNROLL];
-    typename LhsPiece<KIND>::type l[UNROLL][ROWS];
+  typedef typename std::conditional<PACKED, LhsStep<PACKED ? LHS_G * ROWS : 4>, piece_t>::type lhs_t;
+  auto load_lhs = [&](lhs_t* l, int64_t block, bool second_kstep) {
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      const int64_t off = ((j0 + WAVES * u) << 10) + 16 * lane;
-      const bool inside = off < a.tile_bytes;
-      v[u] = make_uint4(0, 0, 0, 0);
-      if (TWO_KSTEPS && inside && off + 16 > a.tile_bytes) {
-        // An odd K: the stream ends after this lane's first k step.
-        const uint2 half = *(const uint2*)(rhs_tile + off);
-        v[u].x = half.x;
-        v[u].y = half.y;
-      } else if (inside) {
-        if constexpr (STREAMED) v[u] = __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4i32*)(rhs_tile + off)));
-        else v[u] = *(const uint4*)(rhs_tile + off);
-      }
-      // The lhs piece of this lane's k step.
-      const int64_t kstep = inside ? ((j0 + WAVES * u) << (10 - log2_kstep_bytes)) + kstep_in_block : 0;
+    for (int m = 0; m < LHS_ROWS; ++m) {
+      const uint8_t* p = lhs_row[m] + block * lhs_block;
+      if constexpr (PACKED && LHS_G * ROWS == 2) l[m].dwords[0] = *(const uint16_t*)p;
+      else if constexpr (PACKED) l[m] = *(const lhs_t*)p;
+      else if constexpr (TWO_KSTEPS) l[m] = make_uint2((uint32_t)p[0] | ((second_kstep ? p[lhs_kstep_bytes] : 0u) << 8), 0);
+      else l[m] = load_lhs_piece<KIND, G>(p);
+    }
+  };
+  auto multiply = [&](const uint4 v, const lhs_t* l) {
 #pragma unroll
-      for (int m = 0; m < ROWS; ++m) {
-        if constexpr (TWO_KSTEPS) {
-          const uint8_t* p = lhs_row[m] + kstep * lhs_kstep_bytes;
-          const uint32_t second = kstep + 1 < a.K ? p[lhs_kstep_bytes] : 0u;
-          l[u][m] = make_uint2((uint32_t)p[0] | (second << 8), 0);
-        } else {
-          l[u][m] = load_lhs_piece<KIND, G>(lhs_row[m] + kstep * lhs_kstep_bytes);
-        }
-        if (!inside) l[u][m] = typename LhsPiece<KIND>::type{};  // 0 * 0, whatever the lhs holds there
+    for (int m = 0; m < ROWS; ++m) {
+      if constexpr (PACKED) {
+        const uint32_t* d = l[0].dwords;
+        piece_t piece;
+        if constexpr (G == 2) piece = make_uint2(m & 1 ? d[m / 2] >> 16 : d[m / 2] & 0xFFFFu, 0);
+        else if constexpr (G == 4) piece = make_uint2(d[m], 0);
+        else piece = make_uint2(d[2 * m], d[2 * m + 1]);
+        multiply_piece<KIND, G>(v, piece, acc + m * R);
+      } else {
+        multiply_piece<KIND, G>(v, l[m], acc + m * R);
       }
     }
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u)
-#pragma unroll
-      for (int m = 0; m < ROWS; ++m) multiply_piece<KIND, G>(v[u], l[u][m], acc[m]);
+  };
+
+  // The blocks are dealt to the wavefronts in turn. What is left behind the last whole one goes to the last wavefront:
+  // lanes beyond the stream's end multiply zeros, whatever the lhs holds there.
+  const int32_t full = (int32_t)(a.tile_bytes >> 10);
+  const int32_t rest_bytes = (int32_t)(a.tile_bytes & 1023);
+  const bool has_rest = wave == WAVES - 1 && rest_bytes != 0;
+  uint4 rest_v = make_uint4(0, 0, 0, 0);
+  lhs_t rest_l[LHS_ROWS] = {};
+  if (has_rest && 16 * lane < rest_bytes) {
+    const uint8_t* p = rhs + ((int64_t)full << 10);
+    if (TWO_KSTEPS && 16 * lane + 16 > rest_bytes) {
+      // An odd K: the stream ends after this lane's first k step.
+      const uint2 half = *(const uint2*)p;
+      rest_v.x = half.x;
+      rest_v.y = half.y;
+    } else {
+      rest_v = *(const uint4*)p;
+    }
+    load_lhs(rest_l, full, 16 * lane + 16 <= rest_bytes);
   }
 
+  uint4 v[UNROLL];
+  lhs_t l[UNROLL][LHS_ROWS];
+  int32_t left = (full + WAVES - 1 - wave) / WAVES;
+  int64_t block = wave;
+  auto load = [&](int u) {
+    const uint8_t* p = rhs + ((block + u * WAVES) << 10);
+    if constexpr (STREAMED) v[u] = __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4i32*)p));
+    else v[u] = *(const uint4*)p;
+    load_lhs(l[u], block + u * WAVES, true);
+  };
+  auto next_batch = [&] {
+    left -= UNROLL;
+    block += UNROLL * WAVES;
+  };
+  if (left >= UNROLL) {
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) load(u);
+    next_batch();
+    while (left >= UNROLL) {
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        multiply(v[u], l[u]);
+        load(u);
+        __builtin_amdgcn_sched_barrier(0);  // (no load moves in front of the multiplication of what its registers hold)
+      }
+      next_batch();
+    }
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      multiply(v[u], l[u]);
+      if (u < left) load(u);
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < UNROLL - 1; ++u)
+      if (u < left) load(u);
+  }
+#pragma unroll
+  for (int u = 0; u < UNROLL - 1; ++u)
+    if (u < left) multiply(v[u], l[u]);
+  if (has_rest) multiply(rest_v, rest_l);
+
   // Lanes that are a multiple of lanes_per_kstep apart hold the same rhs rows.
-  for (int s = 1 << log2_lanes_per_kstep; s < 64; s <<= 1) {
-#pragma unroll
-    for (int m = 0; m < ROWS; ++m)
-#pragma unroll
-      for (int r = 0; r < R; ++r) acc[m][r] += exchange(acc[m][r], s);
-  }
-  if (lane < (1 << log2_lanes_per_kstep)) {
-#pragma unroll
-    for (int m = 0; m < ROWS; ++m)
-#pragma unroll
-      for (int r = 0; r < R; ++r) partial[wave][m][R * lane + r] = acc[m][r];
-  }
+  const int32_t lanes_per_kstep = 1 << log2_lanes_per_kstep;
+  sum_lanes<32, ROWS * R>(acc, lane, lanes_per_kstep, 0, [&](int first, const acc_t* sums, int count) {
+    for (int i = 0; i < count; ++i)
+      partial[wave][(first + i) / R][R * (lane & (lanes_per_kstep - 1)) + (first + i) % R] = sums[i];
+  });
   __syncthreads();
   const int t = threadIdx.x;
   const int slab_row = t >> a.log2_N0, j0 = t & (N0 - 1);
@@ -445,20 +547,30 @@ bool make_args(const Mmt4dArgs& a, bool probe_only, int* kind, int* piece_bytes,
   return true;
 }
 
-template <int KIND, int G, int WAVES, bool STREAMED, bool NARROW>
+// PACKED_UNROLL: UNROLL for an lhs tile of 2 or 4 rows that is aligned to its k steps. Other lhs have a load for each row
+// beside one of the rhs, and more registers to each step (3 x 4096 x 4096 f32 of 8-byte pieces: 17.8 us with eight wavefronts
+// of four blocks, 12.1 of two).
+template <int KIND, int G, int WAVES, int PACKED_UNROLL, bool STREAMED, bool NARROW>
 hipError_t launch_slabs(const SkinnyArgs& all_rows, hipStream_t stream) {
-  // Fewer lhs rows leave registers for more of the rhs stream in flight. More
-  // than 8 rows: one launch per slab of 8.
-  constexpr int SHARE = WAVES / 4;
   void (*kernel)(const SkinnyArgs);
   SkinnyArgs s = all_rows;
+  auto launch = [&] { return launch_kernel(kernel, (unsigned)all_rows.N, 64 * WAVES, 0, stream, s); };
+  if constexpr (G > 1 && (KIND == kI8 || KIND == kI16 || KIND == kF16 || KIND == kBF16 || KIND == kF32)) {
+    const int kstep = G * s.rows;
+    if (s.rows == 1 << s.log2_M0 && (s.rows == 2 || s.rows == 4) && (uintptr_t)s.lhs % (kstep < 16 ? kstep : 16) == 0) {
+      kernel = s.rows == 2 ? mmt4d_skinny_kernel<KIND, G, 2, WAVES, PACKED_UNROLL, STREAMED, NARROW, true>
+                           : mmt4d_skinny_kernel<KIND, G, 4, WAVES, PACKED_UNROLL, STREAMED, NARROW, true>;
+      return launch();
+    }
+  }
+  // More than 8 rows: one launch per slab of 8.
   for (s.row0 = 0; s.row0 < s.rows; s.row0 += 8) {
     const int left = s.rows - s.row0;
-    if (left <= 1) kernel = mmt4d_skinny_kernel<KIND, G, 1, WAVES, 16 / SHARE, STREAMED, NARROW>;
-    else if (left <= 2) kernel = mmt4d_skinny_kernel<KIND, G, 2, WAVES, 16 / SHARE, STREAMED, NARROW>;
-    else if (left <= 4) kernel = mmt4d_skinny_kernel<KIND, G, 4, WAVES, 8 / SHARE, STREAMED, NARROW>;
-    else kernel = mmt4d_skinny_kernel<KIND, G, 8, WAVES, 4 / SHARE, STREAMED, NARROW>;
-    const hipError_t e = launch_kernel(kernel, (unsigned)all_rows.N, 64 * WAVES, 0, stream, s);
+    if (left <= 1) kernel = mmt4d_skinny_kernel<KIND, G, 1, WAVES, 4, STREAMED, NARROW, false>;
+    else if (left <= 2) kernel = mmt4d_skinny_kernel<KIND, G, 2, WAVES, 4, STREAMED, NARROW, false>;
+    else if (left <= 4) kernel = mmt4d_skinny_kernel<KIND, G, 4, WAVES, G == 8 && WAVES == 8 ? 2 : 4, STREAMED, NARROW, false>;
+    else kernel = mmt4d_skinny_kernel<KIND, G, 8, WAVES, 2, STREAMED, NARROW, false>;
+    const hipError_t e = launch();
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -467,16 +579,29 @@ hipError_t launch_slabs(const SkinnyArgs& all_rows, hipStream_t stream) {
 template <int KIND, int G, bool NARROW>
 hipError_t launch_piece(const SkinnyArgs& s, hipStream_t stream) {
   const int64_t bytes = s.tile_bytes * s.N;
-  // No more tile rows than compute units, and long ones: eight wavefronts (4 x 512 x 8192 bf16 14.4 -> 10.3 us, 1 x 512 x
-  // 4096 5.0 -> 3.9; against four that stream, 4 x 4096 x 14336 int8 22.5 -> 14.3 with its 59 MB held, 22.4 -> 18.8 from
-  // HBM). With shorter ones, or several to a unit, the summing at the end costs more than it gives.
-  if (s.N <= 256 && s.tile_bytes >= 128 * 1024) return launch_slabs<KIND, G, 8, false, NARROW>(s, stream);
-  // One byte or less per rhs element against more than two rows is bound by the vector ALU, which streaming does not help:
-  // 4 x 14336 x 4096 int8 17.6 us, streamed 20.6, from HBM 20.9 both; only beyond what the caches can hold it does (235
-  // MB: 60.8 -> 56.8).
-  const bool alu_bound = (KIND == kI8 || KIND == kI8I4 || KIND == kI16U4 || KIND == kI16I8) && s.rows > 2;
-  if (alu_bound ? bytes > (128ll << 20) : comes_from_hbm(bytes)) return launch_slabs<KIND, G, 4, true, NARROW>(s, stream);
-  return launch_slabs<KIND, G, 4, false, NARROW>(s, stream);
+  // No more tile rows than compute units: eight wavefronts, 4 KiB in flight each (1 x 880 x 8918 bf16 9.3 -> 6.5 us, with 8
+  // KiB in each of four 7.3; 2 x 1984 x 4991 f16 7.1 -> 5.5, 6.1).
+  if (s.N <= 256) return launch_slabs<KIND, G, 8, 4, false, NARROW>(s, stream);
+  // One byte or less per rhs element against more than two rows is slowed down by streaming: 4 x 14336 x 4096 int8 17.6 us,
+  // streamed 20.6, from HBM 20.9 both; only beyond what the caches can hold it gains (235 MB: 60.8 -> 56.8).
+  const bool one_byte = KIND == kI8 || KIND == kI8I4 || KIND == kI16U4 || KIND == kI16I8;
+  const bool streamed = one_byte && s.rows > 2 ? bytes > (128ll << 20) : comes_from_hbm(bytes);
+  // One row and more than two tile rows a unit, from HBM: 12 KiB in flight in each of four wavefronts (1 x 24320 x 3664 int8
+  // 15.4 -> 14.3, 1 x 16816 x 7722 23.4 -> 22.7), but eight wavefronts for tiles of whole 64 KiB (1 x 14336 x 4096 bf16 20.1
+  // -> 19.0, 1 x 28672 x 8192 int8 35.7 -> 34.7) unless they lie a multiple of 256 KiB apart, on few memory channels (f32 1 x
+  // 14336 x 4096 41.5 us, with four 35.5); from the caches eight for tiles of 64 KiB and more.
+  if (s.rows == 1 && s.N > 512) {
+    const bool eight = streamed ? s.rhs_stride_bytes % (64 * 1024) == 0 && s.rhs_stride_bytes % (256 * 1024) != 0 : s.tile_bytes >= 64 * 1024;
+    if (streamed)
+      return eight ? launch_kernel<SkinnyArgs>(mmt4d_skinny_kernel<KIND, G, 1, 8, 4, true, NARROW, false>, (unsigned)s.N, 512, 0, stream, s)
+                   : launch_kernel<SkinnyArgs>(mmt4d_skinny_kernel<KIND, G, 1, 4, 12, true, NARROW, false>, (unsigned)s.N, 256, 0, stream, s);
+    if (eight) return launch_slabs<KIND, G, 8, 4, false, NARROW>(s, stream);
+  }
+  // Several rows and more than two tile rows a unit: 8 KiB in flight (4 x 9616 x 6381 f16 23.7, with 4 KiB 25.1; 4 x 5312 x
+  // 6146 int8, two to a unit, 8.9 and 8.1).
+  if (s.rows > 1 && s.N > 512)
+    return streamed ? launch_slabs<KIND, G, 4, 8, true, NARROW>(s, stream) : launch_slabs<KIND, G, 4, 8, false, NARROW>(s, stream);
+  return streamed ? launch_slabs<KIND, G, 4, 4, true, NARROW>(s, stream) : launch_slabs<KIND, G, 4, 4, false, NARROW>(s, stream);
 }
 
 template <int KIND, bool NARROW>

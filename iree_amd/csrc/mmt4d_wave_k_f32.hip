@@ -11,12 +11,10 @@ hipError_t launch_shape(const MfmaArgs& m, int shape, bool streamed, hipStream_t
   if constexpr (SHAPE < (int)(sizeof kWaveKShapesF32 / sizeof kWaveKShapesF32[0])) {
     constexpr WaveKShape s = kWaveKShapesF32[SHAPE];
     if (shape != SHAPE) return launch_shape<G, SHAPE + 1>(m, shape, streamed, stream);
-    // One fragment either way, K long: the multiplies of one step are over before the next one is there (64 x 528 x 4500
-    // 9.5 us with one step in flight, 8.5 with two; below K = 1600 two take up to 9 % longer).
     if constexpr (SHAPE == 0) {
-      if (m.chunks > 112) return launch_wave_k_tile<kF32, false, false, G, 1, 1, 8, 2>(m, streamed, stream);
+      if (m.chunks >= 32) return launch_wave_k_tile<kF32, false, false, G, 1, 1, 8, 3>(m, streamed, stream);
     }
-    return launch_wave_k_tile<kF32, false, false, G, s.fa, s.fb, 8, 1>(m, streamed, stream);
+    return launch_wave_k_tile<kF32, false, false, G, s.fa, s.fb, 8, 2>(m, streamed, stream);
   } else {
     return hipErrorInvalidValue;
   }

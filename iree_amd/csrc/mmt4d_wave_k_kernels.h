@@ -6,13 +6,12 @@
 // fewer tiles than compute units has nothing to hide that behind. Here a
 // workgroup of 8 wavefronts owns a (16*FA) x (16*FB) tile and every wavefront
 // multiplies the WHOLE tile over its own share of K: operands go from
-// global memory straight to the MFMA's registers, a batch of UNROLL 64-byte
-// steps in flight while the previous batch is multiplied, with no LDS and no
-// barrier until the partial tiles are summed through LDS at the end, in
-// wavefront order (results do not depend on scheduling). A workgroup thus has
-// 128 to 256 KiB of loads in flight and, where the caches hold the operands, is
-// bound by what a compute unit's load path moves: (16*FA + 16*FB) * 64 bytes per
-// step at 70 to 90 bytes a nanosecond.
+// global memory straight to the MFMA's registers, DEPTH - 1 64-byte steps in
+// flight while one is multiplied, with no LDS and no barrier until the partial
+// tiles are summed through LDS at the end, in wavefront order (results do not
+// depend on scheduling). Where the caches hold the operands a workgroup is bound
+// by what a compute unit's load path moves, (16*FA + 16*FB) * 64 bytes per step
+// at 70 to 90 bytes a nanosecond, f32 by the matrix pipe.
 //
 // Operand registers. Fragments are 16 rows x 64 bytes of K
 // (v_mfma_i32_16x16x64_i8, v_mfma_f32_16x16x32_{f16,bf16}, four
@@ -182,7 +181,7 @@ struct Operand {
   }
 };
 
-template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int UNROLL, bool STREAMED, bool PIECES>
+template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int DEPTH, bool STREAMED, bool PIECES>
 __global__ __launch_bounds__(64 * WAVES)
 __attribute__((amdgpu_waves_per_eu(2, FA * FB >= 16 ? 2 : 4)))
 void mmt4d_wave_k_kernel(const MfmaArgs a) {
@@ -192,7 +191,7 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
   static_assert(!PIECES || G == 4, "4-byte pieces");
   constexpr bool STAGED = G < 16 && !PIECES;  // operands pass through LDS
   static_assert(!RHS_I4 || (KIND == kI8 && G == 16), "int4 rhs");
-  // The wavefronts' staging of narrow row pieces, [WAVES][UNROLL][FA + FB][1 KiB]; then [WAVES][FA * FB][64] partial sums.
+  // The wavefronts' staging of narrow row pieces, [WAVES][FA + FB][1 KiB]; then [WAVES][FA * FB][64] partial sums.
   extern __shared__ uint4 ring[];
 
   int tile_row, tile_col;
@@ -242,95 +241,112 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
   rhs_t rhs;
   set_up(lhs, a.lhs, first_row, a.M, a.log2_M0, a.lhs_stride_bytes, a.lhs_rb, a.log2_lhs_rb, RHS_I4 ? 32 : 16);
   set_up(rhs, a.rhs, first_col, a.N, a.log2_N0, a.rhs_stride_bytes, a.rhs_rb, a.log2_rhs_rb, 16);
-  uint8_t* const staging = (uint8_t*)ring + wave * (UNROLL * (FA + FB) * 1024);  // (narrow pieces only)
+  uint8_t* const staging = (uint8_t*)ring + wave * ((FA + FB) * 1024);  // (narrow pieces only)
 
   acc_t acc[FA][FB];
 #pragma unroll
   for (int i = 0; i < FA; ++i)
 #pragma unroll
     for (int j = 0; j < FB; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
-  // Batches of UNROLL steps, whose loads are in flight together, are dealt out to the wavefronts in turn: at any time
-  // the workgroup reads one contiguous stretch of every row panel. (A contiguous share of K per wavefront puts all
-  // loads of a launch at the same few offsets modulo the share: 5 to 10 % slower.)
+  // The steps are dealt out to the wavefronts in turn: at any time the workgroup reads one contiguous stretch of every row
+  // panel. (A contiguous share of K per wavefront puts all loads of a launch at the same few offsets modulo the share: 5 to
+  // 10 % slower.)
   const int32_t ksteps_per_step = (RHS_I4 ? 128 : 64) >> a.log2_lhs_rb;
   const int32_t steps = (a.K + ksteps_per_step - 1) / ksteps_per_step;
-  const int32_t all_batches = a.K / ksteps_per_step / UNROLL;
-  const int32_t batches = (all_batches - wave + WAVES - 1) / WAVES;
+  const int32_t whole = a.K / ksteps_per_step;
+  const int32_t count = (whole - wave + WAVES - 1) / WAVES;
 
-  struct Batch {
-    uint4 l[UNROLL][lhs_t::RAW], r[UNROLL][rhs_t::RAW];
+  struct Step {
+    uint4 l[lhs_t::RAW], r[rhs_t::RAW];
   };
-  auto fetch = [&](int32_t b, Batch& to) {
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      const int32_t s = (b * WAVES + wave) * UNROLL + u;
-      rhs.template load<false, STREAMED>(s, 0, 0, to.r[u]);
-      lhs.template load<false, false>(s, 0, 0, to.l[u]);
-    }
+  auto fetch = [&](int32_t b, Step& to) {
+    rhs.template load<false, STREAMED>(b * WAVES + wave, 0, 0, to.r);
+    lhs.template load<false, false>(b * WAVES + wave, 0, 0, to.l);
   };
-  // What is left after the full batches (at most UNROLL steps, K's end among them) goes to the last wavefront.
-  const bool has_rest = wave == WAVES - 1 && all_batches * UNROLL < steps;
-  auto fetch_rest = [&](Batch& to) {
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      const int32_t s = all_batches * UNROLL + u;
-      rhs.template load<true, false>(s, s * ksteps_per_step, a.K, to.r[u]);
-      lhs.template load<true, false>(s, s * ksteps_per_step, a.K, to.l[u]);
-    }
+  // A step that K ends in goes to the last wavefront.
+  const bool has_rest = wave == WAVES - 1 && whole < steps;
+  auto fetch_rest = [&](Step& to) {
+    rhs.template load<true, false>(whole, whole * ksteps_per_step, a.K, to.r);
+    lhs.template load<true, false>(whole, whole * ksteps_per_step, a.K, to.l);
   };
-  auto zero_rest = [&](Batch& of) {
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      const int32_t k0 = (all_batches * UNROLL + u) * ksteps_per_step;
-      rhs.zero_beyond(k0, a.K, of.r[u]);
-      lhs.zero_beyond(k0, a.K, of.l[u]);
-    }
+  auto zero_rest = [&](Step& of) {
+    rhs.zero_beyond(whole * ksteps_per_step, a.K, of.r);
+    lhs.zero_beyond(whole * ksteps_per_step, a.K, of.l);
   };
-  auto multiply = [&](const Batch& from) {
+  auto multiply = [&](const Step& from) {
     if constexpr (STAGED) {
-#pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        lhs.to_lds(from.l[u], staging + u * (FA + FB) * 1024);
-        rhs.to_lds(from.r[u], staging + u * (FA + FB) * 1024 + FA * 1024);
-      }
+      lhs.to_lds(from.l, staging);
+      rhs.to_lds(from.r, staging + FA * 1024);
       __builtin_amdgcn_wave_barrier();
     }
+    if constexpr (RHS_I4) {
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      if constexpr (RHS_I4) {
-#pragma unroll
-        for (int j = 0; j < FB; ++j) {
-          const uint4 w = from.r[u][j];
-          const uint4 lo = widen_i4_times16(make_uint2(w.x, w.y)), hi = widen_i4_times16(make_uint2(w.z, w.w));
-#pragma unroll
-          for (int i = 0; i < FA; ++i) {
-            acc[i][j] = mfma16<KIND>(lo, from.l[u][2 * i], acc[i][j]);
-            acc[i][j] = mfma16<KIND>(hi, from.l[u][2 * i + 1], acc[i][j]);
-          }
-        }
-      } else {
-        uint8_t* const lds = staging + u * (FA + FB) * 1024;
-        uint4 fa[FA];
+      for (int j = 0; j < FB; ++j) {
+        const uint4 w = from.r[j];
+        const uint4 lo = widen_i4_times16(make_uint2(w.x, w.y)), hi = widen_i4_times16(make_uint2(w.z, w.w));
 #pragma unroll
         for (int i = 0; i < FA; ++i) {
-          if constexpr (STAGED) fa[i] = lhs.from_lds(lds, i, lane); else fa[i] = from.l[u][i];
+          acc[i][j] = mfma16<KIND>(lo, from.l[2 * i], acc[i][j]);
+          acc[i][j] = mfma16<KIND>(hi, from.l[2 * i + 1], acc[i][j]);
         }
+      }
+    } else {
+      uint4 fa[FA];
 #pragma unroll
-        for (int j = 0; j < FB; ++j) {
-          uint4 fb;
-          if constexpr (STAGED) fb = rhs.from_lds(lds + FA * 1024, j, lane); else fb = from.r[u][j];
+      for (int i = 0; i < FA; ++i) {
+        if constexpr (STAGED) fa[i] = lhs.from_lds(staging, i, lane); else fa[i] = from.l[i];
+      }
 #pragma unroll
-          for (int i = 0; i < FA; ++i) acc[i][j] = mfma16<KIND>(fb, fa[i], acc[i][j]);
-        }
+      for (int j = 0; j < FB; ++j) {
+        uint4 fb;
+        if constexpr (STAGED) fb = rhs.from_lds(staging + FA * 1024, j, lane); else fb = from.r[j];
+#pragma unroll
+        for (int i = 0; i < FA; ++i) acc[i][j] = mfma16<KIND>(fb, fa[i], acc[i][j]);
       }
     }
   };
-  {
-    Batch p, n;
+  if constexpr (DEPTH > 2) {
+    // A ring: each step's registers are loaded again as soon as they are multiplied. What is left at the end, any number of
+    // steps, is one batch of loads.
+    Step ring_of[DEPTH], rest;
+    if (has_rest) fetch_rest(rest);
     int32_t b = 0;
-    if (batches > 0) {
+    if (count >= DEPTH) {
+#pragma unroll
+      for (int u = 0; u < DEPTH; ++u) fetch(u, ring_of[u]);
+      b = DEPTH;
+      for (; b + DEPTH <= count; b += DEPTH) {
+#pragma unroll
+        for (int u = 0; u < DEPTH; ++u) {
+          multiply(ring_of[u]);
+          __builtin_amdgcn_sched_barrier(0);
+          fetch(b + u, ring_of[u]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < DEPTH; ++u) {
+        multiply(ring_of[u]);
+        if (b + u < count) fetch(b + u, ring_of[u]);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < DEPTH - 1; ++u)
+        if (u < count) fetch(u, ring_of[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < DEPTH - 1; ++u)
+      if (b + u < count) multiply(ring_of[u]);
+    if (has_rest) {
+      zero_rest(rest);
+      multiply(rest);
+    }
+  } else {
+    Step p, n;
+    int32_t b = 0;
+    if (count > 0) {
       fetch(0, p);
-      for (; b + 2 < batches; b += 2) {
+      for (; b + 2 < count; b += 2) {
         fetch(b + 1, n);
         __builtin_amdgcn_sched_barrier(0);
         multiply(p);
@@ -340,7 +356,7 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
         multiply(n);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (b + 1 < batches) {
+      if (b + 1 < count) {
         fetch(b + 1, n);
         multiply(p);
         if (has_rest) fetch_rest(p);
@@ -408,16 +424,16 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
   }
 }
 
-template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int UNROLL, bool PIECES>
+template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int DEPTH, bool PIECES>
 hipError_t launch_wave_k_loads(MfmaArgs m, bool streamed, hipStream_t stream) {
   unsigned grid;
   set_tile_grid(&m, 16 * FA, 16 * FB, &grid);
-  constexpr int staging_kib = G < 16 && !PIECES ? WAVES * UNROLL * (FA + FB) : 0, partial_kib = WAVES * FA * FB;
+  constexpr int staging_kib = G < 16 && !PIECES ? WAVES * (FA + FB) : 0, partial_kib = WAVES * FA * FB;
   constexpr int lds_bytes = 1024 * (staging_kib > partial_kib ? staging_kib : partial_kib);
   static_assert(lds_bytes <= 160 * 1024, "partial sums do not fit the LDS");
-  auto kernel = mmt4d_wave_k_kernel<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, false, PIECES>;
+  auto kernel = mmt4d_wave_k_kernel<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, DEPTH, false, PIECES>;
   if constexpr (G == 16) {
-    if (streamed) kernel = mmt4d_wave_k_kernel<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, true, PIECES>;
+    if (streamed) kernel = mmt4d_wave_k_kernel<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, DEPTH, true, PIECES>;
   }
   if (lds_bytes > 65536) {
     const hipError_t attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
@@ -426,31 +442,39 @@ hipError_t launch_wave_k_loads(MfmaArgs m, bool streamed, hipStream_t stream) {
   return launch_kernel<MfmaArgs>(kernel, grid, 64 * WAVES, lds_bytes, stream, m);
 }
 
-template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int UNROLL>
+template <int KIND, bool RHS_I4, bool NARROW, int G, int FA, int FB, int WAVES, int DEPTH>
 hipError_t launch_wave_k_tile(const MfmaArgs& m, bool streamed, hipStream_t stream) {
   if constexpr (G != 4) {
-    return launch_wave_k_loads<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, false>(m, streamed, stream);
+    return launch_wave_k_loads<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, DEPTH, false>(m, streamed, stream);
   } else if constexpr (KIND == kF32) {
-    return launch_wave_k_loads<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, true>(m, streamed, stream);
+    return launch_wave_k_loads<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, DEPTH, true>(m, streamed, stream);
   } else {
     return wave_k_loads_pieces(m, KIND, G, FA, FB)
-               ? launch_wave_k_loads<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, true>(m, streamed, stream)
-               : launch_wave_k_loads<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, UNROLL, false>(m, streamed, stream);
+               ? launch_wave_k_loads<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, DEPTH, true>(m, streamed, stream)
+               : launch_wave_k_loads<KIND, RHS_I4, NARROW, G, FA, FB, WAVES, DEPTH, false>(m, streamed, stream);
   }
 }
 
-// One 64-byte step of K in flight ahead of the one that is multiplied, for each of eight wavefronts. (What is left of K
-// after whole batches is one wavefront's work, and longer batches leave more: four and two steps a batch for the tiles of one
-// and of two to four fragments took 3 to 12 % longer near where these tiles are the best, 2 % less nowhere.)
+// One 64-byte step of K in flight ahead of the one that is multiplied, for each of eight wavefronts; two for tiles of one
+// fragment and 32 steps and more, whose multiplication is over before the next step is there: f16 16x16x1 16 x 560 x 7148 8.7
+// -> 7.6 us, f32 32 x 352 x 8740 15.5 -> 13.5, bf16 16 x 1360 x 6576 7.2 -> 7.0. (int8 in 16-byte pieces 1 % slower. Three
+// and more, or two for larger tiles, give nothing, and longer batches leave more to the one wavefront that has K's rest.)
+template <int KIND, int G>
+constexpr bool kTwoStepsAhead = KIND != kI8 || G < 16;
+
 template <int KIND, bool RHS_I4, bool NARROW, int G>
 hipError_t launch_wave_k_piece(const MfmaArgs& m, int shape, bool streamed, hipStream_t stream) {
   switch (shape) {
-    case 0: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 1, 8, 1>(m, streamed, stream);
-    case 1: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 2, 8, 1>(m, streamed, stream);
-    case 2: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 2, 2, 8, 1>(m, streamed, stream);
-    case 3: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 2, 4, 8, 1>(m, streamed, stream);
-    case 4: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 4, 2, 8, 1>(m, streamed, stream);
-    case 5: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 4, 4, 8, 1>(m, streamed, stream);
+    case 0:
+      if constexpr (kTwoStepsAhead<KIND, G>) {
+        if (m.chunks >= 32) return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 1, 8, 3>(m, streamed, stream);
+      }
+      return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 1, 8, 2>(m, streamed, stream);
+    case 1: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 2, 8, 2>(m, streamed, stream);
+    case 2: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 2, 2, 8, 2>(m, streamed, stream);
+    case 3: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 2, 4, 8, 2>(m, streamed, stream);
+    case 4: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 4, 2, 8, 2>(m, streamed, stream);
+    case 5: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 4, 4, 8, 2>(m, streamed, stream);
     default: return hipErrorInvalidValue;
   }
 }

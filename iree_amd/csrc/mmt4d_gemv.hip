@@ -320,7 +320,7 @@ __device__ __forceinline__ uint4 lhs_bytes_even_then_odd(uint4 v) {
 // TN rhs tiles per workgroup share each lhs operand: with 16 lhs rows the lhs
 // is twice the bytes of one rhs tile per step (int8 against int4), all of it
 // through L2 for every workgroup. The ring of UNROLL loads and SPLIT as in mmt4d_gemv_kernel.
-template <int TN, int UNROLL, int kWaves, int SPLIT, bool STREAMED>
+template <int TN, int UNROLL, int kWaves, bool STREAMED, int SPLIT>
 __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_i4_kernel(const GemvArgs a) {
   static_assert(TN == 1 || SPLIT == 1, "several tiles to a workgroup or several workgroups to a tile");
   constexpr int ROWS = 16 / SPLIT;
@@ -708,17 +708,17 @@ hipError_t launch_gemv(const Mmt4dArgs& a, hipStream_t stream, const char** name
     // 18.3 -> 16.3, 1 x 14336 x 6912 10.5 -> 9.8; 1 x 11008 x 11008 12.9, with two 13.4).
     const int rows = g.M << g.log2_M0;
     if (rows > 8 && streamed && g.N > units && g.N <= 4 * (int64_t)units)
-      return launch_kernel<GemvArgs>(mmt4d_gemv_i4_kernel<4, 3, 4, 1, true>, (g.N + 3) / 4, 256, 0, stream, g);
+      return launch_kernel<GemvArgs>(mmt4d_gemv_i4_kernel<4, 3, 4, true, 1>, (g.N + 3) / 4, 256, 0, stream, g);
     if ((rows > 8 && g.N > units) || (streamed && g.N > 3 * (int64_t)units))
-      return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<2, 4, 4, 1, true> : mmt4d_gemv_i4_kernel<2, 4, 4, 1, false>,
+      return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<2, 4, 4, true, 1> : mmt4d_gemv_i4_kernel<2, 4, 4, false, 1>,
                                      (g.N + 1) / 2, 256, 0, stream, g);
     if (rows <= 8 && (g.N <= units / 2 || (g.N > units && g.N <= units * 3 / 2)))
-      return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<1, 8, 4, 2, true> : mmt4d_gemv_i4_kernel<1, 8, 4, 2, false>,
+      return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<1, 8, 4, true, 2> : mmt4d_gemv_i4_kernel<1, 8, 4, false, 2>,
                                      g.N * 2, 256, 0, stream, g);
     if (g.steps <= 16)
-      return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<1, 4, 4, 1, true> : mmt4d_gemv_i4_kernel<1, 4, 4, 1, false>,
+      return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<1, 4, 4, true, 1> : mmt4d_gemv_i4_kernel<1, 4, 4, false, 1>,
                                      g.N, 256, 0, stream, g);
-    return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<1, 6, 4, 1, true> : mmt4d_gemv_i4_kernel<1, 6, 4, 1, false>,
+    return launch_kernel<GemvArgs>(streamed ? mmt4d_gemv_i4_kernel<1, 6, 4, true, 1> : mmt4d_gemv_i4_kernel<1, 6, 4, false, 1>,
                                    g.N, 256, 0, stream, g);
   }
   if (kind == kI8) return launch_kind<kI8>(g, stream, name);

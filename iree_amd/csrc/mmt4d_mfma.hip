@@ -56,6 +56,9 @@ double wave_k_cost_f32(const MfmaArgs& m, const WaveKShape& s, int64_t tiles, bo
   const int fragments = s.fa * s.fb;
   // (K below what was measured: the output is all there is, which the block kernels write as fast.)
   if (m.chunks < 4 && tiles > 256) return 1e30;
+  // (Four steps a wavefront and less, four tiles a unit and more: summing and writing, which the block kernels do as they go
+  // along, is most of it. 464 x 13248 x 268 40.0 us with the block kernel, 46.8 in 80x64 tiles.)
+  if (m.chunks < 32 && tiles > 1024) return 1e30;
   // A chunk's multiplies at the pipe's rate, or its loads. Workgroups beside each other start and end beside each other too.
   const double multiplies = (staged ? 0.02 : 0.0142) * fragments, loads = (staged ? 0.0159 : 0.0107) * (s.fa + s.fb);
   const double us = 1.9 + (tiles > 256 ? tiles / 256.0 : 1.0) * (0.7 + 0.125 * fragments) +
@@ -76,6 +79,8 @@ double block_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
     start_us = 6.8;  // (and the summing of the partial tiles)
   } else {
     choose_tile(m, kind, rhs_i4, gather, direct, &us_per_chunk);
+    // (int4, K cut behind the loop: 336 x 1696 x 288 4.9 us, 4.3 in 64x64 tiles of the other kernel)
+    if (rhs_i4 && ((int64_t)m.K * m.lhs_rb) % 64 != 0) start_us += 0.4;
     if (!direct) us_per_chunk *= 2.2;       // staged through registers
     // Few rows and more 64x64 tiles than units: the unit's second tile, row pieces of 4 and 8 bytes, is dearer than the
     // table's (from 16-byte pieces, many rows): bf16 16 x 20720 x 7396, 16x16x2 tiles, 0.28 us and not 0.195. Without the

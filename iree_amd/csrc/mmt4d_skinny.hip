@@ -581,6 +581,14 @@ hipError_t launch_piece(const SkinnyArgs& s, hipStream_t stream) {
   const int64_t bytes = s.tile_bytes * s.N;
   // No more tile rows than compute units: eight wavefronts, 4 KiB in flight each (1 x 880 x 8918 bf16 9.3 -> 6.5 us, with 8
   // KiB in each of four 7.3; 2 x 1984 x 4991 f16 7.1 -> 5.5, 6.1).
+  // int8, up to two rows and tiles of 128 KiB and more: 8 KiB each (2 x 592 x 9334 4.7, 4.8 with four, 1 x 816 x 9740 4.4, 4.7;
+  // near 256 tile rows 2 to 7 % behind four: 2 x 4096 x 14336 10.7, 10.3).
+  if constexpr (KIND == kI8 && G > 1) {
+    if (s.N <= 256 && s.rows <= 2 && s.tile_bytes >= 128 * 1024) {
+      if (s.rows == 1) return launch_kernel<SkinnyArgs>(mmt4d_skinny_kernel<KIND, G, 1, 8, 8, false, NARROW, false>, (unsigned)s.N, 512, 0, stream, s);
+      return launch_slabs<KIND, G, 8, 8, false, NARROW>(s, stream);
+    }
+  }
   if (s.N <= 256) return launch_slabs<KIND, G, 8, 4, false, NARROW>(s, stream);
   // One byte or less per rhs element against more than two rows is slowed down by streaming: 4 x 14336 x 4096 int8 17.6 us,
   // streamed 20.6, from HBM 20.9 both; only beyond what the caches can hold it gains (235 MB: 60.8 -> 56.8).

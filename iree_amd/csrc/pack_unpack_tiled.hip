@@ -252,6 +252,32 @@ __device__ __forceinline__ void store_tiled(uint4 vec, uint8_t* p) {
   else __builtin_nontemporal_store(v, (v4i32*)p);
 }
 
+// The first `count` elements, fewer than all, of a vector of the 2-D side (unpack): 8, 4, 2 and 1 bytes as they are needed.
+// (Element by element, a row's last vector is a chain of 7 or 15 conditional stores: f16 [23, 843] from 16x16 tiles 5.2 ->
+// 4.2 us. With 4-byte elements, three stores, this is 2 to 4 % slower.)
+template <int E>
+__device__ __forceinline__ void store_edge_vec(uint8_t* g, uint4 v, int32_t count) {
+  typedef uint32_t v2a1 __attribute__((ext_vector_type(2), aligned(1)));
+  typedef uint32_t u32a1 __attribute__((aligned(1)));
+  typedef uint16_t u16a1 __attribute__((aligned(1)));
+  const int32_t bytes = count * E;
+  uint32_t next = v.x, after = v.y;
+  if (bytes & 8) {
+    *(v2a1*)g = v2a1{next, after};
+    next = v.z;
+    after = v.w;
+  }
+  if (bytes & 4) {
+    *(u32a1*)(g + (bytes & 8)) = next;
+    next = after;
+  }
+  if (bytes & 2) {
+    *(u16a1*)(g + (bytes & 12)) = (uint16_t)next;
+    next >>= 16;
+  }
+  if (E < 2 && (bytes & 1)) g[bytes & 14] = (uint8_t)next;
+}
+
 constexpr int kBlockBytes = 16384;  // bytes of the 2-D matrix per workgroup
 
 // E: element bytes. W: vector bytes on the 2-D side (16 needs 4-byte aligned
@@ -392,9 +418,14 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
           } else
           *(flat_vec_t*)g = regs[u].vec;
         } else if (row < a.size0) {
+          if constexpr (E < 4 && W == 16 && !STRIDED) {
+            if (col < a.size1)
+              store_edge_vec<E>(g, make_uint4(regs[u].vec.x, regs[u].vec.y, regs[u].vec.z, regs[u].vec.w), (int32_t)(a.size1 - col));
+          } else {
 #pragma unroll
-          for (int i = 0; i < EPV; ++i)
-            if (col + i < a.size1) ((elem_t*)g)[STRIDED ? i * a.flat_stride1 : i] = regs[u].elem[i];
+            for (int i = 0; i < EPV; ++i)
+              if (col + i < a.size1) ((elem_t*)g)[STRIDED ? i * a.flat_stride1 : i] = regs[u].elem[i];
+          }
         }
       }
     }
@@ -403,6 +434,19 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
   union TiledVec {
     uint4 vec;
     piece_t piece[PIECES];
+  };
+
+  // How far in the LDS image the pieces of the vector at `e` lie from its first one. A thread's vectors are 4 KiB apart, a
+  // whole number of tiles up to that size: all of them are then the same pieces of their tiles, and one look will do (with
+  // one for each vector it took longer than the memory did: f16 [96, 512]
+  // from 16x1 tiles with inner transposes 5.3 -> 4.0 us, [3712, 2624] 10.0 -> 7.7, s32 [272, 448] from 8x8 4.6 -> 3.8).
+  auto piece_offsets = [&](int32_t e, const TiledCoord& first, int32_t* offset) {
+    offset[0] = 0;
+#pragma unroll
+    for (int q = 1; q < PIECES; ++q) {
+      const TiledCoord c = tiled_coord(a, e + q * PL, tile0_base, tile1_base);
+      offset[q] = (c.row - first.row) * a.pitch_bytes + (c.col - first.col) * E;
+    }
   };
 
   // ---- tiled side <-> LDS ----
@@ -419,19 +463,16 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
         }
       }
     }
+    const bool same_pieces = a.log2_t0 + a.log2_t1 + LOG2_E <= 12;
+    int32_t offset[PIECES];
+    if (same_pieces) piece_offsets(tid * VE, first[0], offset);
 #pragma unroll
     for (int u = 0; u < TILED_PER_THREAD; ++u) {
       if (!first[u].in_range) continue;
-      const int32_t e = (tid + 256 * u) * VE;
+      if (!same_pieces) piece_offsets((tid + 256 * u) * VE, first[u], offset);
 #pragma unroll
       for (int q = 0; q < PIECES; ++q) {
-        int32_t row = first[u].row, col = first[u].col;
-        if (q > 0) {
-          const TiledCoord c = tiled_coord(a, e + q * PL, tile0_base, tile1_base);
-          row = c.row;
-          col = c.col;
-        }
-        piece_t* l = (piece_t*)(lds + row * a.pitch_bytes + col * E);
+        piece_t* l = (piece_t*)(lds + first[u].row * a.pitch_bytes + first[u].col * E + offset[q]);
         if constexpr (UNPACK) *l = regs[u].piece[q]; else regs[u].piece[q] = *l;
       }
       if constexpr (!UNPACK) {
@@ -481,20 +522,15 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
             regs[u].vec = load_tiled<kStream>(g);
         }
       }
+      int32_t offset[PIECES];
+      piece_offsets(tid * VE, first[0], offset);
 #pragma unroll
       for (int u = 0; u < MAX_TILED; ++u) {
         if (!wanted[u]) continue;
         taken_whole(&regs[u].vec);
 #pragma unroll
-        for (int q = 0; q < PIECES; ++q) {
-          int32_t row = first[u].row, col = first[u].col;
-          if (q > 0) {
-            const TiledCoord c = tiled_coord(a, (tid + 256 * u) * VE + q * PL, tile0_base, tile1_base);
-            row = c.row;
-            col = c.col;
-          }
-          *(piece_t*)(lds + row * a.pitch_bytes + col * E) = regs[u].piece[q];
-        }
+        for (int q = 0; q < PIECES; ++q)
+          *(piece_t*)(lds + first[u].row * a.pitch_bytes + first[u].col * E + offset[q]) = regs[u].piece[q];
       }
     } else {
 #pragma unroll
@@ -547,9 +583,14 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
           typedef int v4a1 __attribute__((ext_vector_type(4), aligned(1)));
           __builtin_nontemporal_store(v4a1{(int)out[u].vec.x, (int)out[u].vec.y, (int)out[u].vec.z, (int)out[u].vec.w}, (v4a1*)g);
         } else if (row < a.size0) {
+          if constexpr (E < 4) {
+            if (col < a.size1)
+              store_edge_vec<E>(g, make_uint4(out[u].vec.x, out[u].vec.y, out[u].vec.z, out[u].vec.w), (int32_t)(a.size1 - col));
+          } else {
 #pragma unroll
-          for (int i = 0; i < EPV; ++i)
-            if (col + i < a.size1) ((elem_t*)g)[i] = out[u].elem[i];
+            for (int i = 0; i < EPV; ++i)
+              if (col + i < a.size1) ((elem_t*)g)[i] = out[u].elem[i];
+          }
         }
       }
     }

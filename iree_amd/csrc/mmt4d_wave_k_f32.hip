@@ -12,7 +12,7 @@ hipError_t launch_shape(const MfmaArgs& m, int shape, bool streamed, hipStream_t
     constexpr WaveKShape s = kWaveKShapesF32[SHAPE];
     if (shape != SHAPE) return launch_shape<G, SHAPE + 1>(m, shape, streamed, stream);
     if constexpr (SHAPE == 0) {
-      if (m.chunks >= 32) return launch_wave_k_tile<kF32, false, false, G, 1, 1, 8, 3>(m, streamed, stream);
+      if (two_steps_ahead<kF32, G>(m)) return launch_wave_k_tile<kF32, false, false, G, 1, 1, 8, 3>(m, streamed, stream);
     }
     return launch_wave_k_tile<kF32, false, false, G, s.fa, s.fb, 8, 2>(m, streamed, stream);
   } else {

@@ -455,19 +455,26 @@ hipError_t launch_wave_k_tile(const MfmaArgs& m, bool streamed, hipStream_t stre
   }
 }
 
-// One 64-byte step of K in flight ahead of the one that is multiplied, for each of eight wavefronts; two for tiles of one
-// fragment and 32 steps and more, whose multiplication is over before the next step is there: f16 16x16x1 16 x 560 x 7148 8.7
-// -> 7.6 us, f32 32 x 352 x 8740 15.5 -> 13.5, bf16 16 x 1360 x 6576 7.2 -> 7.0. (int8 in 16-byte pieces 1 % slower. Three
-// and more, or two for larger tiles, give nothing, and longer batches leave more to the one wavefront that has K's rest.)
+// One 64-byte step of K in flight ahead of the one that is multiplied, for each of eight wavefronts. With one fragment either
+// way that step is multiplied before the next one is there, and a long K has two in flight: f16 16x16x1 16 x 560 x 7148 8.7
+// -> 7.6 us, f32 32 x 352 x 8740 15.5 -> 13.5, bf16 16 x 1360 x 6576 7.2 -> 7.0. With fewer steps the ring's longer code
+// costs more than it hides, and with few tiles a step is there sooner. Two ahead against one, 1300 problems: 32 to 72 chunks
+// of 64 bytes 4 to 5 % slower, 80 to 100 1 to 2 %, 100 to 120 2 % slower with less than 128 tiles and 2 % faster with more,
+// 3 to 8 % faster beyond (f32 6 % slower at 64 to 80, 4 % at 100 to 120, 4 % faster beyond); 16-byte pieces of f16 and bf16
+// level at 32 to 48 chunks, 1 to 4 % faster from there on, of int8 1 % slower. Three and more, or two for larger tiles, give nothing.
 template <int KIND, int G>
-constexpr bool kTwoStepsAhead = KIND != kI8 || G < 16;
+bool two_steps_ahead(const MfmaArgs& m) {
+  if (G == 16 && KIND != kF32) return KIND != kI8 && m.chunks >= 48;
+  const int64_t tiles = ((((int64_t)m.M << m.log2_M0) + 15) / 16) * ((((int64_t)m.N << m.log2_N0) + 15) / 16);
+  return m.chunks >= (tiles >= 128 ? 100 : 120);
+}
 
 template <int KIND, bool RHS_I4, bool NARROW, int G>
 hipError_t launch_wave_k_piece(const MfmaArgs& m, int shape, bool streamed, hipStream_t stream) {
   switch (shape) {
     case 0:
-      if constexpr (kTwoStepsAhead<KIND, G>) {
-        if (m.chunks >= 32) return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 1, 8, 3>(m, streamed, stream);
+      if constexpr (KIND != kI8 || G < 16) {
+        if (two_steps_ahead<KIND, G>(m)) return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 1, 8, 3>(m, streamed, stream);
       }
       return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 1, 8, 2>(m, streamed, stream);
     case 1: return launch_wave_k_tile<KIND, RHS_I4, NARROW, G, 1, 2, 8, 2>(m, streamed, stream);

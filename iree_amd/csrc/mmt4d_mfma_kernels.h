@@ -99,16 +99,19 @@ constexpr WaveKShape kWaveKShapesF32[] = {
     {3, 5, "mmt4d_mfma_wave_k_48x80"}, {5, 3, "mmt4d_mfma_wave_k_80x48"}, {4, 4, "mmt4d_mfma_wave_k_64x64"},
     {4, 5, "mmt4d_mfma_wave_k_64x80"}, {5, 4, "mmt4d_mfma_wave_k_80x64"}};
 // Whether it loads the 4-byte row pieces of a tile of fa x fb fragments one at a time rather than through LDS. An instruction
-// then covers 16 rows at four k steps, contiguous with 16-row tiles (bf16 16x16x2, 512 x 2048 x 8192 29.1 -> 23.9 us, 64 x
-// 432 x 3712 5.44 -> 4.37; f32 16x16x1, 288 x 1584 x 4064 46.7 -> 41.2), and not where lhs tiles of 4 rows and a second row
-// of them break it up (bf16 4x16x2, 512 x 2048 x 8192 35.4 -> 38.4). 8x8 tiles: int8 gains from 8 fragments on (8x8x4, 512 x
-// 2048 x 2048 8.09 -> 7.29, one fragment, 32 x 1680 x 6784, 5.8 -> 6.9), bf16 loses 3 to 5 %; f32, bound by the matrix
-// pipe, gains with any tile (8x8x1, 128 x 4096 x 2048 26.5 -> 21.8).
+// then covers 16 rows at four k steps. Over 855 products of int8 and bf16 (operand tiles of 4, 8 and 16 rows, every tile of
+// this kernel, K of 300 to 12280) that takes 7 % less time in the mean, 4 % with one fragment, 11 % with 16, whatever the
+// tile shapes (bf16 16x16x2, 512 x 2048 x 8192 29.1 -> 23.9 us; int8 8x8x4, 32 x 1680 x 6784 6.8 -> 5.8), and f32, bound
+// by the matrix pipe, gains 12 to 20 % (8x8x1, 128 x 4096 x 2048 26.5 -> 21.8). Only where the 16 rows are those of four
+// tiles a multiple of 512 bytes apart, on the same memory channels, it is up to 25 % slower (int8 4x8x4, 64 x 4096 x 8192 in
+// 64x32 tiles; at 108 x 3072 x 8552 15.4 -> 13.1 us); not for the lhs with rhs tiles of 16 rows and more
+// fragments of those (4x16x4 and 4x16x2 2 to 9 % faster there too).
 inline bool wave_k_loads_pieces(const MfmaArgs& m, int kind, int gather, int fa, int fb) {
   if (gather != 4) return false;
   if (kind == kF32) return true;
-  if (kind == kI8 && fa * fb != 2 && fa * fb != 4) return fa * fb >= 8;
-  return m.log2_N0 == 4 && (m.log2_M0 >= 3 || m.M == 1);
+  if (m.log2_N0 <= 2 && m.N > 1 && m.rhs_stride_bytes % 512 == 0) return false;
+  if (m.log2_M0 <= 2 && m.M > 1 && m.lhs_stride_bytes % 512 == 0) return m.log2_N0 == 4 && fb > fa;
+  return true;
 }
 hipError_t launch_wave_k_i8(const MfmaArgs& m, int gather, bool rhs_i4, int shape, bool streamed, hipStream_t stream);
 hipError_t launch_wave_k_f16(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);

@@ -36,16 +36,25 @@ def test_f32_long_K(gpu_lib, K0):  # noqa: F811
         run_case(gpu_lib, abi.MMT4D_TYPE_F32F32F32, 3, 5, -(-depth // K0), 16, 16, K0, "mmt4d_mfma_wave_k_16x16", accumulate=n % 2 == 1, seed=n)
 
 
-@pytest.mark.parametrize("flags,M0,N0,K0", [
+# Rows, columns and bytes of K, and the tile they take: K that leaves the rows of 4-row operand tiles no round number of bytes
+# apart, and K that leaves them a multiple of 512 apart (staged, test_mmt4d_choice_on_host.py).
+FOUR_BYTE_LAYOUTS = [
     (abi.MMT4D_TYPE_S8S8S32, 16, 16, 4), (abi.MMT4D_TYPE_S8S8S32, 8, 8, 4), (abi.MMT4D_TYPE_S8S8S32, 4, 16, 4),
+    (abi.MMT4D_TYPE_S8S8S32, 4, 8, 4), (abi.MMT4D_TYPE_S8S8S32, 8, 4, 4),
     (abi.MMT4D_TYPE_BF16BF16F32, 16, 16, 2), (abi.MMT4D_TYPE_BF16BF16F32, 8, 16, 2), (abi.MMT4D_TYPE_BF16BF16F32, 8, 8, 2),
-    (abi.MMT4D_TYPE_BF16BF16F32, 4, 16, 2), (abi.MMT4D_TYPE_F16F16F32, 16, 8, 2), (abi.MMT4D_TYPE_F16F16F16, 16, 16, 2)])
+    (abi.MMT4D_TYPE_BF16BF16F32, 4, 16, 2), (abi.MMT4D_TYPE_F16F16F32, 16, 8, 2), (abi.MMT4D_TYPE_F16F16F16, 16, 16, 2)]
+FOUR_BYTE_SIZES = [(20, 24, 2100, "16x16"), (20, 3000, 700, "16x32"), (100, 1500, 2700, "32x32"), (100, 3000, 1600, "32x64"),
+                   (330, 1500, 1200, "64x64")]
+FOUR_BYTE_ROUND_SIZES = [(20, 3000, 1536, "16x32"), (100, 1500, 2560, "32x32"), (40, 5000, 768, "32x64"), (264, 3000, 2560, "64x64")]
+
+
+@pytest.mark.parametrize("flags,M0,N0,K0", FOUR_BYTE_LAYOUTS)
 def test_four_byte_pieces(gpu_lib, flags, M0, N0, K0):  # noqa: F811
     e = 1 if flags == abi.MMT4D_TYPE_S8S8S32 else 2
-    for n, (rows, cols, row_bytes) in enumerate([(4, 3000, 300), (20, 24, 2100), (100, 1500, 2700), (72, 5000, 68), (330, 1500, 1200),
-                                                 (460, 1900, 1100)]):
-        run_case(gpu_lib, flags, -(-rows // M0), -(-cols // N0), -(-row_bytes // (K0 * e)) + n % 2, M0, N0, K0, "mmt4d_*",
-                 lhs_pad=16 * n, rhs_pad=16 * n, out_pad=4 * (n % 2), accumulate=n % 3 == 1, seed=n)
+    for n, (rows, cols, row_bytes, tile) in enumerate(FOUR_BYTE_SIZES + FOUR_BYTE_ROUND_SIZES):
+        pad = 16 * (n % 2) if row_bytes % 128 else 0
+        run_case(gpu_lib, flags, -(-rows // M0), -(-cols // N0), row_bytes // (K0 * e), M0, N0, K0, "mmt4d_mfma_wave_k_" + tile,
+                 lhs_pad=pad, rhs_pad=pad, out_pad=4 * (n % 2), accumulate=n % 3 == 1, seed=n)
 
 
 def test_what_lies_behind_K_does_not_count(gpu_lib):  # noqa: F811

@@ -7,6 +7,7 @@ import pytest
 
 from iree_amd import abi
 from host_launches import recorder  # noqa: F401
+from test_gpu_wave_k_f32_tiles import FOUR_BYTE_LAYOUTS, FOUR_BYTE_ROUND_SIZES, FOUR_BYTE_SIZES
 
 LAYOUTS = {"bf16": (abi.MMT4D_TYPE_BF16BF16F32, 16, 16, 16), "s8": (abi.MMT4D_TYPE_S8S8S32, 16, 16, 64),
            "s8s4": (abi.MMT4D_TYPE_S8S4S32, 16, 16, 32), "f16, 2-byte pieces": (abi.MMT4D_TYPE_F16F16F32, 16, 16, 1),
@@ -110,3 +111,19 @@ def test_wave_k_looks_two_steps_ahead_with_a_long_K_only(recorder, layout, two_f
             m = re.search(r"mmt4d_wave_k_kernelILi\dELb0ELb0ELi\d+ELi(\d)ELi(\d)ELi8ELi(\d)E", mangled)
             assert m and (m[1] + m[2] != "11" or int(m[3]) == (3 if steps >= threshold else 2)), (steps, mangled)
             assert n > 240 or m[1] + m[2] == "11", (steps, mangled)
+
+
+# 4-byte row pieces are loaded one at a time, but through LDS where 16 rows are four tiles a multiple of 512 bytes apart: of the
+# rhs always, of the lhs unless there are more fragments of an rhs in 16-row tiles. (The last template argument; the tile is
+# the one that test_gpu_wave_k_f32_tiles.py expects.)
+@pytest.mark.parametrize("flags,M0,N0,K0", FOUR_BYTE_LAYOUTS)
+def test_four_byte_pieces_pass_through_lds_where_rows_share_memory_channels(recorder, flags, M0, N0, K0):  # noqa: F811
+    e = 1 if flags == abi.MMT4D_TYPE_S8S8S32 else 2
+    if flags == abi.MMT4D_TYPE_F16F16F16:
+        flags |= abi.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS
+    for rows, cols, row_bytes, tile in FOUR_BYTE_SIZES + FOUR_BYTE_ROUND_SIZES:
+        mangled, kernel = recorder.mmt4d(flags, -(-rows // M0), -(-cols // N0), row_bytes // (K0 * e), M0, N0, K0)
+        assert kernel == "mmt4d_mfma_wave_k_" + tile
+        pieces = re.search(r"ELi4ELi\dELi\dELi8ELi\dELb0ELb(\d)E", mangled)[1] == "1"
+        round_rows = row_bytes % 128 == 0 and (N0 == 4 or (M0 == 4 and not (N0 == 16 and tile in ("16x32", "32x64"))))
+        assert pieces == (not round_rows), (rows, cols, row_bytes, mangled)

@@ -313,7 +313,11 @@ __device__ __forceinline__ void sum_lanes(const T* v, int lane, int period, int 
 
 // Bytes of an lhs k step in registers, where one load takes the pieces of all rows.
 template <int BYTES>
-struct alignas(BYTES < 16 ? BYTES : 16) LhsStep { uint32_t dwords[BYTES < 4 ? 1 : BYTES / 4]; };
+struct alignas(BYTES < 16 ? BYTES : 16) LhsStep { uint32_t dwords[BYTES / 4]; };
+
+// Whether the lhs's row pieces are as long as the rhs's, and two rows of them whole dwords.
+template <int KIND, int G>
+constexpr bool kPackedLhs = G > 1 && (KIND == kI8 || KIND == kI16 || KIND == kF16 || KIND == kBF16 || KIND == kF32);
 
 // G: bytes of a row piece; ROWS: lhs rows the kernel keeps accumulators for
 // (a.rows <= ROWS); UNROLL: 1 KiB blocks of the rhs stream a wavefront has in
@@ -326,7 +330,7 @@ struct alignas(BYTES < 16 ? BYTES : 16) LhsStep { uint32_t dwords[BYTES < 4 ? 1 
 template <int KIND, int G, int ROWS, int WAVES, int UNROLL, bool STREAMED, bool NARROW, bool PACKED>
 __global__ __launch_bounds__(64 * WAVES) void mmt4d_skinny_kernel(const SkinnyArgs a) {
   static_assert(!NARROW || KIND == kF16 || KIND == kBF16, "16-bit outputs are floats");
-  static_assert(!PACKED || KIND == kI8 || KIND == kI16 || KIND == kF16 || KIND == kBF16 || KIND == kF32, "lhs pieces as long as the rhs's");
+  static_assert(!PACKED || (kPackedLhs<KIND, G> && ROWS > 1), "k steps of whole dwords");
   typedef typename Acc<KIND>::type acc_t;
   typedef typename LhsPiece<KIND>::type piece_t;
   // (One-byte pieces of int8: 8-row tiles, two k steps per lane.)
@@ -364,8 +368,7 @@ __global__ __launch_bounds__(64 * WAVES) void mmt4d_skinny_kernel(const SkinnyAr
 #pragma unroll
     for (int m = 0; m < LHS_ROWS; ++m) {
       const uint8_t* p = lhs_row[m] + block * lhs_block;
-      if constexpr (PACKED && LHS_G * ROWS == 2) l[m].dwords[0] = *(const uint16_t*)p;
-      else if constexpr (PACKED) l[m] = *(const lhs_t*)p;
+      if constexpr (PACKED) l[m] = *(const lhs_t*)p;
       else if constexpr (TWO_KSTEPS) l[m] = make_uint2((uint32_t)p[0] | ((second_kstep ? p[lhs_kstep_bytes] : 0u) << 8), 0);
       else l[m] = load_lhs_piece<KIND, G>(p);
     }
@@ -547,6 +550,12 @@ bool make_args(const Mmt4dArgs& a, bool probe_only, int* kind, int* piece_bytes,
   return true;
 }
 
+// Whether the lhs is one tile of 2 or 4 rows that is aligned to its k steps.
+bool lhs_is_packed(const SkinnyArgs& s, int piece_bytes) {
+  const int kstep = piece_bytes * s.rows;
+  return s.rows == 1 << s.log2_M0 && (s.rows == 2 || s.rows == 4) && (uintptr_t)s.lhs % (kstep < 16 ? kstep : 16) == 0;
+}
+
 // PACKED_UNROLL: UNROLL for an lhs tile of 2 or 4 rows that is aligned to its k steps. Other lhs have a load for each row
 // beside one of the rhs, and more registers to each step (3 x 4096 x 4096 f32 of 8-byte pieces: 17.8 us with eight wavefronts
 // of four blocks, 12.1 of two).
@@ -555,9 +564,8 @@ hipError_t launch_slabs(const SkinnyArgs& all_rows, hipStream_t stream) {
   void (*kernel)(const SkinnyArgs);
   SkinnyArgs s = all_rows;
   auto launch = [&] { return launch_kernel(kernel, (unsigned)all_rows.N, 64 * WAVES, 0, stream, s); };
-  if constexpr (G > 1 && (KIND == kI8 || KIND == kI16 || KIND == kF16 || KIND == kBF16 || KIND == kF32)) {
-    const int kstep = G * s.rows;
-    if (s.rows == 1 << s.log2_M0 && (s.rows == 2 || s.rows == 4) && (uintptr_t)s.lhs % (kstep < 16 ? kstep : 16) == 0) {
+  if constexpr (kPackedLhs<KIND, G>) {
+    if (lhs_is_packed(s, G)) {
       kernel = s.rows == 2 ? mmt4d_skinny_kernel<KIND, G, 2, WAVES, PACKED_UNROLL, STREAMED, NARROW, true>
                            : mmt4d_skinny_kernel<KIND, G, 4, WAVES, PACKED_UNROLL, STREAMED, NARROW, true>;
       return launch();
@@ -586,7 +594,7 @@ hipError_t launch_piece(const SkinnyArgs& s, hipStream_t stream) {
   if constexpr (KIND == kI8 && G > 1) {
     if (s.N <= 256 && s.rows <= 2 && s.tile_bytes >= 128 * 1024) {
       if (s.rows == 1) return launch_kernel<SkinnyArgs>(mmt4d_skinny_kernel<KIND, G, 1, 8, 8, false, NARROW, false>, (unsigned)s.N, 512, 0, stream, s);
-      return launch_slabs<KIND, G, 8, 8, false, NARROW>(s, stream);
+      if (lhs_is_packed(s, G)) return launch_kernel<SkinnyArgs>(mmt4d_skinny_kernel<KIND, G, 2, 8, 8, false, NARROW, true>, (unsigned)s.N, 512, 0, stream, s);
     }
   }
   if (s.N <= 256) return launch_slabs<KIND, G, 8, 4, false, NARROW>(s, stream);

@@ -127,3 +127,18 @@ def test_four_byte_pieces_pass_through_lds_where_rows_share_memory_channels(reco
         pieces = re.search(r"ELi4ELi\dELi\dELi8ELi\dELb0ELb(\d)E", mangled)[1] == "1"
         round_rows = row_bytes % 128 == 0 and (N0 == 4 or (M0 == 4 and not (N0 == 16 and tile in ("16x32", "32x64"))))
         assert pieces == (not round_rows), (rows, cols, row_bytes, mangled)
+
+
+def skinny_form(mangled):
+    """Lhs rows, wavefronts, blocks of 1 KiB in flight in each and whether the rhs is streamed, of the few-row kernel."""
+    m = re.search(r"mmt4d_skinny_kernelILi\dELi\dELi(\d)ELi(\d)ELi(\d+)ELb(\d)E", mangled)
+    assert m, mangled
+    return int(m[1]), int(m[2]), int(m[3]), m[4] == "1"
+
+
+# Two int8 rows, at most a tile row a unit and long ones: 8 KiB in flight for a packed lhs, 4 KiB otherwise.
+def test_two_int8_rows(recorder):  # noqa: F811
+    s8 = abi.MMT4D_TYPE_S8S8S32
+    assert skinny_form(recorder.mmt4d(s8, 1, 200, 4200, 2, 16, 2)[0]) == (2, 8, 8, False)
+    assert skinny_form(recorder.mmt4d(s8, 2, 200, 4200, 1, 16, 2)[0]) == (2, 8, 4, False)
+    assert skinny_form(recorder.mmt4d(s8, 1, 200, 4200, 2, 16, 2, lhs=(1 << 40) + 2)[0]) == (2, 8, 4, False)

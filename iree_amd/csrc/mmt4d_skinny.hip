@@ -603,11 +603,14 @@ hipError_t launch_piece(const SkinnyArgs& s, hipStream_t stream) {
   const bool one_byte = KIND == kI8 || KIND == kI8I4 || KIND == kI16U4 || KIND == kI16I8;
   const bool streamed = one_byte && s.rows > 2 ? bytes > (128ll << 20) : comes_from_hbm(bytes);
   // One row and more than two tile rows a unit, from HBM: 12 KiB in flight in each of four wavefronts (1 x 24320 x 3664 int8
-  // 15.4 -> 14.3, 1 x 16816 x 7722 23.4 -> 22.7), but eight wavefronts for tiles of whole 64 KiB (1 x 14336 x 4096 bf16 20.1
-  // -> 19.0, 1 x 28672 x 8192 int8 35.7 -> 34.7) unless they lie a multiple of 256 KiB apart, on few memory channels (f32 1 x
-  // 14336 x 4096 41.5 us, with four 35.5); from the caches eight for tiles of 64 KiB and more.
+  // 15.4 -> 14.3, 1 x 16816 x 7722 23.4 -> 22.7). Their rings take 48 KiB of a tile and eight wavefronts' 32 KiB, and what is
+  // left of the tile is read with fewer loads in flight: tiles of 64 to 96 and of 128 to 144 KiB leave less to eight (290
+  // problems, 32 to 560 KiB: 2.5 % faster in the mean there, 1 x 14336 x 4096 bf16 20.6 -> 19.4 and x 4160 21.5 -> 20.8, 1 x
+  // 16352 x 2964 f16 17.8 -> 16.4, 1 x 20000 x 5120 int8 17.6 -> 16.4); elsewhere eight are 1.2 % slower, at 256 KiB 4.5 %.
+  // From the caches eight for tiles of 64 KiB and more.
   if (s.rows == 1 && s.N > 512) {
-    const bool eight = streamed ? s.rhs_stride_bytes % (64 * 1024) == 0 && s.rhs_stride_bytes % (256 * 1024) != 0 : s.tile_bytes >= 64 * 1024;
+    const int64_t kib = s.tile_bytes >> 10;
+    const bool eight = streamed ? (kib >= 64 && kib < 96) || (kib >= 128 && kib < 144) : kib >= 64;
     if (streamed)
       return eight ? launch_kernel<SkinnyArgs>(mmt4d_skinny_kernel<KIND, G, 1, 8, 4, true, NARROW, false>, (unsigned)s.N, 512, 0, stream, s)
                    : launch_kernel<SkinnyArgs>(mmt4d_skinny_kernel<KIND, G, 1, 4, 12, true, NARROW, false>, (unsigned)s.N, 256, 0, stream, s);

@@ -1,7 +1,7 @@
 """The few-row kernel for narrow row pieces (mmt4d_skinny.hip) where its wavefronts' shares of the stream are empty, shorter
 than the ring of loads, one ring, one and some; with streams that end inside a block of 1 KiB; for lhs tiles of 1, 2 and 4 rows
 that are loaded a k step at a time, the same rows misaligned or in several tiles, which are not, and 8 rows; on both sides of
-the lines at which the number of wavefronts and loads in flight changes (256 and 512 tile rows, 64 and 256 KiB a tile).
+the lines at which the number of wavefronts and loads in flight changes (256 and 512 tile rows, 64, 96, 128 and 144 KiB a tile).
 
 Integers are compared bit for bit with a float64 product, floats within 1e-3 of max(|ref|, rms(ref)): sums of at most
 8200 products of unit-scale values in 32 bits differ by about 1e-6 of that in any order.
@@ -36,6 +36,7 @@ def test_shares(gpu_lib, flags, N0, K0, M, M0):  # noqa: F811
 @pytest.mark.parametrize("M0", [1, 2, 4])
 def test_tile_sizes(gpu_lib, flags, K0, M0):  # noqa: F811
     kib = 1024 // (16 * K0 * BYTES[flags])
-    for N, tile_kib in [(16, 256), (256, 64), (257, 63), (512, 20), (513, 63), (513, 64), (600, 100), (520, 128), (200, 256)]:
-        if N * tile_kib < 70 << 10:
+    for N, tile_kib in [(16, 256), (256, 64), (257, 63), (512, 20), (513, 63), (513, 64), (600, 95), (600, 96), (600, 100), (520, 127), (520, 128), (513, 143),
+                        (513, 144), (200, 256)]:
+        if N * tile_kib < 76 << 10:
             run_case(gpu_lib, flags, 1, N, tile_kib * kib, M0, 16, K0, "mmt4d_skinny", seed=N)

@@ -142,3 +142,17 @@ def test_two_int8_rows(recorder):  # noqa: F811
     assert skinny_form(recorder.mmt4d(s8, 1, 200, 4200, 2, 16, 2)[0]) == (2, 8, 8, False)
     assert skinny_form(recorder.mmt4d(s8, 2, 200, 4200, 1, 16, 2)[0]) == (2, 8, 4, False)
     assert skinny_form(recorder.mmt4d(s8, 1, 200, 4200, 2, 16, 2, lhs=(1 << 40) + 2)[0]) == (2, 8, 4, False)
+
+
+# One row from HBM, more than two tile rows a unit: eight wavefronts for tiles of 64 to 96 and 128 to 144 KiB, however far apart
+# the tile rows lie.
+@pytest.mark.parametrize("flags,K0,e", [(abi.MMT4D_TYPE_BF16BF16F32, 2, 2), (abi.MMT4D_TYPE_S8S8S32, 2, 1), (abi.MMT4D_TYPE_F32F32F32, 1, 4),
+                                        (abi.MMT4D_TYPE_F16F16F32, 1, 2)])
+def test_one_row_from_hbm(recorder, flags, K0, e):  # noqa: F811
+    for tile_kib, eight in ((50, False), (63, False), (64, True), (65, True), (95, True), (96, False), (127, False), (128, True), (130, True),
+                            (143, True), (144, False), (192, False), (256, False)):
+        K = tile_kib * 1024 // (16 * K0 * e)
+        for steps_off in (0, 1, 3):
+            for pad in (0, 16, 1024):
+                form = skinny_form(recorder.mmt4d(flags, 1, 1100, K + steps_off, 1, 16, K0, rhs_pad=pad)[0])
+                assert form == ((1, 8, 4, True) if eight else (1, 4, 12, True)), (tile_kib, steps_off, pad, form)

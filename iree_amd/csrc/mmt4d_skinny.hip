@@ -563,7 +563,7 @@ template <int KIND, int G, int WAVES, int PACKED_UNROLL, bool STREAMED, bool NAR
 hipError_t launch_slabs(const SkinnyArgs& all_rows, hipStream_t stream) {
   void (*kernel)(const SkinnyArgs);
   SkinnyArgs s = all_rows;
-  auto launch = [&] { return launch_kernel(kernel, (unsigned)all_rows.N, 64 * WAVES, 0, stream, s); };
+  auto launch = [&](int waves = WAVES) { return launch_kernel(kernel, (unsigned)all_rows.N, 64 * waves, 0, stream, s); };
   if constexpr (kPackedLhs<KIND, G>) {
     if (lhs_is_packed(s, G)) {
       kernel = s.rows == 2 ? mmt4d_skinny_kernel<KIND, G, 2, WAVES, PACKED_UNROLL, STREAMED, NARROW, true>
@@ -571,14 +571,18 @@ hipError_t launch_slabs(const SkinnyArgs& all_rows, hipStream_t stream) {
       return launch();
     }
   }
-  // More than 8 rows: one launch per slab of 8.
+  // More than 8 rows: one launch per slab of 8. Five rows and more have a ring of two blocks (8 x 4096 x 4096 s16u4 9.9 us, of
+  // four 19.7, s16s8 10.8 and 11.4, int8 in 4x16x2 tiles 8.0 and 9.1, f32 in 2x16x1 12.6 and 13.8). int4
+  // in 1-byte pieces, 32 sums a row, does not fit the registers that eight wavefronts leave (31 spilled) and has four (8 x
+  // 4096 x 4096 9.6 -> 8.0, 8 x 1024 x 1024 5.7 -> 4.8).
+  constexpr int WAVES_8_ROWS = KIND == kI8I4 && G == 1 ? 4 : WAVES;
   for (s.row0 = 0; s.row0 < s.rows; s.row0 += 8) {
     const int left = s.rows - s.row0;
     if (left <= 1) kernel = mmt4d_skinny_kernel<KIND, G, 1, WAVES, 4, STREAMED, NARROW, false>;
     else if (left <= 2) kernel = mmt4d_skinny_kernel<KIND, G, 2, WAVES, 4, STREAMED, NARROW, false>;
     else if (left <= 4) kernel = mmt4d_skinny_kernel<KIND, G, 4, WAVES, G == 8 && WAVES == 8 ? 2 : 4, STREAMED, NARROW, false>;
-    else kernel = mmt4d_skinny_kernel<KIND, G, 8, WAVES, 2, STREAMED, NARROW, false>;
-    const hipError_t e = launch();
+    else kernel = mmt4d_skinny_kernel<KIND, G, 8, WAVES_8_ROWS, 2, STREAMED, NARROW, false>;
+    const hipError_t e = launch(left <= 4 ? WAVES : WAVES_8_ROWS);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

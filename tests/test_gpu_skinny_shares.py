@@ -40,3 +40,10 @@ def test_tile_sizes(gpu_lib, flags, K0, M0):  # noqa: F811
                         (513, 144), (200, 256)]:
         if N * tile_kib < 76 << 10:
             run_case(gpu_lib, flags, 1, N, tile_kib * kib, M0, 16, K0, "mmt4d_skinny", seed=N)
+
+
+@pytest.mark.parametrize("M,M0,N0", [(1, 1, 16), (1, 2, 16), (1, 4, 16), (1, 8, 16), (3, 4, 16), (7, 1, 32)])
+def test_int4_one_byte_pieces_long_streams(gpu_lib, M, M0, N0):  # noqa: F811
+    for n, (N, tile_kib) in enumerate([(16, 40), (256, 64), (257, 100), (513, 41), (600, 100)]):
+        K = tile_kib * 1024 // N0 + n
+        run_case(gpu_lib, abi.MMT4D_TYPE_S8S4S32, M, N, K, M0, N0, 2, "mmt4d_skinny", accumulate=n % 2 == 1, seed=n)

@@ -572,16 +572,17 @@ hipError_t launch_slabs(const SkinnyArgs& all_rows, hipStream_t stream) {
     }
   }
   // More than 8 rows: one launch per slab of 8. Five rows and more have a ring of two blocks (8 x 4096 x 4096 s16u4 9.9 us, of
-  // four 19.7, s16s8 10.8 and 11.4, int8 in 4x16x2 tiles 8.0 and 9.1, f32 in 2x16x1 12.6 and 13.8). int4
+  // four 19.7, s16s8 10.8 and 11.4, int8 in 4x16x2 tiles 8.0 and 9.1, f32 in 2x16x1 12.6 and 13.8), but s16 in 4-byte pieces
+  // from HBM, which needs the bytes in flight, one of four (16 x 14336 x 4096 64.2 -> 57.4, 8 x 14336 x 4096 24.8 -> 23.1). int4
   // in 1-byte pieces, 32 sums a row, does not fit the registers that eight wavefronts leave (31 spilled) and has four (8 x
   // 4096 x 4096 9.6 -> 8.0, 8 x 1024 x 1024 5.7 -> 4.8).
-  constexpr int WAVES_8_ROWS = KIND == kI8I4 && G == 1 ? 4 : WAVES;
+  constexpr int WAVES_8_ROWS = KIND == kI8I4 && G == 1 ? 4 : WAVES, UNROLL_8_ROWS = KIND == kI16 && G == 4 && STREAMED ? 4 : 2;
   for (s.row0 = 0; s.row0 < s.rows; s.row0 += 8) {
     const int left = s.rows - s.row0;
     if (left <= 1) kernel = mmt4d_skinny_kernel<KIND, G, 1, WAVES, 4, STREAMED, NARROW, false>;
     else if (left <= 2) kernel = mmt4d_skinny_kernel<KIND, G, 2, WAVES, 4, STREAMED, NARROW, false>;
     else if (left <= 4) kernel = mmt4d_skinny_kernel<KIND, G, 4, WAVES, G == 8 && WAVES == 8 ? 2 : 4, STREAMED, NARROW, false>;
-    else kernel = mmt4d_skinny_kernel<KIND, G, 8, WAVES_8_ROWS, 2, STREAMED, NARROW, false>;
+    else kernel = mmt4d_skinny_kernel<KIND, G, 8, WAVES_8_ROWS, UNROLL_8_ROWS, STREAMED, NARROW, false>;
     const hipError_t e = launch(left <= 4 ? WAVES : WAVES_8_ROWS);
     if (e != hipSuccess) return e;
   }

@@ -158,11 +158,13 @@ def test_one_row_from_hbm(recorder, flags, K0, e):  # noqa: F811
                 assert form == ((1, 8, 4, True) if eight else (1, 4, 12, True)), (tile_kib, steps_off, pad, form)
 
 
-# Five rows and more have a ring of two blocks; int4 in 1-byte pieces has four wavefronts always.
+# Five rows and more have a ring of two blocks, int16 from HBM one of four; int4 in 1-byte pieces has four wavefronts always.
 def test_five_to_eight_rows(recorder):  # noqa: F811
     s16, u4, i4 = abi.MMT4D_TYPE_S16S16S32, abi.MMT4D_TYPE_S16U4S32, abi.MMT4D_TYPE_S8S4S32
+    assert skinny_form(recorder.mmt4d(s16, 1, 900, 2048, 8, 16, 2)[0]) == (8, 4, 4, True)
     assert skinny_form(recorder.mmt4d(s16, 1, 900, 800, 8, 16, 2)[0]) == (8, 4, 2, False)
     assert skinny_form(recorder.mmt4d(s16, 1, 200, 2048, 8, 16, 2)[0]) == (8, 8, 2, False)
+    assert skinny_form(recorder.mmt4d(s16, 1, 900, 4096, 8, 8, 2)[0]) == (8, 4, 4, True)
     assert skinny_form(recorder.mmt4d(u4, 1, 200, 512, 8, 32, 8)[0]) == (8, 8, 2, False)
     for M, M0 in ((1, 8), (5, 1), (2, 8), (2, 4)):
         assert skinny_form(recorder.mmt4d(i4, M, 64, 512, M0, 16, 2)[0]) == (8, 4, 2, False)

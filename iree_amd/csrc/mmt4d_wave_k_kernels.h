@@ -132,8 +132,7 @@ struct Operand {
           for (int d = 0; d < 4; ++d) {
             global_u32_t from = (global_u32_t)(at[d] + off[f]);
             if constexpr (CHECKED) from = (global_u32_t)((global_bytes_t)from - back[d]);
-            if constexpr (STREAMED) piece[d] = __builtin_nontemporal_load(from);
-            else piece[d] = *from;
+            piece[d] = *from;
           }
           to = make_uint4(piece[0], piece[1], piece[2], piece[3]);
         } else {
@@ -188,7 +187,7 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
   typedef typename Acc16<KIND>::type acc_t;
   typedef Operand<G, FA, RHS_I4, PIECES> lhs_t;
   typedef Operand<G, FB, false, PIECES> rhs_t;
-  static_assert(!PIECES || G == 4, "4-byte pieces");
+  static_assert(!PIECES || (G == 4 && !STREAMED), "4-byte pieces, which are read through the caches");
   constexpr bool STAGED = G < 16 && !PIECES;  // operands pass through LDS
   static_assert(!RHS_I4 || (KIND == kI8 && G == 16), "int4 rhs");
   // The wavefronts' staging of narrow row pieces, [WAVES][FA + FB][1 KiB]; then [WAVES][FA * FB][64] partial sums.

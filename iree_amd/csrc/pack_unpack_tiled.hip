@@ -252,15 +252,14 @@ __device__ __forceinline__ void store_tiled(uint4 vec, uint8_t* p) {
   else __builtin_nontemporal_store(v, (v4i32*)p);
 }
 
-// The first `count` elements, fewer than all, of a vector of the 2-D side (unpack): 8, 4, 2 and 1 bytes as they are needed.
-// (Element by element, a row's last vector is a chain of 7 or 15 conditional stores: f16 [23, 843] from 16x16 tiles 5.2 ->
-// 4.2 us. With 4-byte elements, three stores, this is 2 to 4 % slower.)
-template <int E>
+// The first `count` elements of 2 bytes, fewer than eight, of a vector of the 2-D side (unpack): 8, 4 and 2 bytes as they
+// are needed. (Element by element, a row's last vector is a chain of seven conditional stores: f16 [23, 843] from 16x16 tiles
+// 5.2 -> 4.2 us. With 4-byte elements, three stores, this is 2 to 4 % slower.)
 __device__ __forceinline__ void store_edge_vec(uint8_t* g, uint4 v, int32_t count) {
   typedef uint32_t v2a1 __attribute__((ext_vector_type(2), aligned(1)));
   typedef uint32_t u32a1 __attribute__((aligned(1)));
   typedef uint16_t u16a1 __attribute__((aligned(1)));
-  const int32_t bytes = count * E;
+  const int32_t bytes = count * 2;
   uint32_t next = v.x, after = v.y;
   if (bytes & 8) {
     *(v2a1*)g = v2a1{next, after};
@@ -271,11 +270,7 @@ __device__ __forceinline__ void store_edge_vec(uint8_t* g, uint4 v, int32_t coun
     *(u32a1*)(g + (bytes & 8)) = next;
     next = after;
   }
-  if (bytes & 2) {
-    *(u16a1*)(g + (bytes & 12)) = (uint16_t)next;
-    next >>= 16;
-  }
-  if (E < 2 && (bytes & 1)) g[bytes & 14] = (uint8_t)next;
+  if (bytes & 2) *(u16a1*)(g + (bytes & 12)) = (uint16_t)next;
 }
 
 constexpr int kBlockBytes = 16384;  // bytes of the 2-D matrix per workgroup
@@ -418,9 +413,9 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
           } else
           *(flat_vec_t*)g = regs[u].vec;
         } else if (row < a.size0) {
-          if constexpr (E < 4 && W == 16 && !STRIDED) {
+          if constexpr (E == 2 && W == 16 && !STRIDED) {
             if (col < a.size1)
-              store_edge_vec<E>(g, make_uint4(regs[u].vec.x, regs[u].vec.y, regs[u].vec.z, regs[u].vec.w), (int32_t)(a.size1 - col));
+              store_edge_vec(g, make_uint4(regs[u].vec.x, regs[u].vec.y, regs[u].vec.z, regs[u].vec.w), (int32_t)(a.size1 - col));
           } else {
 #pragma unroll
             for (int i = 0; i < EPV; ++i)
@@ -436,16 +431,15 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
     piece_t piece[PIECES];
   };
 
-  // How far in the LDS image the pieces of the vector at `e` lie from its first one. A thread's vectors are 4 KiB apart, a
-  // whole number of tiles up to that size: all of them are then the same pieces of their tiles, and one look will do (with
-  // one for each vector it took longer than the memory did: f16 [96, 512]
-  // from 16x1 tiles with inner transposes 5.3 -> 4.0 us, [3712, 2624] 10.0 -> 7.7, s32 [272, 448] from 8x8 4.6 -> 3.8).
-  auto piece_offsets = [&](int32_t e, const TiledCoord& first, int32_t* offset) {
-    offset[0] = 0;
+  // How far in the LDS image piece q of a vector lies from its first one: as far as element q * PL of the block from element
+  // 0, whatever the vector, which starts at a multiple of 16 bytes where all extents are powers of two. (With a look for each
+  // vector of a thread these took longer than the memory did: f16 [96, 512] from 16x1 tiles with inner transposes 5.3 -> 4.0
+  // us, [3712, 2624] 10.0 -> 7.7, s32 [272, 448] from 8x8 4.6 -> 3.8.)
+  auto piece_offsets = [&](int32_t* offset) {
 #pragma unroll
-    for (int q = 1; q < PIECES; ++q) {
-      const TiledCoord c = tiled_coord(a, e + q * PL, tile0_base, tile1_base);
-      offset[q] = (c.row - first.row) * a.pitch_bytes + (c.col - first.col) * E;
+    for (int q = 0; q < PIECES; ++q) {
+      const TiledCoord c = tiled_coord(a, q * PL, tile0_base, tile1_base);
+      offset[q] = c.row * a.pitch_bytes + c.col * E;
     }
   };
 
@@ -463,13 +457,11 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
         }
       }
     }
-    const bool same_pieces = a.log2_t0 + a.log2_t1 + LOG2_E <= 12;
     int32_t offset[PIECES];
-    if (same_pieces) piece_offsets(tid * VE, first[0], offset);
+    piece_offsets(offset);
 #pragma unroll
     for (int u = 0; u < TILED_PER_THREAD; ++u) {
       if (!first[u].in_range) continue;
-      if (!same_pieces) piece_offsets((tid + 256 * u) * VE, first[u], offset);
 #pragma unroll
       for (int q = 0; q < PIECES; ++q) {
         piece_t* l = (piece_t*)(lds + first[u].row * a.pitch_bytes + first[u].col * E + offset[q]);
@@ -523,7 +515,7 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
         }
       }
       int32_t offset[PIECES];
-      piece_offsets(tid * VE, first[0], offset);
+      piece_offsets(offset);
 #pragma unroll
       for (int u = 0; u < MAX_TILED; ++u) {
         if (!wanted[u]) continue;
@@ -583,9 +575,9 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
           typedef int v4a1 __attribute__((ext_vector_type(4), aligned(1)));
           __builtin_nontemporal_store(v4a1{(int)out[u].vec.x, (int)out[u].vec.y, (int)out[u].vec.z, (int)out[u].vec.w}, (v4a1*)g);
         } else if (row < a.size0) {
-          if constexpr (E < 4) {
+          if constexpr (E == 2) {
             if (col < a.size1)
-              store_edge_vec<E>(g, make_uint4(out[u].vec.x, out[u].vec.y, out[u].vec.z, out[u].vec.w), (int32_t)(a.size1 - col));
+              store_edge_vec(g, make_uint4(out[u].vec.x, out[u].vec.y, out[u].vec.z, out[u].vec.w), (int32_t)(a.size1 - col));
           } else {
 #pragma unroll
             for (int i = 0; i < EPV; ++i)
@@ -1269,7 +1261,9 @@ template <bool UNPACK, int POLICY>
 hipError_t launch_plan(const Plan& p, hipStream_t stream) {
   if (p.flat_vec_bytes != 16) return hipErrorInvalidValue;
   switch (p.elem_bytes) {
-    case 1: return launch_e<1, UNPACK, POLICY>(p, stream);
+    case 1:  // (no unpack has elements of one byte)
+      if constexpr (!UNPACK) return launch_e<1, UNPACK, POLICY>(p, stream);
+      return hipErrorInvalidValue;
     case 2: return launch_e<2, UNPACK, POLICY>(p, stream);
     case 4: return launch_e<4, UNPACK, POLICY>(p, stream);
     default: return hipErrorInvalidValue;

@@ -4,7 +4,7 @@ rhs tile is dealt to one, two or four workgroups (3/16, 1/2, 1 and 3/2 of 256 co
 lhs rows in one tile and in several, strided and accumulating.
 
 Integers are compared bit for bit with a float64 product, floats within 1e-3 of max(|ref|, rms(ref)): sums of at most
-4500 products of unit-scale values in 32 bits differ by about 1e-6 of that in any order.
+67600 products of unit-scale values in 32 bits differ by about 1e-6 of that in any order.
 """
 import pytest
 
@@ -44,3 +44,18 @@ def test_int4_shares(gpu_lib, K0, M, M0):  # noqa: F811
                      accumulate=n % 3 == 1, seed=n)
     for N in (770, 1025, 1030):
         run_case(gpu_lib, abi.MMT4D_TYPE_S8S4S32, M, N, 8320 // K0, M0, 16, K0, "mmt4d_gemv", seed=N)
+
+
+# Few tiles dealt to two or four workgroups whose rhs is more than 48 MiB and read past the caches.
+@pytest.mark.parametrize("flags,K0", [(BF16, 8), (F16, 16), (S8, 64), (S8, 16)])
+@pytest.mark.parametrize("M,M0,N,row_bytes", [(1, 1, 320, 10304), (1, 8, 384, 8720), (1, 4, 300, 11000), (1, 1, 48, 66000), (3, 1, 47, 67584),
+                                              (1, 8, 128, 25104)])
+def test_split_tiles_from_hbm(gpu_lib, flags, K0, M, M0, N, row_bytes):  # noqa: F811
+    K = row_bytes // (K0 * (1 if flags == S8 else 2))
+    run_case(gpu_lib, flags, M, N, K, M0, 16, K0, "mmt4d_gemv", accumulate=M == 3, seed=N)
+
+
+@pytest.mark.parametrize("K0", [32, 64])
+@pytest.mark.parametrize("M,M0,N,depth", [(1, 1, 384, 16512), (1, 8, 300, 21216), (5, 1, 128, 49984)])
+def test_int4_split_tiles_from_hbm(gpu_lib, K0, M, M0, N, depth):  # noqa: F811
+    run_case(gpu_lib, abi.MMT4D_TYPE_S8S4S32, M, N, depth // K0, M0, 16, K0, "mmt4d_gemv", accumulate=M == 5, seed=N)

@@ -18,26 +18,26 @@ LAYOUTS = {"bf16": (abi.MMT4D_TYPE_BF16BF16F32, 16, 16, 16), "s8": (abi.MMT4D_TY
 # Microseconds with operands held by the cache (150 MB in turn) and from HBM (640 MB in turn): the tiles of the kernel that
 # splits K over wavefronts, and the block kernel that the problem would take.
 TIMES = [
-    ("bf16", 32, 11008, 2048, {"32x64": (9.8, 12.5), "64x64": (10.0, 12.8), "16x32": (10.4, 13.8), "block": (11.9, 13.2)}),
-    ("bf16", 64, 4096, 4096, {"32x32": (9.2, 13.1), "16x32": (11.2, 16.0), "32x64": (11.0, 16.5), "block": (19.7, 21.0)}),
-    ("bf16", 96, 14336, 4096, {"block": (23.9, 32.6), "64x64": (26.6, 38.4), "32x64": (27.5, 40.7)}),
-    ("bf16", 512, 4096, 4096, {"block": (24.5, 30.0), "64x64": (26.4, 35.1), "64x32": (32.1, 42.4)}),
-    ("s8", 64, 14336, 4096, {"64x64": (14.2, 14.7), "block": (12.8, 16.5), "32x64": (14.7, 19.3)}),
-    ("s8", 128, 4096, 14336, {"32x64": (22.2, 26.9), "64x32": (22.1, 27.3), "32x32": (27.8, 33.1), "block": (32.0, 35.9)}),
-    ("s8s4", 32, 28672, 8192, {"32x64": (25.4, 26.1), "16x32": (24.1, 33.9), "64x64": (28.4, 28.8), "block": (27.2, 30.7)}),
-    ("s8s4", 96, 14336, 4096, {"block": (16.2, 16.3), "64x64": (15.8, 17.9), "32x64": (16.2, 19.3)}),
-    ("s8s4", 96, 11008, 2048, {"block": (10.2, 10.3), "32x64": (10.8, 11.8), "64x64": (10.4, 12.4)}),
-    ("s8s4", 192, 8192, 4096, {"64x64": (15.3, 17.9), "block": (16.6, 16.7), "32x64": (16.6, 18.7)}),
-    ("f16, 2-byte pieces", 64, 4096, 4096, {"32x32": (10.8, 13.9), "16x32": (13.3, 16.7), "64x32": (14.0, 17.5), "block": (37.6, 37.9)}),
-    ("s8, 4-byte pieces", 128, 2048, 2048, {"32x32": (5.6, 5.9), "16x32": (6.1, 6.4), "32x64": (6.5, 6.9), "block": (7.8, 7.9)}),
-    ("bf16, 8-byte pieces", 32, 14336, 4096, {"32x64": (20.5, 25.2), "block": (19.9, 26.0), "64x64": (21.8, 26.6)}),
-    ("s8, 2-byte pieces", 256, 11008, 2048, {"block": (15.5, 17.6), "64x64": (21.2, 23.8), "64x32": (28.1, 31.4)}),
-    ("s8, 2-byte pieces", 304, 1632, 272, {"64x32": (4.0, 4.1), "64x64": (4.7, 4.9), "block": (4.8, 5.0)}),
-    ("s8, 4-byte pieces", 16, 20000, 3000, {"16x32": (12.4, 15.2), "16x16": (13.3, 17.0), "block": (14.5, 17.4)}),
-    ("s8, 2-byte pieces", 96, 10112, 10112, {"32x64": (31.5, 39.0), "block": (44.3, 44.6), "64x64": (42.0, 48.4)}),
-    ("bf16, 4-byte pieces", 16, 10112, 10112, {"32x64": (41.7, 41.7), "16x32": (47.6, 47.6), "16x16": (45.1, 45.0), "block": (48.3, 48.1)}),
-    ("bf16, 4-byte pieces", 16, 20000, 3000, {"16x32": (20.8, 25.9), "16x16": (20.6, 28.0), "block": (24.4, 29.5)}),
-    ("f32", 64, 2048, 2048, {"16x32": (10.2, 10.8), "16x16": (12.2, 13.0), "32x32": (15.9, 16.7), "block": (37.4, 37.5)}),
+    ("bf16", 32, 11008, 2048, {"32x64": (9.57, 11.77), "64x64": (9.86, 12.13), "block": (10.58, 12.48)}),
+    ("bf16", 64, 4096, 4096, {"32x32": (8.69, 12.70), "32x64": (10.77, 16.34), "64x32": (10.90, 16.43), "block": (17.16, 21.26)}),
+    ("bf16", 96, 14336, 4096, {"block": (23.49, 31.51), "64x64": (25.34, 36.39), "32x64": (26.84, 40.35)}),
+    ("bf16", 512, 4096, 4096, {"block": (22.84, 29.98), "64x64": (25.84, 36.22), "64x32": (32.44, 44.09)}),
+    ("s8", 64, 14336, 4096, {"block": (12.42, 15.92), "64x64": (13.66, 14.76), "32x64": (14.27, 18.84)}),
+    ("s8", 128, 4096, 14336, {"64x32": (22.03, 26.97), "32x64": (22.11, 27.09), "32x32": (27.61, 33.56), "block": (28.32, 36.02)}),
+    ("s8s4", 32, 28672, 8192, {"32x64": (23.48, 25.34), "64x64": (26.08, 27.28), "16x32": (22.52, 33.90), "block": (26.98, 28.57)}),
+    ("s8s4", 96, 14336, 4096, {"64x64": (14.24, 16.24), "32x64": (14.95, 18.03), "block": (16.32, 16.52)}),
+    ("s8s4", 96, 11008, 2048, {"32x32": (9.08, 10.18), "block": (10.07, 10.32), "64x64": (9.95, 11.34)}),
+    ("s8s4", 192, 8192, 4096, {"64x64": (14.30, 17.13), "32x64": (15.45, 18.00), "block": (16.75, 16.76)}),
+    ("f16, 2-byte pieces", 64, 4096, 4096, {"32x32": (9.45, 14.99), "16x32": (12.09, 17.08), "64x32": (12.10, 17.23), "block": (33.79, 34.58)}),
+    ("s8, 4-byte pieces", 128, 2048, 2048, {"32x32": (4.92, 5.50), "16x32": (5.65, 6.29), "32x64": (5.75, 6.56), "block": (6.96, 8.05)}),
+    ("bf16, 8-byte pieces", 32, 14336, 4096, {"block": (19.08, 24.37), "32x64": (19.61, 24.94), "64x64": (20.61, 25.55)}),
+    ("s8, 2-byte pieces", 256, 11008, 2048, {"block": (15.04, 17.74), "64x64": (19.34, 22.14), "32x32": (22.02, 27.20)}),
+    ("s8, 2-byte pieces", 304, 1632, 272, {"64x32": (3.96, 4.32), "32x32": (4.11, 4.33), "block": (4.70, 5.03)}),
+    ("s8, 4-byte pieces", 16, 20000, 3000, {"16x32": (11.77, 14.76), "32x32": (11.93, 15.10), "64x32": (12.92, 16.03), "block": (14.22, 16.88)}),
+    ("s8, 2-byte pieces", 96, 10112, 10112, {"32x64": (27.09, 38.19), "32x32": (30.49, 42.96), "64x64": (34.90, 44.45), "block": (39.44, 40.53)}),
+    ("bf16, 4-byte pieces", 16, 10112, 10112, {"32x64": (30.28, 41.46), "64x64": (30.69, 43.56), "16x16": (32.05, 44.58), "block": (39.52, 43.97)}),
+    ("bf16, 4-byte pieces", 16, 20000, 3000, {"16x32": (19.15, 25.76), "32x32": (19.47, 26.00), "16x16": (19.16, 27.17), "block": (23.92, 28.90)}),
+    ("f32", 64, 2048, 2048, {"16x32": (7.97, 10.13), "16x16": (8.82, 11.53), "32x32": (11.16, 12.52), "block": (36.92, 37.41)}),
 ]
 
 

@@ -5,10 +5,9 @@
 // straight into MFMA operand registers, no LDS: for N0 = 16 a wavefront's
 // 16-row x 64-byte operand (lane l: row l & 15, 16-byte column l >> 4) covers
 // whole consecutive k steps of one tile, i.e. each load instruction reads 1 KiB
-// of contiguous memory. The (small, L2-resident) lhs is loaded the same way and
-// shared by the TN rhs tiles a wavefront works on. The wavefronts of a
-// workgroup split K between them and reduce through LDS in a fixed order, so
-// results do not depend on scheduling. The matrix pipe is mostly idle here by
+// of contiguous memory. The (small, L2-resident) lhs is loaded the same way. The
+// wavefronts of a workgroup split K between them and reduce through LDS in a
+// fixed order, so results do not depend on scheduling. The matrix pipe is mostly idle here by
 // design; it is used because its operand layout matches the tiled rhs exactly
 // and it keeps the VALU out of the inner loop.
 //

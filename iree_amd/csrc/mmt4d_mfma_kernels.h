@@ -1074,8 +1074,8 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     }
   };
   // Where that happens: behind the loop, in front of the last chunk's step, or in the step that reads its fragments. A
-  // branch in every step costs the smaller tiles (int8 1024^3 in 64x64 tiles 5.86 -> 5.35 us without it, f16 384 x 2912 x
-  // 2848 in 128x64 tiles 17.2 -> 14.8) and all int4 ones (128x128 and 64x128 11 to 14 %). The larger tiles hide it, and
+  // branch in every step costs the smaller tiles (f16 384 x 2912 x 2848 in 128x64 tiles 17.2 -> 14.8 us without it; int8
+  // 1024^3 in 64x64 tiles 5.86 -> 5.35, level with the wave-K tile that it takes) and all int4 ones (128x128 and 64x128 11 to 14 %). The larger tiles hide it, and
   // lose more by the further step that the code then has behind the loop, run once and fetched from memory (192x192
   // tiles 1 us of 16).
   constexpr bool CUT_BEHIND_LOOP = RHS_I4 || AM * BN <= 4;

@@ -54,10 +54,13 @@ double wave_k_cost_f32(const MfmaArgs& m, const WaveKShape& s, int64_t tiles, bo
   const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
   const double megabytes = 1e-6 * (double)(rows * m.lhs_rb + cols * m.rhs_rb) * m.K;
   const int fragments = s.fa * s.fb;
-  // (K below what was measured: the output is all there is, which the block kernels write as fast.)
+  // (The output is all there is, which the block kernels write faster: 2048 x 2048 x 16 8.3 us, in 32x64 tiles 12.8, 512 x 4096
+  // x 48 6.9 and 8.1.)
   if (m.chunks < 4 && tiles > 256) return 1e30;
   // (Four steps a wavefront and less, four tiles a unit and more: summing and writing, which the block kernels do as they go
-  // along, is most of it. 464 x 13248 x 268 40.0 us with the block kernel, 46.8 in 80x64 tiles.)
+  // along, is most of it. One problem in 400 of K < 512 has another kernel for it; of 24 such, those kernels take 4 % less
+  // in the mean: 464 x 13248 x 268 40.0 us with the block kernel, 46.8 in 80x64 tiles, 1008 x 6528 x 389 54.5 and 64.3, but 224
+  // x 13136 x 496 34.7 and in 32x64 tiles 29.9.)
   if (m.chunks < 32 && tiles > 1024) return 1e30;
   // A chunk's multiplies at the pipe's rate, or its loads. Workgroups beside each other start and end beside each other too.
   const double multiplies = (staged ? 0.02 : 0.0142) * fragments, loads = (staged ? 0.0159 : 0.0107) * (s.fa + s.fb);

@@ -37,6 +37,11 @@ TIMES = [
     ("s8, 2-byte pieces", 96, 10112, 10112, {"32x64": (27.09, 38.19), "32x32": (30.49, 42.96), "64x64": (34.90, 44.45), "block": (39.44, 40.53)}),
     ("bf16, 4-byte pieces", 16, 10112, 10112, {"32x64": (30.28, 41.46), "64x64": (30.69, 43.56), "16x16": (32.05, 44.58), "block": (39.52, 43.97)}),
     ("bf16, 4-byte pieces", 16, 20000, 3000, {"16x32": (19.15, 25.76), "32x32": (19.47, 26.00), "16x16": (19.16, 27.17), "block": (23.92, 28.90)}),
+    ("s8, 2-byte pieces", 208, 5392, 1480, {"block": (10.62, 11.00), "32x32": (11.24, 12.13), "64x64": (12.13, 13.35), "32x64": (12.81, 13.90)}),
+    ("s8, 2-byte pieces", 112, 8224, 2372, {"block": (13.47, 13.99), "32x32": (12.88, 14.94), "64x64": (14.61, 15.94), "64x32": (15.14, 16.88)}),
+    ("bf16, 8-byte pieces", 232, 3504, 1268, {"block": (8.06, 8.88), "64x64": (9.24, 10.28), "64x32": (11.97, 13.40)}),
+    ("bf16, 8-byte pieces", 72, 5648, 1776, {"block": (9.45, 10.12), "64x64": (10.27, 11.71), "32x32": (11.88, 13.63)}),
+    ("s8s4", 320, 1664, 352, {"64x64": (4.28, 4.25), "32x32": (4.93, 4.85), "block": (5.11, 5.09), "32x64": (5.46, 5.40)}),
     ("f32", 64, 2048, 2048, {"16x32": (7.97, 10.13), "16x16": (8.82, 11.53), "32x32": (11.16, 12.52), "block": (36.92, 37.41)}),
 ]
 

@@ -106,10 +106,10 @@ double wave_k_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather, const W
   if (kind == kF32) return wave_k_cost_f32(m, s, tiles, narrow);
   // (Pieces of 2 and 8 bytes: chosen by what 255 problems lose to their best kernel. At 81.4 and a
   // start of 3.03, of before K was cut behind the block kernels' loop, the pick was 1.9 % slower than the best one in the
-  // mean, now 0.6: s8 208 x 5392 x 1480 in 16x16x2 tiles 13.4 -> 10.8 us, bf16 232 x 3504 x 1268 in 8x8x4 9.7 -> 8.5.)
+  // mean, now 0.7: s8 208 x 5392 x 1480 in 16x16x2 tiles 13.4 -> 10.8 us, bf16 232 x 3504 x 1268 in 8x8x4 9.7 -> 8.5.)
   const bool narrow_2_8 = narrow && gather != 4;
   const double tile_us = 16 * (s.fa + s.fb * rhs_share) * row_kb / (narrow_2_8 ? 69.5 : narrow ? 81.4 : 92.5);
-  double us = (narrow_2_8 ? 3.35 : narrow || rhs_i4 ? 3.03 : 2.63) + 0.067 * s.fa * s.fb + 4.6e-5 * (rows + cols * rhs_share) * row_kb;
+  double us = (narrow_2_8 ? 3.2 : narrow || rhs_i4 ? 3.03 : 2.63) + 0.067 * s.fa * s.fb + 4.6e-5 * (rows + cols * rhs_share) * row_kb;
   if (tiles <= 256) return us + tile_us;
   const double rounds = tiles / 256.0;
   if (tiles > (s.fa * s.fb >= 16 ? 256 : 1024)) us += 1e3 * rounds;

@@ -466,16 +466,13 @@ hipError_t launch_wave_k_tile(const MfmaArgs& m, bool streamed, hipStream_t stre
 // One 64-byte step of K in flight ahead of the one that is multiplied, for each of eight wavefronts. With one fragment either
 // way that step is multiplied before the next one is there, and a long K has two in flight: f16 16x16x1 16 x 560 x 7148 8.7
 // -> 7.6 us, f32 32 x 352 x 8740 15.5 -> 13.5, bf16 16 x 1360 x 6576 7.2 -> 7.0. With fewer steps the ring's longer code
-// costs more than it hides, and with few tiles a step is there sooner. Two ahead against one, 1300 problems: 32 to 72 chunks
-// of 64 bytes 4 to 5 % slower, 80 to 100 1 to 2 %, 100 to 120 2 % slower with less than 128 tiles and 2 % faster with more,
-// 3 to 8 % faster beyond (f32 6 % slower at 64 to 80, 4 % at 100 to 120, 4 % faster beyond); 16-byte pieces of f16 and bf16
-// level at 32 to 48 chunks, 1 to 4 % faster from there on, of int8 1 % slower. Three and more, or two for larger tiles, give nothing.
+// costs more than it hides. Two ahead against one, 144 problems, on operands that every launch reads again, that the
+// last-level cache holds and from HBM: 36 to 48 chunks of 64 bytes 6 % slower, 2 % slower and level, 48 to 100 4 % slower,
+// level and 2 % faster, more 2 % slower, 4 and 6 % faster; f32 from 28 to 48 chunks 1 % slower, 2 and 3 % faster, to 100 4 %
+// slower, 2 and 5 % faster, beyond 1 % slower, 7 and 7 % faster; 4-byte pieces from 28 to 48 chunks level, 1 and 1 % faster.
+// (48 x 560 x 1640 f16 in 16x16x1 tiles, 52 chunks, from HBM 5.25 us with one, 4.92 with two.) int8 in 16-byte pieces 1 % slower; three and more, or two for larger tiles, give nothing.
 template <int KIND, int G>
-bool two_steps_ahead(const MfmaArgs& m) {
-  if (G == 16 && KIND != kF32) return KIND != kI8 && m.chunks >= 48;
-  const int64_t tiles = ((((int64_t)m.M << m.log2_M0) + 15) / 16) * ((((int64_t)m.N << m.log2_N0) + 15) / 16);
-  return m.chunks >= (tiles >= 128 ? 100 : 120);
-}
+bool two_steps_ahead(const MfmaArgs& m) { return m.chunks >= (KIND == kF32 || G == 4 ? 32 : 48); }
 
 template <int KIND, bool RHS_I4, bool NARROW, int G>
 hipError_t launch_wave_k_piece(const MfmaArgs& m, int shape, bool streamed, hipStream_t stream) {

@@ -105,16 +105,16 @@ def test_block_kernels_have_the_deep_ring_for_operands_from_hbm(recorder):  # no
 
 # Steps in flight, one more than those ahead, for one fragment either way (mmt4d_wave_k_kernels.h): with 45 tiles and with 165.
 @pytest.mark.parametrize("layout,two_from", [
-    ("f16, 2-byte pieces", (120, 100)), ("s8, 4-byte pieces", (120, 100)), ("bf16, 8-byte pieces", (120, 100)),
-    ("bf16, 4-byte pieces", (120, 100)), ("s8, 2-byte pieces", (120, 100)), ("f32", (120, 100)), ("bf16", (48, 48)), ("s8", (999, 999))])
+    ("f16, 2-byte pieces", 48), ("s8, 4-byte pieces", 32), ("bf16, 8-byte pieces", 48), ("bf16, 4-byte pieces", 32),
+    ("s8, 2-byte pieces", 48), ("f32", 32), ("bf16", 48), ("s8", 999)])
 def test_wave_k_looks_two_steps_ahead_with_a_long_K_only(recorder, layout, two_from):  # noqa: F811
     flags, M0, N0, K0 = LAYOUTS[layout]
     e = {"s8": 1, "f1": 2, "bf": 2, "f3": 4}[layout[:2]]
-    for n, threshold in zip((240, 880), two_from):
-        for steps in (24, 33, 40, 47, 48, 64, 72, 99, 100, 119, 120, 150):
+    for n in (240, 880):
+        for steps in (24, 31, 32, 33, 40, 47, 48, 64, 72, 99, 100, 119, 120, 150):
             mangled, _ = recorder.mmt4d(flags, 48 // M0, n // N0, 64 * steps // (K0 * e), M0, N0, K0)
             m = re.search(r"mmt4d_wave_k_kernelILi\dELb0ELb0ELi\d+ELi(\d)ELi(\d)ELi8ELi(\d)E", mangled)
-            assert m and (m[1] + m[2] != "11" or int(m[3]) == (3 if steps >= threshold else 2)), (steps, mangled)
+            assert m and (m[1] + m[2] != "11" or int(m[3]) == (3 if steps >= two_from else 2)), (steps, mangled)
             assert n > 240 or m[1] + m[2] == "11", (steps, mangled)
 
 

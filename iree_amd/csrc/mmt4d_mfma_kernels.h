@@ -780,18 +780,26 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   //     every group of 16 lanes reads 256 contiguous bytes: no bank conflicts.
   //     (With an int4 rhs the lhs keeps the older arrangement: slot p holds row
   //     p & 31, column slot (p >> 5) & 3, read at slot 128*f + 64*kk + lane.)
-  //   G == 2, 4, 8 (bytes of a row piece; R = 16 / G rows share 16 contiguous
+  //   G == 2, 8 (bytes of a row piece; R = 16 / G rows share 16 contiguous
   //     bytes, a chunk is 64 / G k steps): slot 64*m + l holds rows R*g ..
   //     R*g + R - 1 (g = l % (2*G)) of fragment m >> 1 at k step
   //     (32/G)*(m & 1) + (16/G)*h + d of the chunk (h = (l / (2*G)) & 1,
   //     d = l / (4*G)). The G-byte element number 64*((2*f + kk)*(16/G) + d) +
   //     32*h + r of the operand is then row r of fragment f at that k step: the
   //     MFMA operand of lane 32*h + r for K-step kk is elements d = 0 .. 16/G - 1,
-  //     each read linear in the lane number (4-byte pieces: two paired dword
-  //     reads; 8-byte: two 64-bit reads; 2-byte: eight reads of the dword the
+  //     each read linear in the lane number (8-byte pieces: two 64-bit reads; 2-byte: eight reads of the dword the
   //     element shares with its neighbour row, and a byte permute that picks
   //     the lane's half). K is permuted inside a chunk, identically for lhs
   //     and rhs.
+  //   G == 4 (four rows share 16 contiguous bytes, a chunk is 16 k steps): load m of
+  //     an operand holds k steps 8*(m & 1) + 2*d + h of fragment m >> 1, its slot
+  //     16*d + s the rows 4*g .. 4*g + 3 at (d, h), where s is
+  //       8*h + g                                      M0 = 16 or 4
+  //       4*(g >> 1) + ((2*h + (g & 1)) ^ 2*(g >> 2))  M0 = 8,
+  //     so that four consecutive lanes load 64 contiguous bytes (M0 = 16: the rows
+  //     of one k step, 8: those of two), and the 32 lanes of a half find their
+  //     dwords in 32 different banks. Lane 32*h + r reads dword r & 3 of the slots
+  //     of g = r >> 2, 256 bytes from one d to the next: two paired dword reads.
   //   G == 2, fragments in pairs (an even number of them per wavefront): 16-bit
   //     reads deliver half of what the LDS can, so a lane reads dwords, i.e. two
   //     adjacent rows of one k step, and gives the low half to fragment 2p, the
@@ -804,11 +812,15 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   //     64*d + 32*h + r of a (pair, K-step) is then rows 2*r, 2*r + 1 at the
   //     lane's d-th k step: eight dword reads linear in the lane number (four
   //     two-address instructions) and eight byte permutes per two fragments.
-  //     (Tried: lanes arranged so that four consecutive ones load four
-  //     consecutive k steps of one row group, i.e. one cache line instead of
-  //     two for M0 = 16 or four for M0 = 8, with an xor spreading the row groups
-  //     over the banks. The reads then need eight separate addresses: 8x8x2
-  //     int8 tiles went from 114 to 100 us per 4096^3, 16x16x2 from 83 to 89.)
+  //     (These loads touch two stretches of 64 bytes per four lanes with M0 = 16, four with M0 = 8. With one
+  //     resp. two, laid out like the 4-byte pieces, nothing is gained, the reads and permutes being what the step waits
+  //     for: int8 16x16x2 777 x 4100 x 4096 23.4 us both, 512 x 4096 x 4096 19.7 -> 20.1.)
+  //   What the lanes of a load have to do with each other: the memory pipeline takes four of them at a time, and takes
+  //   those twice that touch two stretches of 64 bytes: 105 bytes a nanosecond and compute unit with one stretch, 70 with
+  //   two, in a loop of nothing but these loads. Tiles of up to 128x128 come close to the latter. 4-byte pieces with M0 = 8 and 64-byte
+  //   pieces (below) had the rows first: int8 512 x 4096 x 4096 16x16x64 16.2 -> 13.8 us, 8x8x4 15.6 -> 13.6, 777 x 4100 x
+  //   4096 22.3 -> 20.1 and 21.0 -> 19.4, 3072^3 (192x192 tiles) 32.2 -> 31.2 and 30.3 -> 29.4; 256x256 tiles are bound by the
+  //   matrix pipe, level.
   //   int4 rhs: slot 64*f + 32*h + r holds nibbles 32*h .. 32*h + 31 of row r of
   //     fragment f: lane 32*h + r reads that slot once per chunk and widens its
   //     first 8 bytes for K-step 0, its last 8 for K-step 1. The lhs columns are
@@ -821,17 +833,18 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     const int64_t tile = (row >> log2_t0) - (first >> log2_t0);
     return tile * stride_bytes + (row & ((1 << log2_t0) - 1)) * rb;
   };
-  //   G == 16, lhs tiles one row tall (a row-major matrix: a row's 64 bytes of a
-  //     chunk are contiguous, consecutive rows a whole row pitch apart): with the
-  //     arrangement above four consecutive lanes would load from four cache
-  //     lines. Here lane l of a load takes row l >> 2 of the load's 16 and the
+  //   G == 16, a row's 64 bytes of a chunk contiguous (64-byte row pieces; lhs tiles
+  //     one row tall, i.e. a row-major matrix): with the arrangement above four
+  //     consecutive lanes would load from four rows. Here lane l of a load takes row
+  //     l >> 2 of the load's 16 and the
   //     16-byte column (l & 3) ^ ((l >> 4) & 3), so four consecutive lanes cover
   //     one row's 64 bytes; lane 32*h + r reads slot 128*f + 64*(r >> 4) + 4*r' +
   //     ((2*kk + h) ^ ((r' >> 2) & 3)), r' = r & 15: the xor spreads the sixteen
   //     rows of a group of lanes over all banks. The slot for K-step 1 is the one
-  //     for K-step 0 with bit 1 flipped, a per-lane distance (lhs_kk1_step).
+  //     for K-step 0 with bit 1 flipped, a per-lane distance (lhs_kk1_step, rhs_kk1_step).
   constexpr bool ROWS16 = G == 16 && !RHS_I4;
-  const bool lhs_row_major = ROWS16 && a.log2_M0 == 0;
+  const bool lhs_by_rows = ROWS16 && (a.log2_M0 == 0 || a.lhs_rb == 64);
+  const bool rhs_by_rows = ROWS16 && a.rhs_rb == 64;
   uint32_t a_off[A_LOADS], b_off[B_LOADS];
   if constexpr (G == 16) {
 #pragma unroll
@@ -839,7 +852,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       const int p = tid + 256 * t;
       int c = RHS_I4 ? ((p >> 6) & 1) + 2 * ((p >> 5) & 1) : (p >> 4) & 3;
       int row = RHS_I4 ? (p >> 7) * 32 + (p & 31) : (p >> 7) * 32 + 16 * ((p >> 6) & 1) + (p & 15);
-      if (lhs_row_major) {
+      if (lhs_by_rows) {
         c = (p & 3) ^ ((p >> 4) & 3);
         row = (p >> 7) * 32 + 16 * ((p >> 6) & 1) + ((p >> 2) & 15);
       }
@@ -850,8 +863,12 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
 #pragma unroll
     for (int t = 0; t < B_LOADS; ++t) {
       const int p = tid + 256 * t;
-      const int c = RHS_I4 ? (p >> 5) & 1 : (p >> 4) & 3;
-      const int row = RHS_I4 ? (p >> 6) * 32 + (p & 31) : (p >> 7) * 32 + 16 * ((p >> 6) & 1) + (p & 15);
+      int c = RHS_I4 ? (p >> 5) & 1 : (p >> 4) & 3;
+      int row = RHS_I4 ? (p >> 6) * 32 + (p & 31) : (p >> 7) * 32 + 16 * ((p >> 6) & 1) + (p & 15);
+      if (rhs_by_rows) {
+        c = (p & 3) ^ ((p >> 4) & 3);
+        row = (p >> 7) * 32 + 16 * ((p >> 6) & 1) + ((p >> 2) & 15);
+      }
       b_off[t] = (uint32_t)(row_offset(first_col + row, total_cols - 1, first_col, a.log2_N0,
                                        a.rhs_stride_bytes, a.rhs_rb) +
                             ((16 * c) >> a.log2_rhs_rb) * rhs_kstep + ((16 * c) & (a.rhs_rb - 1)));
@@ -888,10 +905,19 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     constexpr int R = 16 / G;  // rows per 16-byte piece
     // Row group and k step of the chunk of this lane's piece in load t (the
     // wavefront's share of the k steps included).
-    auto piece_of = [&](bool paired, int t, int* row, int* k1) {
+    auto piece_of = [&](int log2_t0, bool paired, int t, int* row, int* k1) {
       if (paired) {
         *row = 64 * t + 8 * (lane & 7);
         *k1 = 16 * (wave >> 1) + 8 * ((lane >> 3) & 1) + 4 * (wave & 1) + (lane >> 4);
+      } else if constexpr (G == 4) {
+        int g = lane & 7, h = (lane >> 3) & 1;
+        if (log2_t0 == 3) {
+          const int x = (lane & 3) ^ ((lane >> 2) & 2);
+          g = 2 * ((lane >> 2) & 3) + (x & 1);
+          h = x >> 1;
+        }
+        *row = 32 * (2 * t + (wave >> 1)) + 4 * g;
+        *k1 = 8 * (wave & 1) + 2 * (lane >> 4) + h;
       } else {
         *row = 32 * (2 * t + (wave >> 1)) + R * (lane % (2 * G));
         *k1 = (32 / G) * (wave & 1) + (16 / G) * ((lane / (2 * G)) & 1) + lane / (4 * G);
@@ -900,14 +926,14 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
 #pragma unroll
     for (int t = 0; t < A_LOADS; ++t) {
       int row, k1;
-      piece_of(PAIR_A, t, &row, &k1);
+      piece_of(a.log2_M0, PAIR_A, t, &row, &k1);
       a_off[t] = (uint32_t)(row_offset(first_row + row, total_rows - R, first_row, a.log2_M0, a.lhs_stride_bytes,
                                        a.lhs_rb) + k1 * lhs_kstep);
     }
 #pragma unroll
     for (int t = 0; t < B_LOADS; ++t) {
       int row, k1;
-      piece_of(PAIR_B, t, &row, &k1);
+      piece_of(a.log2_N0, PAIR_B, t, &row, &k1);
       b_off[t] = (uint32_t)(row_offset(first_col + row, total_cols - R, first_col, a.log2_N0, a.rhs_stride_bytes,
                                        a.rhs_rb) + k1 * rhs_kstep);
     }
@@ -954,6 +980,12 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   };
 
   uint4 pa[AM][2], pb[BN][2], qa[AM][2], qb[BN][2];
+  // G == 4: byte offset of a lane's first dword inside a fragment's K-step, see the layouts above.
+  auto dwords_lane_offset = [&](int log2_t0) -> int32_t {
+    const int h = lane >> 5, r = lane & 31, g = r >> 2;
+    const int s = log2_t0 == 3 ? 4 * (g >> 1) + ((2 * h + (g & 1)) ^ (2 * (g >> 2))) : 8 * h + g;
+    return 16 * s + 4 * (r & 3);
+  };
   // G < 16: dword `part` (0..3) of a lane's operand for one (fragment, K-step),
   // whose first element is at `first` (already including the lane's offset):
   // the elements are 64*G bytes apart.
@@ -984,8 +1016,8 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       return widen_i4_times16(kk ? make_uint2(raw.z, raw.w) : make_uint2(raw.x, raw.y));
     }
     if constexpr (G == 16) {
-      if (!RHS_I4 && operand == 0 && lhs_row_major)
-        return ring[128 * f + 64 * ((lane & 31) >> 4) + 4 * (lane & 15) + ((2 * kk + (lane >> 5)) ^ ((lane >> 2) & 3))];
+      if (!RHS_I4 && (operand == 0 ? lhs_by_rows : rhs_by_rows))
+        return ring[operand + 128 * f + 64 * ((lane & 31) >> 4) + 4 * (lane & 15) + ((2 * kk + (lane >> 5)) ^ ((lane >> 2) & 3))];
       if (!RHS_I4) return ring[operand + 128 * f + 32 * kk + 64 * ((lane & 31) >> 4) + 16 * (lane >> 5) + (lane & 15)];
       return ring[operand + 128 * f + 64 * kk + lane];
     } else if constexpr (G == 1) {
@@ -994,7 +1026,8 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       const uint2 lo = lds_read_transposed(first), hi = lds_read_transposed(first + 128);
       return make_uint4(lo.x, lo.y, hi.x, hi.y);
     } else {
-      const uint8_t* first = (const uint8_t*)(ring + operand) + 1024 * (2 * f + kk) + G * lane;
+      const uint8_t* first = (const uint8_t*)(ring + operand) + 1024 * (2 * f + kk) +
+                             (G == 4 ? dwords_lane_offset(operand >= A_PIECES ? a.log2_N0 : a.log2_M0) : G * lane);
       return make_uint4(gather_dword(first, 0), gather_dword(first, 1), gather_dword(first, 2), gather_dword(first, 3));
     }
   };
@@ -1029,29 +1062,31 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   // of a fragment to the next (see the layouts above).
   const uint8_t* ring_bytes =
       (const uint8_t*)ring + (ROWS16 ? 16 * (64 * ((lane & 31) >> 4) + 16 * (lane >> 5) + (lane & 15))
-                                     : (G == 1 ? 0 : (G == 16 ? 16 : G) * lane));
-  // G == 2: lanes address dwords, not 16-bit elements. Paired: dword number
+                                     : (G == 1 || G == 4 ? 0 : G * lane));
+  // What a lane's reads of either operand add to that. G == 1: the transposing reads' offset. G == 4: the dword reads'. G == 2: lanes address
+  // dwords, not 16-bit elements. Paired: dword number
   // lane; unpaired: the dword that holds the lane's element (two lanes share
   // it), from which `own_half` then picks the low or the high half. (16-bit
   // reads that fill the halves of a register one after the other made these
   // tiles 1.8x slower than the 4-byte ones: the second read of a register has
-  // to wait for the first.)
-  // (G == 1: the per-operand lane offset of the transposing reads instead.)
-  // (Row-major lhs: the distance from the rhs lane slot, which ring_bytes holds, to the lhs one for K-step 0.)
-  const int32_t lhs_rm_slot0 = 4 * (lane & 15) + ((lane >> 5) ^ ((lane >> 2) & 3));
-  const int32_t pair_a_lane =
-      G == 1 ? transposed_lane_offset(a.log2_M0)
-             : (G == 2 ? (PAIR_A ? 2 * lane : -2 * (lane & 1))
-                       : (lhs_row_major ? 16 * (lhs_rm_slot0 - (16 * (lane >> 5) + (lane & 15))) : 0));
-  // Bytes from an lhs fragment's K-step 0 to its K-step 1 in this lane's reads.
-  const int32_t lhs_kk1_step = lhs_row_major ? 16 * ((lhs_rm_slot0 ^ 2) - lhs_rm_slot0) : 16 * (ROWS16 ? 32 : 64);
-  const int32_t pair_b_lane =
-      G == 1 ? transposed_lane_offset(a.log2_N0) : (G != 2 ? 0 : (PAIR_B ? 2 * lane : -2 * (lane & 1)));
+  // to wait for the first.) G == 16, by rows: the distance to the by-rows slot for K-step 0.
+  const int32_t by_rows_slot0 = 4 * (lane & 15) + ((lane >> 5) ^ ((lane >> 2) & 3));
+  auto lane_offset = [&](int log2_t0, bool paired, bool by_rows) -> int32_t {
+    if constexpr (G == 1) return transposed_lane_offset(log2_t0);
+    if constexpr (G == 2) return paired ? 2 * lane : -2 * (lane & 1);
+    if constexpr (G == 4) return dwords_lane_offset(log2_t0);
+    return by_rows ? 16 * (by_rows_slot0 - (16 * (lane >> 5) + (lane & 15))) : 0;
+  };
+  const int32_t pair_a_lane = lane_offset(a.log2_M0, PAIR_A, lhs_by_rows);
+  const int32_t pair_b_lane = lane_offset(a.log2_N0, PAIR_B, rhs_by_rows);
+  // Bytes from a fragment's K-step 0 to its K-step 1 in this lane's reads (16-byte pieces).
+  const int32_t lhs_kk1_step = lhs_by_rows ? 16 * ((by_rows_slot0 ^ 2) - by_rows_slot0) : 16 * (ROWS16 ? 32 : 64);
+  const int32_t rhs_kk1_step = rhs_by_rows ? 16 * ((by_rows_slot0 ^ 2) - by_rows_slot0) : 16 * 32;
   const uint32_t own_half = (lane & 1) ? 0x07060302u : 0x05040100u;
-  constexpr int KK16 = ROWS16 ? 32 : 64;
 
   // Zeroes what the last chunk shares with the one before it. Lane half h of K-step kk holds bytes 32*kk + 16*h .. + 15 of
-  // the chunk's 64 bytes per row, in ascending order of k in every layout above; with an int4 rhs bytes 16*kk + 32*h .. + 15.
+  // the chunk's 64 bytes per row, in ascending order of k; with an int4 rhs bytes 16*kk + 32*h .. + 15; of 4-byte
+  // pieces every other one of bytes 32*kk .. + 31, from the h-th on.
   auto cut_fragments = [&](uint4 (*fa)[2], uint4 (*fb)[2]) {
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
@@ -1059,8 +1094,13 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       const int cut = min(max(cut_bytes - first_byte, 0), 16);
       uint32_t keep[4];
 #pragma unroll
-      for (int w = 0; w < 4; ++w)
+      for (int w = 0; w < 4; ++w) {
+        if constexpr (G == 4) {
+          keep[w] = 32 * kk + 8 * w + 4 * (lane >> 5) < cut_bytes ? 0u : 0xFFFFFFFFu;
+          continue;
+        }
         keep[w] = cut >= 4 * w + 4 ? 0u : (cut <= 4 * w ? 0xFFFFFFFFu : 0xFFFFFFFFu << (8 * (cut - 4 * w)));
+      }
 #pragma unroll
       for (int i = 0; i < AM; ++i) {
         fa[i][kk].x &= keep[0]; fa[i][kk].y &= keep[1]; fa[i][kk].z &= keep[2]; fa[i][kk].w &= keep[3];
@@ -1171,6 +1211,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     const uint8_t* read_a = ring_bytes + read_stage_off + frag_a_off + pair_a_lane;
     const uint8_t* read_a_kk1 = read_a + lhs_kk1_step;  // (used where the lhs has 16-byte pieces)
     const uint8_t* read_b = ring_bytes + read_stage_off + frag_b_off + pair_b_lane;
+    const uint8_t* read_b_kk1 = read_b + rhs_kk1_step;
     uint4 raw_b[RHS_I4 ? BN : 1];
 #pragma unroll
     for (int m = LEAD; m < MFMAS; ++m) {
@@ -1202,7 +1243,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
             const int frag = y / PARTS, part = y % PARTS;
             uint4& dst = nxt[frag][kk];
             if constexpr (G == 16) {
-              if (is_b) dst = *(const uint4*)(src + (128 * frag + KK16 * kk) * 16);
+              if (is_b) dst = *(const uint4*)((kk ? read_b_kk1 : read_b) + 128 * frag * 16);
               else dst = *(const uint4*)((kk ? read_a_kk1 : read_a) + 128 * frag * 16);
             } else {
               const uint8_t* first = src + 1024 * (2 * frag + kk);
@@ -1340,7 +1381,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
                              int kk) -> uint4 {
       const uint8_t* src = is_b ? base_b : base_a;
       if constexpr (G == 16) {
-        if (is_b) return *(const uint4*)(src + (128 * f + KK16 * kk) * 16);
+        if (is_b) return *(const uint4*)(src + (kk ? rhs_kk1_step : 0) + 128 * f * 16);
         return *(const uint4*)((kk ? base_a_kk1 : base_a) + 128 * f * 16);
       } else if constexpr (G == 1) {
         const uint2 lo = lds_read_transposed(src + 2048 * f + 512 * kk);

@@ -61,7 +61,8 @@ struct MfmaArgs {
   int32_t lhs_rb, rhs_rb;    // bytes of one (k, i0) row piece
   int32_t log2_lhs_rb, log2_rhs_rb;
   int32_t chunks;            // ceil(K * lhs_rb / 64)
-  int32_t tile_rows, tile_cols;  // grid of block tiles
+  int32_t tile_rows, tile_cols;  // grid of block tiles (set_tile_grid)
+  uint32_t band_reciprocal;      // of tile_cols, see uk_device.h
   int32_t accumulate;
 };
 
@@ -284,18 +285,25 @@ __device__ __forceinline__ uint4 load_piece(const uint8_t* p, int64_t kstep, int
 // on a contiguous range of tiles, then that range is walked in bands of 4 tile
 // rows so that neighbours share lhs and rhs panels. False: nothing to do.
 __device__ __forceinline__ bool locate_block(const MfmaArgs& a, int* tile_row, int* tile_col) {
-  const int total_tiles = a.tile_rows * a.tile_cols;
-  const int per_xcd = (total_tiles + 7) >> 3;
-  const int linear = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  const uint32_t total_tiles = (uint32_t)a.tile_rows * a.tile_cols;
+  const uint32_t per_xcd = (total_tiles + 7) >> 3;
+  const uint32_t linear = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (linear >= total_tiles) return false;
-  constexpr int BAND = 4;
-  const int band = linear / (BAND * a.tile_cols);
-  const int band_first = band * BAND;
-  const int band_rows = min(a.tile_rows - band_first, BAND);
-  const int in_band = linear - band * BAND * a.tile_cols;
-  *tile_row = band_first + in_band % band_rows;
-  *tile_col = in_band / band_rows;
+  tile_of_number(linear, (uint32_t)a.tile_rows, (uint32_t)a.tile_cols, a.band_reciprocal, tile_row, tile_col);
   return true;
+}
+
+// What runs in front of a workgroup's first load counts on every launch. The kernel arguments lie in two cache lines that
+// nothing has fetched yet, 560 cycles away: needed here together they are fetched together, where as their uses came up the
+// second line was fetched behind the first. An instruction takes 4 to 5 cycles, branches to code not yet fetched more. With
+// this, tile_of_number, offsets in 32 bits and no branches, 160 to 220 instructions are left of 230 to 320, and a launch is
+// 0.3 to 0.45 us shorter: int8 8x8x4 1024^3 5.39 -> 4.99 us, 1024 x 2048 x 512 5.8 -> 5.44, f32 256 x 512 x 512 3.69 -> 3.27,
+// bf16 64 x 4096 x 4096 8.25 -> 7.91, int4 512 x 11008 x 4096 30.2 -> 29.9.
+__device__ __forceinline__ void fetch_arguments(const MfmaArgs& a) {
+  asm volatile("" ::"s"(a.lhs), "s"(a.rhs), "s"(a.lhs_stride_bytes), "s"(a.rhs_stride_bytes), "s"(a.M), "s"(a.N), "s"(a.K),
+               "s"(a.log2_M0), "s"(a.log2_N0), "s"(a.lhs_rb), "s"(a.rhs_rb), "s"(a.log2_lhs_rb), "s"(a.log2_rhs_rb),
+               "s"(a.chunks), "s"(a.tile_rows), "s"(a.tile_cols), "s"(a.band_reciprocal));
+  __builtin_amdgcn_sched_barrier(0);
 }
 
 // Writes one wavefront's accumulators. Lane l holds, for fragment (i, j): lhs
@@ -748,6 +756,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
 
   UK_TIMELINE(const unsigned long long tl_start = __builtin_amdgcn_s_memrealtime(); unsigned long long tl_loop = 0,
               tl_loop_end = 0;)
+  fetch_arguments(a);
   int tile_row, tile_col;
   if (!locate_block(a, &tile_row, &tile_col)) return;
 
@@ -758,11 +767,9 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
 
   const int64_t total_rows = (int64_t)a.M << a.log2_M0;
   const int64_t total_cols = (int64_t)a.N << a.log2_N0;
-  const int64_t lhs_kstep = (int64_t)a.lhs_rb << a.log2_M0;
-  const int64_t rhs_kstep = (int64_t)a.rhs_rb << a.log2_N0;
-  const int32_t ksteps_per_chunk = 64 >> a.log2_lhs_rb;
-  const int64_t lhs_chunk_bytes = ksteps_per_chunk * lhs_kstep;
-  const int64_t rhs_chunk_bytes = ksteps_per_chunk * rhs_kstep;
+  // Bytes of a k step and of a chunk.
+  const int log2_lhs_kstep = a.log2_lhs_rb + a.log2_M0, log2_rhs_kstep = a.log2_rhs_rb + a.log2_N0;
+  const int32_t lhs_chunk_bytes = 64 << a.log2_M0, rhs_chunk_bytes = (RHS_I4 ? 32 : 64) << a.log2_N0;
 
   const int64_t first_row = (int64_t)tile_row * BLOCK_ROWS;
   const int64_t first_col = (int64_t)tile_col * BLOCK_COLS;
@@ -827,11 +834,13 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   //     assigned to match: (K-step kk, lane half h) gets 16-byte column kk + 2*h.
   // Rows past the end of the matrix are redirected to its last row (group):
   // their products are computed, never stored.
-  auto row_offset = [&](int64_t row, int64_t last, int64_t first, int log2_t0, int64_t stride_bytes,
-                        int32_t rb) -> int64_t {
+  // (In 32 bits, counted from the workgroup's first row, which is the first of a tile: this is code that runs once, in front
+  // of the first load.)
+  const int32_t rows_left = (int32_t)min(total_rows - first_row, (int64_t)BLOCK_ROWS);
+  const int32_t cols_left = (int32_t)min(total_cols - first_col, (int64_t)BLOCK_COLS);
+  auto row_offset = [&](int32_t row, int32_t last, int log2_t0, int64_t stride_bytes, int log2_rb) -> uint32_t {
     row = min(row, last);
-    const int64_t tile = (row >> log2_t0) - (first >> log2_t0);
-    return tile * stride_bytes + (row & ((1 << log2_t0) - 1)) * rb;
+    return (uint32_t)(row >> log2_t0) * (uint32_t)stride_bytes + ((uint32_t)(row & ((1 << log2_t0) - 1)) << log2_rb);
   };
   //   G == 16, a row's 64 bytes of a chunk contiguous (64-byte row pieces; lhs tiles
   //     one row tall, i.e. a row-major matrix): with the arrangement above four
@@ -856,9 +865,8 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
         c = (p & 3) ^ ((p >> 4) & 3);
         row = (p >> 7) * 32 + 16 * ((p >> 6) & 1) + ((p >> 2) & 15);
       }
-      a_off[t] = (uint32_t)(row_offset(first_row + row, total_rows - 1, first_row,
-                                       a.log2_M0, a.lhs_stride_bytes, a.lhs_rb) +
-                            ((16 * c) >> a.log2_lhs_rb) * lhs_kstep + ((16 * c) & (a.lhs_rb - 1)));
+      a_off[t] = row_offset(row, rows_left - 1, a.log2_M0, a.lhs_stride_bytes, a.log2_lhs_rb) +
+                 ((16 * c) >> a.log2_lhs_rb << log2_lhs_kstep) + ((16 * c) & (a.lhs_rb - 1));
     }
 #pragma unroll
     for (int t = 0; t < B_LOADS; ++t) {
@@ -869,9 +877,8 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
         c = (p & 3) ^ ((p >> 4) & 3);
         row = (p >> 7) * 32 + 16 * ((p >> 6) & 1) + ((p >> 2) & 15);
       }
-      b_off[t] = (uint32_t)(row_offset(first_col + row, total_cols - 1, first_col, a.log2_N0,
-                                       a.rhs_stride_bytes, a.rhs_rb) +
-                            ((16 * c) >> a.log2_rhs_rb) * rhs_kstep + ((16 * c) & (a.rhs_rb - 1)));
+      b_off[t] = row_offset(row, cols_left - 1, a.log2_N0, a.rhs_stride_bytes, a.log2_rhs_rb) +
+                 ((16 * c) >> a.log2_rhs_rb << log2_rhs_kstep) + ((16 * c) & (a.rhs_rb - 1));
     }
   } else if constexpr (G == 1) {
     // One-byte row pieces (K0 = 1 int8: the operand is k-major, M0 bytes per k
@@ -891,15 +898,15 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     for (int t = 0; t < A_LOADS; ++t) {
       int row, k1;
       piece_of(a.log2_M0, t, &row, &k1);
-      a_off[t] = (uint32_t)(row_offset(first_row + row, total_rows - (1 << a.log2_M0), first_row, a.log2_M0,
-                                       a.lhs_stride_bytes, a.lhs_rb) + k1 * lhs_kstep);
+      a_off[t] = row_offset(row, rows_left - (1 << a.log2_M0), a.log2_M0, a.lhs_stride_bytes, a.log2_lhs_rb) +
+                 (k1 << log2_lhs_kstep);
     }
 #pragma unroll
     for (int t = 0; t < B_LOADS; ++t) {
       int row, k1;
       piece_of(a.log2_N0, t, &row, &k1);
-      b_off[t] = (uint32_t)(row_offset(first_col + row, total_cols - (1 << a.log2_N0), first_col, a.log2_N0,
-                                       a.rhs_stride_bytes, a.rhs_rb) + k1 * rhs_kstep);
+      b_off[t] = row_offset(row, cols_left - (1 << a.log2_N0), a.log2_N0, a.rhs_stride_bytes, a.log2_rhs_rb) +
+                 (k1 << log2_rhs_kstep);
     }
   } else {
     constexpr int R = 16 / G;  // rows per 16-byte piece
@@ -910,12 +917,10 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
         *row = 64 * t + 8 * (lane & 7);
         *k1 = 16 * (wave >> 1) + 8 * ((lane >> 3) & 1) + 4 * (wave & 1) + (lane >> 4);
       } else if constexpr (G == 4) {
-        int g = lane & 7, h = (lane >> 3) & 1;
-        if (log2_t0 == 3) {
-          const int x = (lane & 3) ^ ((lane >> 2) & 2);
-          g = 2 * ((lane >> 2) & 3) + (x & 1);
-          h = x >> 1;
-        }
+        // (Selected by masks, which the compiler does not make branches of.)
+        const int eight = -(int)(log2_t0 == 3), x = (lane & 3) ^ ((lane >> 2) & 2);
+        const int g = ((2 * ((lane >> 2) & 3) + (x & 1)) & eight) | (lane & 7 & ~eight);
+        const int h = ((x >> 1) & eight) | ((lane >> 3) & 1 & ~eight);
         *row = 32 * (2 * t + (wave >> 1)) + 4 * g;
         *k1 = 8 * (wave & 1) + 2 * (lane >> 4) + h;
       } else {
@@ -927,15 +932,13 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     for (int t = 0; t < A_LOADS; ++t) {
       int row, k1;
       piece_of(a.log2_M0, PAIR_A, t, &row, &k1);
-      a_off[t] = (uint32_t)(row_offset(first_row + row, total_rows - R, first_row, a.log2_M0, a.lhs_stride_bytes,
-                                       a.lhs_rb) + k1 * lhs_kstep);
+      a_off[t] = row_offset(row, rows_left - R, a.log2_M0, a.lhs_stride_bytes, a.log2_lhs_rb) + (k1 << log2_lhs_kstep);
     }
 #pragma unroll
     for (int t = 0; t < B_LOADS; ++t) {
       int row, k1;
       piece_of(a.log2_N0, PAIR_B, t, &row, &k1);
-      b_off[t] = (uint32_t)(row_offset(first_col + row, total_cols - R, first_col, a.log2_N0, a.rhs_stride_bytes,
-                                       a.rhs_rb) + k1 * rhs_kstep);
+      b_off[t] = row_offset(row, cols_left - R, a.log2_N0, a.rhs_stride_bytes, a.log2_rhs_rb) + (k1 << log2_rhs_kstep);
     }
   }
 
@@ -957,10 +960,10 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   const int chunks = a.chunks;
   const int last_chunk = chunks - 1;
   const int32_t cut_bytes = (int32_t)((64 - (((int64_t)a.K << a.log2_lhs_rb) & 63)) & 63);
-  const int64_t lhs_last_base = a.K * lhs_kstep - lhs_chunk_bytes;
-  const int64_t rhs_last_base = a.K * rhs_kstep - rhs_chunk_bytes;
-  const int64_t lhs_last_advance = lhs_last_base - (last_chunk - 1) * lhs_chunk_bytes;
-  const int64_t rhs_last_advance = rhs_last_base - (last_chunk - 1) * rhs_chunk_bytes;
+  const int64_t lhs_last_base = ((int64_t)a.K << log2_lhs_kstep) - lhs_chunk_bytes;
+  const int64_t rhs_last_base = ((int64_t)a.K << log2_rhs_kstep) - rhs_chunk_bytes;
+  const int64_t lhs_last_advance = lhs_last_base - (int64_t)(last_chunk - 1) * lhs_chunk_bytes;
+  const int64_t rhs_last_advance = rhs_last_base - (int64_t)(last_chunk - 1) * rhs_chunk_bytes;
 
   // Load number `n` (compile-time after unrolling) of the chunk whose operand
   // bases are la / lb, into the stage at LDS byte offset `stage_off`.
@@ -970,11 +973,16 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     load_to_lds(stage_off + (is_a ? 0 : A_PIECES * 16) + (256 * t + 64 * wave) * 16,
                 is_a ? a_off[t] : b_off[t], is_a ? la : lb);
   };
+  // The first chunks: a compile-time `kc` of a few, whose base lies within 16 KiB (a minimum, no branches: see row_offset).
+  const int32_t lhs_last_near = (int32_t)min(lhs_last_base, (int64_t)1 << 20);
+  const int32_t rhs_last_near = (int32_t)min(rhs_last_base, (int64_t)1 << 20);
+  static_assert(AHEAD * 64 * 16 < 1 << 20, "chunks that the minimum is right for");
+  auto lhs_near = [&](int kc) { return lhs_base + (uint32_t)min(kc * lhs_chunk_bytes, lhs_last_near); };
+  auto rhs_near = [&](int kc) { return rhs_base + (uint32_t)min(kc * rhs_chunk_bytes, rhs_last_near); };
   auto issue_chunk = [&](int kc) {
-    const int idx = min(kc, last_chunk);
     const uint32_t stage_off = (uint32_t)(kc % STAGES) * (STAGE_PIECES * 16);
-    const uint8_t* la = lhs_base + (idx == last_chunk ? lhs_last_base : idx * lhs_chunk_bytes);
-    const uint8_t* lb = rhs_base + (idx == last_chunk ? rhs_last_base : idx * rhs_chunk_bytes);
+    const uint8_t* la = lhs_near(kc);
+    const uint8_t* lb = rhs_near(kc);
 #pragma unroll
     for (int n = 0; n < LOADS; ++n) issue_load(n, stage_off, la, lb);
   };
@@ -982,8 +990,8 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   uint4 pa[AM][2], pb[BN][2], qa[AM][2], qb[BN][2];
   // G == 4: byte offset of a lane's first dword inside a fragment's K-step, see the layouts above.
   auto dwords_lane_offset = [&](int log2_t0) -> int32_t {
-    const int h = lane >> 5, r = lane & 31, g = r >> 2;
-    const int s = log2_t0 == 3 ? 4 * (g >> 1) + ((2 * h + (g & 1)) ^ (2 * (g >> 2))) : 8 * h + g;
+    const int h = lane >> 5, r = lane & 31, g = r >> 2, eight = -(int)(log2_t0 == 3);
+    const int s = ((4 * (g >> 1) + ((2 * h + (g & 1)) ^ (2 * (g >> 2)))) & eight) | ((8 * h + g) & ~eight);
     return 16 * s + 4 * (r & 3);
   };
   // G < 16: dword `part` (0..3) of a lane's operand for one (fragment, K-step),
@@ -1051,8 +1059,8 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   // chunk number (64-bit multiplies on the scalar unit, in front of the step's
   // first MFMA).
   constexpr uint32_t STAGE_BYTES = STAGE_PIECES * 16, RING_BYTES = STAGES * STAGE_BYTES;
-  const uint8_t* load_a = lhs_base + (AHEAD >= last_chunk ? lhs_last_base : AHEAD * lhs_chunk_bytes);
-  const uint8_t* load_b = rhs_base + (AHEAD >= last_chunk ? rhs_last_base : AHEAD * rhs_chunk_bytes);
+  const uint8_t* load_a = lhs_near(AHEAD);
+  const uint8_t* load_b = rhs_near(AHEAD);
   int load_chunk = AHEAD;
   uint32_t load_stage_off = AHEAD * STAGE_BYTES % RING_BYTES;
   uint32_t read_stage_off = STAGE_BYTES;
@@ -1713,6 +1721,7 @@ void mmt4d_mfma_split_k_kernel(const MfmaArgs a) {
   constexpr int MFMAS = KKW * AMF * 2;
   static_assert(MFMAS == 8 && LOADS <= 8 && READS <= 8, "the step below deals memory work over four of eight MFMAs");
 
+  fetch_arguments(a);
   int tile_row, tile_col;
   if (!locate_block(a, &tile_row, &tile_col)) return;
   const int tid = threadIdx.x;
@@ -1922,6 +1931,7 @@ void set_tile_grid(MfmaArgs* m, int block_rows, int block_cols, unsigned* grid) 
   m->tile_rows = (int32_t)((rows + block_rows - 1) / block_rows);
   m->tile_cols = (int32_t)((cols + block_cols - 1) / block_cols);
   const int64_t tiles = (int64_t)m->tile_rows * m->tile_cols;
+  m->band_reciprocal = band_reciprocal((uint32_t)m->tile_cols);
   *grid = (unsigned)(((tiles + 7) / 8) * 8);
 }
 

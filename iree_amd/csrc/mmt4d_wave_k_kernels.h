@@ -193,6 +193,7 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
   // The wavefronts' staging of narrow row pieces, [WAVES][FA + FB][1 KiB]; then [WAVES][FA * FB][64] partial sums.
   extern __shared__ uint4 ring[];
 
+  fetch_arguments(a);
   int tile_row, tile_col;
   if (!locate_block(a, &tile_row, &tile_col)) return;
   const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
@@ -200,25 +201,27 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
   const int64_t total_rows = (int64_t)a.M << a.log2_M0, total_cols = (int64_t)a.N << a.log2_N0;
   const int64_t first_row = (int64_t)tile_row * (16 * FA), first_col = (int64_t)tile_col * (16 * FB);
 
-  // Tiles past the end of the matrix are redirected to its last one: computed, never stored.
+  // Tiles past the end of the matrix are redirected to its last one: computed, never stored. (32 bits: offsets from the
+  // workgroup's first tile, which the plan has checked. This runs once, in front of the first load.)
   auto set_up = [&](auto& op, const uint8_t* base, int64_t first, int32_t tiles, int log2_t0, int64_t stride, int32_t rb,
                     int log2_rb, int32_t lane_bytes) {
-    const int64_t kstep = (int64_t)rb << log2_t0;
+    const uint32_t kstep = (uint32_t)rb << log2_t0;
     const int32_t first_tile = (int32_t)(first >> log2_t0);
+    const int32_t last_tile = tiles - 1 - first_tile;
     op.base = (global_bytes_t)uniform_pointer(base + first_tile * stride);
     op.step_bytes = (uint32_t)(4 * lane_bytes) << log2_t0;
-    op.kstep_bytes = (uint32_t)kstep;
+    op.kstep_bytes = kstep;
     int32_t row;  // of the fragment
-    int64_t lane_off;
+    uint32_t lane_off;
     if constexpr (PIECES) {
       row = r;
       op.k_lane = q;
-      lane_off = q * kstep;
+      lane_off = (uint32_t)q << (log2_rb + log2_t0);
       op.lds_slot = 0;
     } else if constexpr (G == 16) {
       row = r;
       op.k_lane = (lane_bytes * q) >> log2_rb;
-      lane_off = op.k_lane * kstep + ((lane_bytes * q) & (rb - 1));
+      lane_off = ((uint32_t)op.k_lane << (log2_rb + log2_t0)) + ((lane_bytes * q) & (rb - 1));
       op.lds_slot = 0;
     } else {
       // Lanes go along a tile's step (64 bytes per row, contiguous), then to the fragment's next tile.
@@ -227,13 +230,13 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
       const int32_t group = in_tile & ((1 << log2_lanes_per_kstep) - 1);
       op.k_lane = in_tile >> log2_lanes_per_kstep;
       row = ((lane >> (2 + log2_t0)) << log2_t0) + group * (16 / G);
-      lane_off = op.k_lane * kstep;
+      lane_off = (uint32_t)op.k_lane << (log2_rb + log2_t0);
       op.lds_slot = (uint32_t)(op.k_lane * 16 + row) * G;
     }
 #pragma unroll
     for (int f = 0; f < (int)(sizeof op.off / sizeof op.off[0]); ++f) {
-      const int32_t tile = min(first_tile + ((16 * f + row) >> log2_t0), tiles - 1) - first_tile;
-      op.off[f] = (uint32_t)(tile * stride + (row & ((1 << log2_t0) - 1)) * rb + lane_off);
+      const int32_t tile = min((16 * f + row) >> log2_t0, last_tile);
+      op.off[f] = (uint32_t)tile * (uint32_t)stride + ((uint32_t)(row & ((1 << log2_t0) - 1)) << log2_rb) + lane_off;
     }
   };
   lhs_t lhs;
@@ -250,10 +253,11 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
   // The steps are dealt out to the wavefronts in turn: at any time the workgroup reads one contiguous stretch of every row
   // panel. (A contiguous share of K per wavefront puts all loads of a launch at the same few offsets modulo the share: 5 to
   // 10 % slower.)
-  const int32_t ksteps_per_step = (RHS_I4 ? 128 : 64) >> a.log2_lhs_rb;
-  const int32_t steps = (a.K + ksteps_per_step - 1) / ksteps_per_step;
-  const int32_t whole = a.K / ksteps_per_step;
-  const int32_t count = (whole - wave + WAVES - 1) / WAVES;
+  static_assert(WAVES == 8, "a shift by three");
+  const int32_t log2_ksteps = (RHS_I4 ? 7 : 6) - a.log2_lhs_rb, ksteps_per_step = 1 << log2_ksteps;
+  const int32_t steps = (a.K + ksteps_per_step - 1) >> log2_ksteps;
+  const int32_t whole = a.K >> log2_ksteps;
+  const int32_t count = (whole - wave + WAVES - 1) >> 3;
 
   struct Step {
     uint4 l[lhs_t::RAW], r[rhs_t::RAW];

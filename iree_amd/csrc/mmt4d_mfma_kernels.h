@@ -677,6 +677,12 @@ __global__ __launch_bounds__(256, MIN_BLOCKS) void mmt4d_mfma_kernel(const MfmaA
 // fragment instead of one 128-bit read, and the loads are arranged so that
 // those reads are linear in the lane number (conflict-free).
 //
+// A wavefront alone on its SIMD issues an instruction every four to six cycles, and a step of the smaller tiles takes as long
+// as its instructions: 46 for 4 MFMAs on the 128x64 tile (57 before the first chunk took what is odd about K, see below, and
+// loads came in pairs). bf16 512 x 4096 x 4096 23.0 -> 21.6 us, 304 x 5008 x 3008 16.4 -> 15.5, int8 8x8x4 512 x 4096 x 4096
+// 13.7 -> 12.9; int4 512 x 11008 x 4096 (256x128) 29.2 -> 27.4, 784 x 4112 x 4096 (128x128) 21.5 -> 20.1; 192-wide tiles 2
+// to 5 %, 256x256 up to 2 % (int8 16x16x2, 4096^3, bound by power, 71.4 -> 72.1).
+//
 // The loads are issued from inline assembly: the compiler cannot see that they
 // write LDS, so it does not serialise the LDS reads against them; ordering is
 // enforced by hand with s_waitcnt vmcnt + a workgroup barrier once per chunk.
@@ -692,13 +698,23 @@ __device__ unsigned long long uk_timeline[256 * 8];
 #define UK_TIMELINE(...)
 #endif
 
-// One wavefront-wide load of 64 x 16 bytes to LDS byte offset `lds_off`
-// (wavefront-uniform) from `base` (uniform) + per-lane byte offset `voff`.
+// One wavefront-wide load of 64 x 16 bytes to LDS byte offset `lds_off` + FURTHER (wavefront-uniform) from `base`
+// (uniform) + per-lane byte offset `voff`.
+template <uint32_t FURTHER = 0>
 __device__ __forceinline__ void load_to_lds(uint32_t lds_off, uint32_t voff, const uint8_t* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                :
-               : "s"(lds_off), "v"(voff), "s"(base)
-               : "memory");
+               : "s"(lds_off), "v"(voff), "s"(base), "n"(FURTHER)
+               : "memory", "scc");
+}
+// Two, the second to LDS 1 KiB further on. The instruction's offset is added to both addresses: the caller has taken the
+// 1 KiB off `voff1`.
+template <uint32_t FURTHER>
+__device__ __forceinline__ void load_two_to_lds(uint32_t lds_off, uint32_t voff0, uint32_t voff1, const uint8_t* base) {
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %3\n\tglobal_load_lds_dwordx4 %2, %3 offset:1024"
+               :
+               : "s"(lds_off), "v"(voff0), "v"(voff1), "s"(base), "n"(FURTHER)
+               : "memory", "scc");
 }
 
 // 8 bytes per lane from LDS, transposed within each group of 16 lanes
@@ -719,6 +735,15 @@ __device__ __forceinline__ const uint8_t* uniform_pointer(const uint8_t* p) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
   const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
   return (const uint8_t*)(((uint64_t)hi << 32) | lo);
+}
+
+// f(0), .. f(N - 1), each number a type of its own.
+template <int N, typename F>
+__device__ __forceinline__ void each_of(F f) {
+  if constexpr (N > 0) {
+    each_of<N - 1>(f);
+    f(std::integral_constant<int, N - 1>());
+  }
 }
 
 template <int N>
@@ -777,7 +802,13 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   const uint8_t* rhs_base = uniform_pointer(a.rhs + (first_col >> a.log2_N0) * a.rhs_stride_bytes);
 
   // Load t of wavefront w fills the 16-byte LDS slots 64*m .. 64*m + 63 of its
-  // operand, m = 4*t + w, lane l the slot 64*m + l.
+  // operand, lane l the slot 64*m + l; m = 4*t + w or, where an operand's loads are issued together, loads*w + t.
+  // Together (one or two of them): on tiles whose steps are as long as their instructions take to issue, 64x64 and
+  // 128x64 and those of an int4 rhs up to 128x128, and where the operands come from HBM (ten stages: bf16 384 x 8192 x
+  // 4096 29.5 -> 29.1 us, 8x8x4 28.5 -> 28.0). The 128x128 tile of four stages, bound by the LDS, is 1 % faster one by one.
+  constexpr bool TOGETHER = AM * BN <= 2 || (AM * BN <= 4 && (RHS_I4 || STAGES == 10));
+  auto a_number = [&](int t) { return TOGETHER ? A_LOADS * wave + t : 4 * t + wave; };
+  auto b_number = [&](int t) { return TOGETHER ? B_LOADS * wave + t : 4 * t + wave; };
   //   G == 16: slot p holds fragment p >> 7, rows 16*((p >> 6) & 1) + (p & 15),
   //     16-byte column c = (p >> 4) & 3 (K-step c >> 1, lane half c & 1 of the
   //     MFMA operand): one load covers 16 rows x 64 bytes, which for 64-byte row
@@ -858,7 +889,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   if constexpr (G == 16) {
 #pragma unroll
     for (int t = 0; t < A_LOADS; ++t) {
-      const int p = tid + 256 * t;
+      const int p = 64 * a_number(t) + lane;
       int c = RHS_I4 ? ((p >> 6) & 1) + 2 * ((p >> 5) & 1) : (p >> 4) & 3;
       int row = RHS_I4 ? (p >> 7) * 32 + (p & 31) : (p >> 7) * 32 + 16 * ((p >> 6) & 1) + (p & 15);
       if (lhs_by_rows) {
@@ -870,7 +901,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     }
 #pragma unroll
     for (int t = 0; t < B_LOADS; ++t) {
-      const int p = tid + 256 * t;
+      const int p = 64 * b_number(t) + lane;
       int c = RHS_I4 ? (p >> 5) & 1 : (p >> 4) & 3;
       int row = RHS_I4 ? (p >> 6) * 32 + (p & 31) : (p >> 7) * 32 + 16 * ((p >> 6) & 1) + (p & 15);
       if (rhs_by_rows) {
@@ -883,61 +914,59 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   } else if constexpr (G == 1) {
     // One-byte row pieces (K0 = 1 int8: the operand is k-major, M0 bytes per k
     // step). A load brings one group of 16 rows x 64 k steps = 1 KiB, group
-    // m = 4*t + w of the operand (fragment m >> 1), into slots 64*m .. 64*m + 63:
+    // m of the operand (fragment m >> 1), into slots 64*m .. 64*m + 63:
     // 16-row tiles: lane l the 16 rows at k step l; 8-row tiles: lane l the 8
     // rows of tile l & 1 of the group at k steps 2*(l >> 1) and + 1. Either
     // way a k step's 16 rows lie within 32 bytes of LDS and the transposing
     // read (lds_read_transposed) hands lane (r, h) 8 consecutive k of row r; two
     // of them make a K-step's 16 bytes, in ascending k like every layout here.
-    auto piece_of = [&](int log2_t0, int t, int* row, int* k1) {
-      const int group = 4 * t + wave;
+    auto piece_of = [&](int log2_t0, int group, int* row, int* k1) {
       *row = 16 * group + (log2_t0 == 4 ? 0 : 8 * (lane & 1));
       *k1 = log2_t0 == 4 ? lane : 2 * (lane >> 1);
     };
 #pragma unroll
     for (int t = 0; t < A_LOADS; ++t) {
       int row, k1;
-      piece_of(a.log2_M0, t, &row, &k1);
+      piece_of(a.log2_M0, a_number(t), &row, &k1);
       a_off[t] = row_offset(row, rows_left - (1 << a.log2_M0), a.log2_M0, a.lhs_stride_bytes, a.log2_lhs_rb) +
                  (k1 << log2_lhs_kstep);
     }
 #pragma unroll
     for (int t = 0; t < B_LOADS; ++t) {
       int row, k1;
-      piece_of(a.log2_N0, t, &row, &k1);
+      piece_of(a.log2_N0, b_number(t), &row, &k1);
       b_off[t] = row_offset(row, cols_left - (1 << a.log2_N0), a.log2_N0, a.rhs_stride_bytes, a.log2_rhs_rb) +
                  (k1 << log2_rhs_kstep);
     }
   } else {
     constexpr int R = 16 / G;  // rows per 16-byte piece
-    // Row group and k step of the chunk of this lane's piece in load t (the
-    // wavefront's share of the k steps included).
-    auto piece_of = [&](int log2_t0, bool paired, int t, int* row, int* k1) {
+    // Row group and k step of the chunk of this lane's piece in load m.
+    auto piece_of = [&](int log2_t0, bool paired, int m, int* row, int* k1) {
       if (paired) {
-        *row = 64 * t + 8 * (lane & 7);
-        *k1 = 16 * (wave >> 1) + 8 * ((lane >> 3) & 1) + 4 * (wave & 1) + (lane >> 4);
+        *row = 64 * (m >> 2) + 8 * (lane & 7);
+        *k1 = 16 * ((m >> 1) & 1) + 8 * ((lane >> 3) & 1) + 4 * (m & 1) + (lane >> 4);
       } else if constexpr (G == 4) {
         // (Selected by masks, which the compiler does not make branches of.)
         const int eight = -(int)(log2_t0 == 3), x = (lane & 3) ^ ((lane >> 2) & 2);
         const int g = ((2 * ((lane >> 2) & 3) + (x & 1)) & eight) | (lane & 7 & ~eight);
         const int h = ((x >> 1) & eight) | ((lane >> 3) & 1 & ~eight);
-        *row = 32 * (2 * t + (wave >> 1)) + 4 * g;
-        *k1 = 8 * (wave & 1) + 2 * (lane >> 4) + h;
+        *row = 32 * (m >> 1) + 4 * g;
+        *k1 = 8 * (m & 1) + 2 * (lane >> 4) + h;
       } else {
-        *row = 32 * (2 * t + (wave >> 1)) + R * (lane % (2 * G));
-        *k1 = (32 / G) * (wave & 1) + (16 / G) * ((lane / (2 * G)) & 1) + lane / (4 * G);
+        *row = 32 * (m >> 1) + R * (lane % (2 * G));
+        *k1 = (32 / G) * (m & 1) + (16 / G) * ((lane / (2 * G)) & 1) + lane / (4 * G);
       }
     };
 #pragma unroll
     for (int t = 0; t < A_LOADS; ++t) {
       int row, k1;
-      piece_of(a.log2_M0, PAIR_A, t, &row, &k1);
+      piece_of(a.log2_M0, PAIR_A, a_number(t), &row, &k1);
       a_off[t] = row_offset(row, rows_left - R, a.log2_M0, a.lhs_stride_bytes, a.log2_lhs_rb) + (k1 << log2_lhs_kstep);
     }
 #pragma unroll
     for (int t = 0; t < B_LOADS; ++t) {
       int row, k1;
-      piece_of(a.log2_N0, PAIR_B, t, &row, &k1);
+      piece_of(a.log2_N0, PAIR_B, b_number(t), &row, &k1);
       b_off[t] = row_offset(row, cols_left - R, a.log2_N0, a.rhs_stride_bytes, a.log2_rhs_rb) + (k1 << log2_rhs_kstep);
     }
   }
@@ -950,41 +979,53 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
 
-  // K may end inside the last chunk. That chunk is then
-  // loaded from where a full chunk ends at K, so it overlaps the chunk before
-  // it and every load stays inside the operands, and the overlap, i.e. the
-  // first `cut_bytes` of its 64 bytes per row, is zeroed in the fragments of
-  // both operands (0 * 0 adds nothing, whatever the data; with an int4 rhs, where 0 * anything
-  // does, in the lhs alone). int4 with an odd number of k steps of 32 went to the register-staged kernel
-  // before: 1360 x 1712 x 1440 23.1 -> 11.6 us, 2512 x 4352 x 1504 51.2 -> 26.1.
+  // K in whole chunks but for the first: where K is none, chunk 0 is the first 64 bytes of every row all the same and
+  // chunk 1 begins where chunk 0 without its last `cut_bytes` ends. Every load stays inside the operands (there is a whole
+  // chunk at least), and what chunk 0 shares with chunk 1 is zeroed in its fragments of both operands once, in front of the
+  // loop (0 * 0 adds nothing, whatever the data; with an int4 rhs, where 0 * anything does, in the lhs alone). (The last
+  // chunk was the odd one before: a mask in every step, which the compiler makes unconditional, 24 of a step's 120
+  // instructions on the 256x128 tile, or a further step behind the loop, and four more scalar selects for where the last
+  // chunk lies.)
   const int chunks = a.chunks;
   const int last_chunk = chunks - 1;
   const int32_t cut_bytes = (int32_t)((64 - (((int64_t)a.K << a.log2_lhs_rb) & 63)) & 63);
-  const int64_t lhs_last_base = ((int64_t)a.K << log2_lhs_kstep) - lhs_chunk_bytes;
-  const int64_t rhs_last_base = ((int64_t)a.K << log2_rhs_kstep) - rhs_chunk_bytes;
-  const int64_t lhs_last_advance = lhs_last_base - (int64_t)(last_chunk - 1) * lhs_chunk_bytes;
-  const int64_t rhs_last_advance = rhs_last_base - (int64_t)(last_chunk - 1) * rhs_chunk_bytes;
+  const int32_t lhs_cut = cut_bytes << a.log2_M0, rhs_cut = cut_bytes << a.log2_N0 >> (RHS_I4 ? 1 : 0);
 
-  // Load number `n` (compile-time after unrolling) of the chunk whose operand
-  // bases are la / lb, into the stage at LDS byte offset `stage_off`.
-  auto issue_load = [&](int n, uint32_t stage_off, const uint8_t* la, const uint8_t* lb) {
-    const bool is_a = n < A_LOADS;
-    const int t = is_a ? n : n - A_LOADS;
-    load_to_lds(stage_off + (is_a ? 0 : A_PIECES * 16) + (256 * t + 64 * wave) * 16,
-                is_a ? a_off[t] : b_off[t], is_a ? la : lb);
+  // Loads number `n` (compile-time after unrolling) of the chunk whose operand bases are la / lb, into the stage at LDS byte
+  // offset `stage_off`, the wavefront's first slots included.
+  constexpr int A_ISSUES = TOGETHER ? 1 : A_LOADS, ISSUES = A_ISSUES + (TOGETHER ? 1 : B_LOADS);
+  const int32_t b_from_a = 16 * A_PIECES + 1024 * (b_number(0) - a_number(0));
+  if constexpr (TOGETHER) {
+    static_assert(A_LOADS <= 2 && B_LOADS <= 2, "one pair");
+    if constexpr (A_LOADS == 2) a_off[0] += 1024;  // (see load_two_to_lds; the bases are 1 KiB lower)
+    if constexpr (B_LOADS == 2) b_off[0] += 1024;
+  }
+  auto issue_load = [&](auto number, uint32_t stage_off, const uint8_t* la, const uint8_t* lb) {
+    constexpr int n = decltype(number)::value;
+    if constexpr (TOGETHER) {
+      if constexpr (n == 0) {
+        if constexpr (A_LOADS == 2) load_two_to_lds<0>(stage_off, a_off[0], a_off[1], la);
+        else load_to_lds(stage_off, a_off[0], la);
+      } else {
+        if constexpr (B_LOADS == 2) load_two_to_lds<0>(stage_off + b_from_a, b_off[0], b_off[1], lb);
+        else load_to_lds(stage_off + b_from_a, b_off[0], lb);
+      }
+    } else {
+      if constexpr (n < A_LOADS) load_to_lds<4096 * n>(stage_off, a_off[n], la);
+      else load_to_lds<16 * A_PIECES + 4096 * (n - A_LOADS)>(stage_off, b_off[n - A_LOADS], lb);
+    }
   };
-  // The first chunks: a compile-time `kc` of a few, whose base lies within 16 KiB (a minimum, no branches: see row_offset).
-  const int32_t lhs_last_near = (int32_t)min(lhs_last_base, (int64_t)1 << 20);
-  const int32_t rhs_last_near = (int32_t)min(rhs_last_base, (int64_t)1 << 20);
-  static_assert(AHEAD * 64 * 16 < 1 << 20, "chunks that the minimum is right for");
-  auto lhs_near = [&](int kc) { return lhs_base + (uint32_t)min(kc * lhs_chunk_bytes, lhs_last_near); };
-  auto rhs_near = [&](int kc) { return rhs_base + (uint32_t)min(kc * rhs_chunk_bytes, rhs_last_near); };
+  const uint8_t* lhs_from = lhs_base - (TOGETHER && A_LOADS == 2 ? 1024 : 0);
+  const uint8_t* rhs_from = rhs_base - (TOGETHER && B_LOADS == 2 ? 1024 : 0);
+  // The first chunks: a compile-time `kc` of a few. (Minima and maxima, no branches: see row_offset. Chunks beyond the last
+  // one are that one again.)
+  auto lhs_near = [&](int kc) { return lhs_from + (uint32_t)max(min(kc, last_chunk) * lhs_chunk_bytes - lhs_cut, 0); };
+  auto rhs_near = [&](int kc) { return rhs_from + (uint32_t)max(min(kc, last_chunk) * rhs_chunk_bytes - rhs_cut, 0); };
   auto issue_chunk = [&](int kc) {
-    const uint32_t stage_off = (uint32_t)(kc % STAGES) * (STAGE_PIECES * 16);
+    const uint32_t stage_off = (uint32_t)(kc % STAGES) * (STAGE_PIECES * 16) + 1024 * a_number(0);
     const uint8_t* la = lhs_near(kc);
     const uint8_t* lb = rhs_near(kc);
-#pragma unroll
-    for (int n = 0; n < LOADS; ++n) issue_load(n, stage_off, la, lb);
+    each_of<ISSUES>([&](auto n) { issue_load(n, stage_off, la, lb); });
   };
 
   uint4 pa[AM][2], pb[BN][2], qa[AM][2], qb[BN][2];
@@ -1062,7 +1103,8 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   const uint8_t* load_a = lhs_near(AHEAD);
   const uint8_t* load_b = rhs_near(AHEAD);
   int load_chunk = AHEAD;
-  uint32_t load_stage_off = AHEAD * STAGE_BYTES % RING_BYTES;
+  const uint32_t load_ring_begin = 1024 * a_number(0), load_ring_end = RING_BYTES + load_ring_begin;
+  uint32_t load_stage_off = AHEAD * STAGE_BYTES % RING_BYTES + load_ring_begin;
   uint32_t read_stage_off = STAGE_BYTES;
   const uint32_t frag_a_off = (uint32_t)((wave_m * AM) * 128) * 16;
   const uint32_t frag_b_off = (uint32_t)(A_PIECES + (wave_n * BN) * (RHS_I4 ? 64 : 128)) * 16;
@@ -1092,22 +1134,22 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   const int32_t rhs_kk1_step = rhs_by_rows ? 16 * ((by_rows_slot0 ^ 2) - by_rows_slot0) : 16 * 32;
   const uint32_t own_half = (lane & 1) ? 0x07060302u : 0x05040100u;
 
-  // Zeroes what the last chunk shares with the one before it. Lane half h of K-step kk holds bytes 32*kk + 16*h .. + 15 of
+  // Zeroes what chunk 0 shares with chunk 1. Lane half h of K-step kk holds bytes 32*kk + 16*h .. + 15 of
   // the chunk's 64 bytes per row, in ascending order of k; with an int4 rhs bytes 16*kk + 32*h .. + 15; of 4-byte
   // pieces every other one of bytes 32*kk .. + 31, from the h-th on.
   auto cut_fragments = [&](uint4 (*fa)[2], uint4 (*fb)[2]) {
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
       const int first_byte = RHS_I4 ? 16 * kk + 32 * (lane >> 5) : 32 * kk + 16 * (lane >> 5);
-      const int cut = min(max(cut_bytes - first_byte, 0), 16);
+      const int kept = min(max(64 - cut_bytes - first_byte, 0), 16);
       uint32_t keep[4];
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
         if constexpr (G == 4) {
-          keep[w] = 32 * kk + 8 * w + 4 * (lane >> 5) < cut_bytes ? 0u : 0xFFFFFFFFu;
+          keep[w] = 32 * kk + 8 * w + 4 * (lane >> 5) < 64 - cut_bytes ? 0xFFFFFFFFu : 0u;
           continue;
         }
-        keep[w] = cut >= 4 * w + 4 ? 0u : (cut <= 4 * w ? 0xFFFFFFFFu : 0xFFFFFFFFu << (8 * (cut - 4 * w)));
+        keep[w] = kept >= 4 * w + 4 ? 0xFFFFFFFFu : (kept <= 4 * w ? 0u : (1u << (8 * (kept - 4 * w))) - 1);
       }
 #pragma unroll
       for (int i = 0; i < AM; ++i) {
@@ -1121,13 +1163,6 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       }
     }
   };
-  // Where that happens: behind the loop, in front of the last chunk's step, or in the step that reads its fragments. A
-  // branch in every step costs the smaller tiles (f16 384 x 2912 x 2848 in 128x64 tiles 17.2 -> 14.8 us without it; int8
-  // 1024^3 in 64x64 tiles 5.86 -> 5.35, level with the wave-K tile that it takes) and all int4 ones (128x128 and 64x128 11 to 14 %). The larger tiles hide it, and
-  // lose more by the further step that the code then has behind the loop, run once and fetched from memory (192x192
-  // tiles 1 us of 16).
-  constexpr bool CUT_BEHIND_LOOP = RHS_I4 || AM * BN <= 4;
-
   // One pipeline step for the chunk whose fragments are in `cur`:
   //   a few MFMAs first (they only need registers, and keep the matrix pipe
   //   fed across the barrier); wait until this wavefront's loads of the next
@@ -1212,10 +1247,6 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       wait_loads_but<LOADS*(AHEAD - 2)>();
     }
     __builtin_amdgcn_s_barrier();
-    // The fragments read during this step are those of chunk load_chunk - AHEAD + 1.
-    // (The variants with the staggered tail are launched for K in whole chunks only: nothing to cut there, and the
-    // masking, which the compiler makes unconditional, 64 instructions per step, is left out.)
-    const bool cut_next = !CUT_BEHIND_LOOP && STAGGER == 0 && cut_bytes != 0 && load_chunk - AHEAD + 1 == last_chunk;
     const uint8_t* read_a = ring_bytes + read_stage_off + frag_a_off + pair_a_lane;
     const uint8_t* read_a_kk1 = read_a + lhs_kk1_step;  // (used where the lhs has 16-byte pieces)
     const uint8_t* read_b = ring_bytes + read_stage_off + frag_b_off + pair_b_lane;
@@ -1225,9 +1256,10 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     for (int m = LEAD; m < MFMAS; ++m) {
       const int slot = m - LEAD;
       if (slot < SLOTS) {
-#pragma unroll
-        for (int n = slot * LOADS / SLOTS; n < (slot + 1) * LOADS / SLOTS; ++n)
-          issue_load(n, load_stage_off, load_a, load_b);
+        each_of<ISSUES>([&](auto n) {
+          if (n.value >= slot * ISSUES / SLOTS && n.value < (slot + 1) * ISSUES / SLOTS)
+            issue_load(n, load_stage_off, load_a, load_b);
+        });
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = slot * READS / SLOTS; u < (slot + 1) * READS / SLOTS; ++u) {
@@ -1291,16 +1323,15 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       if (m == MFMAS - 1) {
         // Advance the running state (clamped at the last chunk: the loads
         // issued beyond it are redundant, their stages are never read).
-        const bool more = load_chunk < last_chunk, to_last = load_chunk + 1 == last_chunk;
-        load_a += more ? (to_last ? lhs_last_advance : lhs_chunk_bytes) : 0;
-        load_b += more ? (to_last ? rhs_last_advance : rhs_chunk_bytes) : 0;
+        const bool more = load_chunk < last_chunk;
+        load_a += (uint32_t)(more ? lhs_chunk_bytes : 0);
+        load_b += (uint32_t)(more ? rhs_chunk_bytes : 0);
         ++load_chunk;
-        load_stage_off = load_stage_off + STAGE_BYTES == RING_BYTES ? 0 : load_stage_off + STAGE_BYTES;
+        load_stage_off = load_stage_off + STAGE_BYTES == load_ring_end ? load_ring_begin : load_stage_off + STAGE_BYTES;
         read_stage_off = read_stage_off + STAGE_BYTES == RING_BYTES ? 0 : read_stage_off + STAGE_BYTES;
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (cut_next) cut_fragments(nxt_a, nxt_b);
   };
   auto step = [&](const uint4 (*cur_a)[2], const uint4 (*cur_b)[2], uint4 (*nxt_a)[2], uint4 (*nxt_b)[2],
                   bool held_loads_behind = false) {
@@ -1556,6 +1587,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       }
     }
   }
+  if (!TAILED && cut_bytes != 0) cut_fragments(pa, pb);
   UK_TIMELINE(tl_loop = __builtin_amdgcn_s_memrealtime();)
   int kc = 0;
   if constexpr (TAILED) {
@@ -1641,30 +1673,11 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     tail(pa, pb);
     return;
   }
-  if constexpr (CUT_BEHIND_LOOP) {
-    for (; kc + 2 < chunks; kc += 2) {
-      step(pa, pb, qa, qb);
-      step(qa, qb, pa, pb);
-    }
-    if (kc + 1 < chunks) {
-      step(pa, pb, qa, qb);
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-#pragma unroll
-        for (int i = 0; i < AM; ++i) pa[i][kk] = qa[i][kk];
-#pragma unroll
-        for (int j = 0; j < BN; ++j) pb[j][kk] = qb[j][kk];
-      }
-    }
-    if (cut_bytes != 0) cut_fragments(pa, pb);
+  for (; kc + 1 < chunks; kc += 2) {
     step(pa, pb, qa, qb);
-  } else {
-    for (; kc + 1 < chunks; kc += 2) {
-      step(pa, pb, qa, qb);
-      step(qa, qb, pa, pb);
-    }
-    if (kc < chunks) step(pa, pb, qa, qb);
+    step(qa, qb, pa, pb);
   }
+  if (kc < chunks) step(pa, pb, qa, qb);
   // No load may still be writing LDS when the workgroup's allocation is freed.
   wait_loads_but<0>();
   UK_TIMELINE(tl_loop_end = __builtin_amdgcn_s_memrealtime();)

@@ -36,6 +36,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "uk_device.h"
 #include "uk_internal.h"
 
 namespace uk {
@@ -70,7 +71,37 @@ struct TiledArgs {
   // linear_block_of: consecutive blocks that one XCD takes, workgroups per XCD
   // that are dealt out that way, and blocks per XCD of the rest.
   int32_t group, grouped_slots, rest_per_xcd;
+  // What a workgroup divides by to find its block, with reciprocals (set_bands).
+  int32_t band_blocks, last_band, last_band_rows;
+  uint32_t group_reciprocal, band_blocks_reciprocal, band_reciprocal, last_band_reciprocal;
 };
+
+// Fills in what block_of and linear_block_of divide by.
+void set_bands(TiledArgs* a) {
+  const int32_t blocks1 = a->blocks1 < 1 ? 1 : a->blocks1, blocks0 = a->total_blocks < blocks1 ? 1 : a->total_blocks / blocks1;
+  const int64_t band_blocks = (int64_t)a->band * blocks1;
+  a->band_blocks = (int32_t)(band_blocks < INT32_MAX ? band_blocks : INT32_MAX);  // (fewer blocks than that in all)
+  a->last_band = (blocks0 - 1) / a->band;
+  a->last_band_rows = blocks0 - a->last_band * a->band;
+  a->group_reciprocal = reciprocal_of((uint32_t)a->group);
+  a->band_blocks_reciprocal = reciprocal_of((uint32_t)a->band_blocks);
+  a->band_reciprocal = reciprocal_of((uint32_t)a->band);
+  a->last_band_reciprocal = reciprocal_of((uint32_t)a->last_band_rows);
+}
+
+// The kernel arguments lie in three cache lines that nothing has fetched yet, 560 cycles away: needed here together they are
+// fetched together. As their uses came up five trips followed one another, with four divisions of 35 instructions between:
+// some 220 instructions in front of a workgroup's first load, of which 100 are left. bf16 [2048, 5504] into 16x16 tiles, both
+// transposes, 8.40 -> 7.66 us, f32 [2329, 1590] 5.92 -> 5.58, [1000, 4100] unpacked 6.75 -> 6.50, s32 [2048, 4100] 11.5 ->
+// 11.3, the int8 chain of 512 x 2048 x 2048 14.2 -> 13.6; f32 [8191, 8190], bound by memory, packed and unpacked 168.9 -> 167.7.
+__device__ __forceinline__ void fetch_arguments(const TiledArgs& a) {
+  asm volatile("" ::"s"(a.src), "s"(a.dst), "s"(a.flat_stride0), "s"(a.tiled_stride0), "s"(a.size0), "s"(a.size1), "s"(a.outer0),
+               "s"(a.outer1), "s"(a.log2_t0), "s"(a.log2_t1), "s"(a.log2_s3), "s"(a.log2_br), "s"(a.log2_bc));
+  asm volatile("" ::"s"(a.pitch_bytes), "s"(a.blocks1), "s"(a.total_blocks), "s"(a.tr_inner), "s"(a.tr_outer), "s"(a.band),
+               "s"(a.group), "s"(a.grouped_slots), "s"(a.rest_per_xcd), "s"(a.band_blocks), "s"(a.last_band), "s"(a.last_band_rows),
+               "s"(a.group_reciprocal), "s"(a.band_blocks_reciprocal), "s"(a.band_reciprocal), "s"(a.last_band_reciprocal));
+  __builtin_amdgcn_sched_barrier(0);
+}
 
 // Coordinates of an element of the tiled side within a block.
 struct TiledCoord {
@@ -120,17 +151,13 @@ __device__ __forceinline__ TiledCoord tiled_coord(const TiledArgs& a, int32_t e,
 // other's runs (measured on 16384^2 int8 into [n][k][16][16]: 4.9 TB/s with
 // band 1, 5.9 TB/s with 16).
 __device__ __forceinline__ void block_of(const TiledArgs& a, int32_t linear, int64_t* block0, int64_t* block1) {
-  if (a.band <= 1) {
-    *block0 = linear / a.blocks1;
-    *block1 = linear % a.blocks1;
-    return;
-  }
-  const int32_t blocks0 = a.total_blocks / a.blocks1;
-  const int32_t g = linear / (a.band * a.blocks1), first = g * a.band;
-  const int32_t rows_here = min(a.band, blocks0 - first);
-  const int32_t i = linear - g * a.band * a.blocks1;
-  *block0 = first + i % rows_here;
-  *block1 = i / rows_here;
+  const uint32_t g = divide((uint32_t)linear, (uint32_t)a.band_blocks, a.band_blocks_reciprocal);
+  const uint32_t i = (uint32_t)linear - g * (uint32_t)a.band_blocks;
+  const bool last = g == (uint32_t)a.last_band;
+  const uint32_t rows_here = (uint32_t)(last ? a.last_band_rows : a.band);
+  const uint32_t column = divide(i, rows_here, last ? a.last_band_reciprocal : a.band_reciprocal);
+  *block0 = g * (uint32_t)a.band + (i - column * rows_here);
+  *block1 = column;
 }
 
 // Workgroup id -> block number. Consecutive workgroup ids land on different
@@ -150,12 +177,10 @@ __device__ __forceinline__ void block_of(const TiledArgs& a, int32_t linear, int
 // stretches, so that no XCD is left with a group more than the others.
 __device__ __forceinline__ int32_t linear_block_of(const TiledArgs& a) {
   const uint32_t xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, group = (uint32_t)a.group;
-  if (slot < (uint32_t)a.grouped_slots) {
-    const uint32_t g = slot / group;
-    return (int32_t)((g * 8 + xcd) * group + (slot - g * group));
-  }
-  const uint32_t r = slot - (uint32_t)a.grouped_slots;
-  return (int32_t)((uint32_t)a.grouped_slots * 8 + xcd * (uint32_t)a.rest_per_xcd + r);
+  const uint32_t g = divide(slot, group, a.group_reciprocal);
+  const uint32_t grouped = (g * 8 + xcd) * group + (slot - g * group);
+  const uint32_t rest = (uint32_t)a.grouped_slots * 8 + xcd * (uint32_t)a.rest_per_xcd + (slot - (uint32_t)a.grouped_slots);
+  return (int32_t)(slot < (uint32_t)a.grouped_slots ? grouped : rest);
 }
 
 // 16 bytes without an alignment requirement: the hardware's multi-dword
@@ -320,6 +345,7 @@ __global__ __launch_bounds__(256) void tiled_kernel(const TiledArgs a) {
   constexpr int LOG2_W = W == 16 ? 4 : W == 8 ? 3 : W == 4 ? 2 : W == 2 ? 1 : 0;
 
   const int tid = threadIdx.x;
+  fetch_arguments(a);
   const int32_t linear = linear_block_of(a);
   if (linear >= a.total_blocks) return;
   int64_t block0, block1;
@@ -656,6 +682,7 @@ __global__ __launch_bounds__(256) void pack_transposing_wide_kernel(const TiledA
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int lane_row = lane >> 4, cg = lane & 15;
+  fetch_arguments(a);
   const int32_t linear = linear_block_of(a);
   if (linear >= a.total_blocks) return;
   int64_t block0, block1;
@@ -772,6 +799,7 @@ __global__ __launch_bounds__(256) void pack_transposing_kernel(const TiledArgs a
   constexpr int TILED_PER_THREAD = kBlockBytes / 16 / 256;
 
   const int tid = threadIdx.x;
+  fetch_arguments(a);
   const int32_t linear = linear_block_of(a);
   if (linear >= a.total_blocks) return;
   int64_t block0, block1;
@@ -1105,10 +1133,11 @@ bool make_plan(const uint8_t* flat, const uint8_t* tiled, int64_t flat_stride0, 
     const int64_t group = a.band > 1 ? (int64_t)a.band * a.blocks1 : 64;
     const int64_t grouped_slots = a.total_blocks / (8 * group) * group;
     const int64_t rest = a.total_blocks - 8 * grouped_slots;
-    a.group = (int32_t)group;
+    a.group = (int32_t)(group < INT32_MAX ? group : INT32_MAX);
     a.grouped_slots = (int32_t)grouped_slots;
     a.rest_per_xcd = (int32_t)((rest + 7) / 8);
     plan->grid = (unsigned)((grouped_slots + a.rest_per_xcd) * 8);
+    set_bands(&a);
   }
   plan->lds_bytes = (size_t)br * a.pitch_bytes;
   return plan->lds_bytes <= 49152;

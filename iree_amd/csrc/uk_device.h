@@ -92,19 +92,22 @@ __host__ __device__ __forceinline__ uint16_t narrow16(float f) {
   return (uint16_t)(sign | r);
 }
 
-// Tile number `linear` of a grid of tile_rows x tile_cols tiles that are walked in bands of kBandRows rows, a band column by
-// column. Divisions by multiplication: the compiler's, of 25 dependent instructions each, were a fifth of what ran in front of
-// a workgroup's first load. tile_cols below 2^29.
-constexpr uint32_t kBandRows = 4;
-// ceil(2^32 / tiles of a band)
-__host__ __device__ __forceinline__ uint32_t band_reciprocal(uint32_t tile_cols) {
-  return 0xFFFFFFFFu / (kBandRows * tile_cols) + 1;
+// n / d, exactly, by multiplication with a reciprocal that the host has computed. (The compiler's division of 32 bits is 25
+// dependent instructions, 100 to 150 cycles, and a workgroup divides before it can load.)
+__host__ __device__ __forceinline__ uint32_t reciprocal_of(uint32_t d) { return 0xFFFFFFFFu / d; }
+__host__ __device__ __forceinline__ uint32_t divide(uint32_t n, uint32_t d, uint32_t reciprocal) {
+  const uint32_t q = (uint32_t)((uint64_t)n * reciprocal >> 32);  // one too few at most
+  return q + (n - q * d >= d ? 1 : 0);
 }
+
+// Tile number `linear` of a grid of tile_rows x tile_cols tiles that are walked in bands of kBandRows rows, a band column by
+// column. tile_cols below 2^29.
+constexpr uint32_t kBandRows = 4;
+__host__ __device__ __forceinline__ uint32_t band_reciprocal(uint32_t tile_cols) { return reciprocal_of(kBandRows * tile_cols); }
 __host__ __device__ __forceinline__ void tile_of_number(uint32_t linear, uint32_t tile_rows, uint32_t tile_cols,
                                                         uint32_t reciprocal, int* tile_row, int* tile_col) {
   const uint32_t band_tiles = kBandRows * tile_cols;
-  uint32_t band = (uint32_t)((uint64_t)linear * reciprocal >> 32);  // one too many at most
-  band -= band * band_tiles > linear ? 1 : 0;
+  const uint32_t band = divide(linear, band_tiles, reciprocal);
   const uint32_t band_first = band * kBandRows, rows_left = tile_rows - band_first;
   const uint32_t band_rows = rows_left < kBandRows ? rows_left : kBandRows;
   const uint32_t in_band = linear - band * band_tiles;

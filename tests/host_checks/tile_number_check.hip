@@ -1,5 +1,5 @@
-// tile_of_number (iree_amd/csrc/uk_device.h) against plain divisions: every tile of small grids, and the tiles around the
-// ends of bands and of the grid of large ones.
+// divide and tile_of_number (iree_amd/csrc/uk_device.h) against plain divisions: divisors up to the largest with the numbers
+// around their multiples; every tile of small grids, and the tiles around the ends of bands and of the grid of large ones.
 #include <stdint.h>
 #include <stdio.h>
 
@@ -18,7 +18,20 @@ static void check(uint32_t linear, uint32_t rows, uint32_t cols) {
   }
 }
 
+static void check_divide(uint32_t n, uint32_t d) {
+  ++checked;
+  const uint32_t q = uk::divide(n, d, uk::reciprocal_of(d));
+  if (q != n / d && wrong++ < 10) printf("%u / %u: %u\n", n, d, q);
+}
+
 int main() {
+  for (uint64_t d = 1; d < 1ull << 32; d = d < 5000 ? d + 1 : d + d / 37)
+    for (uint64_t q : {0ull, 1ull, 2ull, 3ull, 100ull, 65535ull, 0xFFFFFFFFull / d / 2, 0xFFFFFFFFull / d - 1, 0xFFFFFFFFull / d})
+      for (int64_t e = -2; e <= 2; ++e) {
+        const int64_t n = (int64_t)(q * d) + e;
+        if (n >= 0 && n < 1ll << 32) check_divide((uint32_t)n, (uint32_t)d);
+      }
+  for (uint32_t d : {1u, 2u, 3u, 7u, 64u, 0x7FFFFFFFu, 0x80000000u, 0xFFFFFFFFu}) check_divide(0xFFFFFFFFu, d);
   for (uint32_t rows = 1; rows <= 40; ++rows)
     for (uint32_t cols = 1; cols <= 130; ++cols)
       for (uint32_t i = 0; i < rows * cols; ++i) check(i, rows, cols);

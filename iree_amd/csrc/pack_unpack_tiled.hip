@@ -1260,11 +1260,17 @@ int plan_transposing(Plan* p) {
 // both transposes 5.74 -> 5.83 (six or four workgroups: in between; three or two: 5.0-5.8), unpack 6.06 -> 6.17. Over
 // tiles 16x1, 8x8, 16x16, the four transpose combinations and [2048, 16384] ... [1024, 65536], buffers rotated
 // so that the last-level cache does not hold them: pack -3 to +8 %, unpack -6 to +12 %, about +2 % in the mean for
-// both. Not for 1- and 2-byte elements (-1 to -19 %) and not for matrices the last-level cache holds (4096^2:
-// -1 to -5 %, 3000^2: -2 to -8 %).
+// both. Not for 1-byte elements (int8 10000^2 -1 % with six, -13 % with five) and not for matrices the last-level cache
+// holds (4096^2: -1 to -5 %, 3000^2: -2 to -8 %).
+// 2-byte elements: six, for what exceeds kKeepInputBytes. 26 matrices of 101 to 400 MB, every tile shape and order, packed and
+// unpacked: 2.2 % less time in the mean, at best 6, never more than 0.1 % more (bf16 [4096, 14336], both transposes, 42.2 ->
+// 41.5 us, f16 [8192, 8192] in 16x1 tiles 57.0 -> 54.3, [8135, 21925] unpacked 133.7 -> 127.3; with seven half of that, with
+// five 42.2 -> 45.7). Below, 4 to 100 MB, up to 14 % more.
 void limit_resident_blocks(Plan* p) {
-  constexpr size_t kLdsAskedFor = 32 * 1024;
-  if (p->elem_bytes == 4 && p->args.total_blocks >= 8192 && p->lds_bytes < kLdsAskedFor) p->lds_bytes = kLdsAskedFor;
+  size_t asked_for = 0;
+  if (p->elem_bytes == 4 && p->args.total_blocks >= 8192) asked_for = 32 * 1024;
+  if (p->elem_bytes == 2 && p->args.total_blocks > kKeepInputBytes / kBlockBytes) asked_for = 24 * 1024;
+  if (p->lds_bytes < asked_for) p->lds_bytes = asked_for;
 }
 
 template <int E, bool UNPACK, int POLICY>

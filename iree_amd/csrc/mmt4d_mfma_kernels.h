@@ -737,6 +737,12 @@ __device__ __forceinline__ const uint8_t* uniform_pointer(const uint8_t* p) {
   return (const uint8_t*)(((uint64_t)hi << 32) | lo);
 }
 
+// (Overloads on scalars rather than a bit cast of a vector element.)
+__device__ __forceinline__ uint32_t value_bits(int32_t v) { return (uint32_t)v; }
+__device__ __forceinline__ uint32_t value_bits(float v) { return __float_as_uint(v); }
+__device__ __forceinline__ void set_from_bits(int32_t& v, uint32_t bits) { v = (int32_t)bits; }
+__device__ __forceinline__ void set_from_bits(float& v, uint32_t bits) { v = __uint_as_float(bits); }
+
 // f(0), .. f(N - 1), each number a type of its own.
 template <int N, typename F>
 __device__ __forceinline__ void each_of(F f) {
@@ -758,8 +764,8 @@ __device__ __forceinline__ void wait_loads_but() {
 // STAGGER: 0 = every accumulator stored after the last MFMA; 1 = staggered tail (see below); 2 = the same for
 // an accumulating call, the destination read in the tail; 3 = accumulating call with the destination read and
 // added during the main loop (needs enough steps), tail as in 1.
-template <int KIND, bool RHS_I4, bool NARROW, int G, int AM, int BN, int STAGES, int STAGGER = 0>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, AM * BN >= 9 ? 1 : (AM * BN >= 4 ? 2 : 4))))
+template <int KIND, bool RHS_I4, bool NARROW, int G, int AM, int BN, int STAGES, int STAGGER = 0, int GROUPS = 1>
+__global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(GROUPS, AM * BN >= 9 ? 1 : (AM * BN >= 4 ? 2 : 4))))
 void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   typedef typename AccType<KIND>::type acc_t;
   static_assert(!RHS_I4 || (G == 16 && BN >= 2), "int4 rhs: 16-byte pieces, at least one fragment per wavefront");
@@ -785,9 +791,9 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   int tile_row, tile_col;
   if (!locate_block(a, &tile_row, &tile_col)) return;
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = threadIdx.x & 63;
+  const int wave_of_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int group = GROUPS == 1 ? 0 : wave_of_all >> 2, wave = GROUPS == 1 ? wave_of_all : wave_of_all & 3;
   const int wave_m = wave >> 1, wave_n = wave & 1;
 
   const int64_t total_rows = (int64_t)a.M << a.log2_M0;
@@ -986,10 +992,14 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   // chunk was the odd one before: a mask in every step, which the compiler makes unconditional, 24 of a step's 120
   // instructions on the 256x128 tile, or a further step behind the loop, and four more scalar selects for where the last
   // chunk lies.)
-  const int chunks = a.chunks;
+  // Two groups: chunk i of group g is chunk 2*i + g of K, or one less where K has an odd number of chunks; the first group's
+  // first is none then, loaded as chunk 0 and zeroed whole.
+  const int chunks = GROUPS == 1 ? a.chunks : (a.chunks + 1) >> 1;
   const int last_chunk = chunks - 1;
-  const int32_t cut_bytes = (int32_t)((64 - (((int64_t)a.K << a.log2_lhs_rb) & 63)) & 63);
-  const int32_t lhs_cut = cut_bytes << a.log2_M0, rhs_cut = cut_bytes << a.log2_N0 >> (RHS_I4 ? 1 : 0);
+  const int group_from = GROUPS == 1 ? 0 : group - (a.chunks & 1);
+  const int32_t cut_of_row = (int32_t)((64 - (((int64_t)a.K << a.log2_lhs_rb) & 63)) & 63);
+  const int32_t lhs_cut = cut_of_row << a.log2_M0, rhs_cut = cut_of_row << a.log2_N0 >> (RHS_I4 ? 1 : 0);
+  const int32_t cut_bytes = group_from < 0 ? 64 : (group_from == 0 ? cut_of_row : 0);
 
   // Loads number `n` (compile-time after unrolling) of the chunk whose operand bases are la / lb, into the stage at LDS byte
   // offset `stage_off`, the wavefront's first slots included.
@@ -1019,10 +1029,17 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   const uint8_t* rhs_from = rhs_base - (TOGETHER && B_LOADS == 2 ? 1024 : 0);
   // The first chunks: a compile-time `kc` of a few. (Minima and maxima, no branches: see row_offset. Chunks beyond the last
   // one are that one again.)
-  auto lhs_near = [&](int kc) { return lhs_from + (uint32_t)max(min(kc, last_chunk) * lhs_chunk_bytes - lhs_cut, 0); };
-  auto rhs_near = [&](int kc) { return rhs_from + (uint32_t)max(min(kc, last_chunk) * rhs_chunk_bytes - rhs_cut, 0); };
+  auto lhs_near = [&](int kc) {
+    return lhs_from + (uint32_t)max((GROUPS * min(kc, last_chunk) + group_from) * lhs_chunk_bytes - lhs_cut, 0);
+  };
+  auto rhs_near = [&](int kc) {
+    return rhs_from + (uint32_t)max((GROUPS * min(kc, last_chunk) + group_from) * rhs_chunk_bytes - rhs_cut, 0);
+  };
+  // The group's ring.
+  const uint32_t ring_off = (uint32_t)group * (STAGES * STAGE_PIECES * 16);
+  const uint4* const own_ring = ring + ring_off / 16;
   auto issue_chunk = [&](int kc) {
-    const uint32_t stage_off = (uint32_t)(kc % STAGES) * (STAGE_PIECES * 16) + 1024 * a_number(0);
+    const uint32_t stage_off = ring_off + (uint32_t)(kc % STAGES) * (STAGE_PIECES * 16) + 1024 * a_number(0);
     const uint8_t* la = lhs_near(kc);
     const uint8_t* lb = rhs_near(kc);
     each_of<ISSUES>([&](auto n) { issue_load(n, stage_off, la, lb); });
@@ -1061,21 +1078,21 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   // Fragment f of an operand at 16-byte slot `operand` of the ring, K-step kk.
   auto read_frag = [&](int operand, int f, int kk) -> uint4 {
     if (RHS_I4 && operand >= A_PIECES) {
-      const uint4 raw = ring[operand + 64 * f + lane];
+      const uint4 raw = own_ring[operand + 64 * f + lane];
       return widen_i4_times16(kk ? make_uint2(raw.z, raw.w) : make_uint2(raw.x, raw.y));
     }
     if constexpr (G == 16) {
       if (!RHS_I4 && (operand == 0 ? lhs_by_rows : rhs_by_rows))
-        return ring[operand + 128 * f + 64 * ((lane & 31) >> 4) + 4 * (lane & 15) + ((2 * kk + (lane >> 5)) ^ ((lane >> 2) & 3))];
-      if (!RHS_I4) return ring[operand + 128 * f + 32 * kk + 64 * ((lane & 31) >> 4) + 16 * (lane >> 5) + (lane & 15)];
-      return ring[operand + 128 * f + 64 * kk + lane];
+        return own_ring[operand + 128 * f + 64 * ((lane & 31) >> 4) + 4 * (lane & 15) + ((2 * kk + (lane >> 5)) ^ ((lane >> 2) & 3))];
+      if (!RHS_I4) return own_ring[operand + 128 * f + 32 * kk + 64 * ((lane & 31) >> 4) + 16 * (lane >> 5) + (lane & 15)];
+      return own_ring[operand + 128 * f + 64 * kk + lane];
     } else if constexpr (G == 1) {
-      const uint8_t* first = (const uint8_t*)(ring + operand) + 2048 * f + 512 * kk +
+      const uint8_t* first = (const uint8_t*)(own_ring + operand) + 2048 * f + 512 * kk +
                              transposed_lane_offset(operand >= A_PIECES ? a.log2_N0 : a.log2_M0);
       const uint2 lo = lds_read_transposed(first), hi = lds_read_transposed(first + 128);
       return make_uint4(lo.x, lo.y, hi.x, hi.y);
     } else {
-      const uint8_t* first = (const uint8_t*)(ring + operand) + 1024 * (2 * f + kk) +
+      const uint8_t* first = (const uint8_t*)(own_ring + operand) + 1024 * (2 * f + kk) +
                              (G == 4 ? dwords_lane_offset(operand >= A_PIECES ? a.log2_N0 : a.log2_M0) : G * lane);
       return make_uint4(gather_dword(first, 0), gather_dword(first, 1), gather_dword(first, 2), gather_dword(first, 3));
     }
@@ -1103,7 +1120,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   const uint8_t* load_a = lhs_near(AHEAD);
   const uint8_t* load_b = rhs_near(AHEAD);
   int load_chunk = AHEAD;
-  const uint32_t load_ring_begin = 1024 * a_number(0), load_ring_end = RING_BYTES + load_ring_begin;
+  const uint32_t load_ring_begin = ring_off + 1024 * a_number(0), load_ring_end = RING_BYTES + load_ring_begin;
   uint32_t load_stage_off = AHEAD * STAGE_BYTES % RING_BYTES + load_ring_begin;
   uint32_t read_stage_off = STAGE_BYTES;
   const uint32_t frag_a_off = (uint32_t)((wave_m * AM) * 128) * 16;
@@ -1111,7 +1128,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   // Lane 32*h + r's byte offset into a fragment, and the slots from one K-step
   // of a fragment to the next (see the layouts above).
   const uint8_t* ring_bytes =
-      (const uint8_t*)ring + (ROWS16 ? 16 * (64 * ((lane & 31) >> 4) + 16 * (lane >> 5) + (lane & 15))
+      (const uint8_t*)own_ring + (ROWS16 ? 16 * (64 * ((lane & 31) >> 4) + 16 * (lane >> 5) + (lane & 15))
                                      : (G == 1 || G == 4 ? 0 : G * lane));
   // What a lane's reads of either operand add to that. G == 1: the transposing reads' offset. G == 4: the dword reads'. G == 2: lanes address
   // dwords, not 16-bit elements. Paired: dword number
@@ -1324,8 +1341,8 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
         // Advance the running state (clamped at the last chunk: the loads
         // issued beyond it are redundant, their stages are never read).
         const bool more = load_chunk < last_chunk;
-        load_a += (uint32_t)(more ? lhs_chunk_bytes : 0);
-        load_b += (uint32_t)(more ? rhs_chunk_bytes : 0);
+        load_a += (uint32_t)(more ? GROUPS * lhs_chunk_bytes : 0);
+        load_b += (uint32_t)(more ? GROUPS * rhs_chunk_bytes : 0);
         ++load_chunk;
         load_stage_off = load_stage_off + STAGE_BYTES == load_ring_end ? load_ring_begin : load_stage_off + STAGE_BYTES;
         read_stage_off = read_stage_off + STAGE_BYTES == RING_BYTES ? 0 : read_stage_off + STAGE_BYTES;
@@ -1566,7 +1583,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
 #pragma unroll
           for (int part = 0; part < 4; ++part)
             split_pair_part(
-                read_pair_part((const uint8_t*)(ring + A_PIECES) + 2048 * (frag_b0 + j) + 2048 * kk + 4 * lane, part),
+                read_pair_part((const uint8_t*)(own_ring + A_PIECES) + 2048 * (frag_b0 + j) + 2048 * kk + 4 * lane, part),
                 part, pb[j][kk], pb[j + 1][kk]);
         }
       } else {
@@ -1579,7 +1596,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
         if (i % 2 == 0) {
 #pragma unroll
           for (int part = 0; part < 4; ++part)
-            split_pair_part(read_pair_part((const uint8_t*)ring + 2048 * (frag_a0 + i) + 2048 * kk + 4 * lane, part),
+            split_pair_part(read_pair_part((const uint8_t*)own_ring + 2048 * (frag_a0 + i) + 2048 * kk + 4 * lane, part),
                             part, pa[i][kk], pa[i + 1][kk]);
         }
       } else {
@@ -1682,6 +1699,50 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   wait_loads_but<0>();
   UK_TIMELINE(tl_loop_end = __builtin_amdgcn_s_memrealtime();)
 
+  if constexpr (GROUPS == 2) {
+    // Group g takes the wavefront's fragments (i, j) with half of the i (or, AM = 1, of the j) and adds what the other group
+    // has of them, the first group's sum first. sums[wavefront of all][fragment][4 registers of 16][lane]
+    constexpr bool BY_ROWS = AM == 2;
+    static_assert((AM == 2 && BN <= 2) || (AM == 1 && BN == 2), "halves of one row or column of fragments");
+    static_assert(!PAIR_A && !PAIR_B && STAGGER == 0, "fragments on their own");
+    constexpr int HALF = AM * BN / 2;
+    static_assert(8 * HALF * 4 * 64 * 16 <= 2 * STAGES * STAGE_PIECES * 16, "the rings take the sums");
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    u32x4* const sums = (u32x4*)ring;
+    __syncthreads();  // nobody reads operands from the rings any more
+    auto fragment = [&](int of_group, int f) -> acc_t& { return BY_ROWS ? acc[of_group][f] : acc[0][of_group]; };
+#pragma unroll
+    for (int f = 0; f < HALF; ++f) {
+      acc_t other = fragment(1, f);
+      if (group == 1) other = fragment(0, f);
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        sums[((wave_of_all * HALF + f) * 4 + v) * 64 + lane] =
+            u32x4{value_bits(other[4 * v]), value_bits(other[4 * v + 1]), value_bits(other[4 * v + 2]), value_bits(other[4 * v + 3])};
+    }
+    __syncthreads();
+    acc_t total[1][BY_ROWS ? BN : 1];
+#pragma unroll
+    for (int f = 0; f < HALF; ++f) {
+      acc_t own = fragment(0, f), part;
+      if (group == 1) own = fragment(1, f);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const u32x4 bits = sums[(((wave_of_all ^ 4) * HALF + f) * 4 + v) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          typename AccType<KIND>::scalar value;
+          set_from_bits(value, bits[e]);
+          part[4 * v + e] = value;
+        }
+      }
+      total[0][f] = own + part;
+    }
+    store_block<KIND, RHS_I4, NARROW, 1, BY_ROWS ? BN : 1>(
+        a, total, first_row + wave_m * (32 * AM) + (BY_ROWS ? 32 * group : 0),
+        first_col + wave_n * (32 * BN) + (BY_ROWS ? 0 : 32 * group), lane);
+    return;
+  }
   store_block<KIND, RHS_I4, NARROW, AM, BN, PAIR_A, PAIR_B>(a, acc, first_row + wave_m * (32 * AM),
                                                             first_col + wave_n * (32 * BN), lane);
   UK_TIMELINE(asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1691,12 +1752,6 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
                 t[4] = __builtin_amdgcn_s_memrealtime();
               })
 }
-
-// (Overloads on scalars rather than a bit cast of a vector element.)
-__device__ __forceinline__ uint32_t value_bits(int32_t v) { return (uint32_t)v; }
-__device__ __forceinline__ uint32_t value_bits(float v) { return __float_as_uint(v); }
-__device__ __forceinline__ void set_from_bits(int32_t& v, uint32_t bits) { v = (int32_t)bits; }
-__device__ __forceinline__ void set_from_bits(float& v, uint32_t bits) { v = __uint_as_float(bits); }
 
 // ---------------------------------------------------------------------------
 // A 128x64 block tile whose four wavefronts split K instead of the tile, for 65 to
@@ -1949,14 +2004,15 @@ void set_tile_grid(MfmaArgs* m, int block_rows, int block_cols, unsigned* grid) 
 }
 
 // Direct-to-LDS kernel on (64*AM) x (64*BN) block tiles with a ring of STAGES stages.
-template <int KIND, bool RHS_I4, bool NARROW, int G, int AM, int BN, int STAGES>
+// GROUPS: of four wavefronts, that share K.
+template <int KIND, bool RHS_I4, bool NARROW, int G, int AM, int BN, int STAGES, int GROUPS = 1>
 hipError_t launch_direct(MfmaArgs m, hipStream_t stream, bool staggered_tail = true) {
   unsigned grid;
   set_tile_grid(&m, 64 * AM, 64 * BN, &grid);
   constexpr int stage_pieces = 256 * AM + (RHS_I4 ? 128 : 256) * BN;
-  constexpr size_t lds_bytes = (size_t)STAGES * 16 * stage_pieces;
+  constexpr size_t lds_bytes = (size_t)GROUPS * STAGES * 16 * stage_pieces;
   static_assert(lds_bytes <= 160 * 1024, "ring does not fit the LDS");
-  void (*kernel)(const MfmaArgs) = mmt4d_mfma_direct_kernel<KIND, RHS_I4, NARROW, G, AM, BN, STAGES>;
+  void (*kernel)(const MfmaArgs) = mmt4d_mfma_direct_kernel<KIND, RHS_I4, NARROW, G, AM, BN, STAGES, 0, GROUPS>;
   // The 256x256 tile with the staggered tail: K in whole chunks, enough of them.
   if constexpr (AM == 4 && BN == 4 && !RHS_I4 && G != 2 && KIND != kF32) {
     if (staggered_tail && ((int64_t)m.K * m.lhs_rb) % 64 == 0 && m.chunks >= 2 * STAGES) {
@@ -1973,7 +2029,7 @@ hipError_t launch_direct(MfmaArgs m, hipStream_t stream, bool staggered_tail = t
         hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
     if (attr != hipSuccess) return attr;
   }
-  return launch_kernel<MfmaArgs>(kernel, grid, 256, lds_bytes, stream, m);
+  return launch_kernel<MfmaArgs>(kernel, grid, 256 * GROUPS, lds_bytes, stream, m);
 }
 
 template <int KIND, bool NARROW>
@@ -2016,6 +2072,20 @@ inline bool streams_operands(const MfmaArgs& m, int block_rows, int block_cols) 
   return tiles <= 256 && comes_from_hbm((rows * m.lhs_rb + cols * m.rhs_rb) * m.K);
 }
 
+// One workgroup per compute unit at most, and K long enough: two groups of four wavefronts with a ring each multiply the tile
+// over every other chunk of K, so that each SIMD has two wavefronts, one issuing while the other waits, and are summed at the
+// end through LDS (1.2 us, and twice the first loads). 16-bit operands, 128x128: 784 x 4112 x 4096 33.4 -> 31.9 us (8x8x4
+// tiles 32.4 -> 30.4, bf16 output 33.8 -> 30.4), 640 x 4000 x 4096 31.2 -> 27.8, 512 x 5008 x 4000 31.0 -> 26.8, 1504^2 x 3008 24.4 ->
+// 21.3, 2048^2 x 3712 34.0 -> 32.3, x 6144 53.3 -> 49.7. The fewer tiles there are the less
+// K it takes, the clock being higher: 160 tiles gain 4 % at 64 chunks, 231 lose up to 5 there and gain 2.5 at 80 to 96, 256
+// lose up to 4 at 96 and gain 1.5 to 4 at 112. int4, 64x128: 1 to 4 % at 64 chunks, 6 % at 128 (256 x 8192 x 8192 26.3 -> 24.8;
+// 56 chunks -2 to +2 %); 128x128 gains nothing below 96 chunks and 1 to 3 % there, int8 loses up to 14 %: not taken.
+inline bool two_groups(const MfmaArgs& m, bool rhs_i4, int block_rows, int block_cols) {
+  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
+  const int64_t tiles = ((rows + block_rows - 1) / block_rows) * ((cols + block_cols - 1) / block_cols);
+  return tiles <= 256 && m.chunks >= 64 && (rhs_i4 || 2 * m.chunks >= tiles - 32);
+}
+
 template <int KIND, bool RHS_I4, int G, bool NARROW>
 hipError_t launch_variant(const MfmaArgs& m, hipStream_t stream, const char** name) {
   const bool direct = direct_covers<RHS_I4, G>(m);
@@ -2043,6 +2113,9 @@ hipError_t launch_variant(const MfmaArgs& m, hipStream_t stream, const char** na
       if constexpr (!RHS_I4 && KIND != kF32) {
         if (direct && streams_operands(m, 128, 128)) return launch_direct<KIND, RHS_I4, NARROW, G, 2, 2, 10>(m, stream);
       }
+      if constexpr (G != 2 && (KIND == kF16 || KIND == kBF16)) {
+        if (direct && two_groups(m, RHS_I4, 128, 128)) return launch_direct<KIND, RHS_I4, NARROW, G, 2, 2, 4, 2>(m, stream);
+      }
       if (direct) return launch_direct<KIND, RHS_I4, NARROW, G, 2, 2, 4>(m, stream);
       return launch_staged<KIND, RHS_I4, NARROW, G, 2, 2, 2>(m, stream);
     // (The conditions are choose_tile's: these shapes are not instantiated where it does not take them.)
@@ -2068,7 +2141,10 @@ hipError_t launch_variant(const MfmaArgs& m, hipStream_t stream, const char** na
       return hipErrorInvalidValue;
     case 5:
       *name = "mmt4d_mfma_64x128";
-      if constexpr (RHS_I4) return launch_direct<KIND, RHS_I4, NARROW, G, 1, 2, 8>(m, stream);
+      if constexpr (RHS_I4) {
+        if (two_groups(m, RHS_I4, 64, 128)) return launch_direct<KIND, RHS_I4, NARROW, G, 1, 2, 8, 2>(m, stream);
+        return launch_direct<KIND, RHS_I4, NARROW, G, 1, 2, 8>(m, stream);
+      }
       [[fallthrough]];
     case 3:
       *name = "mmt4d_mfma_128x64";

@@ -140,8 +140,33 @@ inline bool split_k_covers(const MfmaArgs& m) {
   return rows > 64 && rows <= 128 && cols <= 256 * 64 && row_bytes % 128 == 0 && row_bytes >= 8192;
 }
 
+constexpr TileChoice kBlockTiles[] = {{4, 4, false}, {4, 2, true}, {2, 2, false}, {2, 1, true}, {1, 1, false}, {1, 2, true},
+                                      {3, 3, true},  {2, 3, true}, {3, 2, true},  {4, 3, true}, {3, 4, true}};
+
+// One workgroup per compute unit at most, and K long enough: two groups of four wavefronts with a ring each multiply the tile
+// over every other chunk of K, so that each SIMD has two wavefronts, one issuing while the other waits, and are summed at the
+// end through LDS (1.4 us, and twice the first loads). 128x128 tiles, and 64x128 ones of an int4 rhs: bf16 784 x 4112 x 4096
+// 33.4 -> 31.9 us (8x8x4 tiles 32.4 -> 30.4, bf16 output 33.8 -> 30.4), 512 x 5008 x 4000 31.0 -> 26.8, 1504^2 x 3008 24.4 -> 21.3,
+// 2048^2 x 3712 34.0 -> 32.3, x 6144 53.3 -> 49.7; int8 8x8x8 3064 x 944 x 5232 23.7 -> 20.9; int4 576 x 5104 x 4704 21.6 -> 20.1, 256 x
+// 8192 x 8192 25.9 -> 24.3. The fewer tiles there are the less K it takes, the clock being higher. 16-bit: 1 to 6 % slower at
+// 24 to 35 chunks of K, 3 to 6 % faster at 40 to 50 with up to 220 tiles; with 231 of them up to 5 % slower at 64 and 2.5 %
+// faster at 80, with 256 up to 4 % slower at 96 and 1.5 to 4 % faster at 112. int8 and the 128x128 tile of int4: 3 to 8 % faster
+// from 42 chunks on with up to 170 tiles, 11 % at 82 with 192; 2 % slower at 64 with 231, 1 to 3 % faster at 96 with 256. int4
+// 64x128: level at 36 to 48, 4 to 9 % faster at 54 with 140 tiles, 1 to 4 % at 64 with 256.
+// (2-byte pieces: pairs of fragments, which a group's half does not have whole. f32 is bound by the matrix pipe. Operands from
+// HBM: a ring of ten stages is as fast or faster, 784 x 4112 x 8192 60.2 and 62.8, see streams_operands.)
+inline bool two_groups(const MfmaArgs& m, int kind, bool rhs_i4, int gather, bool direct, const TileChoice& t) {
+  if (!direct || gather == 2 || kind == kF32 || t.bn != 2 || t.am != (rhs_i4 && t.am == 1 ? 1 : 2)) return false;
+  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
+  const int64_t tiles = ((rows + 64 * t.am - 1) / (64 * t.am)) * ((cols + 127) / 128);
+  if (tiles > 256 || m.chunks < 44 || comes_from_hbm((rows * m.lhs_rb + cols * m.rhs_rb) * m.K)) return false;
+  if (t.am == 1) return 2 * (int64_t)m.chunks >= tiles - 128;
+  return kind == kI8 ? 10 * (int64_t)m.chunks >= 7 * (tiles - 100) : 2 * (int64_t)m.chunks >= tiles - 32;
+}
+
 // The tile that a problem takes: the least time for 64 bytes of K per row over all of its workgroups, from the time that
-// one workgroup per compute unit takes and, where two fit a compute unit (LDS: up to 128x128), two beside each other.
+// one workgroup per compute unit takes and, where two fit a compute unit (LDS: up to 128x192), two beside each other; less
+// with two groups of wavefronts (two_groups).
 // Microseconds on the direct-to-LDS kernel, fitted to 24 shapes (M 160..4096, N 464..13952, K 700..8192) with every tile
 // for bf16 / f16 16x16x16, bf16 8x8x4, int8 8x8x4 and 16x16x64, f16 16x16x1 and int8 16x16x2 (2-byte pieces: fragments
 // come in pairs, which an odd number of them does not have), int4 16x16x32. The tile picked is 0.1 to 1.3 % slower in the
@@ -149,8 +174,6 @@ inline bool split_k_covers(const MfmaArgs& m) {
 // matrix pipe whatever the tile, which leaves the number of rounds (in units of a 128x128 tile; the large tiles, which
 // move fewer bytes, are favoured by 10 %).
 // `us_per_chunk`: that least time.
-constexpr TileChoice kBlockTiles[] = {{4, 4, false}, {4, 2, true}, {2, 2, false}, {2, 1, true}, {1, 1, false}, {1, 2, true},
-                                      {3, 3, true},  {2, 3, true}, {3, 2, true},  {4, 3, true}, {3, 4, true}};
 inline int choose_tile(const MfmaArgs& m, int kind, bool rhs_i4, int gather, bool direct, double* us_per_chunk) {
   constexpr int kCount = sizeof kBlockTiles / sizeof kBlockTiles[0];
   // Per class of operands and tile, 0: no such instantiation.
@@ -160,7 +183,8 @@ inline int choose_tile(const MfmaArgs& m, int kind, bool rhs_i4, int gather, boo
                                        {.61f, .40f, .285f, .251f, .25f, 0, 0, 0, 0, .52f, .523f},
                                        {.62f, .324f, .237f, 0, .129f, .172f, 0, 0, .26f, 0, 0},
                                        {3.45f, 1.87f, 1.0f, .53f, .27f, 0, 0, 0, 0, 0, 0}};
-  static const float kTwo[][kCount] = {{0, 0, .345f, .31f, .195f}, {0, 0, .44f, .345f, .23f}, {0, 0, .48f, .52f, .35f},
+  static const float kTwo[][kCount] = {{0, 0, .345f, .31f, .195f, 0, 0, .43f, .43f}, {0, 0, .44f, .345f, .23f, 0, 0, .41f, .41f},
+                                       {0, 0, .48f, .52f, .35f},
                                        {0, 0, .345f, 0, .195f, .263f}, {0, 0, 2.0f, 1.06f, .54f}};
   const int what = kind == kF32 ? kFloat32 : rhs_i4 ? kInt4 : gather == 2 ? kTwoBytePieces : kind == kI8 ? kInt8 : kSixteenBit;
   const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
@@ -176,7 +200,9 @@ inline int choose_tile(const MfmaArgs& m, int kind, bool rhs_i4, int gather, boo
     const int64_t br = 64 * t.am, bc = 64 * t.bn;
     const int64_t rounds = (((rows + br - 1) / br) * ((cols + bc - 1) / bc) + 255) / 256;
     const double one = kOne[what][i], two = kTwo[what][i];
-    const double cost = two > 0 ? (rounds & 1) * one + (rounds >> 1) * two : rounds * one;
+    double cost = two > 0 ? (rounds & 1) * one + (rounds >> 1) * two : rounds * one;
+    if (two_groups(m, kind, rhs_i4, gather, direct, t))
+      cost = t.am == 1 ? .84 * one + 1.0 / m.chunks : .78 * one + 1.4 / m.chunks;
     if (best < 0 || cost < best_cost) {
       best = i;
       best_cost = cost;
@@ -2072,20 +2098,6 @@ inline bool streams_operands(const MfmaArgs& m, int block_rows, int block_cols) 
   return tiles <= 256 && comes_from_hbm((rows * m.lhs_rb + cols * m.rhs_rb) * m.K);
 }
 
-// One workgroup per compute unit at most, and K long enough: two groups of four wavefronts with a ring each multiply the tile
-// over every other chunk of K, so that each SIMD has two wavefronts, one issuing while the other waits, and are summed at the
-// end through LDS (1.2 us, and twice the first loads). 16-bit operands, 128x128: 784 x 4112 x 4096 33.4 -> 31.9 us (8x8x4
-// tiles 32.4 -> 30.4, bf16 output 33.8 -> 30.4), 640 x 4000 x 4096 31.2 -> 27.8, 512 x 5008 x 4000 31.0 -> 26.8, 1504^2 x 3008 24.4 ->
-// 21.3, 2048^2 x 3712 34.0 -> 32.3, x 6144 53.3 -> 49.7. The fewer tiles there are the less
-// K it takes, the clock being higher: 160 tiles gain 4 % at 64 chunks, 231 lose up to 5 there and gain 2.5 at 80 to 96, 256
-// lose up to 4 at 96 and gain 1.5 to 4 at 112. int4, 64x128: 1 to 4 % at 64 chunks, 6 % at 128 (256 x 8192 x 8192 26.3 -> 24.8;
-// 56 chunks -2 to +2 %); 128x128 gains nothing below 96 chunks and 1 to 3 % there, int8 loses up to 14 %: not taken.
-inline bool two_groups(const MfmaArgs& m, bool rhs_i4, int block_rows, int block_cols) {
-  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
-  const int64_t tiles = ((rows + block_rows - 1) / block_rows) * ((cols + block_cols - 1) / block_cols);
-  return tiles <= 256 && m.chunks >= 64 && (rhs_i4 || 2 * m.chunks >= tiles - 32);
-}
-
 template <int KIND, bool RHS_I4, int G, bool NARROW>
 hipError_t launch_variant(const MfmaArgs& m, hipStream_t stream, const char** name) {
   const bool direct = direct_covers<RHS_I4, G>(m);
@@ -2113,8 +2125,9 @@ hipError_t launch_variant(const MfmaArgs& m, hipStream_t stream, const char** na
       if constexpr (!RHS_I4 && KIND != kF32) {
         if (direct && streams_operands(m, 128, 128)) return launch_direct<KIND, RHS_I4, NARROW, G, 2, 2, 10>(m, stream);
       }
-      if constexpr (G != 2 && (KIND == kF16 || KIND == kBF16)) {
-        if (direct && two_groups(m, RHS_I4, 128, 128)) return launch_direct<KIND, RHS_I4, NARROW, G, 2, 2, 4, 2>(m, stream);
+      if constexpr (G != 2 && KIND != kF32) {
+        if (two_groups(m, KIND, RHS_I4, G, direct, kBlockTiles[2]))
+          return launch_direct<KIND, RHS_I4, NARROW, G, 2, 2, 4, 2>(m, stream);
       }
       if (direct) return launch_direct<KIND, RHS_I4, NARROW, G, 2, 2, 4>(m, stream);
       return launch_staged<KIND, RHS_I4, NARROW, G, 2, 2, 2>(m, stream);
@@ -2142,7 +2155,8 @@ hipError_t launch_variant(const MfmaArgs& m, hipStream_t stream, const char** na
     case 5:
       *name = "mmt4d_mfma_64x128";
       if constexpr (RHS_I4) {
-        if (two_groups(m, RHS_I4, 64, 128)) return launch_direct<KIND, RHS_I4, NARROW, G, 1, 2, 8, 2>(m, stream);
+        if (two_groups(m, KIND, RHS_I4, G, direct, kBlockTiles[5]))
+          return launch_direct<KIND, RHS_I4, NARROW, G, 1, 2, 8, 2>(m, stream);
         return launch_direct<KIND, RHS_I4, NARROW, G, 1, 2, 8>(m, stream);
       }
       [[fallthrough]];

@@ -14,6 +14,7 @@
 // Covers s8s8s32, f16f16f32 and bf16bf16f32 with N0 = 16 and 16, 32 or 64
 // bytes per (k, row) piece, and s8s4s32 (int4 weights) with N0 = 16 and
 // K0 = 32 or 64 (mmt4d_gemv_i4_kernel below).
+#include "uk_device.h"
 #include "uk_internal.h"
 
 namespace uk {
@@ -37,6 +38,10 @@ struct GemvArgs {
   int32_t rb, log2_rb;  // bytes of one (k, row) piece
   int32_t steps;        // MFMA K-steps: ceil(K * rb / 64); int4: whole ones of 128 values
   int32_t accumulate;
+  // The kernels of one workgroup per unit: how many there are, its reciprocal (divide), and whether each has as many whole tiles.
+  int32_t units;
+  uint32_t units_reciprocal;
+  int32_t rounds;
 };
 
 template <int KIND> struct Acc { typedef v4i32 type; };
@@ -167,6 +172,35 @@ __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_kernel(const GemvArgs 
   *dst = acc;
 }
 
+// Some value, at no instruction's cost.
+__device__ __forceinline__ void any_value(uint4* v) {
+  v4i32 some;
+  asm volatile("" : "=v"(some));
+  *v = __builtin_bit_cast(uint4, some);
+}
+
+// All of them are needed at once: in one trip to memory, not in two.
+__device__ __forceinline__ void fetch_arguments(const GemvArgs& a) {
+  asm volatile("" ::"s"(a.lhs), "s"(a.rhs), "s"(a.lhs_stride_bytes), "s"(a.rhs_stride_bytes), "s"(a.M), "s"(a.N), "s"(a.log2_M0),
+               "s"(a.rb), "s"(a.log2_rb), "s"(a.units), "s"(a.units_reciprocal), "s"(a.rounds));
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// The half tiles of the rhs that a workgroup of a.units takes, as even shares as whole ones make. (64-bit divisions, and the
+// number of workgroups read from the launch's own record, were 300 of the 550 instructions in front of the first load.)
+struct Halves {
+  uint32_t first, end;
+};
+__device__ __forceinline__ Halves halves_of(const GemvArgs& a) {
+  const uint32_t n = blockIdx.x * (2 * (uint32_t)a.N);  // (at most 8 tiles for each of some hundred units)
+  return Halves{divide(n, (uint32_t)a.units, a.units_reciprocal), divide(n + 2 * (uint32_t)a.N, (uint32_t)a.units, a.units_reciprocal)};
+}
+void set_units(GemvArgs* g, int units) {
+  g->units = units;
+  g->units_reciprocal = reciprocal_of((uint32_t)units);
+  g->rounds = g->N % units == 0;
+}
+
 // The same product for more than 4 lhs rows, where the lhs operand of a K-step
 // is as large as a rhs tile's (1 KiB) and the kernel above pulls all of it
 // through L2 again for every rhs tile. Here one workgroup per compute unit
@@ -177,8 +211,8 @@ __global__ __launch_bounds__(64 * kWaves) void mmt4d_gemv_kernel(const GemvArgs 
 // The rhs is dealt out in HALF tiles (rhs rows 0-7 or 8-15 of a tile: 128
 // contiguous bytes of every k step for 16-byte row pieces) so that every unit
 // gets the same number of bytes also when tiles / units is not whole (896 tiles
-// on 256 units: 3.5); a half tile is a tile with half the lanes' loads masked,
-// its missing rows multiply as zeros and are not stored. Partial sums meet in
+// on 256 units: 3.5); a half tile is a tile with half the lanes' loads masked, whose
+// missing rows' columns are not stored. Partial sums meet in
 // LDS in wavefront order: results do not depend on scheduling.
 // Needs steps == kWaves * UNROLL (one batch of loads per wavefront and tile).
 template <int KIND, int kWaves, int UNROLL, int MAX_TILES>
@@ -188,47 +222,48 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(UNR
 void mmt4d_gemv_resident_lhs_kernel(const GemvArgs a) {
   typedef typename Acc<KIND>::type acc_t;
   extern __shared__ uint4 gemv_lds[];  // [kWaves][UNROLL][64] lhs operands; then [MAX_TILES][kWaves][64] partial sums
+  fetch_arguments(a);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row = lane & 15, g = lane >> 4;
   const int32_t M0 = 1 << a.log2_M0;
   const int32_t lhs_rows = a.M << a.log2_M0;  // <= 16
 
   // This unit's range of half tiles.
-  const int64_t halves = 2 * (int64_t)a.N;
-  const int64_t h0 = (int64_t)blockIdx.x * halves / gridDim.x, h1 = ((int64_t)blockIdx.x + 1) * halves / gridDim.x;
+  const Halves own = halves_of(a);
+  const uint32_t h0 = own.first, h1 = own.end;
   if (h1 <= h0) return;
   const int64_t t0 = h0 >> 1, t1 = (h1 - 1) >> 1;
   const int tiles = (int)(t1 - t0 + 1);  // <= MAX_TILES (checked on the host)
   const bool skip_low_half_of_first = h0 & 1, skip_high_half_of_last = h1 & 1;
-  // When every unit gets whole tiles and equally many, it takes one of every round of gridDim.x tiles instead of
+  // When every unit gets whole tiles and equally many, it takes one of every round of a.units tiles instead of
   // its range: ranges of 4 tiles of 128 KiB put the units' streams 512 KiB apart, a power of two that the memory
   // channels do not like (16 x 16384 x 4096 bf16: 5.59 -> 5.80 TB/s; with half tiles in play the ranges are the
   // faster deal, 5.83 against 5.67 at 14336).
-  const bool rounds = a.N % gridDim.x == 0;
-  auto tile_of = [&](int u) -> int64_t { return rounds ? blockIdx.x + (int64_t)gridDim.x * u : t0 + u; };
+  const int64_t first_tile = a.rounds ? blockIdx.x : t0, tile_step = a.rounds ? a.units : 1;
+  auto tile_of = [&](int u) -> int64_t { return first_tile + tile_step * u; };
 
-  const int32_t ksteps_per_step = 64 >> a.log2_rb;
   const int32_t k1_lane = (16 * g) >> a.log2_rb;
   const int32_t within = (16 * g) & (a.rb - 1);
-  const int64_t rhs_kstep = (int64_t)a.rb * 16;
-  const int64_t lhs_kstep = (int64_t)a.rb << a.log2_M0;
   const bool lhs_valid = row < lhs_rows;
-  const int64_t k1_first = (int64_t)(wave * UNROLL) * ksteps_per_step;  // this wavefront's share of K
+  const int32_t first_step = wave * UNROLL;  // this wavefront's share of K: 128 steps at most, 32-bit offsets
   const uint8_t* lhs_lane = a.lhs + (int64_t)(row >> a.log2_M0) * a.lhs_stride_bytes +
-                            (int64_t)(row & (M0 - 1)) * a.rb + (k1_lane + k1_first) * lhs_kstep + within;
-  const uint8_t* rhs_lane = a.rhs + (int64_t)row * a.rb + (k1_lane + k1_first) * rhs_kstep + within;
-  const int64_t rhs_step_bytes = ksteps_per_step * rhs_kstep, lhs_step_bytes = ksteps_per_step * lhs_kstep;
+                            (uint32_t)(((row & (M0 - 1)) << a.log2_rb) + (k1_lane << (a.log2_rb + a.log2_M0)) + within +
+                                       (first_step * 64 << a.log2_M0));
+  const uint8_t* rhs_lane = a.rhs + (uint32_t)((row << a.log2_rb) + (k1_lane << (a.log2_rb + 4)) + within + first_step * 1024);
+  constexpr int32_t rhs_step_bytes = 1024;
+  const int64_t lhs_step_bytes = (int64_t)64 << a.log2_M0;
 
   auto tile_rows_loaded = [&](int u) -> bool {
     if (u == 0 && skip_low_half_of_first && row < 8) return false;
     if (u == tiles - 1 && skip_high_half_of_last && row >= 8) return false;
     return true;
   };
-  // (Lanes whose rows of a half tile belong to another unit load nothing and keep what they held: rhs row n only
-  // ever reaches column n of the result, and those columns are not stored.)
+  // (Lanes whose rows of a half tile belong to another unit load nothing and keep what they held, whatever that is: rhs row n
+  // only ever reaches column n of the result, and those columns are not stored. Zeros here were 128 instructions in front of
+  // the first load; loads of the other half's rows instead cost 2 % where half tiles are many, 11008 x 8192.)
   uint4 r[2][UNROLL];
 #pragma unroll
-  for (int s = 0; s < UNROLL; ++s) r[0][s] = r[1][s] = make_uint4(0, 0, 0, 0);
+  for (int s = 0; s < UNROLL; ++s) any_value(&r[0][s]), any_value(&r[1][s]);
   auto fetch = [&](int u, uint4* dst) {
     const uint8_t* p = rhs_lane + tile_of(u) * a.rhs_stride_bytes;
     const bool loaded = tile_rows_loaded(u);
@@ -449,6 +484,7 @@ template <int kWaves, int UNROLL, int MAX_TILES>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4, 4)))  // (128 registers, as with 16 wavefronts)
 void mmt4d_gemv_i4_resident_lhs_kernel(const GemvArgs a) {
   extern __shared__ uint4 gemv_lds[];  // [kWaves][UNROLL][2][64] lhs operands; then [MAX_TILES][kWaves][64] partial sums
+  fetch_arguments(a);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row = lane & 15, g = lane >> 4;
   const int32_t M0 = 1 << a.log2_M0;
@@ -457,8 +493,8 @@ void mmt4d_gemv_i4_resident_lhs_kernel(const GemvArgs a) {
   const int64_t lhs_kstep = (int64_t)a.rb << a.log2_M0;
   const int64_t lhs_step_bytes = (int64_t)128 << a.log2_M0;
 
-  const int64_t halves = 2 * (int64_t)a.N;
-  const int64_t h0 = (int64_t)blockIdx.x * halves / gridDim.x, h1 = ((int64_t)blockIdx.x + 1) * halves / gridDim.x;
+  const Halves own = halves_of(a);
+  const uint32_t h0 = own.first, h1 = own.end;
   if (h1 <= h0) return;
   const int64_t t0 = h0 >> 1, t1 = (h1 - 1) >> 1;
   const int tiles = (int)(t1 - t0 + 1);  // <= MAX_TILES (checked on the host)
@@ -485,7 +521,7 @@ void mmt4d_gemv_i4_resident_lhs_kernel(const GemvArgs a) {
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d)
 #pragma unroll
-    for (int s = 0; s < UNROLL; ++s) r[d][s] = make_uint4(0, 0, 0, 0);
+    for (int s = 0; s < UNROLL; ++s) any_value(&r[d][s]);
   auto fetch = [&](int u, uint4* dst) {
     const uint8_t* p = rhs_lane + (int64_t)u * a.rhs_stride_bytes;
     const bool loaded = tile_rows_loaded(u);
@@ -597,6 +633,9 @@ bool make_args(const Mmt4dArgs& a, bool probe_only, int* kind, GemvArgs* g) {
   g->log2_rb = log2_exact(rb);
   g->steps = i4 ? (int32_t)((int64_t)a.K * a.K0 / 128) : (int32_t)(((int64_t)a.K * rb + 63) / 64);
   g->accumulate = (a.flags & IREE_UK_FLAG_MMT4D_ACCUMULATE) ? 1 : 0;
+  g->units = 0;
+  g->units_reciprocal = 0;
+  g->rounds = 0;
   return true;
 }
 
@@ -639,7 +678,9 @@ bool launch_resident_lhs(const GemvArgs& g, hipStream_t stream, hipError_t* stat
     int used = units;
     for (int u = units; u >= units - units / 16; --u)
       if (g.N % u == 0) { used = u; break; }
-    *status = launch_kernel<GemvArgs>(kernel, used, 64 * waves, lds_bytes, stream, g);
+    GemvArgs with_units = g;
+    set_units(&with_units, used);
+    *status = launch_kernel<GemvArgs>(kernel, used, 64 * waves, lds_bytes, stream, with_units);
   };
   // (8 wavefronts with 16 loads each in flight twice over; 16 wavefronts x 8 measured no better than the kernel above.)
   switch (g.steps) {
@@ -696,6 +737,7 @@ hipError_t launch_gemv(const Mmt4dArgs& a, hipStream_t stream, const char** name
       const hipError_t attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
       if (attr != hipSuccess) return attr;
       *name = "mmt4d_gemv_resident_lhs";
+      set_units(&g, units);
       return launch_kernel(kernel, units, g.steps == 64 ? 1024 : 512, lds_bytes, stream, g);
     }
     // Otherwise four wavefronts with six steps' loads in flight, or four steps' where that is all a wavefront has (1 x 25168

@@ -769,6 +769,14 @@ __device__ __forceinline__ uint32_t value_bits(float v) { return __float_as_uint
 __device__ __forceinline__ void set_from_bits(int32_t& v, uint32_t bits) { v = (int32_t)bits; }
 __device__ __forceinline__ void set_from_bits(float& v, uint32_t bits) { v = __uint_as_float(bits); }
 
+// What a step of the kernel below takes its place from.
+template <typename Read, typename Load, typename Advance>
+struct StepPlace {
+  Read read_from;
+  Load load;
+  Advance advance;
+};
+
 // f(0), .. f(N - 1), each number a type of its own.
 template <int N, typename F>
 __device__ __forceinline__ void each_of(F f) {
@@ -1036,20 +1044,26 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     if constexpr (A_LOADS == 2) a_off[0] += 1024;  // (see load_two_to_lds; the bases are 1 KiB lower)
     if constexpr (B_LOADS == 2) b_off[0] += 1024;
   }
-  auto issue_load = [&](auto number, uint32_t stage_off, const uint8_t* la, const uint8_t* lb) {
+  // (`further`: bytes from that stage to the one meant; a, b: per-lane offsets.)
+  auto issue_load_to = [&](auto number, auto further, uint32_t stage_off, uint32_t b_stage_off, const uint32_t* a, const uint32_t* b,
+                           const uint8_t* la, const uint8_t* lb) {
     constexpr int n = decltype(number)::value;
+    constexpr uint32_t FURTHER = decltype(further)::value;
     if constexpr (TOGETHER) {
       if constexpr (n == 0) {
-        if constexpr (A_LOADS == 2) load_two_to_lds<0>(stage_off, a_off[0], a_off[1], la);
-        else load_to_lds(stage_off, a_off[0], la);
+        if constexpr (A_LOADS == 2) load_two_to_lds<FURTHER>(stage_off, a[0], a[1], la);
+        else load_to_lds<FURTHER>(stage_off, a[0], la);
       } else {
-        if constexpr (B_LOADS == 2) load_two_to_lds<0>(stage_off + b_from_a, b_off[0], b_off[1], lb);
-        else load_to_lds(stage_off + b_from_a, b_off[0], lb);
+        if constexpr (B_LOADS == 2) load_two_to_lds<FURTHER>(b_stage_off, b[0], b[1], lb);
+        else load_to_lds<FURTHER>(b_stage_off, b[0], lb);
       }
     } else {
-      if constexpr (n < A_LOADS) load_to_lds<4096 * n>(stage_off, a_off[n], la);
-      else load_to_lds<16 * A_PIECES + 4096 * (n - A_LOADS)>(stage_off, b_off[n - A_LOADS], lb);
+      if constexpr (n < A_LOADS) load_to_lds<FURTHER + 4096 * n>(stage_off, a[n], la);
+      else load_to_lds<FURTHER + 16 * A_PIECES + 4096 * (n - A_LOADS)>(stage_off, b[n - A_LOADS], lb);
     }
+  };
+  auto issue_load = [&](auto number, uint32_t stage_off, const uint8_t* la, const uint8_t* lb) {
+    issue_load_to(number, std::integral_constant<uint32_t, 0>(), stage_off, stage_off + b_from_a, a_off, b_off, la, lb);
   };
   const uint8_t* lhs_from = lhs_base - (TOGETHER && A_LOADS == 2 ? 1024 : 0);
   const uint8_t* rhs_from = rhs_base - (TOGETHER && B_LOADS == 2 ? 1024 : 0);
@@ -1064,8 +1078,10 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   // The group's ring.
   const uint32_t ring_off = (uint32_t)group * (STAGES * STAGE_PIECES * 16);
   const uint4* const own_ring = ring + ring_off / 16;
+  // Chunk c lies in stage c - 1 modulo their number: what step kc reads is in stage kc.
+  const uint4* const first_stage = own_ring + (STAGES - 1) * STAGE_PIECES;
   auto issue_chunk = [&](int kc) {
-    const uint32_t stage_off = ring_off + (uint32_t)(kc % STAGES) * (STAGE_PIECES * 16) + 1024 * a_number(0);
+    const uint32_t stage_off = ring_off + (uint32_t)((kc + STAGES - 1) % STAGES) * (STAGE_PIECES * 16) + 1024 * a_number(0);
     const uint8_t* la = lhs_near(kc);
     const uint8_t* lb = rhs_near(kc);
     each_of<ISSUES>([&](auto n) { issue_load(n, stage_off, la, lb); });
@@ -1104,21 +1120,21 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   // Fragment f of an operand at 16-byte slot `operand` of the ring, K-step kk.
   auto read_frag = [&](int operand, int f, int kk) -> uint4 {
     if (RHS_I4 && operand >= A_PIECES) {
-      const uint4 raw = own_ring[operand + 64 * f + lane];
+      const uint4 raw = first_stage[operand + 64 * f + lane];
       return widen_i4_times16(kk ? make_uint2(raw.z, raw.w) : make_uint2(raw.x, raw.y));
     }
     if constexpr (G == 16) {
       if (!RHS_I4 && (operand == 0 ? lhs_by_rows : rhs_by_rows))
-        return own_ring[operand + 128 * f + 64 * ((lane & 31) >> 4) + 4 * (lane & 15) + ((2 * kk + (lane >> 5)) ^ ((lane >> 2) & 3))];
-      if (!RHS_I4) return own_ring[operand + 128 * f + 32 * kk + 64 * ((lane & 31) >> 4) + 16 * (lane >> 5) + (lane & 15)];
-      return own_ring[operand + 128 * f + 64 * kk + lane];
+        return first_stage[operand + 128 * f + 64 * ((lane & 31) >> 4) + 4 * (lane & 15) + ((2 * kk + (lane >> 5)) ^ ((lane >> 2) & 3))];
+      if (!RHS_I4) return first_stage[operand + 128 * f + 32 * kk + 64 * ((lane & 31) >> 4) + 16 * (lane >> 5) + (lane & 15)];
+      return first_stage[operand + 128 * f + 64 * kk + lane];
     } else if constexpr (G == 1) {
-      const uint8_t* first = (const uint8_t*)(own_ring + operand) + 2048 * f + 512 * kk +
+      const uint8_t* first = (const uint8_t*)(first_stage + operand) + 2048 * f + 512 * kk +
                              transposed_lane_offset(operand >= A_PIECES ? a.log2_N0 : a.log2_M0);
       const uint2 lo = lds_read_transposed(first), hi = lds_read_transposed(first + 128);
       return make_uint4(lo.x, lo.y, hi.x, hi.y);
     } else {
-      const uint8_t* first = (const uint8_t*)(own_ring + operand) + 1024 * (2 * f + kk) +
+      const uint8_t* first = (const uint8_t*)(first_stage + operand) + 1024 * (2 * f + kk) +
                              (G == 4 ? dwords_lane_offset(operand >= A_PIECES ? a.log2_N0 : a.log2_M0) : G * lane);
       return make_uint4(gather_dword(first, 0), gather_dword(first, 1), gather_dword(first, 2), gather_dword(first, 3));
     }
@@ -1147,8 +1163,8 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   const uint8_t* load_b = rhs_near(AHEAD);
   int load_chunk = AHEAD;
   const uint32_t load_ring_begin = ring_off + 1024 * a_number(0), load_ring_end = RING_BYTES + load_ring_begin;
-  uint32_t load_stage_off = AHEAD * STAGE_BYTES % RING_BYTES + load_ring_begin;
-  uint32_t read_stage_off = STAGE_BYTES;
+  uint32_t load_stage_off = (STAGES - 2) * STAGE_BYTES + load_ring_begin;
+  uint32_t read_stage_off = 0;
   const uint32_t frag_a_off = (uint32_t)((wave_m * AM) * 128) * 16;
   const uint32_t frag_b_off = (uint32_t)(A_PIECES + (wave_n * BN) * (RHS_I4 ? 64 : 128)) * 16;
   // Lane 32*h + r's byte offset into a fragment, and the slots from one K-step
@@ -1222,8 +1238,9 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   // (`held_loads_behind`: the eight loads of destination values that variant 3 issues at the start of a phase
   // are younger than the chunk this step waits for, and may stay in flight with it.)
   // `between_mfmas(m)`: extra work placed behind MFMA m of the step (variant 3 adds destination values there).
-  auto step_with = [&](const uint4 (*cur_a)[2], const uint4 (*cur_b)[2], uint4 (*nxt_a)[2], uint4 (*nxt_b)[2],
-                       bool held_loads_behind, auto between_mfmas) {
+  // `place`: where this step's loads go and its fragments come from, and what follows it.
+  auto step_at = [&](const uint4 (*cur_a)[2], const uint4 (*cur_b)[2], uint4 (*nxt_a)[2], uint4 (*nxt_b)[2],
+                     bool held_loads_behind, auto between_mfmas, auto place) {
     constexpr int SUB = SubSteps<KIND>::value;
     constexpr int MFMAS = 2 * AM * BN * SUB;
     // Units a fragment's LDS reads are dealt out in: a 128-bit read; two pairs of
@@ -1290,10 +1307,9 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       wait_loads_but<LOADS*(AHEAD - 2)>();
     }
     __builtin_amdgcn_s_barrier();
-    const uint8_t* read_a = ring_bytes + read_stage_off + frag_a_off + pair_a_lane;
-    const uint8_t* read_a_kk1 = read_a + lhs_kk1_step;  // (used where the lhs has 16-byte pieces)
-    const uint8_t* read_b = ring_bytes + read_stage_off + frag_b_off + pair_b_lane;
-    const uint8_t* read_b_kk1 = read_b + rhs_kk1_step;
+    // (K-step 1 of either: used where it has 16-byte pieces)
+    const uint8_t *read_a, *read_a_kk1, *read_b, *read_b_kk1;
+    place.read_from(&read_a, &read_a_kk1, &read_b, &read_b_kk1);
     uint4 raw_b[RHS_I4 ? BN : 1];
 #pragma unroll
     for (int m = LEAD; m < MFMAS; ++m) {
@@ -1301,7 +1317,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       if (slot < SLOTS) {
         each_of<ISSUES>([&](auto n) {
           if (n.value >= slot * ISSUES / SLOTS && n.value < (slot + 1) * ISSUES / SLOTS)
-            issue_load(n, load_stage_off, load_a, load_b);
+            place.load(n);
         });
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1363,18 +1379,31 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       split_units_of(slot - SPLIT_DELAY);
       multiply(m);
       between_mfmas(m);
-      if (m == MFMAS - 1) {
-        // Advance the running state (clamped at the last chunk: the loads
-        // issued beyond it are redundant, their stages are never read).
-        const bool more = load_chunk < last_chunk;
-        load_a += (uint32_t)(more ? GROUPS * lhs_chunk_bytes : 0);
-        load_b += (uint32_t)(more ? GROUPS * rhs_chunk_bytes : 0);
-        ++load_chunk;
-        load_stage_off = load_stage_off + STAGE_BYTES == load_ring_end ? load_ring_begin : load_stage_off + STAGE_BYTES;
-        read_stage_off = read_stage_off + STAGE_BYTES == RING_BYTES ? 0 : read_stage_off + STAGE_BYTES;
-      }
+      if (m == MFMAS - 1) place.advance();
       __builtin_amdgcn_sched_barrier(0);
     }
+  };
+  // A step anywhere: all of that is running state, advanced by the step (clamped at the last chunk: the loads issued beyond
+  // it are redundant, their stages are never read).
+  auto running_read = [&](const uint8_t** read_a, const uint8_t** read_a_kk1, const uint8_t** read_b, const uint8_t** read_b_kk1) {
+    *read_a = ring_bytes + read_stage_off + frag_a_off + pair_a_lane;
+    *read_a_kk1 = *read_a + lhs_kk1_step;
+    *read_b = ring_bytes + read_stage_off + frag_b_off + pair_b_lane;
+    *read_b_kk1 = *read_b + rhs_kk1_step;
+  };
+  auto running_load = [&](auto n) { issue_load(n, load_stage_off, load_a, load_b); };
+  auto running_advance = [&]() {
+    const bool more = load_chunk < last_chunk;
+    load_a += (uint32_t)(more ? GROUPS * lhs_chunk_bytes : 0);
+    load_b += (uint32_t)(more ? GROUPS * rhs_chunk_bytes : 0);
+    ++load_chunk;
+    load_stage_off = load_stage_off + STAGE_BYTES == load_ring_end ? load_ring_begin : load_stage_off + STAGE_BYTES;
+    read_stage_off = read_stage_off + STAGE_BYTES == RING_BYTES ? 0 : read_stage_off + STAGE_BYTES;
+  };
+  auto step_with = [&](const uint4 (*cur_a)[2], const uint4 (*cur_b)[2], uint4 (*nxt_a)[2], uint4 (*nxt_b)[2],
+                       bool held_loads_behind, auto between_mfmas) {
+    step_at(cur_a, cur_b, nxt_a, nxt_b, held_loads_behind, between_mfmas,
+            StepPlace<decltype(running_read), decltype(running_load), decltype(running_advance)>{running_read, running_load, running_advance});
   };
   auto step = [&](const uint4 (*cur_a)[2], const uint4 (*cur_b)[2], uint4 (*nxt_a)[2], uint4 (*nxt_b)[2],
                   bool held_loads_behind = false) {
@@ -1609,7 +1638,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
 #pragma unroll
           for (int part = 0; part < 4; ++part)
             split_pair_part(
-                read_pair_part((const uint8_t*)(own_ring + A_PIECES) + 2048 * (frag_b0 + j) + 2048 * kk + 4 * lane, part),
+                read_pair_part((const uint8_t*)(first_stage + A_PIECES) + 2048 * (frag_b0 + j) + 2048 * kk + 4 * lane, part),
                 part, pb[j][kk], pb[j + 1][kk]);
         }
       } else {
@@ -1622,7 +1651,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
         if (i % 2 == 0) {
 #pragma unroll
           for (int part = 0; part < 4; ++part)
-            split_pair_part(read_pair_part((const uint8_t*)own_ring + 2048 * (frag_a0 + i) + 2048 * kk + 4 * lane, part),
+            split_pair_part(read_pair_part((const uint8_t*)first_stage + 2048 * (frag_a0 + i) + 2048 * kk + 4 * lane, part),
                             part, pa[i][kk], pa[i + 1][kk]);
         }
       } else {
@@ -1715,6 +1744,69 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     UK_TIMELINE(tl_loop_end = __builtin_amdgcn_s_memrealtime();)
     tail(pa, pb);
     return;
+  }
+  // Four steps at a time while all of their loads are of chunks that exist: where a step reads and loads is then a constant
+  // beyond one base each, and the four chunks' offsets are registers. 28 instructions a step of the 128x64 tile where a step
+  // anywhere has 46, 21 of 38 for 64x64, 64 of 80 for 64x128 and an int4 rhs. bf16 8x8x4 512 x 4096 x 4096 24.3 -> 22.4 us,
+  // 16x16x16 22.8 -> 22.0, int8 16x16x2 19.2 -> 18.2, int4 256 x 8000 x 3008 13.0 -> 12.4, 784 x 4112 x 4096 (128x128) 21.4 -> 21.0.
+  // Not for a K of few rounds, which the preparation costs 1 %, nor where it was level: 4-byte pieces of int8 (128x64 -4 to
+  // +2 %) and the 128x128 tile of others, bound by the LDS (-2 to +2 %).
+  constexpr bool BY_FOUR = STAGES % 4 == 0 && KIND != kF32 && (RHS_I4 ? AM * BN <= 4 : AM * BN <= 2 && !(KIND == kI8 && G == 4));
+  if constexpr (BY_FOUR) if (last_chunk >= AHEAD + 8) {
+    constexpr uint32_t FOUR = 4 * STAGE_BYTES;
+    uint32_t fast_a[4][A_LOADS], fast_b[4][B_LOADS];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int t = 0; t < A_LOADS; ++t) fast_a[c][t] = a_off[t] + c * GROUPS * lhs_chunk_bytes;
+#pragma unroll
+      for (int t = 0; t < B_LOADS; ++t) fast_b[c][t] = b_off[t] + c * GROUPS * rhs_chunk_bytes;
+    }
+    // LDS offsets of the four stages that this round reads, whose last two steps load into the first two of them, and of
+    // those before, which the first two load into (four stages: the same).
+    uint32_t this_four = load_ring_begin, other_four = load_ring_begin + (STAGES == 4 ? 0 : FOUR);
+    static_assert(STAGES == 4 || STAGES == 8, "two fours at most");
+    const uint8_t* from_a = ring_bytes + frag_a_off + pair_a_lane;
+    const uint8_t* from_b = ring_bytes + frag_b_off + pair_b_lane;
+    while (kc + 3 + AHEAD <= last_chunk) {
+      const uint32_t read_off = this_four - load_ring_begin;
+      const uint8_t* base_a = from_a + read_off;
+      const uint8_t* base_b = from_b + read_off;
+      const uint8_t *base_a_kk1 = base_a + lhs_kk1_step, *base_b_kk1 = base_b + rhs_kk1_step;
+      each_of<4>([&](auto number) {
+        constexpr int S = decltype(number)::value;
+        auto read = [&](const uint8_t** read_a, const uint8_t** read_a_kk1, const uint8_t** read_b, const uint8_t** read_b_kk1) {
+          *read_a = base_a + S * STAGE_BYTES;
+          *read_a_kk1 = base_a_kk1 + S * STAGE_BYTES;
+          *read_b = base_b + S * STAGE_BYTES;
+          *read_b_kk1 = base_b_kk1 + S * STAGE_BYTES;
+        };
+        auto load = [&](auto n) {
+          const uint32_t four = S < 2 ? other_four : this_four;
+          issue_load_to(n, std::integral_constant<uint32_t, ((S + 2) % 4) * STAGE_BYTES>(), four, four + b_from_a, fast_a[S],
+                        fast_b[S], load_a, load_b);
+        };
+        auto advance = [] {};
+        StepPlace<decltype(read), decltype(load), decltype(advance)> place{read, load, advance};
+        if constexpr (S % 2 == 0) step_at(pa, pb, qa, qb, false, [](int) {}, place);
+        else step_at(qa, qb, pa, pb, false, [](int) {}, place);
+      });
+      kc += 4;
+      load_a += (uint32_t)(4 * GROUPS * lhs_chunk_bytes);
+      load_b += (uint32_t)(4 * GROUPS * rhs_chunk_bytes);
+      if constexpr (STAGES == 8) {
+        const uint32_t was = this_four;
+        this_four = other_four;
+        other_four = was;
+      }
+    }
+    load_chunk = kc + AHEAD;
+    // (The chunk after the last one, if the rounds came that far, is the last one again.)
+    const bool beyond = kc > 0 && load_chunk > last_chunk;
+    load_a -= (uint32_t)(beyond ? GROUPS * lhs_chunk_bytes : 0);
+    load_b -= (uint32_t)(beyond ? GROUPS * rhs_chunk_bytes : 0);
+    read_stage_off = this_four - load_ring_begin;
+    load_stage_off = other_four + 2 * STAGE_BYTES;
   }
   for (; kc + 1 < chunks; kc += 2) {
     step(pa, pb, qa, qb);

@@ -1749,9 +1749,9 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   // beyond one base each, and the four chunks' offsets are registers. 28 instructions a step of the 128x64 tile where a step
   // anywhere has 46, 21 of 38 for 64x64, 64 of 80 for 64x128 and an int4 rhs. bf16 8x8x4 512 x 4096 x 4096 24.3 -> 22.4 us,
   // 16x16x16 22.8 -> 22.0, int8 16x16x2 19.2 -> 18.2, int4 256 x 8000 x 3008 13.0 -> 12.4, 784 x 4112 x 4096 (128x128) 21.4 -> 21.0.
-  // Not for a K of few rounds, which the preparation costs 1 %, nor where it was level: 4-byte pieces of int8 (128x64 -4 to
-  // +2 %) and the 128x128 tile of others, bound by the LDS (-2 to +2 %).
-  constexpr bool BY_FOUR = STAGES % 4 == 0 && KIND != kF32 && (RHS_I4 ? AM * BN <= 4 : AM * BN <= 2 && !(KIND == kI8 && G == 4));
+  // Not for a K of few rounds, which the preparation costs 1 %, nor where it was level: int8 but for its 2-byte pieces (128x64
+  // -4 to +4 %) and the 128x128 tile of others, bound by the LDS (-2 to +2 %).
+  constexpr bool BY_FOUR = STAGES % 4 == 0 && KIND != kF32 && (RHS_I4 ? AM * BN <= 4 : AM * BN <= 2 && (KIND != kI8 || G == 2));
   if constexpr (BY_FOUR) if (last_chunk >= AHEAD + 8) {
     constexpr uint32_t FOUR = 4 * STAGE_BYTES;
     uint32_t fast_a[4][A_LOADS], fast_b[4][B_LOADS];

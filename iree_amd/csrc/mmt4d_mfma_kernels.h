@@ -894,11 +894,11 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   //     resp. two, laid out like the 4-byte pieces, nothing is gained, the reads and permutes being what the step waits
   //     for: int8 16x16x2 777 x 4100 x 4096 23.4 us both, 512 x 4096 x 4096 19.7 -> 20.1.)
   //   What the lanes of a load have to do with each other: the memory pipeline takes four of them at a time, and takes
-  //   those twice that touch two stretches of 64 bytes: 105 bytes a nanosecond and compute unit with one stretch, 70 with
-  //   two, in a loop of nothing but these loads. Tiles of up to 128x128 come close to the latter. 4-byte pieces with M0 = 8 and 64-byte
+  //   those twice that touch two lines of 128 bytes: 105 bytes a nanosecond and compute unit with one, 70 with two, in a loop
+  //   of nothing but these loads. Tiles of up to 128x128 come close to the latter. 4-byte pieces with M0 = 8 and 64-byte
   //   pieces (below) had the rows first: int8 512 x 4096 x 4096 16x16x64 16.2 -> 13.8 us, 8x8x4 15.6 -> 13.6, 777 x 4100 x
   //   4096 22.3 -> 20.1 and 21.0 -> 19.4, 3072^3 (192x192 tiles) 32.2 -> 31.2 and 30.3 -> 29.4; 256x256 tiles are bound by the
-  //   matrix pipe, level.
+  //   matrix pipe, level. Four rows of 32-byte pieces are one line as they are.
   //   int4 rhs: slot 64*f + 32*h + r holds nibbles 32*h .. 32*h + 31 of row r of
   //     fragment f: lane 32*h + r reads that slot once per chunk and widens its
   //     first 8 bytes for K-step 0, its last 8 for K-step 1. The lhs columns are

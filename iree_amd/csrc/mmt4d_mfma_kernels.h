@@ -1762,7 +1762,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
 #pragma unroll
       for (int t = 0; t < B_LOADS; ++t) fast_b[c][t] = b_off[t] + c * GROUPS * rhs_chunk_bytes;
     }
-    // LDS offsets of the four stages that this round reads, whose last two steps load into the first two of them, and of
+    // LDS offsets of the four stages that four steps read, whose last two steps load into the first two of them, and of
     // those before, which the first two load into (four stages: the same).
     uint32_t this_four = load_ring_begin, other_four = load_ring_begin + (STAGES == 4 ? 0 : FOUR);
     static_assert(STAGES == 4 || STAGES == 8, "two fours at most");

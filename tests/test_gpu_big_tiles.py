@@ -201,8 +201,8 @@ def test_narrow_row_pieces_fall_back_when_the_direct_kernel_cannot_run(gpu_lib):
     run_case(gpu_lib, abi.MMT4D_TYPE_S8S8S32, 9, 11, 33, 16, 16, 2, "mmt4d_mfma_wave_k_16x16", accumulate=True)
 
 
-# K ending inside a 64-byte chunk on the direct-to-LDS kernel: the last chunk overlaps the one before it and the
-# overlap is zeroed in the fragments. Every row piece size, cuts at every granularity (an odd number of k steps,
+# K ending inside a 64-byte chunk on the direct-to-LDS kernel: the second chunk begins inside the first and what they share
+# is zeroed in the first one's fragments. Every row piece size, cuts at every granularity (an odd number of k steps,
 # cuts inside a lane's 16 bytes and at 16- and 32-byte boundaries), one chunk plus a bit, every block tile.
 @pytest.mark.parametrize("flags,M0,N0,K0,Ks", [
     (abi.MMT4D_TYPE_S8S8S32, 8, 8, 4, (17, 21, 24, 27, 31, 45)), (abi.MMT4D_TYPE_S8S8S32, 16, 16, 2, (33, 40, 47, 49, 63, 95)),
@@ -231,31 +231,44 @@ def test_direct_kernel_with_K_ending_inside_a_chunk(gpu_lib, flags, M0, N0, K0, 
                      seed=K + 200)
 
 
-@pytest.mark.parametrize("M,N,kernel", [(5, 6, b"mmt4d_mfma_wave_k_16x16"), (3, 1500, b"mmt4d_mfma_64x64")])
-def test_K_tail_overlap_is_zeroed_in_both_operands(gpu_lib, M, N, kernel):
-    # A block kernel loads the chunk that K ends in overlapping the one before it. An infinity inside the overlap must
-    # count once: were only one operand zeroed there, inf * 0 would turn the outputs into NaN. (The kernel that splits K
-    # over wavefronts zeroes what lies beyond K instead.)
-    K, M0, N0, K0 = 5, 16, 16, 16      # 32-byte row pieces: chunks [k0,k1], [k2,k3], tail k4 -> the last chunk is [k3,k4]
+# (Float problems in 16x16x16 tiles, 32-byte row pieces, two k steps a chunk; the last four have two groups of wavefronts.)
+OVERLAPPING = [(5, 6, 5, "mmt4d_mfma_wave_k_16x16"), (3, 1500, 5, "mmt4d_mfma_64x64"), (8, 562, 129, "mmt4d_mfma_128x64"),
+               (63, 129, 5, "mmt4d_mfma_128x128"), (63, 129, 129, "mmt4d_mfma_128x128"), (63, 129, 130, "mmt4d_mfma_128x128"),
+               (63, 129, 131, "mmt4d_mfma_128x128"), (63, 129, 132, "mmt4d_mfma_128x128")]
+
+
+@pytest.mark.parametrize("M,N,K,kernel", OVERLAPPING)
+def test_K_tail_overlap_is_zeroed_in_both_operands(gpu_lib, M, N, K, kernel):
+    # Where K ends inside a chunk a block kernel's chunk 1 begins inside chunk 0, which has what they share zeroed: of chunks
+    # [k0,k1], [k1,k2], [k3,k4] for K = 5 that is k1. With two groups of wavefronts and an odd number of chunks the first group
+    # has one chunk less, and in its place all of chunk 0, zeroed: k0 and k1. An infinity there must count once: were
+    # only one operand zeroed, inf * 0 would turn the outputs into NaN. (The kernel that splits K over wavefronts zeroes what
+    # lies beyond K instead.) One infinity in either operand in each k step of chunk 0 and in the last one.
+    M0, N0, K0 = 16, 16, 16
     g = torch.Generator(device="cuda").manual_seed(1)
     lhs = (torch.rand(M * K * M0 * K0, device="cuda", generator=g) + 0.5).to(torch.float16)
     rhs = (torch.rand(N * K * N0 * K0, device="cuda", generator=g) + 0.5).to(torch.float16)
-    lhs.view(M, K, M0, K0)[0, 3, 0, 7] = float("inf")      # logical row 0, k step 3
-    rhs.view(N, K, N0, K0)[1, 3, 5, 2] = float("inf")      # logical column 21, k step 3
+    rows, cols = [], []
+    for i, k in enumerate((0, 1, K - 1)):
+        lhs.view(M, K, M0, K0)[i, k, i, 7] = float("inf")
+        rhs.view(N, K, N0, K0)[1 + i, k, 5, 2] = float("inf")
+        rows.append(i * M0 + i)
+        cols.append((1 + i) * N0 + 5)
     out = torch.zeros(M * N * M0 * N0, device="cuda")
     p = mm_params(lhs.data_ptr(), rhs.data_ptr(), out.data_ptr(), M, N, K, M0, N0, K0, abi.MMT4D_TYPE_F16F16F32)
     gpu_lib.iree_uk_mmt4d_p(C.byref(p))
-    assert gpu_lib.iree_uk_mi355x_last_kernel() == kernel
+    assert gpu_lib.iree_uk_mi355x_last_kernel().decode() == kernel
     got = out.view(M, N, M0, N0).permute(0, 2, 1, 3).reshape(M * M0, N * N0)
     assert not bool(torch.isnan(got).any())
     inf = torch.isinf(got)
     want = torch.zeros_like(inf)
-    want[0, :] = True
-    want[:, 21] = True
+    want[rows, :] = True
+    want[:, cols] = True
     assert torch.equal(inf, want)
-    finite = got[1:, :21]
-    ref = logical(lhs, M, K, M0, K0)[1:] @ logical(rhs, N, K, N0, K0)[:21].t()
-    assert bool(((finite.double() - ref).abs() <= REL_TOL * ref.abs()).all())
+    finite_rows = [r for r in range(M * M0) if r not in rows]
+    finite_cols = [c for c in range(N * N0) if c not in cols]
+    ref = logical(lhs, M, K, M0, K0)[finite_rows] @ logical(rhs, N, K, N0, K0)[finite_cols].t()
+    assert bool(((got[finite_rows][:, finite_cols].double() - ref).abs() <= REL_TOL * ref.abs()).all())
 
 
 # Few block tiles against a long K: the tiles whose wavefronts split K and sum their partial tiles at the end. Even and odd

@@ -2,8 +2,11 @@
 the tile, its symbol the rest."""
 import re
 
+import pytest
+
 from iree_amd import abi
 from host_launches import recorder  # noqa: F401
+import test_gpu_four_steps as four_steps
 import test_gpu_two_groups as two_groups
 
 NARROW = (abi.MMT4D_TYPE_F16F16F16, abi.MMT4D_TYPE_BF16BF16BF16)
@@ -34,3 +37,16 @@ def test_two_groups(recorder):  # noqa: F811
         for sizes, expected in ((two_groups.WIDE, (16, "64x128", 8, 2)), (two_groups.TALL, (16, "128x128", 4, 2))):
             for M, N, K, options in two_groups.four_bit_problems(M0, N0, K0, sizes):
                 assert form(recorder, two_groups.S8S4, M, N, K, M0, N0, K0, options) == expected, (M, N, K)
+
+
+@pytest.mark.parametrize("case", four_steps.FORMS, ids=lambda f: "t%x_%dx%dx%d_%s_%d" % f[:6])
+def test_four_steps(recorder, case):  # noqa: F811
+    flags, M0, N0, K0, tile, groups, size, chunks = case
+    e = 1 if flags in (four_steps.S8, four_steps.S8S4) else 2
+    stages = 4 if tile == "128x128" else 8
+    # The loop is entered from twice the ring's depth on, 12 chunks with four stages, and left at every place of it.
+    entered = [c for c in chunks if c - 1 >= stages - 1 + 8]
+    assert {c % stages for c in entered} == set(range(stages))
+    for M, N, K, options in four_steps.problems(flags, M0, N0, K0, groups, size, chunks):
+        assert form(recorder, flags, M, N, K, M0, N0, K0, options) == (16 if flags == four_steps.S8S4 else min(16, K0 * e), tile, stages, groups), (M, N, K)
+        assert (-(-K * K0 * e // 64) + groups - 1) // groups in chunks

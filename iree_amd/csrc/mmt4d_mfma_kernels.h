@@ -42,6 +42,7 @@
 
 #include <type_traits>
 
+#include "mmt4d_chunk_walk.h"
 #include "uk_device.h"
 #include "uk_internal.h"
 
@@ -1019,21 +1020,11 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
 
-  // K in whole chunks but for the first: where K is none, chunk 0 is the first 64 bytes of every row all the same and
-  // chunk 1 begins where chunk 0 without its last `cut_bytes` ends. Every load stays inside the operands (there is a whole
-  // chunk at least), and what chunk 0 shares with chunk 1 is zeroed in its fragments of both operands once, in front of the
-  // loop (0 * 0 adds nothing, whatever the data; with an int4 rhs, where 0 * anything does, in the lhs alone). (The last
-  // chunk was the odd one before: a mask in every step, which the compiler makes unconditional, 24 of a step's 120
-  // instructions on the 256x128 tile, or a further step behind the loop, and four more scalar selects for where the last
-  // chunk lies.)
-  // Two groups: chunk i of group g is chunk 2*i + g of K, or one less where K has an odd number of chunks; the first group's
-  // first is none then, loaded as chunk 0 and zeroed whole.
-  const int chunks = GROUPS == 1 ? a.chunks : (a.chunks + 1) >> 1;
-  const int last_chunk = chunks - 1;
-  const int group_from = GROUPS == 1 ? 0 : group - (a.chunks & 1);
-  const int32_t cut_of_row = (int32_t)((64 - (((int64_t)a.K << a.log2_lhs_rb) & 63)) & 63);
-  const int32_t lhs_cut = cut_of_row << a.log2_M0, rhs_cut = cut_of_row << a.log2_N0 >> (RHS_I4 ? 1 : 0);
-  const int32_t cut_bytes = group_from < 0 ? 64 : (group_from == 0 ? cut_of_row : 0);
+  const GroupChunks<GROUPS> own_chunks(a.chunks, a.K, a.log2_lhs_rb, group);
+  const int chunks = own_chunks.count, last_chunk = own_chunks.last;
+  const int32_t lhs_cut = own_chunks.cut_of_row << a.log2_M0;
+  const int32_t rhs_cut = own_chunks.cut_of_row << a.log2_N0 >> (RHS_I4 ? 1 : 0);
+  const int32_t cut_bytes = own_chunks.cut_bytes;
 
   // Loads number `n` (compile-time after unrolling) of the chunk whose operand bases are la / lb, into the stage at LDS byte
   // offset `stage_off`, the wavefront's first slots included.
@@ -1067,18 +1058,12 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   };
   const uint8_t* lhs_from = lhs_base - (TOGETHER && A_LOADS == 2 ? 1024 : 0);
   const uint8_t* rhs_from = rhs_base - (TOGETHER && B_LOADS == 2 ? 1024 : 0);
-  // The first chunks: a compile-time `kc` of a few. (Minima and maxima, no branches: see row_offset. Chunks beyond the last
-  // one are that one again.)
-  auto lhs_near = [&](int kc) {
-    return lhs_from + (uint32_t)max((GROUPS * min(kc, last_chunk) + group_from) * lhs_chunk_bytes - lhs_cut, 0);
-  };
-  auto rhs_near = [&](int kc) {
-    return rhs_from + (uint32_t)max((GROUPS * min(kc, last_chunk) + group_from) * rhs_chunk_bytes - rhs_cut, 0);
-  };
+  auto lhs_near = [&](int kc) { return lhs_from + own_chunks.offset(kc, lhs_chunk_bytes, lhs_cut); };
+  auto rhs_near = [&](int kc) { return rhs_from + own_chunks.offset(kc, rhs_chunk_bytes, rhs_cut); };
   // The group's ring.
   const uint32_t ring_off = (uint32_t)group * (STAGES * STAGE_PIECES * 16);
   const uint4* const own_ring = ring + ring_off / 16;
-  // Chunk c lies in stage c - 1 modulo their number: what step kc reads is in stage kc.
+  // (Chunk c lies in stage c - 1 modulo their number.)
   const uint4* const first_stage = own_ring + (STAGES - 1) * STAGE_PIECES;
   auto issue_chunk = [&](int kc) {
     const uint32_t stage_off = ring_off + (uint32_t)((kc + STAGES - 1) % STAGES) * (STAGE_PIECES * 16) + 1024 * a_number(0);
@@ -1153,18 +1138,9 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   };
   const int frag_a0 = wave_m * AM, frag_b0 = wave_n * BN;
 
-  // Loop-carried, wavefront-uniform state: where the next chunk to load comes
-  // from and goes to, and the stage the next fragments are read from. Kept as
-  // running values (a few scalar adds per step) rather than recomputed from the
-  // chunk number (64-bit multiplies on the scalar unit, in front of the step's
-  // first MFMA).
+  // Loop-carried, wavefront-uniform state.
   constexpr uint32_t STAGE_BYTES = STAGE_PIECES * 16, RING_BYTES = STAGES * STAGE_BYTES;
-  const uint8_t* load_a = lhs_near(AHEAD);
-  const uint8_t* load_b = rhs_near(AHEAD);
-  int load_chunk = AHEAD;
-  const uint32_t load_ring_begin = ring_off + 1024 * a_number(0), load_ring_end = RING_BYTES + load_ring_begin;
-  uint32_t load_stage_off = (STAGES - 2) * STAGE_BYTES + load_ring_begin;
-  uint32_t read_stage_off = 0;
+  RingPlace<STAGES, GROUPS, STAGE_BYTES> at(lhs_near(AHEAD), rhs_near(AHEAD), ring_off + 1024 * a_number(0));
   const uint32_t frag_a_off = (uint32_t)((wave_m * AM) * 128) * 16;
   const uint32_t frag_b_off = (uint32_t)(A_PIECES + (wave_n * BN) * (RHS_I4 ? 64 : 128)) * 16;
   // Lane 32*h + r's byte offset into a fragment, and the slots from one K-step
@@ -1383,23 +1359,15 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // A step anywhere: all of that is running state, advanced by the step (clamped at the last chunk: the loads issued beyond
-  // it are redundant, their stages are never read).
+  // A step anywhere: all of that is running state, advanced by the step.
   auto running_read = [&](const uint8_t** read_a, const uint8_t** read_a_kk1, const uint8_t** read_b, const uint8_t** read_b_kk1) {
-    *read_a = ring_bytes + read_stage_off + frag_a_off + pair_a_lane;
+    *read_a = ring_bytes + at.read_off + frag_a_off + pair_a_lane;
     *read_a_kk1 = *read_a + lhs_kk1_step;
-    *read_b = ring_bytes + read_stage_off + frag_b_off + pair_b_lane;
+    *read_b = ring_bytes + at.read_off + frag_b_off + pair_b_lane;
     *read_b_kk1 = *read_b + rhs_kk1_step;
   };
-  auto running_load = [&](auto n) { issue_load(n, load_stage_off, load_a, load_b); };
-  auto running_advance = [&]() {
-    const bool more = load_chunk < last_chunk;
-    load_a += (uint32_t)(more ? GROUPS * lhs_chunk_bytes : 0);
-    load_b += (uint32_t)(more ? GROUPS * rhs_chunk_bytes : 0);
-    ++load_chunk;
-    load_stage_off = load_stage_off + STAGE_BYTES == load_ring_end ? load_ring_begin : load_stage_off + STAGE_BYTES;
-    read_stage_off = read_stage_off + STAGE_BYTES == RING_BYTES ? 0 : read_stage_off + STAGE_BYTES;
-  };
+  auto running_load = [&](auto n) { issue_load(n, at.load_off, at.load_a, at.load_b); };
+  auto running_advance = [&]() { at.advance(last_chunk, lhs_chunk_bytes, rhs_chunk_bytes); };
   auto step_with = [&](const uint4 (*cur_a)[2], const uint4 (*cur_b)[2], uint4 (*nxt_a)[2], uint4 (*nxt_b)[2],
                        bool held_loads_behind, auto between_mfmas) {
     step_at(cur_a, cur_b, nxt_a, nxt_b, held_loads_behind, between_mfmas,
@@ -1512,7 +1480,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
     const uint8_t* base_a_kk1[JR];
     const uint8_t* base_b[JR];
     {
-      uint32_t stage_off = read_stage_off;
+      uint32_t stage_off = at.read_off;
 #pragma unroll
       for (int c = 0; c < JR; ++c) {
         base_a[c] = ring_bytes + stage_off + frag_a_off + pair_a_lane;
@@ -1749,11 +1717,11 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   // beyond one base each, and the four chunks' offsets are registers. 28 instructions a step of the 128x64 tile where a step
   // anywhere has 46, 21 of 38 for 64x64, 64 of 80 for 64x128 and an int4 rhs. bf16 8x8x4 512 x 4096 x 4096 24.3 -> 22.4 us,
   // 16x16x16 22.8 -> 22.0, int8 16x16x2 19.2 -> 18.2, int4 256 x 8000 x 3008 13.0 -> 12.4, 784 x 4112 x 4096 (128x128) 21.4 -> 21.0.
-  // Not for a K of few rounds, which the preparation costs 1 %, nor where it was level: int8 but for its 2-byte pieces (128x64
+  // Not where it was level: int8 but for its 2-byte pieces (128x64
   // -4 to +4 %) and the 128x128 tile of others, bound by the LDS (-2 to +2 %).
   constexpr bool BY_FOUR = STAGES % 4 == 0 && KIND != kF32 && (RHS_I4 ? AM * BN <= 4 : AM * BN <= 2 && (KIND != kI8 || G == 2));
-  if constexpr (BY_FOUR) if (last_chunk >= AHEAD + 8) {
-    constexpr uint32_t FOUR = 4 * STAGE_BYTES;
+  typedef FourSteps<STAGES == 8 ? 8 : 4, GROUPS, STAGE_BYTES> Fours;
+  if constexpr (BY_FOUR) if (Fours::pays(last_chunk)) {
     uint32_t fast_a[4][A_LOADS], fast_b[4][B_LOADS];
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -1762,14 +1730,11 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
 #pragma unroll
       for (int t = 0; t < B_LOADS; ++t) fast_b[c][t] = b_off[t] + c * GROUPS * rhs_chunk_bytes;
     }
-    // LDS offsets of the four stages that four steps read, whose last two steps load into the first two of them, and of
-    // those before, which the first two load into (four stages: the same).
-    uint32_t this_four = load_ring_begin, other_four = load_ring_begin + (STAGES == 4 ? 0 : FOUR);
-    static_assert(STAGES == 4 || STAGES == 8, "two fours at most");
+    Fours fours(at);
     const uint8_t* from_a = ring_bytes + frag_a_off + pair_a_lane;
     const uint8_t* from_b = ring_bytes + frag_b_off + pair_b_lane;
-    while (kc + 3 + AHEAD <= last_chunk) {
-      const uint32_t read_off = this_four - load_ring_begin;
+    while (Fours::fits(kc, last_chunk)) {
+      const uint32_t read_off = fours.reads(at);
       const uint8_t* base_a = from_a + read_off;
       const uint8_t* base_b = from_b + read_off;
       const uint8_t *base_a_kk1 = base_a + lhs_kk1_step, *base_b_kk1 = base_b + rhs_kk1_step;
@@ -1782,9 +1747,9 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
           *read_b_kk1 = base_b_kk1 + S * STAGE_BYTES;
         };
         auto load = [&](auto n) {
-          const uint32_t four = S < 2 ? other_four : this_four;
-          issue_load_to(n, std::integral_constant<uint32_t, ((S + 2) % 4) * STAGE_BYTES>(), four, four + b_from_a, fast_a[S],
-                        fast_b[S], load_a, load_b);
+          const uint32_t four = fours.loads(S);
+          issue_load_to(n, std::integral_constant<uint32_t, Fours::loads_into(S) * STAGE_BYTES>(), four, four + b_from_a, fast_a[S],
+                        fast_b[S], at.load_a, at.load_b);
         };
         auto advance = [] {};
         StepPlace<decltype(read), decltype(load), decltype(advance)> place{read, load, advance};
@@ -1792,21 +1757,9 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
         else step_at(qa, qb, pa, pb, false, [](int) {}, place);
       });
       kc += 4;
-      load_a += (uint32_t)(4 * GROUPS * lhs_chunk_bytes);
-      load_b += (uint32_t)(4 * GROUPS * rhs_chunk_bytes);
-      if constexpr (STAGES == 8) {
-        const uint32_t was = this_four;
-        this_four = other_four;
-        other_four = was;
-      }
+      fours.advance(&at, lhs_chunk_bytes, rhs_chunk_bytes);
     }
-    load_chunk = kc + AHEAD;
-    // (The chunk after the last one, if the rounds came that far, is the last one again.)
-    const bool beyond = kc > 0 && load_chunk > last_chunk;
-    load_a -= (uint32_t)(beyond ? GROUPS * lhs_chunk_bytes : 0);
-    load_b -= (uint32_t)(beyond ? GROUPS * rhs_chunk_bytes : 0);
-    read_stage_off = this_four - load_ring_begin;
-    load_stage_off = other_four + 2 * STAGE_BYTES;
+    fours.leave(&at, kc, last_chunk, lhs_chunk_bytes, rhs_chunk_bytes);
   }
   for (; kc + 1 < chunks; kc += 2) {
     step(pa, pb, qa, qb);

@@ -18,31 +18,31 @@ LAYOUTS = {"bf16": (abi.MMT4D_TYPE_BF16BF16F32, 16, 16, 16), "s8": (abi.MMT4D_TY
 # Microseconds with operands held by the cache (150 MB in turn) and from HBM (640 MB in turn): the tiles of the kernel that
 # splits K over wavefronts, and the block kernel that the problem would take.
 TIMES = [
-    ("bf16", 32, 11008, 2048, {"32x64": (9.57, 11.77), "64x64": (9.86, 12.13), "block": (10.58, 12.48)}),
-    ("bf16", 64, 4096, 4096, {"32x32": (8.69, 12.70), "32x64": (10.77, 16.34), "64x32": (10.90, 16.43), "block": (17.16, 21.26)}),
-    ("bf16", 96, 14336, 4096, {"block": (23.49, 31.51), "64x64": (25.34, 36.39), "32x64": (26.84, 40.35)}),
-    ("bf16", 512, 4096, 4096, {"block": (22.84, 29.98), "64x64": (25.84, 36.22), "64x32": (32.44, 44.09)}),
-    ("s8", 64, 14336, 4096, {"block": (12.42, 15.92), "64x64": (13.66, 14.76), "32x64": (14.27, 18.84)}),
-    ("s8", 128, 4096, 14336, {"64x32": (22.03, 26.97), "32x64": (22.11, 27.09), "32x32": (27.61, 33.56), "block": (28.32, 36.02)}),
-    ("s8s4", 32, 28672, 8192, {"32x64": (23.48, 25.34), "64x64": (26.08, 27.28), "16x32": (22.52, 33.90), "block": (26.98, 28.57)}),
-    ("s8s4", 96, 14336, 4096, {"64x64": (14.24, 16.24), "32x64": (14.95, 18.03), "block": (16.32, 16.52)}),
-    ("s8s4", 96, 11008, 2048, {"32x32": (9.08, 10.18), "block": (10.07, 10.32), "64x64": (9.95, 11.34)}),
-    ("s8s4", 192, 8192, 4096, {"64x64": (14.30, 17.13), "32x64": (15.45, 18.00), "block": (16.75, 16.76)}),
-    ("f16, 2-byte pieces", 64, 4096, 4096, {"32x32": (9.45, 14.99), "16x32": (12.09, 17.08), "64x32": (12.10, 17.23), "block": (33.79, 34.58)}),
-    ("s8, 4-byte pieces", 128, 2048, 2048, {"32x32": (4.92, 5.50), "16x32": (5.65, 6.29), "32x64": (5.75, 6.56), "block": (6.96, 8.05)}),
-    ("bf16, 8-byte pieces", 32, 14336, 4096, {"block": (19.08, 24.37), "32x64": (19.61, 24.94), "64x64": (20.61, 25.55)}),
-    ("s8, 2-byte pieces", 256, 11008, 2048, {"block": (15.04, 17.74), "64x64": (19.34, 22.14), "32x32": (22.02, 27.20)}),
-    ("s8, 2-byte pieces", 304, 1632, 272, {"64x32": (3.96, 4.32), "32x32": (4.11, 4.33), "block": (4.70, 5.03)}),
-    ("s8, 4-byte pieces", 16, 20000, 3000, {"16x32": (11.77, 14.76), "32x32": (11.93, 15.10), "64x32": (12.92, 16.03), "block": (14.22, 16.88)}),
-    ("s8, 2-byte pieces", 96, 10112, 10112, {"32x64": (27.09, 38.19), "32x32": (30.49, 42.96), "64x64": (34.90, 44.45), "block": (39.44, 40.53)}),
-    ("bf16, 4-byte pieces", 16, 10112, 10112, {"32x64": (30.28, 41.46), "64x64": (30.69, 43.56), "16x16": (32.05, 44.58), "block": (39.52, 43.97)}),
-    ("bf16, 4-byte pieces", 16, 20000, 3000, {"16x32": (19.15, 25.76), "32x32": (19.47, 26.00), "16x16": (19.16, 27.17), "block": (23.92, 28.90)}),
-    ("s8, 2-byte pieces", 208, 5392, 1480, {"block": (10.62, 11.00), "32x32": (11.24, 12.13), "64x64": (12.13, 13.35), "32x64": (12.81, 13.90)}),
-    ("s8, 2-byte pieces", 112, 8224, 2372, {"block": (13.47, 13.99), "32x32": (12.88, 14.94), "64x64": (14.61, 15.94), "64x32": (15.14, 16.88)}),
-    ("bf16, 8-byte pieces", 232, 3504, 1268, {"block": (8.06, 8.88), "64x64": (9.24, 10.28), "64x32": (11.97, 13.40)}),
-    ("bf16, 8-byte pieces", 72, 5648, 1776, {"block": (9.45, 10.12), "64x64": (10.27, 11.71), "32x32": (11.88, 13.63)}),
-    ("s8s4", 320, 1664, 352, {"64x64": (4.28, 4.25), "32x32": (4.93, 4.85), "block": (5.11, 5.09), "32x64": (5.46, 5.40)}),
-    ("f32", 64, 2048, 2048, {"16x32": (7.97, 10.13), "16x16": (8.82, 11.53), "32x32": (11.16, 12.52), "block": (36.92, 37.41)}),
+    ("bf16", 32, 11008, 2048, {"32x64": (9.16, 12.04), "block": (9.29, 12.33), "64x64": (9.36, 12.44)}),
+    ("bf16", 64, 4096, 4096, {"32x32": (8.19, 12.73), "32x64": (10.28, 15.92), "64x32": (10.37, 15.95), "block": (12.23, 20.59)}),
+    ("bf16", 96, 14336, 4096, {"block": (23.76, 32.71), "64x64": (25.15, 36.98), "32x64": (26.59, 40.29)}),
+    ("bf16", 512, 4096, 4096, {"block": (24.62, 29.93), "64x64": (25.27, 35.74), "64x32": (31.98, 43.48)}),
+    ("s8", 64, 14336, 4096, {"block": (11.68, 15.14), "64x64": (13.28, 13.76), "32x64": (13.68, 18.37)}),
+    ("s8", 128, 4096, 14336, {"32x64": (21.14, 26.62), "64x32": (21.24, 26.71), "block": (24.19, 32.95), "32x32": (26.90, 32.91)}),
+    ("s8s4", 32, 28672, 8192, {"32x64": (23.53, 24.44), "block": (23.80, 30.15), "16x32": (22.42, 32.52), "64x64": (27.07, 27.35)}),
+    ("s8s4", 96, 14336, 4096, {"64x64": (14.45, 16.96), "block": (14.84, 16.94), "32x64": (14.32, 18.05)}),
+    ("s8s4", 96, 11008, 2048, {"block": (8.80, 8.93), "32x32": (8.29, 9.63), "32x64": (9.31, 10.38), "64x64": (9.59, 10.77)}),
+    ("s8s4", 192, 8192, 4096, {"block": (14.54, 15.84), "64x64": (14.81, 16.52), "32x64": (14.80, 17.18)}),
+    ("f16, 2-byte pieces", 64, 4096, 4096, {"32x32": (8.81, 13.17), "32x64": (11.52, 16.57), "16x32": (11.70, 16.33), "64x32": (11.54, 16.66), "block": (29.04, 29.62)}),
+    ("s8, 4-byte pieces", 128, 2048, 2048, {"32x32": (4.48, 5.00), "16x32": (5.15, 5.78), "32x64": (5.29, 6.04), "block": (5.81, 6.69)}),
+    ("bf16, 8-byte pieces", 32, 14336, 4096, {"block": (18.70, 25.03), "32x64": (19.24, 24.96), "32x32": (19.52, 26.51), "64x64": (20.33, 25.92)}),
+    ("s8, 2-byte pieces", 256, 11008, 2048, {"block": (14.27, 17.38), "64x64": (18.53, 21.27), "32x32": (20.95, 26.34)}),
+    ("s8, 2-byte pieces", 304, 1632, 272, {"32x32": (3.92, 3.89), "64x32": (3.92, 3.90), "block": (4.62, 4.59)}),
+    ("s8, 4-byte pieces", 16, 20000, 3000, {"16x32": (11.08, 14.46), "32x32": (11.43, 14.83), "16x16": (11.71, 16.29), "64x32": (12.29, 15.70), "block": (13.00, 16.62)}),
+    ("s8, 2-byte pieces", 96, 10112, 10112, {"32x64": (27.31, 38.10), "block": (34.27, 37.37), "32x32": (30.29, 42.42), "64x64": (35.14, 43.99)}),
+    ("bf16, 4-byte pieces", 16, 10112, 10112, {"32x64": (29.98, 40.50), "block": (29.65, 42.00), "64x64": (30.31, 42.96), "16x16": (31.66, 43.77)}),
+    ("bf16, 4-byte pieces", 16, 20000, 3000, {"16x32": (19.05, 25.29), "16x16": (18.69, 26.41), "32x32": (19.44, 25.62), "block": (21.87, 28.44)}),
+    ("s8, 2-byte pieces", 208, 5392, 1480, {"block": (9.56, 9.83), "32x32": (10.27, 11.53), "64x64": (11.47, 12.75), "32x64": (12.07, 13.20)}),
+    ("s8, 2-byte pieces", 112, 8224, 2372, {"block": (11.66, 12.55), "32x32": (12.01, 14.03), "64x64": (13.85, 15.29), "64x32": (14.07, 15.95)}),
+    ("bf16, 8-byte pieces", 232, 3504, 1268, {"block": (6.78, 8.52), "64x64": (8.66, 9.88), "64x32": (11.34, 12.86)}),
+    ("bf16, 8-byte pieces", 72, 5648, 1776, {"block": (7.50, 9.75), "64x64": (9.80, 11.47), "32x32": (11.27, 12.97)}),
+    ("s8s4", 320, 1664, 352, {"64x64": (4.21, 4.18), "32x32": (4.48, 4.45), "block": (4.93, 4.91), "32x64": (5.01, 4.99)}),
+    ("f32", 64, 2048, 2048, {"16x32": (7.45, 9.43), "16x16": (8.22, 10.93), "32x32": (10.51, 11.78), "block": (37.26, 36.91)}),
 ]
 
 

@@ -82,8 +82,11 @@ double block_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather) {
     start_us = 6.8;  // (and the summing of the partial tiles)
   } else {
     choose_tile(m, kind, rhs_i4, gather, direct, &us_per_chunk);
-    // (int4, K cut behind the loop: 336 x 1696 x 288 4.9 us, 4.3 in 64x64 tiles of the other kernel)
-    if (rhs_i4 && ((int64_t)m.K * m.lhs_rb) % 64 != 0) start_us += 0.4;
+    // (int4, K ending inside a chunk, which is a mask in front of the loop: 0.2 us. With a few chunks of K this decides: 560 x 1760
+    // x 288 5.0 us, 4.4 in 64x64 tiles of the other kernel; of 134 problems of up to 6 chunks that it alone gives to the other
+    // kernel, the block kernel is 7 % slower in the mean. Of 40 such of 9 to 24 chunks it is 2 % faster in the mean and on 14 up to
+    // 12 % slower, of 80 with more 14 % faster and on one 5 % slower: 144 x 6736 x 1568 7.9 us, 10.2 in 32x64 tiles.)
+    if (rhs_i4 && m.chunks <= 24 && ((int64_t)m.K * m.lhs_rb) % 64 != 0) start_us += 0.4;
     if (!direct) us_per_chunk *= 2.2;       // staged through registers
     // Few rows and more 64x64 tiles than units: the unit's second tile, row pieces of 4 and 8 bytes, is dearer than the
     // table's (from 16-byte pieces, many rows): bf16 16 x 20720 x 7396, 16x16x2 tiles, 0.28 us and not 0.195. Without the

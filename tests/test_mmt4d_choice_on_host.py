@@ -10,7 +10,8 @@ from host_launches import recorder  # noqa: F401
 from test_gpu_wave_k_f32_tiles import FOUR_BYTE_LAYOUTS, FOUR_BYTE_ROUND_SIZES, FOUR_BYTE_SIZES
 
 LAYOUTS = {"bf16": (abi.MMT4D_TYPE_BF16BF16F32, 16, 16, 16), "s8": (abi.MMT4D_TYPE_S8S8S32, 16, 16, 64),
-           "s8s4": (abi.MMT4D_TYPE_S8S4S32, 16, 16, 32), "f16, 2-byte pieces": (abi.MMT4D_TYPE_F16F16F32, 16, 16, 1),
+           "s8s4": (abi.MMT4D_TYPE_S8S4S32, 16, 16, 32), "s8s4, rhs tiles of 8": (abi.MMT4D_TYPE_S8S4S32, 16, 8, 32),
+           "f16, 2-byte pieces": (abi.MMT4D_TYPE_F16F16F32, 16, 16, 1),
            "s8, 4-byte pieces": (abi.MMT4D_TYPE_S8S8S32, 8, 8, 4), "bf16, 8-byte pieces": (abi.MMT4D_TYPE_BF16BF16F32, 8, 8, 4),
            "bf16, 4-byte pieces": (abi.MMT4D_TYPE_BF16BF16F32, 16, 16, 2),
            "s8, 2-byte pieces": (abi.MMT4D_TYPE_S8S8S32, 16, 16, 2), "f32": (abi.MMT4D_TYPE_F32F32F32, 16, 16, 4)}
@@ -42,6 +43,11 @@ TIMES = [
     ("bf16, 8-byte pieces", 232, 3504, 1268, {"block": (6.78, 8.52), "64x64": (8.66, 9.88), "64x32": (11.34, 12.86)}),
     ("bf16, 8-byte pieces", 72, 5648, 1776, {"block": (7.50, 9.75), "64x64": (9.80, 11.47), "32x32": (11.27, 12.97)}),
     ("s8s4", 320, 1664, 352, {"64x64": (4.21, 4.18), "32x32": (4.48, 4.45), "block": (4.93, 4.91), "32x64": (5.01, 4.99)}),
+    # K ending inside a chunk of 64: short and long
+    ("s8s4", 560, 1760, 288, {"64x64": (4.41, 4.40), "block": (5.02, 4.99)}),
+    ("s8s4, rhs tiles of 8", 16, 17776, 544, {"16x32": (4.23, 4.69), "block": (4.80, 5.11)}),
+    ("s8s4", 144, 6736, 1568, {"block": (7.86, 7.89), "32x64": (9.92, 10.54)}),
+    ("s8s4", 352, 3120, 1568, {"block": (8.23, 8.04), "32x64": (10.61, 10.31)}),
     ("f32", 64, 2048, 2048, {"16x32": (7.45, 9.43), "16x16": (8.22, 10.93), "32x32": (10.51, 11.78), "block": (37.26, 36.91)}),
 ]
 

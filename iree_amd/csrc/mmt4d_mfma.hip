@@ -28,7 +28,8 @@ struct Plan {
 // the output at the same rate, which is left out. Measured over 741 problems (M 8..1100, N 64..28672, K 64..14336, every
 // type and row piece) with operands from HBM (sets of 640 MB in turn, the condition of weights in a model's layers) and
 // with operands that the last-level cache holds (150 MB), the coefficients fitted to the geometric mean of the two: the
-// kernel picked is 0.5 % slower than the best one in the mean, 5 % and more on one problem in 31. Fitted to repeated operands
+// kernel picked is 0.5 % slower than the best one in the mean, 5 % and more on one problem in 31 (timed again since the kernels
+// got shorter loops and prologues: 260 problems 0.6 %, one in 26; 200 of int4 0.3 %, one in 100). Fitted to repeated operands
 // alone they would pick 32x64 tiles for bf16 96 x 14336 x 4096: 27.5 us held and 40.6 from HBM, where the 128x64 tile with
 // K split takes 23.9 and 32.6; int4 96 x 14336 x 4096 19.1 from HBM against 16.3.
 //
@@ -108,7 +109,7 @@ double wave_k_cost(const MfmaArgs& m, int kind, bool rhs_i4, int gather, const W
   const bool narrow = gather < 16 && !wave_k_loads_pieces(m, kind, gather, s.fa, s.fb);  // row pieces that pass through LDS
   if (kind == kF32) return wave_k_cost_f32(m, s, tiles, narrow);
   // (Pieces of 2 and 8 bytes: chosen by what 255 problems lose to their best kernel. At 81.4 and a
-  // start of 3.03, of before K was cut behind the block kernels' loop, the pick was 1.9 % slower than the best one in the
+  // start of 3.03, of before the end of K left the block kernels' steps, the pick was 1.9 % slower than the best one in the
   // mean, now 0.7: s8 208 x 5392 x 1480 in 16x16x2 tiles 13.4 -> 10.8 us, bf16 232 x 3504 x 1268 in 8x8x4 9.7 -> 8.5.)
   const bool narrow_2_8 = narrow && gather != 4;
   const double tile_us = 16 * (s.fa + s.fb * rhs_share) * row_kb / (narrow_2_8 ? 69.5 : narrow ? 81.4 : 92.5);

@@ -13,8 +13,8 @@
 //   mmt4d_mfma_direct_kernel (the fast path): operands go global memory ->
 //     LDS directly, 16 contiguous bytes per lane, through a ring of LDS stages
 //     filled several chunks ahead; needs 16-byte aligned operand rows and at
-//     least one full chunk of K (a K that ends inside a chunk is handled by
-//     overlapping the last chunk with the one before it).
+//     least one full chunk of K (where K ends inside a chunk, chunk 1 begins
+//     inside chunk 0, which has what they share zeroed: mmt4d_chunk_walk.h).
 //   mmt4d_mfma_kernel (everything else the plan admits: 4-byte aligned
 //     operands, narrow tiles, less than a chunk of K, an int4 rhs of 8-byte row
 //     pieces): global -> registers (issued two chunks ahead) -> LDS -> registers (read one chunk ahead) -> MFMA.
@@ -170,8 +170,10 @@ inline bool two_groups(const MfmaArgs& m, int kind, bool rhs_i4, int gather, boo
 // with two groups of wavefronts (two_groups).
 // Microseconds on the direct-to-LDS kernel, fitted to 24 shapes (M 160..4096, N 464..13952, K 700..8192) with every tile
 // for bf16 / f16 16x16x16, bf16 8x8x4, int8 8x8x4 and 16x16x64, f16 16x16x1 and int8 16x16x2 (2-byte pieces: fragments
-// come in pairs, which an odd number of them does not have), int4 16x16x32. The tile picked is 0.1 to 1.3 % slower in the
-// mean than the best one; without the 192-wide ones and one efficiency per tile it was 4 to 7 %. f32 is bound by the
+// come in pairs, which an odd number of them does not have), int4 16x16x32. Over 200 problems of those ranges, timed since the
+// loops got shorter, the tile picked is slower than the best one in the mean by 0.3 to 0.5 % (16-bit), 0.1 to 0.6 (int8), 1.6
+// (int4) and, of 2-byte pieces, 0.2 (int8) and 2.5 (f16: 464 x 1792 x 8041 60.3 us in 64x64 tiles, 54.3 in 128x64); without
+// the 192-wide ones and one efficiency per tile it was 4 to 7 %. f32 is bound by the
 // matrix pipe whatever the tile, which leaves the number of rounds (in units of a 128x128 tile; the large tiles, which
 // move fewer bytes, are favoured by 10 %).
 // `us_per_chunk`: that least time.
@@ -708,7 +710,8 @@ __global__ __launch_bounds__(256, MIN_BLOCKS) void mmt4d_mfma_kernel(const MfmaA
 // as its instructions: 46 for 4 MFMAs on the 128x64 tile (57 before the first chunk took what is odd about K, see below, and
 // loads came in pairs). bf16 512 x 4096 x 4096 23.0 -> 21.6 us, 304 x 5008 x 3008 16.4 -> 15.5, int8 8x8x4 512 x 4096 x 4096
 // 13.7 -> 12.9; int4 512 x 11008 x 4096 (256x128) 29.2 -> 27.4, 784 x 4112 x 4096 (128x128) 21.5 -> 20.1; 192-wide tiles 2
-// to 5 %, 256x256 up to 2 % (int8 16x16x2, 4096^3, bound by power, 71.4 -> 72.1).
+// to 5 %, 256x256 up to 2 % (2-byte pieces: int8 16x16x2 3072 x 4096 x 4096 57.4 -> 56.1, 4096^2 x 4094 69.8 -> 69.5, but with all
+// units busy and K a power of two 1.4 to 1.7 % slower: 4096^3 69.1 -> 70.3, x 2048 44.1 -> 44.7).
 //
 // The loads are issued from inline assembly: the compiler cannot see that they
 // write LDS, so it does not serialise the LDS reads against them; ordering is

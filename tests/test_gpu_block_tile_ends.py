@@ -1,6 +1,6 @@
 """The end of K on the block tiles (mmt4d_mfma_kernels.h): one chunk of 64 bytes per row, two, three, and K that ends inside
-the second, the third or a later one, for the tiles that cut the last chunk behind their loop (int4, and up to 128x128) and
-for those that do it inside. Sizes that no tile divides, strided and accumulating.
+the second, the third or a later one: the first chunk then shares bytes with the second and is masked in front of the loop. Every
+block tile, sizes that no tile divides, strided and accumulating.
 
 Integers are compared bit for bit with a float64 product, floats within 1e-3 of max(|ref|, rms(ref)): sums of at most
 1100 products of unit-scale values in 32 bits differ by about 1e-6 of that in any order.

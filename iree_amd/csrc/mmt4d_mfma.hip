@@ -21,6 +21,7 @@ struct Plan {
   bool narrow;  // 16-bit output, rounded once at the end
   int gather;   // bytes of a row piece, 16 for 16 and more
   int wave_shape;  // tile of the kernel that splits K over wavefronts, or -1: a block kernel
+  bool wave_tile;  // the kernel whose wavefronts have the whole of a large tile each, instead of either
   MfmaArgs args;
 };
 
@@ -132,6 +133,42 @@ bool wave_k_covers(const MfmaArgs& m, int gather, bool rhs_i4) {
          (m.N == 1 || m.rhs_stride_bytes % 16 == 0);
 }
 
+// Whether the kernel whose wavefronts have a large tile each covers the problem: four lanes' 16-byte pieces, of four consecutive
+// rows, in one 128-byte line; a whole chunk of K; offsets of a tile below its buffers' 2 GiB.
+bool wave_tile_covers(const MfmaArgs& m, int kind, int gather, bool rhs_i4) {
+  if (gather != 16 || kind == kF32 || (kind == kI8 && !rhs_i4) || !wave_k_covers(m, gather, rhs_i4)) return false;
+  if (m.lhs_rb > 32 || m.log2_M0 < 2 || ((int64_t)m.K << m.log2_lhs_rb) < 64) return false;
+  if (m.lhs_stride_bytes < 0 || m.rhs_stride_bytes < 0) return false;
+  const int64_t lhs_reach = (128 >> m.log2_M0) * m.lhs_stride_bytes + (((int64_t)m.K + 8) << (m.log2_lhs_rb + m.log2_M0));
+  const int64_t rhs_reach = (128 >> m.log2_N0) * m.rhs_stride_bytes + (((int64_t)m.K + 8) << (m.log2_rhs_rb + m.log2_N0));
+  return lhs_reach < (1ll << 31) && rhs_reach < (1ll << 31);
+}
+
+// Whether it is the fastest, from 500 problems (M 17..4096, N 256..14336, K 256..8192, half a round of its tiles on the compute
+// units to four) timed beside what was chosen for them, on three sets of operands in turn, which the last-level cache
+// holds, and some on sets of 640 MB, from HBM.
+// 16-bit operands, 128x128 tiles: 200 to 248 tiles and 64 chunks of K or more 4 % faster in the mean, of 28 problems two 1 %
+// slower, from HBM 3 to 13 % faster. With 22 to 48 chunks 2 to 14 % slower (the partial sums), with 140 to 199 tiles
+// between 9 % slower and 7 % faster, a second round of tiles takes half as long again, and operands of more than 48 MiB (see
+// streams_operands) -2 to +3 %.
+// int4, 64x128 tiles: where 64x64 ones are more than a round of the compute units and these are not, and 32x64 ones would be taken.
+// 11 problems 13 to 28 % faster, from HBM between 2 % slower and 19 % faster, 5 in the mean; but where 32-high tiles
+// have less padding, 160 rows and up to 160 that they divide, 3 to 14 % slower. (Where the block kernel's tile would be taken it
+// is up to 5 % faster with 24 to 44 chunks, 17 with more, and from HBM 2 to 14 % slower. Near 256 tiles between 5 % slower and
+// 6 % faster, beyond up to 30 % slower; with up to 256 tiles of 64x64 those take two thirds of the time.)
+bool wave_tile_is_best(const MfmaArgs& m, bool rhs_i4, int wave_shape) {
+  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0;
+  const int64_t col_tiles = (cols + 127) / 128;
+  if (rhs_i4) {
+    const int64_t row_tiles = (rows + 63) / 64;
+    const bool padded = 6 * 64 * row_tiles > 7 * 32 * ((rows + 31) / 32);  // (than 32-high tiles)
+    return wave_shape >= 0 && row_tiles * ((cols + 63) / 64) > 256 && row_tiles * col_tiles <= 240 && !padded && m.chunks >= 24;
+  }
+  const int64_t tiles = ((rows + 127) / 128) * col_tiles;
+  return tiles >= 200 && tiles <= 248 && m.chunks >= 64 && wave_shape < 0 &&
+         !comes_from_hbm((rows * m.lhs_rb + cols * m.rhs_rb) * m.K);
+}
+
 // Fills `plan` if the problem is covered. With `probe_only` only type and tile
 // shape are looked at; without `choose` the kernel is left open.
 bool make_plan(const Mmt4dArgs& a, bool probe_only, bool choose, Plan* plan) {
@@ -220,6 +257,7 @@ bool make_plan(const Mmt4dArgs& a, bool probe_only, bool choose, Plan* plan) {
   if (((uintptr_t)a.rhs % rhs_align) || (a.N > 1 && rhs_stride_bytes % rhs_align)) return false;
   if ((gather == 1 || gather == 2 || gather == 8) && !mfma_direct_covers(m, gather, i4)) return false;
   plan->wave_shape = -1;
+  plan->wave_tile = false;
   if (!choose || !wave_k_covers(m, gather, i4)) return true;
   double best = block_cost(m, kind, i4, gather);
   const int shapes = kind == kF32 ? sizeof kWaveKShapesF32 / sizeof(WaveKShape) : sizeof kWaveKShapes / sizeof(WaveKShape);
@@ -230,6 +268,7 @@ bool make_plan(const Mmt4dArgs& a, bool probe_only, bool choose, Plan* plan) {
       plan->wave_shape = s;
     }
   }
+  plan->wave_tile = wave_tile_covers(m, kind, gather, i4) && wave_tile_is_best(m, i4, plan->wave_shape);
   return true;
 }
 
@@ -257,8 +296,12 @@ hipError_t launch_wave_k(const Plan& plan, hipStream_t stream, const char** name
 hipError_t launch_mfma(const Mmt4dArgs& a, hipStream_t stream, const char** name) {
   Plan plan;
   if (!make_plan(a, false, true, &plan)) return hipErrorInvalidValue;
-  if (plan.wave_shape >= 0) return launch_wave_k(plan, stream, name);
   const MfmaArgs& m = plan.args;
+  if (plan.wave_tile) {
+    *name = "mmt4d_mfma_wave_tile";
+    return launch_wave_tile(m, plan.kind, plan.rhs_i4, plan.narrow, stream);
+  }
+  if (plan.wave_shape >= 0) return launch_wave_k(plan, stream, name);
   switch (plan.kind) {
     case kI8: return launch_mfma_i8(m, plan.gather, plan.rhs_i4, stream, name);
     case kF16: return launch_mfma_f16(m, plan.gather, plan.narrow, stream, name);

@@ -122,6 +122,10 @@ hipError_t launch_wave_k_f32(const MfmaArgs& m, int gather, int shape, bool stre
 hipError_t launch_wave_k_f16_narrow(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);
 hipError_t launch_wave_k_bf16_narrow(const MfmaArgs& m, int gather, int shape, bool streamed, hipStream_t stream);
 
+// The kernel whose wavefronts multiply the whole of a large tile each (mmt4d_wave_tile.hip): 128x128 for 16-bit operands,
+// 64x128 for an int4 rhs.
+hipError_t launch_wave_tile(const MfmaArgs& m, int kind, bool rhs_i4, bool narrow, hipStream_t stream);
+
 // The block tiles of the block kernels. Larger ones move fewer operand bytes per multiply through L2 -> LDS and run the
 // matrix pipe longer between barriers, smaller ones spread a problem over more compute units; those with a side of 192
 // are there for the problems that leave a last round of 128- or 256-wide tiles nearly empty (bf16 752 x 10928 x 2272 has

@@ -388,16 +388,15 @@ __device__ __forceinline__ void store_block(const MfmaArgs& a, typename AccType<
     }
   auto to_float = [](stored_t w) -> quad_t {
     if constexpr (NARROW) {
-      return quad_t{widen16<EBITS>((uint16_t)w.x), widen16<EBITS>((uint16_t)(w.x >> 16)),
-                    widen16<EBITS>((uint16_t)w.y), widen16<EBITS>((uint16_t)(w.y >> 16))};
+      return quad_t{widen16_first<EBITS>(w.x), widen16_second<EBITS>(w.x), widen16_first<EBITS>(w.y), widen16_second<EBITS>(w.y)};
     } else {
       return w;
     }
   };
   auto to_stored = [](quad_t v) -> stored_t {
     if constexpr (NARROW) {
-      return make_uint2((uint32_t)narrow16<EBITS>(v.x) | ((uint32_t)narrow16<EBITS>(v.y) << 16),
-                        (uint32_t)narrow16<EBITS>(v.z) | ((uint32_t)narrow16<EBITS>(v.w) << 16));
+      return make_uint2(narrow16_pair<EBITS>(v.x, v.y),
+                        narrow16_pair<EBITS>(v.z, v.w));
     } else {
       return v;
     }
@@ -1444,16 +1443,15 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   constexpr int OUT_EBITS = KIND == kF16 ? 5 : 8;
   auto out_to_float = [](out_stored_t w) -> out_quad_t {
     if constexpr (NARROW) {
-      return out_quad_t{widen16<OUT_EBITS>((uint16_t)w.x), widen16<OUT_EBITS>((uint16_t)(w.x >> 16)),
-                        widen16<OUT_EBITS>((uint16_t)w.y), widen16<OUT_EBITS>((uint16_t)(w.y >> 16))};
+      return out_quad_t{widen16_first<OUT_EBITS>(w.x), widen16_second<OUT_EBITS>(w.x), widen16_first<OUT_EBITS>(w.y), widen16_second<OUT_EBITS>(w.y)};
     } else {
       return w;
     }
   };
   auto out_to_stored = [](out_quad_t v) -> out_stored_t {
     if constexpr (NARROW) {
-      return make_uint2((uint32_t)narrow16<OUT_EBITS>(v.x) | ((uint32_t)narrow16<OUT_EBITS>(v.y) << 16),
-                        (uint32_t)narrow16<OUT_EBITS>(v.z) | ((uint32_t)narrow16<OUT_EBITS>(v.w) << 16));
+      return make_uint2(narrow16_pair<OUT_EBITS>(v.x, v.y),
+                        narrow16_pair<OUT_EBITS>(v.z, v.w));
     } else {
       return v;
     }

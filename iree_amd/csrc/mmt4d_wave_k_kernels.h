@@ -419,11 +419,9 @@ void mmt4d_wave_k_kernel(const MfmaArgs a) {
       uint2* dst = (uint2*)(a.out + 2 * index);
       if (a.accumulate) {
         const uint2 old = *dst;
-        v += acc_t{widen16<EBITS>((uint16_t)old.x), widen16<EBITS>((uint16_t)(old.x >> 16)),
-                   widen16<EBITS>((uint16_t)old.y), widen16<EBITS>((uint16_t)(old.y >> 16))};
+        v += acc_t{widen16_first<EBITS>(old.x), widen16_second<EBITS>(old.x), widen16_first<EBITS>(old.y), widen16_second<EBITS>(old.y)};
       }
-      *dst = make_uint2((uint32_t)narrow16<EBITS>(v.x) | ((uint32_t)narrow16<EBITS>(v.y) << 16),
-                        (uint32_t)narrow16<EBITS>(v.z) | ((uint32_t)narrow16<EBITS>(v.w) << 16));
+      *dst = make_uint2(narrow16_pair<EBITS>(v.x, v.y), narrow16_pair<EBITS>(v.z, v.w));
     } else {
       acc_t* dst = (acc_t*)(a.out + 4 * index);
       if (a.accumulate) v += *dst;

@@ -275,11 +275,9 @@ void mmt4d_mfma_wave_tile_kernel(const MfmaArgs a) {
         constexpr int EBITS = KIND == kF16 ? 5 : 8;
         if (a.accumulate) {
           const uint2 o = old[i][e];
-          v += v4{widen16<EBITS>((uint16_t)o.x), widen16<EBITS>((uint16_t)(o.x >> 16)),
-                  widen16<EBITS>((uint16_t)o.y), widen16<EBITS>((uint16_t)(o.y >> 16))};
+          v += v4{widen16_first<EBITS>(o.x), widen16_second<EBITS>(o.x), widen16_first<EBITS>(o.y), widen16_second<EBITS>(o.y)};
         }
-        *to = make_uint2((uint32_t)narrow16<EBITS>(v.x) | ((uint32_t)narrow16<EBITS>(v.y) << 16),
-                         (uint32_t)narrow16<EBITS>(v.z) | ((uint32_t)narrow16<EBITS>(v.w) << 16));
+        *to = make_uint2(narrow16_pair<EBITS>(v.x, v.y), narrow16_pair<EBITS>(v.z, v.w));
       } else {
         if (a.accumulate) v += old[i][e];
         *to = v;

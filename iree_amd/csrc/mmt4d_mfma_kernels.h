@@ -347,8 +347,7 @@ __device__ __forceinline__ void fetch_arguments(const MfmaArgs& a) {
 // 32*j + 8*q + 4*(l >> 5) + {0..3} of the wavefront's sub-block, which starts at
 // (wave_row, wave_col) of the logical matrix: four consecutive j0 of one output
 // row, one 128-bit store (64-bit for a NARROW, i.e. 16-bit, output, rounded to
-// nearest even the way common.h:701-770 does). When accumulating, a fragment's
-// loads are issued before its first add, so their latencies overlap.
+// nearest even the way common.h:701-770 does).
 //
 // PAIR_A / PAIR_B: the fragments of that operand were fed in interleaved pairs
 // (2-byte row pieces, see the direct-to-LDS kernel): lane row r of fragments
@@ -395,12 +394,61 @@ __device__ __forceinline__ void store_block(const MfmaArgs& a, typename AccType<
   };
   auto to_stored = [](quad_t v) -> stored_t {
     if constexpr (NARROW) {
-      return make_uint2(narrow16_pair<EBITS>(v.x, v.y),
-                        narrow16_pair<EBITS>(v.z, v.w));
+      return make_uint2(narrow16_pair<EBITS>(v.x, v.y), narrow16_pair<EBITS>(v.z, v.w));
     } else {
       return v;
     }
   };
+  if constexpr (!PAIR_A && !PAIR_B) {
+    if (a.accumulate) {
+      // What the destination holds is asked for several fragments before it is added, as many as 64 registers hold. A
+      // fragment's loads when its turn came waited for memory once a fragment, with a 16-bit output, each converted as it
+      // arrived, four times: int8 8x8x4 344 x 6576 x 336 8.9 -> 7.0 us, 856 x 4480 x 580 11.1 -> 10.3, bf16 8x8x4 1024 x 4096 x
+      // 1024 17.2 -> 15.4, 256x256 tiles 3072 x 5024 x 1264 57.2 -> 53.0, bf16 output 79.2 -> 69.0 (with the conversions of
+      // uk_device.h 48.2). (Pairs of fragments, 32 and 64 registers, gain nothing from it and are up to 8 % slower; a loop for
+      // calls of both kinds costs those that do not accumulate 1 to 2 %.)
+      // (Without conditions: rows and columns behind the last ones read others of the sub-block.)
+      if (wave_row >= total_rows || wave_col >= total_cols) return;
+      uint8_t* row_out[AM];
+      bool row_inside[AM];
+#pragma unroll
+      for (int i = 0; i < AM; ++i) {
+        const int64_t this_row = wave_row + 32 * i + (lane & 31), row = min(this_row, total_rows - 1);
+        row_inside[i] = this_row < total_rows;
+        row_out[i] = wave_out + OUT_BYTES * ((row >> a.log2_M0) * a.out_stride0 + ((row & (M0 - 1)) << a.log2_N0));
+      }
+      constexpr int FIT = 64 / (int)sizeof(stored_t), AHEAD = FIT < AM * BN ? FIT : AM * BN;
+      stored_t old[AHEAD][4];
+      auto fetch = [&](int f) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t off = col_inside >> (4 * (f % BN) + q) & 1 ? col_off[f % BN][q] : 0;
+          old[f % AHEAD][q] = *(const stored_t*)(row_out[f / BN] + off);
+        }
+      };
+#pragma unroll
+      for (int f = 0; f < AHEAD; ++f) fetch(f);
+#pragma unroll
+      for (int f = 0; f < AM * BN; ++f) {
+        typename AccType<KIND>::type frag = acc[f / BN][f % BN];
+        asm volatile("" : "+a"(frag));  // (pinned until its turn, see below)
+        quad_t v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          v[q] = quad_t{frag[4 * q], frag[4 * q + 1], frag[4 * q + 2], frag[4 * q + 3]};
+          if constexpr (RHS_I4) v[q] = v[q] >> 4;
+          v[q] += to_float(old[f % AHEAD][q]);
+        }
+        if (f + AHEAD < AM * BN) fetch(f + AHEAD);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (row_inside[f / BN] && (col_inside >> (4 * (f % BN) + q) & 1))
+            *(stored_t*)(row_out[f / BN] + col_off[f % BN][q]) = to_stored(v[q]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      return;
+    }
+  }
   // With paired lhs fragments, fragments 2p and 2p + 1 hold the even and the odd
   // rows of the same 64: they are written together, so that the stores which
   // make up a cache line of the output (two rows of a 16-wide int32 tile, say)
@@ -448,24 +496,24 @@ __device__ __forceinline__ void store_block(const MfmaArgs& a, typename AccType<
             }
             if constexpr (RHS_I4) v[t][s][q] = v[t][s][q] >> 4;
           }
-      if (a.accumulate) {
-        quad_t old[IS][JS][4];
+      if ((PAIR_A || PAIR_B) && a.accumulate) {
+        stored_t old[IS][JS][4];
 #pragma unroll
         for (int t = 0; t < IS; ++t)
 #pragma unroll
           for (int s = 0; s < JS; ++s)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-              old[t][s][q] = quad_t{0, 0, 0, 0};
+              old[t][s][q] = stored_t{};
               if (row_inside[t] && (col_inside >> (4 * (j0 + s) + q) & 1))
-                old[t][s][q] = to_float(*(const stored_t*)(row_out[t] + col_off[j0 + s][q]));
+                old[t][s][q] = *(const stored_t*)(row_out[t] + col_off[j0 + s][q]);
             }
 #pragma unroll
         for (int t = 0; t < IS; ++t)
 #pragma unroll
           for (int s = 0; s < JS; ++s)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) v[t][s][q] += old[t][s][q];
+            for (int q = 0; q < 4; ++q) v[t][s][q] += to_float(old[t][s][q]);
       }
       // Store order: the pieces of one row right after each other (with paired
       // rhs fragments v[.][0][q] and v[.][1][q] are the two halves of 32
@@ -1443,15 +1491,15 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   constexpr int OUT_EBITS = KIND == kF16 ? 5 : 8;
   auto out_to_float = [](out_stored_t w) -> out_quad_t {
     if constexpr (NARROW) {
-      return out_quad_t{widen16_first<OUT_EBITS>(w.x), widen16_second<OUT_EBITS>(w.x), widen16_first<OUT_EBITS>(w.y), widen16_second<OUT_EBITS>(w.y)};
+      return out_quad_t{widen16_first<OUT_EBITS>(w.x), widen16_second<OUT_EBITS>(w.x),
+                        widen16_first<OUT_EBITS>(w.y), widen16_second<OUT_EBITS>(w.y)};
     } else {
       return w;
     }
   };
   auto out_to_stored = [](out_quad_t v) -> out_stored_t {
     if constexpr (NARROW) {
-      return make_uint2(narrow16_pair<OUT_EBITS>(v.x, v.y),
-                        narrow16_pair<OUT_EBITS>(v.z, v.w));
+      return make_uint2(narrow16_pair<OUT_EBITS>(v.x, v.y), narrow16_pair<OUT_EBITS>(v.z, v.w));
     } else {
       return v;
     }

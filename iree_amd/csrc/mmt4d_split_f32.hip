@@ -17,7 +17,8 @@
 // value other than zero below 2^-100, whose lo may be too small for bf16, or a
 // sum that is no finite number (an infinity splits into infinity and NaN, a value
 // above the largest bf16 rounds to one) computes its tile again with them. Such
-// tiles take the time of both.
+// tiles take the time of both: with one such value in every tile 1024 x 2048 x 2048
+// takes 115 us where the f32 kernel takes 64, 432 x 1936 x 3096 87 where it takes 45.
 //
 // The rest is mmt4d_wave_tile.hip's: wavefronts multiply the whole tile over
 // K in turns of 64 bytes (16 values), operands straight from global memory in registers,

@@ -21,7 +21,6 @@ struct Plan {
   bool narrow;  // 16-bit output, rounded once at the end
   int gather;   // bytes of a row piece, 16 for 16 and more
   int wave_shape;  // tile of the kernel that splits K over wavefronts, or -1: a block kernel
-  int split_shape;  // f32: tile of the kernel that splits values into bf16 pieces, or -1
   bool wave_tile;  // the kernel whose wavefronts have the whole of a large tile each, instead of either
   MfmaArgs args;
 };
@@ -170,39 +169,6 @@ bool wave_tile_is_best(const MfmaArgs& m, bool rhs_i4, int wave_shape) {
          !comes_from_hbm((rows * m.lhs_rb + cols * m.rhs_rb) * m.K);
 }
 
-// Whether the kernel that splits f32 into bf16 pieces covers the problem: aligned loads; a load's lanes in runs of 64 bytes, 32 of
-// single floats; a whole chunk of K; offsets of a tile below its buffers' 2 GiB.
-bool split_f32_covers(const MfmaArgs& m, int gather) {
-  if (gather != 16 && gather != 4) return false;
-  if ((uintptr_t)m.lhs % gather || (uintptr_t)m.rhs % gather) return false;
-  if (m.lhs_stride_bytes % gather || m.rhs_stride_bytes % gather || m.lhs_stride_bytes < 0 || m.rhs_stride_bytes < 0) return false;
-  const int32_t least = gather == 16 ? 64 : 32;
-  if ((m.lhs_rb << m.log2_M0) < least || (m.rhs_rb << m.log2_N0) < least) return false;
-  if (((int64_t)m.K << m.log2_lhs_rb) < 64) return false;
-  const int64_t lhs_reach = (128 >> m.log2_M0) * m.lhs_stride_bytes + (((int64_t)m.K + 16) << (m.log2_lhs_rb + m.log2_M0));
-  const int64_t rhs_reach = (128 >> m.log2_N0) * m.rhs_stride_bytes + (((int64_t)m.K + 16) << (m.log2_rhs_rb + m.log2_N0));
-  return lhs_reach < (1ll << 31) && rhs_reach < (1ll << 31);
-}
-
-// Its time in 64x64 (shape 0) and 64x128 tiles, one workgroup per compute unit at a time, and longer steps the more units there
-// are at work. Fitted to 260 problems (M 17..4096, N 256..14336, K 200..8192, 0.8 to 8.6 GFLOP, row pieces of 16 and 4
-// bytes), each timed in both tiles and with the kernel chosen for it before: off by 4 % (rms). Of 220 others (from 0.4
-// GFLOP) it is taken for 49, which run 1.15 times as fast, from 2 % slower to 1.36; of 60 with operands from HBM for 13,
-// 1.09, from 4 % slower to 1.24. Left out: up to 64 rows, which are 8 to 17 % slower on three problems of five, and few chunks
-// of K, which the prologue and the sums outweigh (floats loaded one at a time, 22 to 26 chunks: 5 % slower to level).
-double split_f32_cost(const MfmaArgs& m, int gather, int shape) {
-  const int64_t rows = (int64_t)m.M << m.log2_M0, cols = (int64_t)m.N << m.log2_N0, width = shape ? 128 : 64;
-  const int64_t tiles = ((rows + 63) / 64) * ((cols + width - 1) / width), rounds = (tiles + 255) / 256;
-  if (rounds > 4 || rows <= 64) return 1e30;  // (more rounds than it is fitted to)
-  const double busy = tiles < 256 ? tiles / 256.0 : 1.0;
-  const bool single = gather == 4;  // floats, loaded one at a time
-  if (m.chunks < (single ? 28 : 16)) return 1e30;
-  const double us = shape ? rounds * (6.04 + (single ? 0.91 : 0) + m.chunks * (single ? 0.271 : 0.2344)) + 0.0536 * busy * m.chunks
-                          : 0.15 + rounds * (5.12 + m.chunks * (single ? 0.1434 : 0.1234)) + 0.0423 * busy * m.chunks;
-  const double memory_us = 2.0 + (double)(rows * m.lhs_rb + cols * m.rhs_rb) * m.K / 6.95e6;
-  return us > memory_us ? us : memory_us;
-}
-
 // Fills `plan` if the problem is covered. With `probe_only` only type and tile
 // shape are looked at; without `choose` the kernel is left open.
 bool make_plan(const Mmt4dArgs& a, bool probe_only, bool choose, Plan* plan) {
@@ -292,7 +258,6 @@ bool make_plan(const Mmt4dArgs& a, bool probe_only, bool choose, Plan* plan) {
   if ((gather == 1 || gather == 2 || gather == 8) && !mfma_direct_covers(m, gather, i4)) return false;
   plan->wave_shape = -1;
   plan->wave_tile = false;
-  plan->split_shape = -1;
   if (!choose || !wave_k_covers(m, gather, i4)) return true;
   double best = block_cost(m, kind, i4, gather);
   const int shapes = kind == kF32 ? sizeof kWaveKShapesF32 / sizeof(WaveKShape) : sizeof kWaveKShapes / sizeof(WaveKShape);
@@ -301,16 +266,6 @@ bool make_plan(const Mmt4dArgs& a, bool probe_only, bool choose, Plan* plan) {
     if (cost < best) {
       best = cost;
       plan->wave_shape = s;
-    }
-  }
-  if (kind == kF32 && split_f32_covers(m, gather)) {
-    for (int s = 0; s < 2; ++s) {
-      // (5 % less and better: what the estimates are off by.)
-      const double cost = split_f32_cost(m, gather, s) / 0.95;
-      if (cost < best) {
-        best = cost;
-        plan->split_shape = s;
-      }
     }
   }
   plan->wave_tile = wave_tile_covers(m, kind, gather, i4) && wave_tile_is_best(m, i4, plan->wave_shape);
@@ -342,7 +297,6 @@ hipError_t launch_mfma(const Mmt4dArgs& a, hipStream_t stream, const char** name
   Plan plan;
   if (!make_plan(a, false, true, &plan)) return hipErrorInvalidValue;
   const MfmaArgs& m = plan.args;
-  if (plan.split_shape >= 0) return launch_split_f32(m, plan.gather, plan.split_shape, stream, name);
   if (plan.wave_tile) {
     *name = "mmt4d_mfma_wave_tile";
     return launch_wave_tile(m, plan.kind, plan.rhs_i4, plan.narrow, stream);

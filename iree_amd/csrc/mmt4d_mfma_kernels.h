@@ -126,9 +126,6 @@ hipError_t launch_wave_k_bf16_narrow(const MfmaArgs& m, int gather, int shape, b
 // 64x128 for an int4 rhs.
 hipError_t launch_wave_tile(const MfmaArgs& m, int kind, bool rhs_i4, bool narrow, hipStream_t stream);
 
-// f32 on the bf16 matrix pipe (mmt4d_split_f32.hip): 64x64 tiles of eight wavefronts (shape 0), 64x128 of four (1).
-hipError_t launch_split_f32(const MfmaArgs& m, int gather, int shape, hipStream_t stream, const char** name);
-
 // The block tiles of the block kernels. Larger ones move fewer operand bytes per multiply through L2 -> LDS and run the
 // matrix pipe longer between barriers, smaller ones spread a problem over more compute units; those with a side of 192
 // are there for the problems that leave a last round of 128- or 256-wide tiles nearly empty (bf16 752 x 10928 x 2272 has

@@ -339,6 +339,13 @@ __device__ __forceinline__ void fetch_arguments(const MfmaArgs& a) {
   __builtin_amdgcn_sched_barrier(0);
 }
 
+// Whether a kernel is for calls that accumulate, for those that do not, or finds out at run time. Apart, a call that does not
+// accumulate has none of the registers and instructions of the other kind: with both in one kernel and the destination read ahead (see
+// store_block), plain calls of a 32-bit output were 0.5 % slower over 250 problems, 256x256 tiles 2 to 3 (32 register moves a step
+// for want of registers), int4 256x128 ones 14 where one workgroup fitted a unit instead of two (3744 x 6032 x 768 29.3 -> 33.4
+// us, apart 29.3). Apart they are 0.3 to 1.3 % faster than with one kernel that asks for every fragment, 320 problems.
+enum Accumulate { kNever, kAlways, kAsked };
+
 // Writes one wavefront's accumulators. Lane l holds, for fragment (i, j): lhs
 // row 32*i + (l & 31) and, in accumulator registers 4*q .. 4*q+3, rhs rows
 // 32*j + 8*q + 4*(l >> 5) + {0..3} of the wavefront's sub-block, which starts at
@@ -352,7 +359,7 @@ __device__ __forceinline__ void fetch_arguments(const MfmaArgs& a) {
 // the columns this means that accumulators e and e + 1 of fragment 2p and of
 // fragment 2p + 1 together are four consecutive j0, so two fragments are
 // written at a time.
-template <int KIND, bool RHS_I4, bool NARROW, int AM, int BN, bool PAIR_A = false, bool PAIR_B = false>
+template <int KIND, bool RHS_I4, bool NARROW, int AM, int BN, bool PAIR_A = false, bool PAIR_B = false, int ACCUMULATE = kAsked>
 __device__ __forceinline__ void store_block(const MfmaArgs& a, typename AccType<KIND>::type (&acc)[AM][BN],
                                             int64_t wave_row, int64_t wave_col, int lane) {
   typedef typename AccType<KIND>::scalar scalar_t;
@@ -396,55 +403,55 @@ __device__ __forceinline__ void store_block(const MfmaArgs& a, typename AccType<
       return v;
     }
   };
-  if constexpr (!PAIR_A && !PAIR_B) {
-    if (a.accumulate) {
-      // What the destination holds is asked for several fragments before it is added, as many as 64 registers hold. A
-      // fragment's loads when its turn came waited for memory once a fragment, with a 16-bit output, each converted as it
-      // arrived, four times: int8 8x8x4 344 x 6576 x 336 8.9 -> 7.0 us, 856 x 4480 x 580 11.1 -> 10.3, bf16 8x8x4 1024 x 4096 x
-      // 1024 17.2 -> 15.4, 256x256 tiles 3072 x 5024 x 1264 57.2 -> 53.0, bf16 output 79.2 -> 69.0 (with the conversions of
-      // uk_device.h 48.2). (Pairs of fragments, 32 and 64 registers, gain nothing from it and are up to 8 % slower; a loop for
-      // calls of both kinds costs those that do not accumulate 1 to 2 %.)
-      // (Without conditions: rows and columns behind the last ones read others of the sub-block.)
-      if (wave_row >= total_rows || wave_col >= total_cols) return;
-      uint8_t* row_out[AM];
-      bool row_inside[AM];
+  static_assert(ACCUMULATE != kAlways || (!PAIR_A && !PAIR_B), "pairs are for calls of both kinds");
+  if constexpr (ACCUMULATE == kAlways) {
+    // What the destination holds is asked for ahead of the fragments that it is added to, as much as 16 registers hold. Asked
+    // for when a fragment's turn came it was waited for once a fragment, with a 16-bit output, each converted as it
+    // arrived, four times: int8 8x8x4 344 x 6576 x 336 8.9 -> 6.8 us, 856 x 4480 x 580 10.9 -> 9.4, bf16 8x8x4 1024 x 4096 x 1024
+    // 15.6 -> 13.9, 256x256 tiles 3072 x 5024 x 1264 48.0 -> 46.7, bf16 output 74.8 -> 43.5 (with the conversions of uk_device.h).
+    // 32 and 64 registers of it are as fast in small tiles and slower in large ones (int4 192x128 tiles, 13 problems, against
+    // none ahead: 1.07 times as fast with 16, 1.04 with 32, 0.99 with 64; 128x128 1.09, 1.06, 1.04). Pairs of fragments, 32 registers
+    // at the least, gain nothing from it and are up to 8 % slower.
+    // (Without conditions: rows and columns behind the last ones read others of the sub-block.)
+    if (wave_row >= total_rows || wave_col >= total_cols) return;
+    uint8_t* row_out[AM];
+    bool row_inside[AM];
 #pragma unroll
-      for (int i = 0; i < AM; ++i) {
-        const int64_t this_row = wave_row + 32 * i + (lane & 31), row = min(this_row, total_rows - 1);
-        row_inside[i] = this_row < total_rows;
-        row_out[i] = wave_out + OUT_BYTES * ((row >> a.log2_M0) * a.out_stride0 + ((row & (M0 - 1)) << a.log2_N0));
-      }
-      constexpr int FIT = 64 / (int)sizeof(stored_t), AHEAD = FIT < AM * BN ? FIT : AM * BN;
-      stored_t old[AHEAD][4];
-      auto fetch = [&](int f) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t off = col_inside >> (4 * (f % BN) + q) & 1 ? col_off[f % BN][q] : 0;
-          old[f % AHEAD][q] = *(const stored_t*)(row_out[f / BN] + off);
-        }
-      };
-#pragma unroll
-      for (int f = 0; f < AHEAD; ++f) fetch(f);
-#pragma unroll
-      for (int f = 0; f < AM * BN; ++f) {
-        typename AccType<KIND>::type frag = acc[f / BN][f % BN];
-        asm volatile("" : "+a"(frag));  // (pinned until its turn, see below)
-        quad_t v[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          v[q] = quad_t{frag[4 * q], frag[4 * q + 1], frag[4 * q + 2], frag[4 * q + 3]};
-          if constexpr (RHS_I4) v[q] = v[q] >> 4;
-          v[q] += to_float(old[f % AHEAD][q]);
-        }
-        if (f + AHEAD < AM * BN) fetch(f + AHEAD);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (row_inside[f / BN] && (col_inside >> (4 * (f % BN) + q) & 1))
-            *(stored_t*)(row_out[f / BN] + col_off[f % BN][q]) = to_stored(v[q]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      return;
+    for (int i = 0; i < AM; ++i) {
+      const int64_t this_row = wave_row + 32 * i + (lane & 31), row = min(this_row, total_rows - 1);
+      row_inside[i] = this_row < total_rows;
+      row_out[i] = wave_out + OUT_BYTES * ((row >> a.log2_M0) * a.out_stride0 + ((row & (M0 - 1)) << a.log2_N0));
     }
+    constexpr int FIT = 16 / (int)sizeof(stored_t), AHEAD = FIT < AM * BN ? FIT : AM * BN;
+    stored_t old[AHEAD][4];
+    auto fetch = [&](int f) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t off = col_inside >> (4 * (f % BN) + q) & 1 ? col_off[f % BN][q] : 0;
+        old[f % AHEAD][q] = *(const stored_t*)(row_out[f / BN] + off);
+      }
+    };
+#pragma unroll
+    for (int f = 0; f < AHEAD; ++f) fetch(f);
+#pragma unroll
+    for (int f = 0; f < AM * BN; ++f) {
+      typename AccType<KIND>::type frag = acc[f / BN][f % BN];
+      asm volatile("" : "+a"(frag));  // (pinned until its turn, see below)
+      quad_t v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        v[q] = quad_t{frag[4 * q], frag[4 * q + 1], frag[4 * q + 2], frag[4 * q + 3]};
+        if constexpr (RHS_I4) v[q] = v[q] >> 4;
+        v[q] += to_float(old[f % AHEAD][q]);
+      }
+      if (f + AHEAD < AM * BN) fetch(f + AHEAD);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (row_inside[f / BN] && (col_inside >> (4 * (f % BN) + q) & 1))
+          *(stored_t*)(row_out[f / BN] + col_off[f % BN][q]) = to_stored(v[q]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    return;
   }
   // With paired lhs fragments, fragments 2p and 2p + 1 hold the even and the odd
   // rows of the same 64: they are written together, so that the stores which
@@ -493,7 +500,7 @@ __device__ __forceinline__ void store_block(const MfmaArgs& a, typename AccType<
             }
             if constexpr (RHS_I4) v[t][s][q] = v[t][s][q] >> 4;
           }
-      if ((PAIR_A || PAIR_B) && a.accumulate) {
+      if (ACCUMULATE == kAsked && a.accumulate) {
         stored_t old[IS][JS][4];
 #pragma unroll
         for (int t = 0; t < IS; ++t)
@@ -853,7 +860,7 @@ __device__ __forceinline__ void wait_loads_but() {
 // STAGGER: 0 = every accumulator stored after the last MFMA; 1 = staggered tail (see below); 2 = the same for
 // an accumulating call, the destination read in the tail; 3 = accumulating call with the destination read and
 // added during the main loop (needs enough steps), tail as in 1.
-template <int KIND, bool RHS_I4, bool NARROW, int G, int AM, int BN, int STAGES, int STAGGER = 0, int GROUPS = 1>
+template <int KIND, bool RHS_I4, bool NARROW, int G, int AM, int BN, int STAGES, int STAGGER = 0, int GROUPS = 1, int ACCUMULATE = kAsked>
 __global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(GROUPS, AM * BN >= 9 ? 1 : (AM * BN >= 4 ? 2 : 4))))
 void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
   typedef typename AccType<KIND>::type acc_t;
@@ -1862,13 +1869,13 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
       }
       total[0][f] = own + part;
     }
-    store_block<KIND, RHS_I4, NARROW, 1, BY_ROWS ? BN : 1>(
+    store_block<KIND, RHS_I4, NARROW, 1, BY_ROWS ? BN : 1, false, false, ACCUMULATE>(
         a, total, first_row + wave_m * (32 * AM) + (BY_ROWS ? 32 * group : 0),
         first_col + wave_n * (32 * BN) + (BY_ROWS ? 0 : 32 * group), lane);
     return;
   }
-  store_block<KIND, RHS_I4, NARROW, AM, BN, PAIR_A, PAIR_B>(a, acc, first_row + wave_m * (32 * AM),
-                                                            first_col + wave_n * (32 * BN), lane);
+  store_block<KIND, RHS_I4, NARROW, AM, BN, PAIR_A, PAIR_B, ACCUMULATE>(a, acc, first_row + wave_m * (32 * AM),
+                                                                        first_col + wave_n * (32 * BN), lane);
   UK_TIMELINE(asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
               if (lane == 0 && wave == 0 && blockIdx.x < 256) {
                 unsigned long long* t = uk_timeline + blockIdx.x * 8;
@@ -1894,7 +1901,7 @@ void mmt4d_mfma_direct_kernel(const MfmaArgs a) {
 // of the kernel above (G == 16) with COLS 16-byte columns: slot p of a
 // fragment holds rows 16*(p / (16*COLS)) + (p & 15), column (p >> 4) & (COLS-1).
 // A load fills 64 consecutive slots of one slice.
-template <int KIND, bool NARROW>
+template <int KIND, bool NARROW, int ACCUMULATE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void mmt4d_mfma_split_k_kernel(const MfmaArgs a) {
   typedef typename AccType<KIND>::type acc_t;
@@ -2096,7 +2103,7 @@ void mmt4d_mfma_split_k_kernel(const MfmaArgs a) {
       if (w == 0) total[o][0] = part; else total[o][0] += part;
     }
   }
-  store_block<KIND, false, NARROW, OWN, 1>(a, total, first_row + 32 * OWN * (wave >> 1), first_col + 32 * (wave & 1), lane);
+  store_block<KIND, false, NARROW, OWN, 1, false, false, ACCUMULATE>(a, total, first_row + 32 * OWN * (wave >> 1), first_col + 32 * (wave & 1), lane);
 }
 
 // Whether the direct-to-LDS kernel covers the problem: every lane can load 16
@@ -2136,7 +2143,11 @@ hipError_t launch_direct(MfmaArgs m, hipStream_t stream, bool staggered_tail = t
   constexpr int stage_pieces = 256 * AM + (RHS_I4 ? 128 : 256) * BN;
   constexpr size_t lds_bytes = (size_t)GROUPS * STAGES * 16 * stage_pieces;
   static_assert(lds_bytes <= 160 * 1024, "ring does not fit the LDS");
-  void (*kernel)(const MfmaArgs) = mmt4d_mfma_direct_kernel<KIND, RHS_I4, NARROW, G, AM, BN, STAGES, 0, GROUPS>;
+  constexpr bool PAIRS = G == 2 && (AM % 2 == 0 || BN % 2 == 0);  // (see store_block)
+  void (*kernel)(const MfmaArgs) = mmt4d_mfma_direct_kernel<KIND, RHS_I4, NARROW, G, AM, BN, STAGES, 0, GROUPS, PAIRS ? kAsked : kNever>;
+  if constexpr (!PAIRS) {
+    if (m.accumulate) kernel = mmt4d_mfma_direct_kernel<KIND, RHS_I4, NARROW, G, AM, BN, STAGES, 0, GROUPS, kAlways>;
+  }
   // The 256x256 tile with the staggered tail: K in whole chunks, enough of them.
   if constexpr (AM == 4 && BN == 4 && !RHS_I4 && G != 2 && KIND != kF32) {
     if (staggered_tail && ((int64_t)m.K * m.lhs_rb) % 64 == 0 && m.chunks >= 2 * STAGES) {
@@ -2161,7 +2172,7 @@ hipError_t launch_split_k(MfmaArgs m, hipStream_t stream) {
   unsigned grid;
   set_tile_grid(&m, 128, 64, &grid);
   constexpr int lds_bytes = 6 * 24576;
-  auto kernel = mmt4d_mfma_split_k_kernel<KIND, NARROW>;
+  auto kernel = m.accumulate ? mmt4d_mfma_split_k_kernel<KIND, NARROW, kAlways> : mmt4d_mfma_split_k_kernel<KIND, NARROW, kNever>;
   const hipError_t attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
   if (attr != hipSuccess) return attr;
   return launch_kernel<MfmaArgs>(kernel, grid, 256, lds_bytes, stream, m);

@@ -147,12 +147,15 @@ bool wave_tile_covers(const MfmaArgs& m, int kind, int gather, bool rhs_i4) {
 // Whether it is the fastest, from 500 problems (M 17..4096, N 256..14336, K 256..8192, half a round of its tiles on the compute
 // units to four) timed beside what was chosen for them, on three sets of operands in turn, which the last-level cache
 // holds, and some on sets of 640 MB, from HBM.
-// 16-bit operands, 128x128 tiles: 200 to 248 tiles and 64 chunks of K or more 4 % faster in the mean, of 28 problems two 1 %
-// slower, from HBM 3 to 13 % faster. With 22 to 48 chunks 2 to 14 % slower (the partial sums), with 140 to 199 tiles
-// between 9 % slower and 7 % faster, a second round of tiles takes half as long again, and operands of more than 48 MiB (see
-// streams_operands) -2 to +3 %.
-// int4, 64x128 tiles: where 64x64 ones are more than a round of the compute units and these are not, and 32x64 ones would be taken.
-// 11 problems 13 to 28 % faster, from HBM between 2 % slower and 19 % faster, 5 in the mean; but where 32-high tiles
+// 16-bit operands, 128x128 tiles: 200 to 248 tiles and 64 chunks of K or more, 82 plain problems with a 32-bit output between 2.2 %
+// slower and 10 % faster, 3.6 in the mean, from HBM 47 others 1 to 25 % faster, 8 in the mean. (249 to 256 tiles would gain
+// too, 37 problems 0 to 10 %, from HBM 28 1 to 27: not taken so far.) With 22 to 48 chunks 2 to 14 % slower (the partial
+// sums), with 140 to 199 tiles between 9 % slower and 7 % faster, a second round of tiles takes half as long again, and
+// operands of more than 48 MiB (see streams_operands) -2 to +3 %.
+// int4, 64x128 tiles: where 64x64 ones are more than a round of the compute units and these are not, and 32x64 ones would be taken
+// and are more than two workgroups per unit: 120 problems 8 to 29 % faster, 18 in the mean, from HBM 120 others between 7 % slower
+// and 16 % faster, 4.5 in the mean (from 94 chunks on 1.4). With up to 512 tiles of 32x64, which the units hold at once, 5 to 14 % slower
+// (21 problems), from HBM 11 to 21 (12): 480 x 2144 x 7872 23.1 us, in 32x64 tiles 19.5. Where 32-high tiles
 // have less padding, 160 rows and up to 160 that they divide, 3 to 14 % slower. (Where the block kernel's tile would be taken it
 // is up to 5 % faster with 24 to 44 chunks, 17 with more, and from HBM 2 to 14 % slower. Near 256 tiles between 5 % slower and
 // 6 % faster, beyond up to 30 % slower; with up to 256 tiles of 64x64 those take two thirds of the time.)
@@ -162,7 +165,8 @@ bool wave_tile_is_best(const MfmaArgs& m, bool rhs_i4, int wave_shape) {
   if (rhs_i4) {
     const int64_t row_tiles = (rows + 63) / 64;
     const bool padded = 6 * 64 * row_tiles > 7 * 32 * ((rows + 31) / 32);  // (than 32-high tiles)
-    return wave_shape >= 0 && row_tiles * ((cols + 63) / 64) > 256 && row_tiles * col_tiles <= 240 && !padded && m.chunks >= 24;
+    return wave_shape >= 0 && row_tiles * ((cols + 63) / 64) > 256 && ((rows + 31) / 32) * ((cols + 63) / 64) > 512 &&
+           row_tiles * col_tiles <= 240 && !padded && m.chunks >= 24;
   }
   const int64_t tiles = ((rows + 127) / 128) * col_tiles;
   return tiles >= 200 && tiles <= 248 && m.chunks >= 64 && wave_shape < 0 &&

@@ -59,3 +59,11 @@ def test_where_it_is_taken(recorder):  # noqa: F811
     # 64x64 tiles that fit a round, 64x128 ones that do.
     assert [i4(304, n, 3360) for n in (3264, 3280)] == [False, True]
     assert [i4(320, 3424, 3360), i4(224, 4944, 2592), i4(160, 6160, 4128), i4(144, 5712, 4640)] == [True, True, False, False]
+
+
+# int4: not where the units hold all tiles of 32x64 at once, two workgroups each.
+def test_four_bit_rhs_of_one_round_of_small_tiles(recorder):  # noqa: F811
+    def i4(rows, cols, k):
+        return takes(recorder, gpu.S8S4, rows // 16, cols // 16, k // 32, 16, 16, 32)
+    assert not any(i4(*size) for size in [(480, 2144, 7872), (608, 1632, 2528), (784, 1264, 5888), (2704, 384, 2656), (224, 4640, 7232)])
+    assert [i4(480, n, 4096) for n in (2176, 2192)] == [False, True]  # 15 rows of 34 and 35 tiles

@@ -150,14 +150,15 @@ constexpr TileChoice kBlockTiles[] = {{4, 4, false}, {4, 2, true}, {2, 2, false}
 
 // One workgroup per compute unit at most, and K long enough: two groups of four wavefronts with a ring each multiply the tile
 // over every other chunk of K, so that each SIMD has two wavefronts, one issuing while the other waits, and are summed at the
-// end through LDS (1.4 us, and twice the first loads). 128x128 tiles, and 64x128 ones of an int4 rhs: bf16 784 x 4112 x 4096
-// 33.4 -> 31.9 us (8x8x4 tiles 32.4 -> 30.4, bf16 output 33.8 -> 30.4), 512 x 5008 x 4000 31.0 -> 26.8, 1504^2 x 3008 24.4 -> 21.3,
-// 2048^2 x 3712 34.0 -> 32.3, x 6144 53.3 -> 49.7; int8 8x8x8 3064 x 944 x 5232 23.7 -> 20.9; int4 576 x 5104 x 4704 21.6 -> 20.1, 256 x
-// 8192 x 8192 25.9 -> 24.3. The fewer tiles there are the less K it takes, the clock being higher. 16-bit: 1 to 6 % slower at
-// 24 to 35 chunks of K, 3 to 6 % faster at 40 to 50 with up to 220 tiles; with 231 of them up to 5 % slower at 64 and 2.5 %
-// faster at 80, with 256 up to 4 % slower at 96 and 1.5 to 4 % faster at 112. int8 and the 128x128 tile of int4: 3 to 8 % faster
-// from 42 chunks on with up to 170 tiles, 11 % at 82 with 192; 2 % slower at 64 with 231, 1 to 3 % faster at 96 with 256. int4
-// 64x128: level at 36 to 48, 4 to 9 % faster at 54 with 140 tiles, 1 to 4 % at 64 with 256.
+// end through LDS (1.4 us, and twice the first loads). 128x128 tiles, and 64x128 ones of an int4 rhs: bf16 512 x 5008 x 4000
+// 31.0 -> 26.8 us, 1504^2 x 3008 24.4 -> 21.3, 784 x 4112 x 4096 in 8x8x4 tiles 32.4 -> 30.4, 2048^2 x 3712 34.0 -> 32.3, x
+// 6144 53.3 -> 49.7; int8 8x8x8 3064 x 944 x 5232 23.7 -> 20.9; int4 576 x 5104 x 4704 21.6 -> 20.1, 256 x 8192 x 8192 25.9 ->
+// 24.3. The fewer tiles there are the less K it takes, the clock being higher. 16-bit: 1 to 6 % slower at 24 to 35 chunks of K,
+// 3 to 6 % faster at 40 to 50 with up to 220 tiles; with 231 of them up to 5 % slower at 64 and 2.5 % faster at 80, with 256 up
+// to 4 % slower at 96 and 1.5 to 4 % faster at 112. (With row pieces of 16 and 32 bytes and four rows a tile or more 200 to 248
+// tiles of 64 chunks and more go to mmt4d_wave_tile.hip before this is asked.) int8 and the 128x128 tile of int4: 3 to 8 %
+// faster from 42 chunks on with up to 170 tiles, 11 % at 82 with 192; 2 % slower at 64 with 231, 1 to 3 % faster at 96 with
+// 256. int4 64x128: level at 36 to 48, 4 to 9 % faster at 54 with 140 tiles, 1 to 4 % at 64 with 256.
 // (2-byte pieces: pairs of fragments, which a group's half does not have whole. f32 is bound by the matrix pipe. Operands from
 // HBM: a ring of ten stages is as fast or faster, 784 x 4112 x 8192 60.2 and 62.8, see streams_operands.)
 inline bool two_groups(const MfmaArgs& m, int kind, bool rhs_i4, int gather, bool direct, const TileChoice& t) {

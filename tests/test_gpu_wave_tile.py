@@ -1,7 +1,6 @@
 """The kernel whose wavefronts multiply the whole of a large tile each (mmt4d_wave_tile.hip): 128x128 tiles of 16-bit operands with
 either output, 64x128 tiles of an int4 rhs. Every remainder of the number of 64-byte chunks by the four
-wavefronts and the two steps that one has in registers, K ending at every place of a chunk that row pieces leave, ragged last tiles. That the problems do take this kernel, which its name does not say, is checked
-in test_wave_tile_on_host.py. Integers are compared bit for bit with a float64 product, floats within 1e-3 of max(|ref|, rms(ref)):
+wavefronts and the two steps that one has in registers, K ending at every place of a chunk that row pieces leave, ragged last tiles. Integers are compared bit for bit with a float64 product, floats within 1e-3 of max(|ref|, rms(ref)):
 sums of at most 4500 products of unit-scale values in 32 bits differ by about 1e-6 of that in any order.
 """
 import ctypes as C

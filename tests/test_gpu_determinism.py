@@ -26,6 +26,9 @@ CASES = [
     (BF16, 8, 562, 512, 16, 16, 8, b"mmt4d_mfma_128x64_split_k"),
     (BF16, 63, 129, 136, 16, 16, 16, b"mmt4d_mfma_128x128"),  # two groups of wavefronts
     (F16, 63, 129, 267, 16, 16, 8, b"mmt4d_mfma_128x128"),    # an odd number of chunks, the first one cut
+    (BF16, 109, 132, 259, 16, 16, 8, b"mmt4d_mfma_wave_tile"),  # the same
+    (F16, 53, 488, 134, 8, 16, 16, b"mmt4d_mfma_wave_tile"),
+    (abi.MMT4D_TYPE_F16F16F16 | SKIP, 109, 132, 130, 16, 16, 16, b"mmt4d_mfma_wave_tile"),
     (F32, 16, 16, 64, 16, 16, 4, b"mmt4d_mfma_"),
     (abi.MMT4D_TYPE_F16F16F16 | SKIP, 16, 16, 64, 16, 16, 16, b"mmt4d_mfma_"),
     (BF16, 1, 100, 300, 16, 16, 8, b"mmt4d_gemv"),
